@@ -6,25 +6,29 @@
 // filters, any stride, the feeding tensor.pad folded into the halo loads and the
 // layout kept on both sides: no transposed copy of either tensor in HBM.
 //
-// Implicit GEMM on the f32 MFMA: rows = output pixels of one row segment,
-// columns = filters, reduction = (channel, tap).  Per chunk of 16 channels a
-// workgroup stages, each in the order it is stored in HBM:
-//   * the input halo: 16 channels x KH rows x (PX + KW - 1) columns (a
-//     channel's row segment is contiguous in NCHW, so lanes load consecutive
-//     words), zero outside the image (the pad) and past C;
-//   * its 64 filters' chunk: 16 channels x KH*KW taps per filter, one
-//     contiguous run in FCHW, each filter's record padded to an odd number of
-//     words.
-// MFMA step s of lane (r, q) takes channel 4q + s of the chunk at one tap:
-// A = halo word (channel, tap row, pixel r + tap column), B = filter r's word
-// (channel, tap).  Sixteen lanes read consecutive halo words or records of odd
-// stride, so neither read has bank conflicts.  A chunk's loads are issued
-// before the barrier that ends the previous chunk's multiply; several
-// workgroups per CU overlap one's staging with another's MFMAs.
+// Implicit GEMM on the f32 MFMA: rows = output pixels, columns = filters,
+// reduction k = (c, kh, kw) in FCHW order, so a filter's operand is its own
+// row, loaded 16 bytes per lane straight into registers, and any filter size
+// and stride run the same code.  A workgroup owns 16 NB pixels x 16 WF filters
+// and splits K over WK groups of its waves: at batch 1 a layer has only 128 to
+// 784 16x16 output blocks, so a workgroup per block with its waves along K is
+// what fills the chip.  Per chunk of channels it stages the input patch its
+// pixels see, zero outside the image (the folded tensor.pad); a table in LDS
+// says where k lies in the patch, and lane (r, q) of MFMA step s reads pixel
+// r's word of k = 16 step + 4q + s.  The K parts' sums meet in LDS and are
+// finished with the bias, the residual and the activation, stored along the
+// pixels.
 //
-// Accumulator: lane (r, q) of pixel block i holds pixels 16 i + 4q .. +3 of
-// the segment for filter r -- four consecutive NCHW outputs -- finished with
-// the bias, the residual (same layout) and the activation.
+// What bounds it: at batch 1 the patches' loads, one word per lane (about 28
+// clocks of the CU's load path each), and the fetch of code that runs once;
+// at larger batches the f32 MFMAs (half of their rate).  Measured against the
+// kernel before it (row segments of 32 or 64 pixels x 64 filters, 16-channel
+// chunks of halo and filters staged between two barriers): 3x3 at batch 1
+// 56x56x64 31.7 -> 8.5 us, 28x28x128 57.6 -> 10.4, 14x14x256 110 -> 16,
+// 7x7x512 215 -> 20, the 7x7/2 stem 31.7 -> 9.5; 56x56x64 at batch 8
+// 79 -> 32 us.
+#include <type_traits>
+
 #include "kernels.hpp"
 #include "npu_device.hpp"
 #include "persistent.hpp"
@@ -34,174 +38,397 @@ namespace npu {
 
 namespace {
 
-constexpr int kNchwChunk = 16;  // channels per staged chunk
+// Division of v < 2^16 by d < 2^16 as a multiply: q = (v * m) >> 32 with
+// m = ceil(2^32 / d) (the error v * (m d - 2^32) / (d 2^32) < 2^-16 cannot
+// carry past the next multiple); d = 1 takes v itself.
+struct FastDiv {
+  uint32_t d, m;
+  explicit FastDiv(int dv = 1) : d((uint32_t)dv), m(dv > 1 ? (uint32_t)(((1ULL << 32) + dv - 1) / dv) : 0u) {}
+  __device__ __forceinline__ int div(int v) const { return d == 1 ? v : (int)__umulhi((uint32_t)v, m); }
+};
 
-template <int KH, int KW, int ST, int NB>
-__global__ __launch_bounds__(256) void conv2d_nchw_kernel(
-    const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
-    const float *__restrict__ res, float *__restrict__ out, int C, int H, int W, int F, int pad,
-    int Ho, int Wo, int nseg, int act) {
-  constexpr int CK = kNchwChunk;
-  constexpr int PX = 16 * NB;                  // pixels of the row segment
-  constexpr int HC = (PX - 1) * ST + KW;       // halo columns (stride ST)
-  constexpr int HROWS = CK * KH;               // halo rows (channel, tap row)
-  constexpr int HALO = HROWS * HC;             // halo words
-  constexpr int TAPS = KH * KW;
-  constexpr int WRUN = CK * TAPS;              // a filter's chunk (words)
-  constexpr int WREC = WRUN + 1;               // its LDS record: an odd stride
-  constexpr int NT = 256;
-  constexpr int HPT = (HALO + NT - 1) / NT;    // halo words per thread
-  constexpr int WPT = (64 * WRUN + NT - 1) / NT;  // filter words per thread
-  __shared__ float halo[HALO];
-  __shared__ float wl[64 * WREC];
+struct NchwArgs {
+  const float *x, *w, *bias, *res;
+  float *out;
+  int C, H, W, F, T, K, pad, st, Ho, Wo, act;
+  int tw, nstrips;       // strip width, strips per image
+  int tiles;             // pixel tiles per strip
+  int npt, grid;         // pixel tiles of the launch, workgroups
+  int hc, ps, npl;       // patch columns, patch words per channel, loads per channel
+  int cc, nchunks;       // channels per chunk
+  FastDiv by_hc, by_tw, by_t, by_kw;
+};
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+constexpr int kStage = 16;  // patch words a thread holds in flight per chunk
+constexpr int kRing = 4;    // k steps whose filters a wave holds in flight
+// LDS words between the patches of consecutive channels, for NPL loads of 64
+// words each: 4 mod 64, so a 1x1 filter's four lane groups (channels 4 apart)
+// read 16 banks apart.
+constexpr int patch_stride(int npl) { return 64 * npl + 4; }
+
+// An unaligned-by-16 run of four floats (filter rows of K % 4 != 0 words);
+// global loads need 4-byte alignment only.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int NB, int WF, int WK, int NPL>
+__global__ __launch_bounds__(64 * WF * WK, WF * WK == 16 || (WF * WK == 8 && NB * NPL <= 16) ? 4 : 2)
+void conv2d_nchw_split_kernel(const NchwArgs a) {
+  constexpr int NW = WF * WK, NT = 64 * NW, PX = 16 * NB;
+  constexpr int CPW = kStage / NPL;  // channels a wave stages per chunk
+  constexpr int PS = patch_stride(NPL);
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  const int KC = a.cc * a.T;                       // reduction length of a whole chunk
+  const int KT = (KC + 15) & ~15;
+  int *const ktab = reinterpret_cast<int *>(smem);             // byte offset of k in a patch
+  float *const patch = reinterpret_cast<float *>(ktab + KT);
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
-  const int seg = blockIdx.x % nseg, orow = blockIdx.x / nseg;  // orow = n * Ho + oh
-  const int n = orow / Ho, oh = orow - n * Ho;
-  const int ow0 = seg * PX;
-  const int f0 = blockIdx.y * 64;
+  const int wf = wave % WF, wk = wave / WF;
+  // filter blocks outermost, cut into eight contiguous ranges, one per XCD:
+  // the pixel tiles that read the same filters share an L2
+  const int per = (a.grid + kXcds - 1) / kXcds, t0 = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
+  if (t0 >= a.grid) return;
+  const int fb = t0 / a.npt, pt = t0 - fb * a.npt;
+  const int strip = pt % a.nstrips, t1 = pt / a.nstrips;
+  const int n = t1 / a.tiles, p0 = (t1 - n * a.tiles) * PX;
+  const int ox0 = strip * a.tw, tw = min(a.tw, a.Wo - ox0);  // tw < a.tw: the last strip
+  const int oy0 = a.by_tw.div(p0);
+  const int f0 = (fb * WF + wf) * 16;
 
-  // Staging slots: halo word e = tid + NT j is (channel e / (KH HC), tap row,
-  // column); filter word e is (filter e / WRUN, word e % WRUN of its chunk).
-  // Addresses are recomputed per chunk (constant divisors; opaque() keeps
-  // the compiler from hoisting them into registers held across the loop).  Loads come from clamped addresses and are masked when
-  // written, so none waits under a condition.
-  static_assert(HPT <= 64 && WPT <= 64, "slot masks fit 64 bits");
-  float hv[HPT], wv[WPT];
-  auto halo_slot = [&](int j, int c0, int &src) __attribute__((always_inline)) {
-    const int t = opaque(tid) + NT * j;
-    const int e = min(t, HALO - 1);
-    const int hr = e / HC, col = e - hr * HC;
-    const int c = hr / KH, kh = hr - c * KH;
-    const int ih = oh * ST + kh - pad, iw = ow0 * ST + col - pad;
-    src = ((n * C + min(c0 + c, C - 1)) * H + min(max(ih, 0), H - 1)) * W + min(max(iw, 0), W - 1);
-    return t < HALO && c0 + c < C && ih >= 0 && ih < H && iw >= 0 && iw < W;
+  // ---- filters: lane (r, q) holds filter r, k = 16 step + 4q .. +3, straight
+  //      from its row of FCHW, in a ring of kRing steps.  Every load is
+  //      unconditional (one under a branch, even a uniform one, makes the
+  //      wave wait for it there).  A run that crosses the end of its row reads
+  //      on into the next row; the last row's is moved back into the buffer.
+  const int wrow = min(f0 + r, a.F - 1) * a.K + 4 * q, wlast = a.F * a.K - 4;
+  auto load_w = [&](int k) __attribute__((always_inline)) {
+    return *reinterpret_cast<const f32x4u *>(a.w + min(wrow + k, wlast));
   };
-  auto filter_slot = [&](int j, int c0, int &src) __attribute__((always_inline)) {
-    const int t = opaque(tid) + NT * j;
-    const int e = min(t, 64 * WRUN - 1);
-    const int fl = e / WRUN, k = e - fl * WRUN, c = k / TAPS;
-    src = (min(f0 + fl, F - 1) * C + min(c0 + c, C - 1)) * TAPS + (k - c * TAPS);
-    return t < 64 * WRUN && f0 + fl < F && c0 + c < C;
+  constexpr int KSTEP = 16 * WK;
+  f32x4 wv[kRing];
+  auto fill_ring = [&](int kbase) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kRing; ++u) wv[u] = load_w(min(kbase + 16 * wk + KSTEP * u, a.K));
   };
-  auto fetch = [&](int c0) __attribute__((always_inline)) {
+  fill_ring(0);
+
+  // ---- staging: this wave's load (j, i) is patch words 64 i + lane of
+  //      channel wave + NW j of the chunk.  A word's place in the plane does
+  //      not depend on the channel, so a load is a uniform base plus a lane
+  //      offset fixed for the whole launch.  Words outside the image load
+  //      the plane's first word and are zeroed on commit.  Channels past C
+  //      (the last chunk's) hold channel C - 1 again: their k are never used.
+  int off[NPL];
+  uint32_t keep = 0;
 #pragma unroll
-    for (int j = 0; j < HPT; ++j) {
-      int src;
-      halo_slot(j, c0, src);
-      hv[j] = x[src];
-    }
+  for (int i = 0; i < NPL; ++i) {
+    const int e = 64 * i + lane, hy = a.by_hc.div(e), hx = e - hy * a.hc;
+    const int iy = oy0 * a.st - a.pad + hy, ix = ox0 * a.st - a.pad + hx;
+    const bool in = (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
+    off[i] = in ? iy * a.W + ix : 0;
+    keep |= (uint32_t)in << i;
+  }
+  const int plane = a.H * a.W;
+  const float *const xn = a.x + (size_t)n * a.C * plane;
+  float st[CPW][NPL];
+  auto stage = [&](int c0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < WPT; ++j) {
-      int src;
-      filter_slot(j, c0, src);
-      wv[j] = w[src];
+    for (int j = 0; j < CPW; ++j) {
+      const float *const xc = xn + min(c0 + wave + NW * j, a.C - 1) * plane;
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) st[j][i] = xc[off[i]];
     }
   };
-  auto commit = [&](int c0) __attribute__((always_inline)) {
+  auto commit = [&](float *buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < HPT; ++j) {
-      int src;
-      const bool in = halo_slot(j, c0, src);
-      const int e = tid + NT * j;
-      if (e < HALO) halo[e] = in ? hv[j] : 0.0f;
-    }
+    for (int j = 0; j < CPW; ++j) {
+      if (wave + NW * j < a.cc) {
+        float *const row = buf + (wave + NW * j) * PS + lane;
 #pragma unroll
-    for (int j = 0; j < WPT; ++j) {
-      int src;
-      const bool in = filter_slot(j, c0, src);
-      const int e = tid + NT * j;
-      if (e < 64 * WRUN) {
-        const int fl = e / WRUN;
-        wl[fl * WREC + (e - fl * WRUN)] = in ? wv[j] : 0.0f;
+        for (int i = 0; i < NPL; ++i) row[64 * i] = (keep >> i) & 1u ? st[j][i] : 0.0f;
       }
     }
   };
+  stage(0);
 
+  // ---- where k lies in the patches
+  for (int k = tid; k < KT; k += NT) {
+    const int c = a.by_t.div(k), t = k - c * a.T, kh = a.by_kw.div(t), kw = t - kh * (int)a.by_kw.d;
+    ktab[k] = k < KC ? (c * PS + kh * a.hc + kw) * 4 : 0;
+  }
+  // patch byte offset of this lane's pixel of each block
+  const int npx = a.tw * a.Ho;  // pixel slots of a strip, the last strip's spare columns among them
+  int pb[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int p = min(p0 + 16 * i + r, npx - 1);
+    const int oy = a.by_tw.div(p), ox = p - oy * a.tw;
+    pb[i] = ((oy - oy0) * a.hc + min(ox, tw - 1)) * a.st * 4;
+  }
   f32x4 acc[NB];
 #pragma unroll
-  for (int i = 0; i < NB; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  const float *const wrow = wl + (wave * 16 + r) * WREC;
+  for (int i = 0; i < NB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  for (int c0 = 0; c0 < C; c0 += CK) {
-    fetch(c0);
-    __syncthreads();  // the previous chunk's reads are done
-    commit(c0);
+  for (int ch = 0; ch < a.nchunks; ++ch) {
+    float *const buf = patch + (ch & 1) * a.cc * PS;
+    commit(buf);
+    // one barrier per chunk: the buffer written next is the one read a chunk ago
     __syncthreads();
-#pragma unroll 1
-    for (int kh = 0; kh < KH; ++kh)
+    if (ch + 1 < a.nchunks) stage((ch + 1) * a.cc);
+    const char *const xb = reinterpret_cast<const char *>(buf);
+    const int kbase = ch * KC, kend = min(KC, a.K - kbase);  // this chunk's k: [0, kend)
+    const int kfull = kend & ~15, klast = a.K - 16;
+    // k steps wk, wk + WK, ... of the chunk, kRing at a time and then the
+    // rest.  No early exit from the ring's loop (its registers would be moved
+    // at the exits, each move waiting for its load), and no second copy of it:
+    // the kernel runs its code once or twice, so its instruction fetches count.
+    auto step = [&](int k, f32x4 &ring) __attribute__((always_inline)) {
+      const i32x4 ko = *reinterpret_cast<const i32x4 *>(ktab + k + 4 * q);
+      float v[4][NB];
 #pragma unroll
-      for (int kw = 0; kw < KW; ++kw) {
+      for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const int c = 4 * q + s;
-          const float b = wrow[c * TAPS + kh * KW + kw];
-          const float *hrow = halo + (c * KH + kh) * HC + r * ST + kw;
+        for (int i = 0; i < NB; ++i) v[s][i] = *reinterpret_cast<const float *>(xb + pb[i] + ko[s]);
 #pragma unroll
-          for (int i = 0; i < NB; ++i)
-            acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(hrow[16 * ST * i], b, acc[i], 0, 0, 0);
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[s][i], ring[s], acc[i], 0, 0, 0);
+      ring = load_w(min(kbase + k + KSTEP * kRing, klast));
+    };
+    int k = 16 * wk;
+    for (; k + KSTEP * (kRing - 1) < kfull; k += KSTEP * kRing)
+#pragma unroll
+      for (int u = 0; u < kRing; ++u) step(k + KSTEP * u, wv[u]);
+#pragma unroll
+    for (int u = 0; u + 1 < kRing; ++u)
+      if (k + KSTEP * u < kfull) step(k + KSTEP * u, wv[u]);
+    // the end of K (its length no multiple of 16): words past it count as
+    // zero on both sides
+    if (kfull < kend && (kfull >> 4) % WK == wk) {
+      const int d = wrow + kbase + kfull - wlast;  // > 0: the run was moved back by d
+      f32x4 wq = load_w(kbase + kfull);
+      if (d > 0) wq = d == 1 ? f32x4{wq[1], wq[2], wq[3], 0.f} : d == 2 ? f32x4{wq[2], wq[3], 0.f, 0.f}
+                                                               : f32x4{wq[3], 0.f, 0.f, 0.f};
+      for (int s = 0; s < 4; ++s) {
+        const bool ok = kfull + 4 * q + s < kend;
+        const int ko = ktab[kfull + 4 * q + s];
+        const float b = s == 0 ? wq[0] : s == 1 ? wq[1] : s == 2 ? wq[2] : wq[3];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+          const float v = *reinterpret_cast<const float *>(xb + pb[i] + ko);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(ok ? v : 0.0f, ok ? b : 0.0f, acc[i], 0, 0, 0);
         }
       }
+    }
+    if (ch + 1 < a.nchunks) fill_ring(kbase + KC);
   }
 
-  const int f = f0 + wave * 16 + r;
-  if (f >= F) return;
-  const float bv = bias ? bias[f] : 0.0f;
-  const ActBounds ab = act_bounds(act);
-  const size_t obase = ((size_t)(n * F + f) * Ho + oh) * Wo;
+  // ---- partial sums of the K parts through LDS, [wk][wf][filter][pixel]
+  constexpr int RS = PX + 4;
+  __syncthreads();
+  float *const red = smem;
 #pragma unroll
   for (int i = 0; i < NB; ++i)
+    *reinterpret_cast<f32x4 *>(red + ((size_t)wave * 16 + r) * RS + 16 * i + 4 * q) = acc[i];
+  __syncthreads();
+  const ActBounds ab = act_bounds(a.act);
+  for (int e = tid; e < 16 * WF * PX; e += NT) {
+    const int px = e % PX, fl = e / PX;  // filter fl: wave fl / 16's block, row fl % 16
+    float v = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int ow = ow0 + 16 * i + 4 * q + e;
-      if (ow < Wo) {
-        float v = acc[i][e] + bv;
-        if (res) v += res[obase + ow];
-        out[obase + ow] = act_clamp(v, ab);
-      }
+    for (int k = 0; k < WK; ++k) v += red[((size_t)(k * WF) * 16 + fl) * RS + px];
+    const int p = p0 + px, oy = a.by_tw.div(p), ox = p - oy * a.tw, f = fb * WF * 16 + fl;
+    if (oy < a.Ho && ox < tw && f < a.F) {
+      const size_t o = ((size_t)(n * a.F + f) * a.Ho + oy) * a.Wo + ox0 + ox;
+      if (a.bias) v += a.bias[f];
+      if (a.res) v += a.res[o];
+      a.out[o] = act_clamp(v, ab);
     }
+  }
 }
 
-template <int KH, int KW, int ST, int NB>
-hipError_t launch_nchw(const ConvArgs &a, hipStream_t s) {
-  constexpr int PX = 16 * NB;
-  const int nseg = (a.Wo + PX - 1) / PX;
-  dim3 grid(a.N * a.Ho * nseg, (a.F + 63) / 64);
-  const int chunks = (a.C + kNchwChunk - 1) / kNchwChunk;
-  npu_launch_plan p = make_plan("conv2d_nchw", grid.x * grid.y,
-                                wg_per_cu(conv2d_nchw_kernel<KH, KW, ST, NB>), grid.x * grid.y, 32);
-  p.load_phases = chunks;  // each chunk's staging waits for its loads
-  p.tile_macs = 64.0 * PX * a.C * KH * KW;
-  // per wave: staging address selects and LDS writes per chunk, the tap loop's
-  // LDS reads, the epilogue
-  p.tile_valu = 4.0 * (chunks * (3.0 * ((KH * ((PX - 1) * ST + KW) * kNchwChunk + 255) / 256 +
-                                         (64 * kNchwChunk * KH * KW + 255) / 256)) + 60.0);
-  p.tile_lds_bytes = chunks * 4.0 * (KH * ((PX - 1) * ST + KW) * kNchwChunk + 64.0 * kNchwChunk * KH * KW) +
-                     chunks * 4.0 * 64 * KH * KW * 4 * (NB + 1) * 4;
-  p.tile_load_bytes = chunks * 4.0 * (KH * ((PX - 1) * ST + KW) * kNchwChunk + 64.0 * kNchwChunk * KH * KW);
-  p.tile_store_bytes = 4.0 * PX * 64 * (a.res ? 2 : 1);
-  p.hbm_bytes = 4.0 * ((double)a.N * a.C * a.H * a.W + (double)a.F * a.C * KH * KW +
-                       (double)a.N * a.F * a.Ho * a.Wo * (a.res ? 2 : 1)) + (a.bias ? 4.0 * a.F : 0.0);
+template <int NB, int WF, int WK>
+bool split_shape(const ConvArgs &c, NchwArgs &a, size_t &lds) {
+  constexpr int NW = WF * WK, PX = 16 * NB;
+  a.x = static_cast<const float *>(c.x); a.w = static_cast<const float *>(c.w);
+  a.bias = c.bias; a.res = static_cast<const float *>(c.res); a.out = static_cast<float *>(c.out);
+  a.C = c.C; a.H = c.H; a.W = c.W; a.F = c.F; a.T = c.KH * c.KW; a.K = c.C * a.T;
+  a.pad = c.pad; a.st = c.stride; a.Ho = c.Ho; a.Wo = c.Wo; a.act = c.act;
+  a.nstrips = (c.Wo + 15) / 16;
+  a.tw = (c.Wo + a.nstrips - 1) / a.nstrips;
+  a.nstrips = (c.Wo + a.tw - 1) / a.tw;
+  const long long npx = (long long)a.tw * c.Ho;
+  if (npx + PX >= 65536) return false;
+  a.tiles = (int)((npx + PX - 1) / PX);
+  const long long npt = (long long)c.N * a.nstrips * a.tiles, grid = npt * ((c.F + 16 * WF - 1) / (16 * WF));
+  if (grid > 0x7fffffff - kXcds) return false;
+  a.npt = (int)npt;
+  a.grid = (int)grid;
+  int span = PX % a.tw == 0 ? PX / a.tw : (PX - 2) / a.tw + 2;  // output rows a tile touches
+  if (span > c.Ho) span = c.Ho;
+  const long long hr = (long long)(span - 1) * c.stride + c.KH;
+  a.hc = (a.tw - 1) * c.stride + c.KW;
+  const long long wwords = (long long)c.F * a.K;  // filter indices stay below 2^31 past a row's end
+  if (hr * a.hc > 64 * kStage || a.T > 4096 || wwords < 4 || wwords > (1LL << 31) - 4096) return false;
+  a.ps = (int)hr * a.hc;
+  const int need = (a.ps + 63) / 64;
+  for (int v : {1, 2, 3, 4, 5, 8, 16})
+    if (need <= (a.npl = v)) break;
+  int cmax = kStage / a.npl * NW;
+  for (;; cmax -= 16) {
+    if (c.C <= cmax) {
+      a.cc = c.C;
+      a.nchunks = 1;
+    } else {
+      if (cmax < 16) return false;
+      const int n = (c.C + cmax / 16 * 16 - 1) / (cmax / 16 * 16);
+      a.cc = ((c.C + n - 1) / n + 15) / 16 * 16;
+      a.nchunks = (c.C + a.cc - 1) / a.cc;
+    }
+    const size_t kt = ((size_t)a.cc * a.T + 15) / 16 * 16;
+    lds = 4 * (kt + (size_t)(a.nchunks > 1 ? 2 : 1) * a.cc * patch_stride(a.npl));
+    if (kt <= 8192 && lds <= 80 * 1024) break;
+    if (cmax <= 16) return false;
+  }
+  const size_t red = (size_t)NW * 16 * (PX + 4) * 4;
+  if (red > lds) lds = red;
+  a.by_hc = FastDiv(a.hc); a.by_tw = FastDiv(a.tw); a.by_t = FastDiv(a.T); a.by_kw = FastDiv(c.KW);
+  return true;
+}
+
+template <int NB, int WF, int WK, int NPL>
+hipError_t launch_split(const ConvArgs &c, const NchwArgs &a, size_t lds, hipStream_t s) {
+  auto kern = conv2d_nchw_split_kernel<NB, WF, WK, NPL>;
+  constexpr int NW = WF * WK, PX = 16 * NB;
+  // the dynamic LDS limit, raised once per device
+  const int ok = cached_per_kernel(reinterpret_cast<const void *>(kern), [&](int) {
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024) == hipSuccess
+               ? 1 : 0;
+  });
+  if (!ok) return hipErrorInvalidValue;
+  const dim3 grid((a.grid + kXcds - 1) / kXcds * kXcds);
+  const double units = NW / 4.0, steps = (a.K + 15) / 16;
+  npu_launch_plan p = make_plan("conv2d_nchw", (int)(a.grid * units), wg_per_cu(kern, 64 * NW),
+                                (int)(a.grid * units), 32);
+  p.load_phases = a.nchunks;
+  p.tile_macs = 16.0 * WF * PX * a.K / units;
+  p.tile_valu = 4.0 * (steps / WK * (8.0 + 4.0 * (NB + 2)) + 12.0 * kStage * a.nchunks + 120.0);
+  p.tile_lds_bytes = (4.0 * a.C * a.ps + WF * steps * 4.0 * 256 * (NB + 4) + 2.0 * NW * 16 * PX * 4) / units;
+  p.tile_load_bytes = (4.0 * a.C * a.ps + 4.0 * 16 * WF * a.K) / units;
+  p.tile_store_bytes = 4.0 * PX * 16 * WF * (c.res ? 2 : 1) / units;
+  p.hbm_bytes = 4.0 * ((double)c.N * c.C * c.H * c.W + (double)c.F * a.K +
+                       (double)c.N * c.F * c.Ho * c.Wo * (c.res ? 2 : 1)) + (c.bias ? 4.0 * c.F : 0.0);
   plans_add(p);
-  hipLaunchKernelGGL((conv2d_nchw_kernel<KH, KW, ST, NB>), grid, dim3(256), 0, s,
-                     static_cast<const float *>(a.x), static_cast<const float *>(a.w), a.bias,
-                     static_cast<const float *>(a.res), static_cast<float *>(a.out), a.C, a.H, a.W,
-                     a.F, a.pad, a.Ho, a.Wo, nseg, a.act);
+  hipLaunchKernelGGL(kern, grid, dim3(64 * NW), lds, s, a);
   return hipGetLastError();
 }
 
-// Row segments of 64 pixels, or of 32 when 64-pixel segments would leave
-// fewer than two workgroups per CU.
-template <int KH, int KW, int ST>
-hipError_t launch_nchw_k(const ConvArgs &a, hipStream_t s) {
-  const long long big = (long long)a.N * a.Ho * ((a.Wo + 63) / 64) * ((a.F + 63) / 64);
-  return big >= 512 ? launch_nchw<KH, KW, ST, 4>(a, s) : launch_nchw<KH, KW, ST, 2>(a, s);
+// A window that is the whole input (no pad, one output pixel: the model zoo's
+// classifiers, 7x7 over the last feature map): out[n, f] = x[n] . w[f], both
+// contiguous in the same (c, kh, kw) order.  What bounds it is reading the
+// filters once from HBM.  A workgroup of eight waves takes FW filters and
+// splits K over its waves; a wave streams FW rows at a time in whole
+// 1 KiB runs, several in flight, and multiplies each by the NI images' run.
+// 512x7x7 -> 1000 at batch 1 (103 MB of filters): 2950 us on the direct
+// kernel (16 workgroups, a load round trip per 16 k), 16.5 us here, 6.2 TB/s.
+template <int FW, int NI, bool VEC>
+__global__ __launch_bounds__(512) void conv2d_nchw_dot_kernel(
+    const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
+    const float *__restrict__ res, float *__restrict__ out, int N, int F, int K, int act) {
+  constexpr int NW = 8, EPL = VEC ? 4 : 1;
+  __shared__ float red[NW][FW * NI];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int f0 = blockIdx.x * FW, n0 = blockIdx.y * NI;
+  const float *wr[FW], *xr[NI];
+#pragma unroll
+  for (int j = 0; j < FW; ++j) wr[j] = w + (size_t)min(f0 + j, F - 1) * K;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) xr[i] = x + (size_t)min(n0 + i, N - 1) * K;
+  float acc[FW][NI];
+#pragma unroll
+  for (int j = 0; j < FW; ++j)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) acc[j][i] = 0.0f;
+  constexpr int RUN = 64 * EPL;  // elements of one wave load
+  constexpr int U = NI == 1 ? 4 : 2;
+  // runs wave, wave + NW, ... of K, U at a time; lanes past K take no part
+  auto step = [&](int k0, auto full) __attribute__((always_inline)) {
+    f32x4 wv[U][FW], xv[U][NI];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + u * NW * RUN + EPL * lane;
+      const int kc = decltype(full)::value ? k : min(k, K - EPL);
+#pragma unroll
+      for (int j = 0; j < FW; ++j) {
+        if constexpr (VEC) wv[u][j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(wr[j] + kc));
+        else wv[u][j][0] = wr[j][kc];
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        if constexpr (VEC) xv[u][i] = *reinterpret_cast<const f32x4 *>(xr[i] + kc);
+        else xv[u][i][0] = xr[i][kc];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool ok = decltype(full)::value || k0 + u * NW * RUN + EPL * lane < K;
+#pragma unroll
+      for (int j = 0; j < FW; ++j)
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int e = 0; e < EPL; ++e)
+            acc[j][i] = fmaf(ok ? wv[u][j][e] : 0.0f, ok ? xv[u][i][e] : 0.0f, acc[j][i]);
+    }
+  };
+  int k0 = wave * RUN;
+  for (; k0 + (U - 1) * NW * RUN + RUN <= K; k0 += U * NW * RUN) step(k0, std::true_type{});
+  if (k0 < K) step(k0, std::false_type{});
+#pragma unroll
+  for (int j = 0; j < FW; ++j)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const float v = wave_sum(acc[j][i]);
+      if (lane == 0) red[wave][j * NI + i] = v;
+    }
+  __syncthreads();
+  if (tid < FW * NI) {
+    const int f = f0 + tid / NI, n = n0 + tid % NI;
+    float v = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) v += red[k][tid];
+    if (f < F && n < N) {
+      const size_t o = (size_t)n * F + f;
+      if (bias) v += bias[f];
+      if (res) v += res[o];
+      out[o] = act_clamp(v, act_bounds(act));
+    }
+  }
 }
 
-// Any filter size and stride (the model zoo's 7x7 stems, 5x5 and 9x9
-// filters, its classifier written as a conv over the last feature map):
-// implicit GEMM with the reduction index k = (c, kh, kw) in FCHW order, so a
+template <int FW, int NI, bool VEC>
+hipError_t launch_dot(const ConvArgs &a, int K, hipStream_t s) {
+  const dim3 grid((a.F + FW - 1) / FW, (a.N + NI - 1) / NI);
+  npu_launch_plan p = make_plan("conv2d_nchw_dot", grid.x * grid.y * 2,
+                                wg_per_cu(conv2d_nchw_dot_kernel<FW, NI, VEC>, 512), grid.x * grid.y * 2, 32);
+  p.tile_valu = 4.0 * (K / 512.0 * (FW * NI + FW + NI) + 60.0);
+  p.tile_load_bytes = 4.0 * K * (FW + NI) / 2;
+  p.tile_store_bytes = 4.0 * FW * NI / 2;
+  p.hbm_bytes = 4.0 * ((double)a.N * K + (double)a.F * K + (double)a.N * a.F * (a.res ? 2 : 1)) +
+                (a.bias ? 4.0 * a.F : 0.0);
+  plans_add(p);
+  hipLaunchKernelGGL((conv2d_nchw_dot_kernel<FW, NI, VEC>), grid, dim3(512), 0, s,
+                     static_cast<const float *>(a.x), static_cast<const float *>(a.w), a.bias,
+                     static_cast<const float *>(a.res), static_cast<float *>(a.out), a.N, a.F, K, a.act);
+  return hipGetLastError();
+}
+
+// What the split kernel's patches do not hold (more than 1024 words per
+// channel: long strides or very large filters) or its index ranges: implicit
+// GEMM with the reduction index k = (c, kh, kw) in FCHW order, so a
 // filter's operand is its own contiguous run of k, and each MFMA step's A
 // word is the input pixel that k and the output pixel address (zero in the
 // pad).  Operands come straight from L2: no staging, no halo reuse.
@@ -326,16 +553,51 @@ hipError_t launch_nchw_direct(const ConvArgs &a, hipStream_t s) {
 
 }  // namespace
 
-// 1x1 and 3x3 filters at stride 1 or 2 take the staged kernel, every other
-// shape the direct one.
-hipError_t launch_conv2d_nchw_f32(const ConvArgs &a, hipStream_t s) {
-  if (a.stride == 1) {
-    if (a.KH == 1 && a.KW == 1) return launch_nchw_k<1, 1, 1>(a, s);
-    if (a.KH == 3 && a.KW == 3) return launch_nchw_k<3, 3, 1>(a, s);
-  } else if (a.stride == 2) {
-    if (a.KH == 1 && a.KW == 1) return launch_nchw_k<1, 1, 2>(a, s);
-    if (a.KH == 3 && a.KW == 3) return launch_nchw_k<3, 3, 2>(a, s);
+namespace {
+
+// The split kernel's shapes, largest tile first (pixels x filters per
+// workgroup 64 x 64, 64 x 32, 64 x 16, 32 x 16, 16 x 16): the first that has
+// kMinWgs workgroups, else the smallest.  Measured at batch 1, 3x3, us: the
+// 112 -> 56 layer of 64 channels (49 / 98 / 196 workgroups of the first three)
+// 22.1 / 15.5 / 12.5; 28x28x128 (28 / 56 / 112 / 200) 29.5 / 18.2 / 12.8 /
+// 10.4; 14x14x256 (16 / .. / 64 / 112 / 208) 53 / 31 / 21.6 / 17.0 / 16.1;
+// batch 8 14x14x256 (128 / 256) 55.7 / 33.3.  Sixteen waves per workgroup
+// were slower than eight (7x7x512 27 against 20 us): their loads queue.  With
+// twice kMinWgs tiles of 64 x 64, K is not split: it takes the same time
+// (56x56x64 at batch 8 33.2 against 32.2 us, 28x28x128 at batch 16 56.8 against
+// 57.4) and every sum runs in k order.
+constexpr long long kMinWgs = 160;
+template <int NB, int WF, int WK>
+bool try_split(const ConvArgs &a, long long min_wgs, hipStream_t s, hipError_t &e) {
+  NchwArgs n;
+  size_t lds;
+  if (!split_shape<NB, WF, WK>(a, n, lds)) return false;
+  if (n.grid < min_wgs) return false;
+  switch (n.npl) {
+    case 1: e = launch_split<NB, WF, WK, 1>(a, n, lds, s); break;
+    case 2: e = launch_split<NB, WF, WK, 2>(a, n, lds, s); break;
+    case 3: e = launch_split<NB, WF, WK, 3>(a, n, lds, s); break;
+    case 4: e = launch_split<NB, WF, WK, 4>(a, n, lds, s); break;
+    case 5: e = launch_split<NB, WF, WK, 5>(a, n, lds, s); break;
+    case 8: e = launch_split<NB, WF, WK, 8>(a, n, lds, s); break;
+    default: e = launch_split<NB, WF, WK, 16>(a, n, lds, s); break;
   }
+  return true;
+}
+
+}  // namespace
+
+hipError_t launch_conv2d_nchw_f32(const ConvArgs &a, hipStream_t s) {
+  const long long K = (long long)a.C * a.KH * a.KW;
+  if (a.Ho == 1 && a.Wo == 1 && a.pad == 0 && a.KH == a.H && a.KW == a.W && K < (1 << 30)) {
+    if (K % 4 == 0) return a.N == 1 ? launch_dot<4, 1, true>(a, (int)K, s) : launch_dot<4, 8, true>(a, (int)K, s);
+    return launch_dot<4, 8, false>(a, (int)K, s);
+  }
+  hipError_t e = hipSuccess;
+  if (try_split<4, 4, 1>(a, 2 * kMinWgs, s, e) || try_split<4, 4, 2>(a, kMinWgs, s, e) || 
+      try_split<4, 2, 4>(a, kMinWgs, s, e) || try_split<4, 1, 8>(a, kMinWgs, s, e) ||
+      try_split<2, 1, 8>(a, kMinWgs, s, e) || try_split<1, 1, 8>(a, 1, s, e))
+    return e;
   return launch_nchw_direct(a, s);
 }
 

@@ -977,6 +977,42 @@ def test_nchw_conv_shapes(cuda, N, C, H, W, F, K, pad, st, act, bias, res):
                 what=f"nchw conv {N}x{C}x{H}x{W} -> {F} {K}x{K}/{st}")
 
 
+@pytest.mark.parametrize("N,C,H,W,F,KH,KW,pad,st,bias,res", [
+    (1, 1, 1, 1, 3, 1, 1, 0, 1, True, False),      # fewer than four filter words: the direct kernel
+    (1, 1, 4, 5, 4, 1, 1, 0, 1, False, False),     # one k; the last filter's run moved back by 3
+    (1, 3, 9, 11, 5, 3, 3, 1, 1, True, True),      # K = 27: a ragged end of K, rows not 16-byte aligned
+    (2, 5, 6, 6, 17, 3, 1, 1, 2, False, False),    # K = 15, a 3x1 filter
+    (1, 300, 7, 7, 33, 3, 3, 1, 1, False, True),   # several channel chunks, the last one partial
+    (1, 131, 5, 5, 16, 2, 2, 0, 1, True, False),   # chunks and a ragged end of K
+    (9, 16, 17, 35, 70, 3, 3, 1, 1, True, False),  # strips of 12 columns, the last narrower; 64-filter tiles
+    (4, 24, 33, 16, 40, 3, 3, 2, 1, False, False),  # pad wider than the filter needs
+    (1, 2, 60, 60, 8, 11, 11, 2, 4, True, False),  # stride 4, 11x11: patches of 16 loads
+    (1, 2, 70, 70, 4, 15, 15, 0, 9, False, False),  # a patch past 1024 words: the direct kernel
+    (2, 520, 4, 4, 24, 1, 1, 0, 1, False, False),  # 1x1 over several chunks
+    (1, 7, 3, 5, 9, 3, 5, 0, 1, True, True),       # window = input, K = 105 (word loads)
+    (2, 36, 4, 4, 130, 4, 4, 0, 1, True, False),   # window = input, two of eight images
+    (11, 8, 2, 2, 5, 2, 2, 0, 3, False, True),     # window = input, two image groups
+])
+def test_nchw_conv_tiles(cuda, N, C, H, W, F, KH, KW, pad, st, bias, res):
+    """Edges of the split-K kernel's tiles, chunks and filter runs, of the
+    whole-window dot kernel and of the rule between them."""
+    x = rng.uniform(34, 0, (N, C, H, W), -1, 1)
+    w = rng.normal(34, 1, (F, C, KH, KW), 0, math.sqrt(2 / (KH * KW * C)))
+    b = rng.uniform(34, 2, (F,), -0.1, 0.1) if bias else None
+    Ho, Wo = (H + 2 * pad - KH) // st + 1, (W + 2 * pad - KW) // st + 1
+    r = rng.uniform(34, 3, (N, F, Ho, Wo), -1, 1) if res else None
+    out = torch.full((N, F, Ho, Wo), float("nan"), device="cuda")
+    args = (_dev(x), _dev(w), None if b is None else _dev(b))
+    if res:
+        groups.fused_conv2d_nchw_bias_res_act(*args, _dev(r), out, pad, "relu", stride=st)
+    else:
+        groups.fused_conv2d_nchw_bias_act(*args, out, pad, "relu", stride=st)
+    torch.cuda.synchronize()
+    ref, mag = refs.conv_nchw_act(x, w, b, r, pad, "relu", stride=st)
+    check_bound(_host(out), ref, mag, RTOL_F32,
+                what=f"nchw conv {N}x{C}x{H}x{W} -> {F} {KH}x{KW}/{st}")
+
+
 def test_nchw_conv_non_finite(cuda):
     """NaN and +-Inf through the NCHW conv on the f32 matrix pipe: the same
     positions and values as the oracle's f32 loops."""
