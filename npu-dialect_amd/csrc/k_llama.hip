@@ -50,52 +50,12 @@ namespace npu {
 
 namespace {
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-
-// Eight bf16 of one column, k = 8g .. 8g+7 of a 32-row k step, from a
-// 16-column B strip in LDS (two transposing reads of four k each; the four
-// 16-bit results of a read are the two dwords of the fragment half).
-__device__ __forceinline__ Frag16 read_wfrag(const unsigned char *strip, int kstep, int lane) {
-  const int g = lane >> 4, j = (lane >> 2) & 3, a = lane & 3;
-  // physical row of logical row 8g + 4r + j (r = 0, 1) is 16r + 4g + j
-  const unsigned char *p0 = strip + (kstep * 32 + 4 * g + j) * 32 + a * 8;
-  const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(p0)));
-  const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(p0 + 16 * 32)));
-  Frag16 f;
-  f.u = u32x4{lo.x, lo.y, hi.x, hi.y};
-  return f;
-}
-
-// Physical row, within a chunk, of chunk row k (see read_wfrag).
-__device__ __forceinline__ int strip_row(int k) {
-  const int kl = k & 31;
-  return (k & ~31) + 16 * ((kl >> 2) & 1) + 4 * (kl >> 3) + (kl & 3);
-}
-
 __device__ __forceinline__ uint2 pack4_bf16(float a, float b, float c, float d) {
   return make_uint2(cvt_pk_bf16(a, b), cvt_pk_bf16(c, d));
 }
 
 __device__ __forceinline__ float bf_lo(uint32_t u) { return __uint_as_float(u << 16); }
 __device__ __forceinline__ float bf_hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
-
-// Tile of this workgroup among tiles_m x tiles_n tiles: with xm > 0 the 2-D
-// XCD blocks of xcd_block_tile; else the N-major tile list cut into 8
-// contiguous ranges, range x on XCD x (blockIdx.x % 8).  Returns false for
-// the padding workgroups of a grid rounded up to a multiple of 8.
-__device__ __forceinline__ bool xcd_tile(int tiles_m, int tiles_n, int xm, int &tm, int &tn) {
-  if (xm > 0) {
-    xcd_block_tile(tiles_m, tiles_n, xm, tm, tn);
-    return true;
-  }
-  const int G = tiles_m * tiles_n, per = (G + 7) / 8;
-  const int t = (blockIdx.x % 8) * per + blockIdx.x / 8;
-  if (t >= G) return false;
-  tn = t / tiles_m;
-  tm = t % tiles_m;
-  return true;
-}
 
 constexpr int APAD = 16;  // A row padding (elements): row stride = 32 mod 64 bytes
 constexpr int GT = 1024;  // GEMM workgroup: 16 waves, four per SIMD

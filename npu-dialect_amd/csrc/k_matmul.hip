@@ -1,4 +1,6 @@
-// k_matmul.hip -- group `fill -> matmul -> generic(bias, act)` in f32.
+// k_matmul.hip -- group `fill -> matmul -> generic(bias, act)` in f32: small
+// outputs on split-K tiles of 16 x 16, large ones on tiles of the bf16 matrix
+// pipe (below).
 //
 // Replaces the tile loops the reference wraps around the outlined call
 // (FusionPass.cpp:306-359 tile-and-fuse of the consumer generic, then
@@ -137,9 +139,257 @@ __global__ __launch_bounds__(kWaves * 64) void matmul_bias_act_f32_kernel(
   if (row < M && ecol < N) out[(size_t)row * N + ecol] = act_clamp(bias ? sum + bias_e : sum, ab);
 }
 
+// ---- large outputs: tiles on the bf16 matrix pipe ------------------------------
+//
+// A BM x BN tile per workgroup of WR x WC waves, K in steps of 32.  Each
+// value is split into its three bf16 parts as it is staged (npu_device.hpp)
+// and a product takes six bf16 MFMAs, 2.7 times the f32 matrix rate, at f32
+// accuracy.  A's rows go to LDS as records of three 64-byte part runs; B's
+// rows as 16-column strips per part, read back as column runs by the
+// transposing LDS read.  The operands are swapped (B's fragment first), so a
+// lane ends with four consecutive columns of one row: 16-byte stores.  Two LDS
+// buffers, one barrier per step: the next step's runs are split and written
+// and the one after's loaded while this one is multiplied.
+//
+// What bounds it: the MFMAs and the split's vector work (34 instructions per
+// 16-byte run), which two waves per SIMD overlap; the larger the tile, the
+// fewer splits per product.
+//
+// A value outside the split's domain (Inf, NaN, |v| >= 2^55, 0 < |v| < 2^-55)
+// makes its workgroup compute its tile again with f32 MFMAs straight from
+// memory.
+template <int BM, int BN, int WR, int WC>
+struct X6Shape {
+  static constexpr int NT = 64 * WR * WC, KC = 32;
+  static constexpr int TM = BM / WR / 16, TN = BN / WC / 16;  // 16 x 16 blocks of a wave
+  static constexpr int AREC = 3 * 64 + 32;                    // A row: 32 mod 64 bytes
+  static constexpr int STRIPS = BN / 16, SB = KC * 32 + 32;   // B strip: 8 banks past a multiple of 64
+  static constexpr int ABYTES = BM * AREC, BUF = ABYTES + 3 * STRIPS * SB;
+  static constexpr int AR = BM * 8 / NT;                      // 16-byte runs per thread and step
+  static constexpr int BITEMS = KC * BN / 4, BR = (BITEMS + NT - 1) / NT;
+  static_assert(BM * 8 % NT == 0 && TM >= 1 && TN >= 1, "whole runs, whole blocks");
+};
+
+template <int BM, int BN, int WR, int WC, bool VEC>
+__global__ __launch_bounds__(64 * WR * WC, 2) void matmul_x6_kernel(
+    const float *__restrict__ A, const float *__restrict__ B, const float *__restrict__ bias,
+    float *__restrict__ out, int M, int N, int K, int act, int tiles_m, int tiles_n, int xm) {
+  using S = X6Shape<BM, BN, WR, WC>;
+  constexpr int NT = S::NT, TM = S::TM, TN = S::TN, KC = S::KC;
+  extern __shared__ __attribute__((aligned(16))) unsigned char x6mem[];
+  __shared__ int missed;
+  int tm, tn;
+  if (!xcd_tile(tiles_m, tiles_n, xm, tm, tn)) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 15, q = lane >> 4;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int wr = wave % WR, wc = wave / WR;
+  if (tid == 0) missed = 0;
+
+  // Runs past M or N read the last row or columns (they feed outputs that
+  // are not stored); runs past K are zeroed when they are split.
+  const float *ap[S::AR];
+  uint32_t adst[S::AR];
+  const int ak = (tid & 7) * 4;
+#pragma unroll
+  for (int i = 0; i < S::AR; ++i) {
+    const int row = (tid + NT * i) >> 3;
+    ap[i] = A + (size_t)min(m0 + row, M - 1) * K;
+    adst[i] = (uint32_t)(row * S::AREC + ak * 2);
+  }
+  int bk[S::BR], bcol[S::BR];
+  uint32_t bdst[S::BR];
+#pragma unroll
+  for (int i = 0; i < S::BR; ++i) {
+    const int it = min(tid + NT * i, S::BITEMS - 1);
+    const int c = it % (BN / 4) * 4;
+    bk[i] = it / (BN / 4);
+    bcol[i] = n0 + c;
+    bdst[i] = (uint32_t)(S::ABYTES + (c >> 4) * S::SB + strip_row(bk[i]) * 32 + (c & 15) * 2);
+  }
+  u32x4 av[S::AR], bv[S::BR];
+  auto fetch = [&](int k0) __attribute__((always_inline)) {
+    const int ka = min(k0 + ak, K - 4);
+#pragma unroll
+    for (int i = 0; i < S::AR; ++i) av[i] = *reinterpret_cast<const u32x4 *>(ap[i] + ka);
+#pragma unroll
+    for (int i = 0; i < S::BR; ++i) {
+      const float *row = B + (size_t)min(k0 + bk[i], K - 1) * N;
+      if constexpr (VEC) {
+        bv[i] = *reinterpret_cast<const u32x4 *>(row + min(bcol[i], N - 4));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bv[i][e] = __float_as_uint(row[min(bcol[i] + e, N - 1)]);
+      }
+    }
+  };
+  SplitDomainBounds dom;
+  auto commit = [&](int k0, unsigned char *buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < S::AR; ++i) {
+      const u32x4 v = masked(av[i], k0 + ak < K);
+      dom.fold(v);
+      const Parts4 p = split_parts(v);
+      *reinterpret_cast<uint2 *>(buf + adst[i]) = p.h;
+      *reinterpret_cast<uint2 *>(buf + adst[i] + 64) = p.m;
+      *reinterpret_cast<uint2 *>(buf + adst[i] + 128) = p.l;
+    }
+#pragma unroll
+    for (int i = 0; i < S::BR; ++i) {
+      const u32x4 v = masked(bv[i], k0 + bk[i] < K);
+      dom.fold(v);
+      const Parts4 p = split_parts(v);
+      if (NT * (i + 1) <= S::BITEMS || tid + NT * i < S::BITEMS) {
+        *reinterpret_cast<uint2 *>(buf + bdst[i]) = p.h;
+        *reinterpret_cast<uint2 *>(buf + bdst[i] + S::STRIPS * S::SB) = p.m;
+        *reinterpret_cast<uint2 *>(buf + bdst[i] + 2 * S::STRIPS * S::SB) = p.l;
+      }
+    }
+  };
+
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](const unsigned char *buf) __attribute__((always_inline)) {
+    Frag16 b[TN][3];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        b[j][p] = read_wfrag(buf + S::ABYTES + (p * S::STRIPS + wc * TN + j) * S::SB, 0, lane);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      Frag16 a[3];
+      const unsigned char *rec = buf + (wr * (BM / WR) + 16 * i + r) * S::AREC + q * 16;
+#pragma unroll
+      for (int p = 0; p < 3; ++p) a[p].u = *reinterpret_cast<const u32x4 *>(rec + 64 * p);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] += dot_x6(b[j], a);
+    }
+  };
+  const int steps = (K + KC - 1) / KC;
+  fetch(0);
+  commit(0, x6mem);
+  fetch(KC);
+  __syncthreads();
+  for (int s = 0; s < steps; ++s) {
+    multiply(x6mem + (s & 1) * S::BUF);
+    if (s + 1 < steps) {
+      commit((s + 1) * KC, x6mem + ((s + 1) & 1) * S::BUF);
+      fetch((s + 2) * KC);
+    }
+    __syncthreads();
+  }
+  if (__builtin_amdgcn_ballot_w64(dom.miss()) != 0 && lane == 0) missed = 1;
+  __syncthreads();
+  if (missed) {
+    // f32 MFMAs, k in order, operands from memory (K % 4 == 0)
+    const float *arow[TM], *bp[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) arow[i] = A + (size_t)min(m0 + wr * (BM / WR) + 16 * i + r, M - 1) * K + q;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) bp[j] = B + (size_t)q * N + min(n0 + wc * (BN / WC) + 16 * j + r, N - 1);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < K; k += 4) {
+      float af[TM], bf[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) af[i] = arow[i][k];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) bf[j] = bp[j][(size_t)k * N];
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j], af[i], acc[i][j], 0, 0, 0);
+    }
+  }
+
+  const ActBounds ab = act_bounds(act);
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + wc * (BN / WC) + 16 * j + 4 * q;
+    f32x4 bj = {0.f, 0.f, 0.f, 0.f};
+    if (bias) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bj[e] = bias[min(n + e, N - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int m = m0 + wr * (BM / WR) + 16 * i + r;
+      if (m >= M) continue;
+      f32x4 v = acc[i][j];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = act_clamp(bias ? v[e] + bj[e] : v[e], ab);
+      float *o = out + (size_t)m * N + n;
+      if constexpr (VEC) {
+        if (n < N) *reinterpret_cast<f32x4 *>(o) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) o[e] = v[e];
+      }
+    }
+  }
+}
+
+template <int BM, int BN, int WR, int WC, bool VEC>
+hipError_t launch_x6(const MatmulArgs &a, hipStream_t s) {
+  using S = X6Shape<BM, BN, WR, WC>;
+  auto kern = matmul_x6_kernel<BM, BN, WR, WC, VEC>;
+  // the dynamic LDS limit, raised once per device
+  const int ok = cached_per_kernel(reinterpret_cast<const void *>(kern), [&](int) {
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, 2 * S::BUF) == hipSuccess
+               ? 1 : 0;
+  });
+  if (!ok) return hipErrorInvalidValue;
+  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
+  const int G = tiles_m * tiles_n, grid = (G + kXcds - 1) / kXcds * kXcds;
+  const double steps = (a.K + S::KC - 1) / S::KC;
+  npu_launch_plan p = make_plan("matmul_f32_bf16x6", G, wg_per_cu(kern, S::NT), G, 16);
+  p.unit_waves = WR * WC;
+  p.load_phases = 1;
+  p.tile_macs = 6.0 * BM * BN * S::KC * steps;
+  p.tile_valu = WR * WC * (steps * (34.0 * (S::AR + S::BR) + 30.0) + 16.0 * S::TM * S::TN + 100.0);
+  p.tile_lds_bytes = steps * (S::BUF + WR * WC * 3.0 * 1024 * (S::TM + S::TN));
+  p.tile_load_bytes = steps * 4.0 * S::KC * (BM + BN);
+  p.tile_store_bytes = 4.0 * BM * BN;
+  p.hbm_bytes = 4.0 * ((double)a.M * a.K + (double)a.K * a.N + (double)a.M * a.N + (a.bias ? a.N : 0));
+  plans_add(p);
+  const int xm = xcd_block_grid(tiles_m, tiles_n, BM, BN, true);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(S::NT), 2 * S::BUF, s, a.A, a.B, a.bias, a.out, a.M, a.N,
+                     a.K, a.act, tiles_m, tiles_n, xm);
+  return hipGetLastError();
+}
+
+template <int BM, int BN, int WR, int WC>
+hipError_t launch_x6(const MatmulArgs &a, hipStream_t s) {
+  return a.N % 4 == 0 ? launch_x6<BM, BN, WR, WC, true>(a, s) : launch_x6<BM, BN, WR, WC, false>(a, s);
+}
+
+// Tiles of 256 x 96 when there are enough to give most CUs one (a workgroup's
+// 153 KB of LDS leave no room for a second), of 64 x 64 when there are enough
+// of those, else the split-K tiles of 16 x 16.  Measured, us, as 16x16 / 64x64
+// / 256x96: 2000x1024x3000 (256 tiles of 256 x 96) 421 / 128 / 82;
+// 1000x2048x1999 (84; 512 of 64 x 64) 403 / 97 / 156; 2000x64x2000 (168) 80 /
+// 12.5 / 11.7; 1024x1024x1024 (256 of 64 x 64) 46 / 30 / 74; 512x1024x2048
+// (256) 50 / 30 / 74; 627x648x900 (150) 22.0 / 20.5 / 50; 64x1024x4096 (64)
+// 17.4 / 27.7 / 73; 512x1024x512 (64) 12.3 / 28 / 72.
+// Error against 64 bits, relative 2-norm: K = 1024 1.2e-7 (16x16: 2.9e-7).
+constexpr int kMinBig = 160, kMinMid = 176;
+
 }  // namespace
 
 hipError_t launch_matmul_bias_act_f32(const MatmulArgs &a, hipStream_t s) {
+  const long long big = (long long)((a.M + 255) / 256) * ((a.N + 95) / 96);
+  const long long mid = (long long)((a.M + 63) / 64) * ((a.N + 63) / 64);
+  if (big >= kMinBig) return launch_x6<256, 96, 4, 2>(a, s);
+  if (mid >= kMinMid) return launch_x6<64, 64, 2, 2>(a, s);
   const int tiles_n = (a.N + 15) / 16, tiles = tiles_n * ((a.M + 15) / 16);
   const int nchunks = (a.K + 15) / 16;
   const bool vec = a.N % 4 == 0;

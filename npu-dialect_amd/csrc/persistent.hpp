@@ -92,6 +92,23 @@ inline int xcd_block_grid(int tiles_m, int tiles_n, int bm, int bn_cols, bool n_
   return best;
 }
 
+// Tile of this workgroup among tiles_m x tiles_n tiles: with xm > 0 the 2-D
+// XCD blocks of xcd_block_tile; else the N-major tile list cut into 8
+// contiguous ranges, range x on XCD x (blockIdx.x % 8).  Returns false for
+// the padding workgroups of a grid rounded up to a multiple of 8.
+__device__ __forceinline__ bool xcd_tile(int tiles_m, int tiles_n, int xm, int &tm, int &tn) {
+  if (xm > 0) {
+    xcd_block_tile(tiles_m, tiles_n, xm, tm, tn);
+    return true;
+  }
+  const int G = tiles_m * tiles_n, per = (G + 7) / 8;
+  const int t = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (t >= G) return false;
+  tn = t / tiles_m;
+  tm = t % tiles_m;
+  return true;
+}
+
 // Index arithmetic that does not depend on the tile would be hoisted out of
 // a tile loop by the compiler and pinned in registers for its whole length;
 // passing a value through an empty asm makes it be recomputed per tile

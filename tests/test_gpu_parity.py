@@ -76,6 +76,52 @@ def test_c1_matmul_shapes(cuda, M, K, N, act, bias):
     check_bound(_host(out), ref, mag, RTOL_F32, what=f"matmul {M}x{K}x{N}")
 
 
+@pytest.mark.parametrize("M,K,N,act,bias", [
+    (769, 36, 960, "relu", True),      # 64x64 tiles: a row and 4 k past a tile
+    (833, 4, 833, "none", False),      # one k run, odd N (word loads and stores)
+    (704, 64, 1021, "relu6", True),    # whole k steps, columns ragged by 1 mod 4
+    (2049, 68, 1732, "relu", True),    # 256x96 tiles, a row past a tile, ragged columns
+    (2305, 32, 1537, "none", True),    # 256x96 tiles, odd N, one whole k step
+])
+def test_c1_matmul_large_tiles(cuda, M, K, N, act, bias):
+    """Edges of the large-output tiles on the bf16 matrix pipe."""
+    A = rng.uniform(41, 0, (M, K), -1, 1)
+    B = rng.uniform(41, 1, (K, N), -1, 1)
+    b = rng.uniform(41, 2, (N,), -1, 1) if bias else None
+    out = torch.full((M, N), float("nan"), device="cuda")
+    groups.fused_matmul_bias_act(_dev(A), _dev(B), None if b is None else _dev(b), out, act)
+    torch.cuda.synchronize()
+    with oracle.threaded():
+        ref, mag = refs.matmul_bias_act(A, B, b, act)
+    check_bound(_host(out), ref, mag, RTOL_F32, what=f"matmul {M}x{K}x{N}")
+
+
+def test_c1_matmul_large_tiles_out_of_split_domain(cuda):
+    """Values the three-part split does not take (Inf, NaN, magnitudes of 2^60
+    and 2^-70, an f32 subnormal) in A or B: their tiles are computed with f32
+    MFMAs, every value and every Inf and NaN where the f32 loops give them."""
+    M, K, N = 769, 40, 960
+    A = rng.uniform(42, 0, (M, K), -1, 1)
+    B = rng.uniform(42, 1, (K, N), -1, 1)
+    A[3, 5], A[70, 39], A[200, 0] = np.inf, np.nan, 2.0 ** 60
+    A[400] = 2.0 ** -70
+    B[7, 130], B[39, 959], B[:, 500] = -np.inf, 2.0 ** -140, 2.0 ** -90
+    out = torch.empty(M, N, device="cuda")
+    groups.fused_matmul_bias_act(_dev(A), _dev(B), None, out, "none")
+    torch.cuda.synchronize()
+    got = _host(out)
+    with oracle.threaded():
+        ref, mag = refs.matmul_bias_act(A, B, None, "none")
+    hit = ~np.isfinite(ref)
+    assert hit.sum() >= N
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    fin = hit & ~np.isnan(ref)
+    assert np.array_equal(got[fin], ref[fin])
+    # f32 subnormal spacing per term where the products are that small
+    check_bound(got[~hit], ref[~hit], mag[~hit], RTOL_F32, atol=K * 2.0 ** -149,
+                what="matmul outside the split's domain")
+
+
 def test_c1_reference_kat_fills(cuda):
     """e2e_verify's closed form on the GPU: fills 0.01 / 0.02 give K * 2e-4."""
     M, K, N = 256, 512, 256
