@@ -9,132 +9,245 @@
 // spatial split the reference picks over Co (test/lit/spatial_tiling_conv2d.mlir:28-34)
 // becomes the grid's y dimension; the pixel dimension is the grid's x.
 //
-// Workgroup tile: 64 pixels x 64 filters, 4 waves as 2 x 2, each wave
-// 32 x 32 = four 16x16 MFMA tiles.  The epilogue (bias add, residual add,
-// act, and the bf16 rounding of the bf16 variant) runs on the accumulators.
+// A workgroup of 2 x 2 waves owns BM pixels x BN filters.  The reduction walks
+// the taps and, within a tap, chunks of 128 bytes of channels; per step the
+// pixels' runs (zero outside the image and past C) and the filters' runs are
+// staged in LDS, double-buffered, the next step's loads in flight while the
+// current one is multiplied, one barrier per step.  The filter fragment is the
+// MFMA's first operand, so a lane ends with four consecutive filters of one
+// pixel: the epilogue (bias add, residual add, act, and the bf16 rounding of
+// the bf16 variant) runs on the accumulators and stores 8 or 16 bytes.
 // C need not be a multiple of an MFMA fragment's 16 (f32) or 32 (bf16)
-// channels: a lane's 16-byte run past C loads zeros.  F need not be a
-// multiple of 16 either: filters past F are zero and not stored.
+// channels: a 16-byte run past C is staged as zero.  F need not be a multiple
+// of 16 either: filters past F read filter F - 1 and are not stored.
 #include "kernels.hpp"
 #include "npu_device.hpp"
+#include "persistent.hpp"
 #include "plans.hpp"
 
 namespace npu {
 
 namespace {
 
-template <class MM, typename T>
-__global__ __launch_bounds__(256) void conv2d_nhwc_kernel(
-    const T *__restrict__ x, const T *__restrict__ w, const float *__restrict__ bias,
-    const T *__restrict__ res, T *__restrict__ out, int Nb, int H, int W, int C, int F, int KH,
-    int KW, int pad, int Ho, int Wo, int act) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+struct ConvTileArgs {
+  const void *x, *w, *res;
+  const float *bias;
+  void *out;
+  int H, W, C, F, KW, taps, pad, Ho, Wo, act, P, npt, nft;
+};
+
+template <class MM, typename T, int BM, int BN>
+__global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs a) {
+  constexpr int ES = sizeof(T), RUN = 16 / ES;        // elements of a 16-byte run
+  constexpr int KC = 128 / ES;                        // channels of a step
+  constexpr int REC = 128 + 32;                       // LDS row: 32 mod 64 bytes
+  constexpr int TM = BM / 32, TN = BN / 32;           // 16 x 16 blocks of a wave
+  constexpr int AR = BM / 32, BR = BN / 32;           // runs per thread and step
+  constexpr int BUF = (BM + BN) * REC;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * BUF];
+  const int per = gridDim.x / kXcds, t = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
+  if (t >= a.npt * a.nft) return;
+  const int pt = t / a.nft, ft = t - pt * a.nft;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, q = lane >> 4;
-  const int P = Nb * Ho * Wo;
-  const int p0 = blockIdx.x * 64 + (wave & 1) * 32;
-  const int f0 = blockIdx.y * 64 + (wave >> 1) * 32;
+  const int wp = wave & 1, wf = wave >> 1;
+  const int p0 = pt * BM, f0 = ft * BN;
+  const T *const x = static_cast<const T *>(a.x);
+  const T *const w = static_cast<const T *>(a.w);
 
-  int pbase[2], poh[2], pow_[2];
-  bool pok[2];
+  // staging: this thread's 16-byte run `seg` of rows tid / 8 + 32 i
+  const int seg = tid & 7, row0 = tid >> 3;
+  int abase[AR], aoh[AR], aow[AR], bbase[BR];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int p = p0 + 16 * i + r;
-    pok[i] = p < P;
-    const int pp = pok[i] ? p : 0;
-    const int n = pp / (Ho * Wo);
-    const int rem = pp - n * Ho * Wo;
-    poh[i] = rem / Wo;
-    pow_[i] = rem - poh[i] * Wo;
-    pbase[i] = n * H * W;  // pixel index of (n, 0, 0) in the input
+  for (int i = 0; i < AR; ++i) {
+    const int p = min(p0 + row0 + 32 * i, a.P - 1);
+    const int n = p / (a.Ho * a.Wo), rem = p - n * a.Ho * a.Wo;
+    const int oh = rem / a.Wo;
+    aoh[i] = oh - a.pad;
+    aow[i] = rem - oh * a.Wo - a.pad;
+    abase[i] = n * a.H * a.W;
   }
-  bool fok[2];
-  int fbase[2];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int f = f0 + 16 * j + r;
-    fok[j] = f < F;
-    fbase[j] = (fok[j] ? f : 0) * KH * KW * C;
-  }
+  for (int i = 0; i < BR; ++i) bbase[i] = min(f0 + row0 + 32 * i, a.F - 1) * a.taps * a.C;
+  // Loads from clamped addresses now, zeros chosen when the runs are written
+  // (a select on a loaded value would make the wave wait for it there).
+  u32x4 av[AR], bv[BR];
+  uint32_t keep = 0;
+  auto fetch = [&](int kh, int kw, int c0) __attribute__((always_inline)) {
+    const int c = c0 + seg * RUN;
+    const bool cin = c < a.C;
+    const int cc = cin ? c : 0;
+    keep = (uint32_t)cin << AR;
+#pragma unroll
+    for (int i = 0; i < AR; ++i) {
+      const int ih = aoh[i] + kh, iw = aow[i] + kw;
+      const bool in = (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
+      av[i] = *reinterpret_cast<const u32x4 *>(x + (size_t)(abase[i] + (in ? ih * a.W + iw : 0)) * a.C + cc);
+      keep |= (uint32_t)(in && cin) << i;
+    }
+    const int tap = (kh * a.KW + kw) * a.C + cc;
+#pragma unroll
+    for (int i = 0; i < BR; ++i) bv[i] = *reinterpret_cast<const u32x4 *>(w + (size_t)(bbase[i] + tap));
+  };
+  unsigned char *const dst = lds + row0 * REC + seg * 16;
+  auto commit = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < AR; ++i)
+      *reinterpret_cast<u32x4 *>(dst + buf * BUF + 32 * i * REC) = masked(av[i], (keep >> i) & 1u);
+#pragma unroll
+    for (int i = 0; i < BR; ++i)
+      *reinterpret_cast<u32x4 *>(dst + buf * BUF + (BM + 32 * i) * REC) = masked(bv[i], (keep >> AR) & 1u);
+  };
 
-  typename MM::acc_t acc[2][2];
+  typename MM::acc_t acc[TM][TN];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = typename MM::acc_t{0, 0, 0, 0};
+    for (int j = 0; j < TN; ++j) acc[i][j] = typename MM::acc_t{0, 0, 0, 0};
 
-  const int cl = q * MM::kPerLane;
-  for (int kh = 0; kh < KH; ++kh) {
-    for (int kw = 0; kw < KW; ++kw) {
-      int aoff[2];
-      bool aok[2];
+  // steps in order (kh, kw, channel chunk); the coordinates of the step being
+  // fetched run one ahead, and stay on the last step past the end
+  const int chunks = (a.C + KC - 1) / KC, steps = a.taps * chunks, KH = a.taps / a.KW;
+  int kh = 0, kw = 0, ch = 0;
+  auto advance = [&]() __attribute__((always_inline)) {
+    if (++ch == chunks) {
+      ch = 0;
+      if (++kw == a.KW) kw = 0, kh = min(kh + 1, KH - 1);
+    }
+  };
+  fetch(0, 0, 0);
+  commit(0);
+  advance();
+  fetch(kh, kw, ch * KC);
+  __syncthreads();
+  const unsigned char *const arow = lds + (wp * (BM / 2) + r) * REC + q * 16;
+  const unsigned char *const brow = lds + (BM + wf * (BN / 2) + r) * REC + q * 16;
+  int mch = 0;  // channel chunk of the step being multiplied
+  for (int s = 0; s < steps; ++s) {
+    const int off = (s & 1) * BUF;
+    const int frags = min(2, (a.C - mch * KC + KC / 2 - 1) / (KC / 2));
+    if (++mch == chunks) mch = 0;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int ih = poh[i] + kh - pad, iw = pow_[i] + kw - pad;
-        aok[i] = pok[i] && ih >= 0 && ih < H && iw >= 0 && iw < W;
-        aoff[i] = (pbase[i] + ih * W + iw) * C + cl;
-      }
-      const int woff = (kh * KW + kw) * C + cl;
-      for (int c0 = 0; c0 < C; c0 += MM::kPerFrag) {
-        const bool cin = c0 + cl < C;  // this lane's run lies within the C channels
-        Frag16 a[2], b[2];
+    for (int f = 0; f < 2; ++f) {
+      if (f < frags) {  // uniform: the last chunk's second half may lie past C
+        Frag16 af[TM], bf[TN];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) a[i] = aok[i] && cin ? load16(x + aoff[i] + c0) : frag_zero();
+        for (int i = 0; i < TM; ++i) af[i].u = *reinterpret_cast<const u32x4 *>(arow + off + 16 * i * REC + 64 * f);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) b[j] = fok[j] && cin ? load16(w + fbase[j] + woff + c0) : frag_zero();
+        for (int j = 0; j < TN; ++j) bf[j].u = *reinterpret_cast<const u32x4 *>(brow + off + 16 * j * REC + 64 * f);
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int st = 0; st < MM::kSteps; ++st)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) MM::mma(acc[i][j], a[i], b[j]);
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) MM::step(acc[i][j], bf[j], af[i], st);
       }
     }
+    if (s + 1 < steps) {
+      commit((s + 1) & 1);
+      advance();
+      fetch(kh, kw, ch * KC);
+    }
+    __syncthreads();
   }
 
-  // Epilogue: rows 4q + e of each 16-pixel block, column r of each 16-filter block.
+  // Epilogue: pixel r of each block, its filters 4q .. +3.
+  const ActBounds ab = act_bounds(a.act);
+  const T *const res = static_cast<const T *>(a.res);
+  T *const out = static_cast<T *>(a.out);
+  const bool vec = a.F % 4 == 0;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int f = f0 + 16 * j + r;
-    if (f >= F) continue;
-    const float bv = bias ? bias[f] : 0.0f;
+  for (int j = 0; j < TN; ++j) {
+    const int f = f0 + wf * (BN / 2) + 16 * j + 4 * q;
+    f32x4 bj = {0.f, 0.f, 0.f, 0.f};
+    if (a.bias) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+      for (int e = 0; e < 4; ++e) bj[e] = a.bias[min(f + e, a.F - 1)];
+    }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int p = p0 + 16 * i + 4 * q + e;
-        if (p >= P) continue;
-        float v = acc[i][j][e] + bv;
-        if constexpr (sizeof(T) == 4) {
-          if (res) v += res[(size_t)p * F + f];
-          out[(size_t)p * F + f] = act_apply(v, act);
+    for (int i = 0; i < TM; ++i) {
+      const int p = p0 + wp * (BM / 2) + 16 * i + r;
+      if (p >= a.P || f >= a.F) continue;
+      const size_t o = (size_t)p * a.F + f;
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] + bj[e];
+      if constexpr (sizeof(T) == 4) {
+        if (vec) {
+          if (res) v += *reinterpret_cast<const f32x4 *>(res + o);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = act_clamp(v[e], ab);
+          *reinterpret_cast<f32x4 *>(out + o) = v;
         } else {
-          if (res) v += bf16_to_f32(res[(size_t)p * F + f]);
-          out[(size_t)p * F + f] = f32_to_bf16(act_apply(v, act));
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (f + e < a.F) out[o + e] = act_clamp(res ? v[e] + res[o + e] : v[e], ab);
+        }
+      } else {
+        if (vec) {
+          if (res) {
+            const uint2 u = *reinterpret_cast<const uint2 *>(res + o);
+            v[0] += __uint_as_float(u.x << 16);
+            v[1] += __uint_as_float(u.x & 0xffff0000u);
+            v[2] += __uint_as_float(u.y << 16);
+            v[3] += __uint_as_float(u.y & 0xffff0000u);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = act_clamp(v[e], ab);
+          *reinterpret_cast<uint2 *>(out + o) = make_uint2(cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (f + e < a.F)
+              out[o + e] = f32_to_bf16(act_clamp(res ? v[e] + bf16_to_f32(res[o + e]) : v[e], ab));
         }
       }
     }
   }
 }
 
+template <class MM, typename T, int BM, int BN>
+hipError_t launch_tile(const ConvArgs &c, hipStream_t s) {
+  auto kern = conv2d_nhwc_kernel<MM, T, BM, BN>;
+  ConvTileArgs a{c.x, c.w, c.res, c.bias, c.out, c.H, c.W, c.C, c.F, c.KW, c.KH * c.KW, c.pad, c.Ho, c.Wo, c.act,
+                 c.N * c.Ho * c.Wo, 0, 0};
+  a.npt = (a.P + BM - 1) / BM;
+  a.nft = (a.F + BN - 1) / BN;
+  const int G = a.npt * a.nft, grid = (G + kXcds - 1) / kXcds * kXcds;
+  const double steps = (double)a.taps * ((a.C + 128 / sizeof(T) - 1) / (128 / sizeof(T)));
+  npu_launch_plan p = make_plan("conv2d_nhwc", G, wg_per_cu(kern), G, 8 * sizeof(T));
+  p.load_phases = 1;  // a step's loads are in flight during the step before
+  p.tile_macs = (double)BM * BN * steps * 128 / sizeof(T);
+  p.tile_valu = 4.0 * (steps * (10.0 * (BM + BN) / 32 + 20.0) + 12.0 * BM * BN / 1024 + 120.0);
+  p.tile_lds_bytes = steps * (128.0 * (BM + BN) + 4.0 * 2 * 1024 * (BM + BN) / 32);
+  p.tile_load_bytes = steps * 128.0 * (BM + BN);
+  p.tile_store_bytes = (double)BM * BN * sizeof(T);
+  p.hbm_bytes = (double)sizeof(T) * ((double)c.N * c.H * c.W * c.C + (double)c.F * c.KH * c.KW * c.C +
+                                     (double)a.P * c.F * (c.res ? 2 : 1)) + (c.bias ? 4.0 * c.F : 0.0);
+  plans_add(p);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+// Tiles of 64 pixels x 64 filters when there are enough to keep more than one
+// workgroup on a CU, with 32 filters where 64 would compute a tenth more
+// padding; then 64 x 32; then 32 x 32.  Measured, us, as 64x64 / 64x32 / 32x32
+// (workgroups of the first), against the kernel before (operands straight from
+// L2): bf16 3x3 28x28x128 at batch 32 (784) 22.7 / 27.7 / 28.9, before 71.3;
+// 14x14x256 (392) 26.2 / 30.1 / 30.6, before 70.5; 7x7x512 (200) 40.9 / 38.2 /
+// 36.9, before 70.0; 28x28x128 at batch 4 (98) 12.1 / 10.4 / 9.3, before 21.7;
+// 1x1 68x67x80 -> 150 at batch 11 (2376) 31.4 / 27.3 / 29.2, before 29.7; f32
+// 1x1 56x56x64 -> 256 at batch 32 (6272) 60.9 / 62.5 / 67.8, before 93.6.
+// Tiles of 128 pixels or filters were slower (fewer workgroups per CU).
+constexpr long long kMinTiles = 384;
+
 template <class MM, typename T>
 hipError_t launch_conv(const ConvArgs &a, hipStream_t s) {
-  const int P = a.N * a.Ho * a.Wo;
-  dim3 grid((P + 63) / 64, (a.F + 63) / 64);
-  const int iters = a.KH * a.KW * ((a.C + MM::kPerFrag - 1) / MM::kPerFrag);
-  npu_launch_plan p = make_plan("conv2d_nhwc", grid.x * grid.y, wg_per_cu(conv2d_nhwc_kernel<MM, T>),
-                                grid.x * grid.y, 8 * sizeof(T));
-  p.load_phases = iters;  // each (tap, channel chunk) step loads, then multiplies
-  p.tile_macs = 64.0 * 64 * iters * MM::kPerFrag;
-  p.tile_valu = 4.0 * (40.0 * iters + 150);  // per wave: addressing per step, epilogue
-  p.tile_load_bytes = iters * 4.0 * 4 * 1024;  // per wave 2 A and 2 B fragments of 1 KB
-  p.tile_store_bytes = 64.0 * 64 * sizeof(T);
-  p.hbm_bytes = (double)sizeof(T) * ((double)a.N * a.H * a.W * a.C + (double)a.F * a.KH * a.KW * a.C +
-                                     (double)P * a.F * (a.res ? 2 : 1)) + (a.bias ? 4.0 * a.F : 0.0);
-  plans_add(p);
-  hipLaunchKernelGGL((conv2d_nhwc_kernel<MM, T>), grid, dim3(256), 0, s,
-                     static_cast<const T *>(a.x), static_cast<const T *>(a.w), a.bias,
-                     static_cast<const T *>(a.res), static_cast<T *>(a.out), a.N, a.H, a.W, a.C,
-                     a.F, a.KH, a.KW, a.pad, a.Ho, a.Wo, a.act);
-  return hipGetLastError();
+  const long long pt = ((long long)a.N * a.Ho * a.Wo + 63) / 64;
+  const int f64 = (a.F + 63) / 64, f32 = (a.F + 31) / 32;
+  if (pt * f64 >= kMinTiles && 2 * f64 * 10 <= f32 * 11) return launch_tile<MM, T, 64, 64>(a, s);
+  if (pt * f32 >= kMinTiles) return launch_tile<MM, T, 64, 32>(a, s);
+  return launch_tile<MM, T, 32, 32>(a, s);
 }
 
 }  // namespace

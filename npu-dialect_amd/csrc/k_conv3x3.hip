@@ -2,10 +2,10 @@
 // generic(bias, act)` for images up to 64 pixels wide: the shape of the
 // conv2d configurations (56x56x64 -> 64).
 //
-// A workgroup owns TR full image rows of one image and 64 (or 16) filters.
+// A workgroup owns one full image row of one image and 16 filters.
 // The reduction runs over stages of NCH channel chunks (a chunk is one MFMA
 // operand run: 16 f32 or 32 bf16 channels).  For each stage the zero-padded
-// (TR+2) x (W+2) input halo is staged once into LDS and all nine taps read
+// 3 x (W+2) input halo is staged once into LDS and all nine taps read
 // their A operands from it with shifted addressing, so each input element
 // leaves HBM/L2 once per stage instead of once per tap.  With several stages
 // the next stage's halo and filter fragments are fetched into registers
@@ -37,7 +37,7 @@ namespace npu {
 
 namespace {
 
-template <class MM, typename T, int TR, int WF, int WMAX, int NCH, int NBUF, int WFIX>
+template <class MM, typename T, int WMAX, int NCH, int NBUF, int WFIX>
 __global__ __launch_bounds__(256) void conv3x3_rows_kernel(
     const T *__restrict__ x, const T *__restrict__ w, const float *__restrict__ bias,
     T *__restrict__ out, int H, int w_rt, int c_rt, int F, int act) {
@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) void conv3x3_rows_kernel(
   // compile-time, so the halo and output index arithmetic folds
   const int W = WFIX > 0 ? WFIX : w_rt;
   const int C = NBUF == 1 ? NCH * MM::kPerFrag : c_rt;
-  constexpr int WP = 4 / WF;                  // waves along pixels
+  constexpr int TR = 1, WP = 4;               // one row per workgroup, waves along its pixels
   constexpr int KPL = MM::kPerLane;           // elements of one lane's 16-byte run
   constexpr int KC = MM::kPerFrag;            // channels per chunk (64 bytes)
   constexpr int SEGP = NCH * 4;               // 16-byte segments per pixel and stage
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(256) void conv3x3_rows_kernel(
   // path of a one-tile workgroup: bf16 56x56x64 5.1 -> 3.7 us); a row
   // stride of 9 C channels plus 32 bytes (32 mod 64 bytes) keeps the 16
   // filters' fragment reads conflict-free.
-  constexpr bool WLDS = NBUF == 1 && WF == 1;
+  constexpr bool WLDS = NBUF == 1;
   constexpr int WST = 9 * NCH * KC + 32 / sizeof(T);
   constexpr int EPR = 16 / sizeof(T);  // elements per 16-byte run
   __shared__ __attribute__((aligned(16))) T halo[NBUF][HR * (WMAX + 2) * REC];
@@ -74,9 +74,9 @@ __global__ __launch_bounds__(256) void conv3x3_rows_kernel(
   int tile = blockIdx.x;
   if (gridDim.x % kXcds == 0) tile = (tile % kXcds) * (gridDim.x / kXcds) + tile / kXcds;
   const int n = tile / tiles_h, h0 = (tile - n * tiles_h) * TR;
-  const int f = (blockIdx.y * WF + (wave % WF)) * 16 + r;
+  const int f = blockIdx.y * 16 + r;
   const bool fok = f < F;
-  const int wp = wave / WF;
+  const int wp = wave;
   const int HC = W + 2, nseg = HR * HC * SEGP;
   const int tile_px = TR * W;
 
@@ -1027,20 +1027,19 @@ hipError_t launch_x6(const ConvArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <class MM, typename T, int TR, int WF, int WMAX, int NCH, int NBUF, int WFIX>
+template <class MM, typename T, int WMAX, int NCH, int NBUF, int WFIX>
 hipError_t launch_rows(const ConvArgs &a, hipStream_t s) {
   if (a.W > WMAX || (WFIX > 0 && a.W != WFIX) || a.C % (MM::kPerFrag * NCH) != 0 ||
       (NBUF == 1 && a.C != MM::kPerFrag * NCH))
     return hipErrorInvalidValue;
-  const int tiles_h = (a.H + TR - 1) / TR;
-  dim3 grid(a.N * tiles_h, (a.F + 16 * WF - 1) / (16 * WF));
+  dim3 grid(a.N * a.H, (a.F + 15) / 16);
   {
-    constexpr int WP = 4 / WF, PBW = ((TR * WMAX + 15) / 16 + WP - 1) / WP;
+    constexpr int TR = 1, WP = 4, PBW = ((TR * WMAX + 15) / 16 + WP - 1) / WP;
     constexpr int REC = NCH * 64 + 32;
     const int nstages = a.C / (MM::kPerFrag * NCH);
     const double es = sizeof(T);
     npu_launch_plan p = make_plan("conv3x3_rows", grid.x * grid.y,
-                                  wg_per_cu(conv3x3_rows_kernel<MM, T, TR, WF, WMAX, NCH, NBUF, WFIX>),
+                                  wg_per_cu(conv3x3_rows_kernel<MM, T, WMAX, NCH, NBUF, WFIX>),
                                   grid.x * grid.y, 8 * sizeof(T));
     p.load_phases = 1;  // later stages are fetched while the previous one computes
     p.tile_macs = 4.0 * PBW * 256 * 9 * a.C;
@@ -1053,19 +1052,19 @@ hipError_t launch_rows(const ConvArgs &a, hipStream_t s) {
     // Otherwise: the first stages' halo and filter staging (260 f32, 400
     // bf16: twice the 16-byte runs), 41 per stage, the epilogue (bias,
     // activation, conversion and the stores of the tile's pixel blocks) 137.
-    constexpr bool WLDS = NBUF == 1 && WF == 1;
-    p.tile_valu = 4.0 * (WFIX > 0 && NBUF == 1 && TR == 1
-                             ? (WLDS ? (sizeof(T) == 4 && NCH == 4 ? 478.0 : 300.0) : 235.0)
+    constexpr bool WLDS = NBUF == 1;
+    p.tile_valu = 4.0 * (WFIX > 0 && NBUF == 1
+                             ? (sizeof(T) == 4 && NCH == 4 ? 478.0 : 300.0)
                              : (sizeof(T) == 4 ? 260.0 : 400.0) + 41.0 * nstages + 137.0);
     p.tile_lds_bytes = (TR + 2.0) * (a.W + 2) * REC * nstages + 4.0 * PBW * 9 * NCH * 1024 * nstages +
                        (WLDS ? 2.0 * 16 * 9 * a.C * es : 0.0);  // filters staged and read
     p.tile_load_bytes = (TR + 2.0) * (a.W + 2) * a.C * es + (WLDS ? 1.0 : 4.0) * 16 * 9 * a.C * es;
-    p.tile_store_bytes = (double)TR * a.W * 16 * WF * es;
+    p.tile_store_bytes = (double)TR * a.W * 16 * es;
     p.hbm_bytes = es * ((double)a.N * a.H * a.W * a.C + 9.0 * a.F * a.C + (double)a.N * a.H * a.W * a.F) +
                   (a.bias ? 4.0 * a.F : 0.0);
     plans_add(p);
   }
-  hipLaunchKernelGGL((conv3x3_rows_kernel<MM, T, TR, WF, WMAX, NCH, NBUF, WFIX>), grid, dim3(256), 0, s,
+  hipLaunchKernelGGL((conv3x3_rows_kernel<MM, T, WMAX, NCH, NBUF, WFIX>), grid, dim3(256), 0, s,
                      static_cast<const T *>(a.x), static_cast<const T *>(a.w), a.bias,
                      static_cast<T *>(a.out), a.H, a.W, a.C, a.F, a.act);
   return hipGetLastError();
@@ -1078,37 +1077,41 @@ hipError_t launch_persistent(const ConvArgs &a, hipStream_t s) {
   return launch_stream<MM, T, WMAX, NCH, WFIX>(a, g, s);
 }
 
-// Launch shapes.  With C of two or four chunks, F a multiple of 64 and at
-// least 48 row pairs (two 56-row images), a persistent kernel (filter
-// fragments held in registers): for f32 the one on the bf16 pipe (32 or 64
-// channels), for bf16 the stream kernel.  Its per-workgroup set-up (filters
-// loaded, for f32 split) costs about 2.5 us once, where the one-workgroup-per-
-// tile kernels refetch the filters and re-stage the halo per tile: on
-// 56x56x64 -> 64 those take 5.4 (f32) and 2.3 us (bf16) per further image,
-// the persistent kernels 1.1 and 0.3.  Else one workgroup per tile: 2 rows x
-// 64 filters (waves split the filters) when tiles are many, 1 row x 16
-// filters (waves split the row) when few, so the grid still spreads over the
-// CUs.  Rows of up to 56 pixels use tiles sized for 56 (7 pixel blocks for 2
-// rows, none wasted); a row width of exactly 56 is also compiled in, so
-// index arithmetic folds.
+// Launch shapes.  With F a multiple of 64 and at least 48 row pairs (two
+// 56-row images), a persistent kernel (filter fragments held in registers):
+// for f32 at 32 or 64 channels the one on the bf16 pipe, for bf16 at 64 the
+// stream kernel.  Its per-workgroup set-up (filters loaded, for f32 split)
+// costs about 2.5 us once, where the one-workgroup-per-tile kernel refetches
+// the filters and re-stages the halo per tile: on 56x56x64 -> 64 that takes
+// 5.4 (f32) and 2.3 us (bf16) per further image, the persistent kernels 1.1
+// and 0.3.  Else one workgroup per row and 16 filters, as long as each has a
+// CU of its own.  Every other shape runs on the pixel x filter tiles of
+// k_conv.hip.  Measured, us, here against those tiles: bf16 batch 32
+// 56x56x64 13.5 / 24.2; batch 1 56x56x64 (224 workgroups) 3.8 / 5.8, 14x14x96
+// (84) 5.3 / 7.9, 28x28x128 (224) 8.0 / 8.1; f32 batch 1 56x56x64 6.3 / 9.6,
+// batch 4 13.0 / 19.7, 14x14x160 (140) 16.9 / 18.7.  Past 256 workgroups, and
+// for the bf16 stream kernel with 128 channels, the tiles win: bf16 28x28x64 at
+// batch 4 (448) 7.8 / 5.9, 28x28x128 at batch 4 17.8 / 9.3 and at batch 32
+// 29.3 / 22.5; 14x14x256 at batch 32 249 / 26 (f32 498 / 105).  Rows of up to
+// 56 pixels use tiles sized for 56 (7 pixel blocks for 2 rows, none wasted); a
+// row width of exactly 56 is also compiled in, so index arithmetic folds.
+bool persistent_shape(const ConvArgs &a, int kc) {
+  return (long long)a.N * ((a.H + 1) / 2) >= 48 && a.F % 64 == 0 &&
+         (kc == 16 ? a.C == 32 || a.C == 64 : a.C == 64);
+}
+
 template <class MM, typename T, int WMAX, int WFIX>
 hipError_t launch_w(const ConvArgs &a, hipStream_t s) {
-  const int pairs = a.N * ((a.H + 1) / 2);
-  const bool big = pairs >= 512;
-  if (pairs >= 48 && a.F % 64 == 0) {
-    if constexpr (sizeof(T) == 4) {  // f32: on the bf16 pipe
-      if (a.C == 32) return launch_x6<WMAX, 1, WFIX>(a, s);
-      if (a.C == 64) return launch_x6<WMAX, 2, WFIX>(a, s);
-    } else {
-      if (a.C == 2 * MM::kPerFrag) return launch_persistent<MM, T, WMAX, 2, WFIX>(a, s);
-      if (a.C == 4 * MM::kPerFrag) return launch_persistent<MM, T, WMAX, 4, WFIX>(a, s);
-    }
+  if (persistent_shape(a, MM::kPerFrag)) {
+    if constexpr (sizeof(T) == 4)  // f32: on the bf16 pipe
+      return a.C == 32 ? launch_x6<WMAX, 1, WFIX>(a, s) : launch_x6<WMAX, 2, WFIX>(a, s);
+    else
+      return launch_persistent<MM, T, WMAX, 2, WFIX>(a, s);
   }
-  if (a.C == 2 * MM::kPerFrag)
-    return big ? launch_rows<MM, T, 2, 4, WMAX, 2, 1, WFIX>(a, s) : launch_rows<MM, T, 1, 1, WMAX, 2, 1, WFIX>(a, s);
+  if (a.C == 2 * MM::kPerFrag) return launch_rows<MM, T, WMAX, 2, 1, WFIX>(a, s);
   if constexpr (sizeof(T) == 4)
-    if (!big && a.C == 4 * MM::kPerFrag) return launch_rows<MM, T, 1, 1, WMAX, 4, 1, WFIX>(a, s);
-  return big ? launch_rows<MM, T, 2, 4, WMAX, 1, 2, WFIX>(a, s) : launch_rows<MM, T, 1, 1, WMAX, 1, 2, WFIX>(a, s);
+    if (a.C == 4 * MM::kPerFrag) return launch_rows<MM, T, WMAX, 4, 1, WFIX>(a, s);
+  return launch_rows<MM, T, WMAX, 1, 2, WFIX>(a, s);
 }
 
 template <class MM, typename T>
@@ -1121,7 +1124,8 @@ hipError_t launch_conv3x3(const ConvArgs &a, hipStream_t s) {
 
 bool conv3x3_rows_supported(const ConvArgs &a, int elem_bytes) {
   const int kc = 64 / elem_bytes;
-  return a.KH == 3 && a.KW == 3 && a.pad == 1 && a.W <= 64 && a.C % kc == 0 && a.F % 16 == 0;
+  if (!(a.KH == 3 && a.KW == 3 && a.pad == 1 && a.W <= 64 && a.C % kc == 0 && a.F % 16 == 0)) return false;
+  return persistent_shape(a, kc) || (long long)a.N * a.H * (a.F / 16) <= 256;
 }
 
 hipError_t launch_conv3x3_f32(const ConvArgs &a, hipStream_t s) {

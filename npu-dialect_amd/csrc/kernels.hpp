@@ -29,7 +29,8 @@ hipError_t launch_conv2d_nhwc_bf16(const ConvArgs &a, hipStream_t s);
 // and stride: ConvArgs with H/W/C/F as named, x [N,C,H,W], w [F,C,KH,KW],
 // out and res [N,F,Ho,Wo].
 hipError_t launch_conv2d_nchw_f32(const ConvArgs &a, hipStream_t s);
-// 3x3 / stride 1 / pad 1 with rows of at most 64 pixels: LDS halo kernel.
+// 3x3 / stride 1 / pad 1 with rows of at most 64 pixels, where the LDS halo
+// kernels are the fastest.
 bool conv3x3_rows_supported(const ConvArgs &a, int elem_bytes);
 hipError_t launch_conv3x3_f32(const ConvArgs &a, hipStream_t s);
 hipError_t launch_conv3x3_bf16(const ConvArgs &a, hipStream_t s);

@@ -1350,6 +1350,51 @@ def test_model_zoo_block_runs_on_the_gpu(cuda, C, M, final_relu):
                 what=f"model-zoo block C={C} M={M}")
 
 
+@pytest.mark.parametrize("N,H,W,C,F,KH,KW,pad,dtype,res", [
+    (3, 65, 64, 8, 128, 3, 3, 1, "bf16", True),    # 64x64 tiles, one run per tap, ragged pixels
+    (1, 157, 157, 72, 64, 1, 1, 0, "bf16", False),  # 64x64 tiles, a second chunk of one run
+    (2, 80, 81, 40, 70, 3, 3, 0, "bf16", True),    # 64x32 tiles, F % 4 != 0, no pad
+    (4, 80, 80, 20, 96, 3, 3, 1, "f32", True),     # 64x32 tiles, C of five runs
+    (1, 160, 156, 36, 61, 1, 3, 1, "f32", False),  # 64x64 tiles, a 1x3 filter, odd F, 64 + 16 bytes of channels
+    (1, 5, 4, 136, 33, 5, 5, 2, "bf16", True),     # 32x32 tiles, three chunks, 20 pixels
+    (2, 66, 70, 64, 24, 3, 3, 1, "f32", False),    # rows past 64 pixels, two chunks
+])
+def test_conv_tiles(cuda, N, H, W, C, F, KH, KW, pad, dtype, res):
+    """Edges of the NHWC conv's pixel x filter tiles: each tile size, ragged
+    pixels and filters, channel runs past C, vector and scalar epilogues."""
+    Ho, Wo = H + 2 * pad - KH + 1, W + 2 * pad - KW + 1
+    x = rng.uniform(51, 0, (N, H, W, C), -1, 1)
+    w = rng.normal(51, 1, (F, KH, KW, C), 0, math.sqrt(2 / (KH * KW * C)))
+    b = rng.uniform(51, 2, (F,), -0.1, 0.1)
+    r = rng.uniform(51, 3, (N, Ho, Wo, F), -1, 1) if res else None
+    if dtype == "bf16":
+        x, w = rng.to_bf16_bits(x), rng.to_bf16_bits(w)
+        r = None if r is None else rng.to_bf16_bits(r)
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    out = torch.full((N, Ho, Wo, F), float("nan"), dtype=tdt, device="cuda")
+    dev = configs.to_device({"x": x, "w": w, "b": b, "r": r})
+    if res:
+        groups.fused_conv2d_nhwc_bias_res_act(dev["x"], dev["w"], dev["b"], dev["r"], out, pad, "relu")
+    else:
+        groups.fused_conv2d_nhwc_bias_act(dev["x"], dev["w"], dev["b"], out, pad, "relu")
+    torch.cuda.synchronize()
+    got = configs.to_host(out)
+    if dtype == "bf16":
+        x, w = bf16(x), bf16(w)
+        r = None if r is None else bf16(r)
+    t = lambda v: torch.from_numpy(np.ascontiguousarray(v)).double()
+    conv = lambda x, w: torch.nn.functional.conv2d(t(x).permute(0, 3, 1, 2), t(w).permute(0, 3, 1, 2),
+                                                   padding=pad).permute(0, 2, 3, 1).numpy()
+    ref, mag = conv(x, w) + b, conv(np.abs(x), np.abs(w)) + np.abs(b)
+    if res:
+        ref, mag = ref + r, mag + np.abs(r)
+    ref = np.maximum(ref, 0)
+    if dtype == "bf16":
+        check_bf16_rounded(got, ref, mag, KH * KW * C + 2, what="conv tiles")
+    else:
+        check_bound(got, ref, mag, RTOL_F32, what="conv tiles")
+
+
 @pytest.mark.parametrize("N,H,W,C,F,dtype", [(2, 9, 13, 24, 40, "f32"), (1, 7, 7, 48, 24, "bf16")])
 def test_conv_residual_and_odd_channels(cuda, N, H, W, C, F, dtype):
     """fused_conv2d_nhwc_bias_res_act with channel counts that are not a
