@@ -38,15 +38,6 @@ namespace npu {
 
 namespace {
 
-// Division of v < 2^16 by d < 2^16 as a multiply: q = (v * m) >> 32 with
-// m = ceil(2^32 / d) (the error v * (m d - 2^32) / (d 2^32) < 2^-16 cannot
-// carry past the next multiple); d = 1 takes v itself.
-struct FastDiv {
-  uint32_t d, m;
-  explicit FastDiv(int dv = 1) : d((uint32_t)dv), m(dv > 1 ? (uint32_t)(((1ULL << 32) + dv - 1) / dv) : 0u) {}
-  __device__ __forceinline__ int div(int v) const { return d == 1 ? v : (int)__umulhi((uint32_t)v, m); }
-};
-
 struct NchwArgs {
   const float *x, *w, *bias, *res;
   float *out;

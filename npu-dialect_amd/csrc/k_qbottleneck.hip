@@ -23,6 +23,8 @@
 // accumulator holds four consecutive output channels of one pixel.  Integer
 // accumulation is exact, so any summation order gives the oracle's result bit
 // for bit.
+#include <type_traits>
+
 #include "kernels.hpp"
 #include "npu_device.hpp"
 #include "persistent.hpp"
@@ -300,24 +302,425 @@ hipError_t launch_qb(const QBottleneckArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Any C and M1 that are multiples of 64, C <= 2048 and M1 <= 512 (ResNet-50's
-// later stages: 512/128, 1024/256, 2048/512), for the counts the tuned
-// instances above do not cover.  Every filter block is read from L2 where it
-// is used, so nothing scales the registers with the channel counts.  A
-// workgroup walks 4 x 4 output tiles; per tile: the x halo (6 x 6 pixels, all
-// C channels, zero outside the image) to LDS; conv1 on the halo, one unit =
-// 16 output channels x 16 halo pixels, requant + ReLU clamp into y1 (zero
-// outside the image: the pad before conv2); conv2, one unit = 16 channels of
-// the 16 output pixels, into y2; conv3, one unit = 16 output channels, with
-// requant, the residual from the halo and the clamp, stored.  The units of a
-// phase are dealt round-robin over the four waves, one barrier per phase.
-__global__ __launch_bounds__(256, 1) void qb_stream_kernel(
+// Large filters (launch_qbottleneck_i8: ResNet-50's 512/128, 1024/256 and
+// 2048/512): any C <= 2048 and M1 <= 512 that are multiples of 64, M1 >= 128.
+// Sixteen waves walk 4 x 7 output tiles (6 x 9 halo pixels); y1 and y2 stay in
+// LDS.  Each of the three convolutions is a matrix product that streams its
+// filters through LDS in chunks of 256 rows of 128 bytes (KP = 1), or, for
+// M1 = 128, of 128 rows of two such runs (KP = 2), conv1 its halo pixels'
+// channels with them; two LDS buffers, two more chunks in registers, one
+// barrier per chunk.  conv3 goes 256 output channels at a time: the residual's
+// tile is staged in LDS, finished in place and stored in 16-byte runs while the
+// next channels are multiplied.
+//
+// Filter chunks lie unpadded, the 16-byte piece p of row f at p ^ (f / 2 % 8),
+// so that 16 rows' reads and a row's writes use every bank once.
+//
+// What bounds it: the instructions around each chunk's four MFMAs per wave
+// (about 1 700 clocks a chunk, 34 chunks a tile at 1024/256).  Loaded straight as
+// MFMA fragments, 16 rows of 64 bytes per instruction, the filters cost the CU's
+// load path 70 clocks per KB (60 us at 1024/256); one chunk in registers instead
+// of two 38.4 us.  Measured, batch 32, us, before (4 x 4 tiles, fragments from
+// L2) and now: 14x14x1024/256 122 -> 36.3, 28x28x512/128 133 -> 68,
+// 7x7x2048/512 367 -> 101.
+constexpr int STH = 4, STW = 7, SHW = STW + 2, SHP = SHW * (STH + 2);  // 54 halo pixels
+constexpr int SOP = STH * STW;                                         // 28 output pixels
+constexpr int SNT = 1024, SROWS = 256;                                 // lanes, filter rows of a chunk
+constexpr int SOS = SROWS + 16;                                        // output tile row (bytes)
+
+struct QStreamArgs {
+  const int8_t *x, *w1, *w2, *w3;
+  const int32_t *m1, *s1, *m2, *s2, *m3, *s3;
+  int8_t *out;
+  int H, W, C, M1, tiles_w, tiles_img, ntiles;
+  FastDiv by_mk;
+};
+
+template <int KP>
+struct QStreamShape {
+  static constexpr int NF1 = 2, NP1 = KP == 1 ? 2 : 1, NF2 = KP == 1 ? 2 : 1;
+  static constexpr int XS = KP * 128 + 32;            // x chunk row: 32 mod 64 bytes
+  static constexpr int XBUF = SHP * XS, XR = (SHP * 8 * KP + SNT - 1) / SNT;
+  static constexpr int NOB = 2;                       // output tiles in LDS
+  static constexpr int FBUF = SROWS * 128;
+  static_assert(NOB * SOP * SOS <= 2 * XBUF, "output tiles fit the x chunks' space");
+  static size_t lds(int M1) { return 2 * FBUF + 2 * XBUF + (size_t)(SHP + 32) * (M1 + 32); }
+};
+
+template <int KP>
+__global__ __launch_bounds__(SNT, 4) void qb_stream_kernel(const QStreamArgs a) {
+  using S = QStreamShape<KP>;
+  constexpr int NF1 = S::NF1, NP1 = S::NP1, NF2 = S::NF2, XS = S::XS, XR = S::XR;
+  extern __shared__ __attribute__((aligned(16))) int8_t qmem[];
+  int8_t *const fbuf = qmem;                     // [2][SROWS][128]
+  int8_t *const xbuf = fbuf + 2 * S::FBUF;       // [2][SHP][XS]; conv3: [NOB][SOP][SOS]
+  int8_t *const y1 = xbuf + 2 * S::XBUF;         // [SHP][YS]
+  const int C = a.C, M1 = a.M1, YS = M1 + 32;
+  int8_t *const y2 = y1 + SHP * YS;              // [32][YS]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int R = min(M1, SROWS), rg = (M1 + R - 1) / R, mk = M1 / 64;  // filter rows of a chunk, row groups
+  // k chunks of a row group, made even (an odd count's last chunk is empty):
+  // chunks go by pairs, each with its own LDS buffer and registers
+  const int kc1 = (C + 256 * KP - 1) / (256 * KP) * 2, kc2 = (9 * M1 + 256 * KP - 1) / (256 * KP) * 2;
+  const int kc3 = (M1 + 255) / 256 * 2, rg3 = (C + SROWS - 1) / SROWS;
+
+  // ---- filter chunks: this thread's 16-byte piece `piece` of slots srow and
+  //      srow + 128 (slot = kpart R + row).  Rows and k past the end load
+  //      from clamped addresses; the first are not stored, the second skipped.
+  const int piece = tid & 7, srow = tid >> 3;
+  const int fdst0 = srow * 128 + 16 * (piece ^ ((srow >> 1) & 7)), fdst1 = fdst0 + 128 * 128;
+  struct Pair {
+    u32x4 lo, hi;
+  } fr0, fr1;  // of the even and the odd chunks
+  auto commit = [&](int buf, const Pair &f) __attribute__((always_inline)) {
+    *reinterpret_cast<u32x4 *>(fbuf + buf * S::FBUF + fdst0) = f.lo;
+    *reinterpret_cast<u32x4 *>(fbuf + buf * S::FBUF + fdst1) = f.hi;
+  };
+  // filter fragment: slot row f (= r mod 16), 64-byte step h of its 128 bytes
+  const int sw = (r >> 1) & 7;
+  auto ffrag = [&](int buf, int f, int h) __attribute__((always_inline)) {
+    return load16(fbuf + buf * S::FBUF + f * 128 + 16 * ((4 * h + q) ^ sw));
+  };
+  // chunk i of the tile's walk over conv1's, conv2's and conv3's chunks
+  const int n1 = rg * kc1, n2 = n1 + rg * kc2, n3 = n2 + rg3 * kc3;
+  // the chunk to fetch next: its place in the walk, its filters' rows, bytes
+  // per row, rows per chunk, k chunks and bytes of k per chunk
+  int fi, fk, fg, f_rows, f_kbytes, f_rper, f_kcn, f_kstep;
+  const int8_t *f_w;
+  auto fetch_start = [&]() __attribute__((always_inline)) {
+    fi = fk = fg = 0;
+    f_w = a.w1, f_rows = M1, f_kbytes = C, f_rper = R, f_kcn = kc1, f_kstep = 128 * KP;
+  };
+  auto fetch_next = [&](Pair &f) __attribute__((always_inline)) {
+    const int kp0 = KP == 1 ? 0 : srow / f_rper, kp1 = KP == 1 ? 0 : (srow + 128) / f_rper;
+    const int row0 = min(fg * f_rper + srow - kp0 * f_rper, f_rows - 1), kb0 = fk * f_kstep + kp0 * 128 + piece * 16;
+    const int row1 = min(fg * f_rper + srow + 128 - kp1 * f_rper, f_rows - 1), kb1 = fk * f_kstep + kp1 * 128 + piece * 16;
+    f.lo = *reinterpret_cast<const u32x4 *>(f_w + (row0 * f_kbytes + (kb0 < f_kbytes ? kb0 : 0)));
+    f.hi = *reinterpret_cast<const u32x4 *>(f_w + (row1 * f_kbytes + (kb1 < f_kbytes ? kb1 : 0)));
+    if (fi + 1 < n3) {
+      ++fi;
+      if (++fk == f_kcn) fk = 0, ++fg;
+      if (fi == n1) {
+        fg = 0;
+        f_w = a.w2, f_kbytes = 9 * M1, f_kcn = kc2;
+      } else if (fi == n2) {
+        fg = 0;
+        f_w = a.w3, f_rows = C, f_kbytes = M1, f_rper = SROWS, f_kcn = kc3, f_kstep = 128;
+      }
+    }
+  };
+  struct Mul4 {
+    i32x4 m, s;
+  };
+  auto load_params = [&](const int32_t *m, const int32_t *sh, int c) __attribute__((always_inline)) {
+    return Mul4{*reinterpret_cast<const i32x4 *>(m + c), *reinterpret_cast<const i32x4 *>(sh + c)};
+  };
+  auto scale = [&](const Mul4 &p) __attribute__((always_inline)) {
+    Scale4 sc;
+    sc.m = p.m;
+    sc.s = p.s;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sc.r[e] = 1LL << (p.s[e] - 1);
+    return sc;
+  };
+
+  const TileWalk walk = tile_walk(a.ntiles);
+  for (int t = walk.first; t < walk.end; t += walk.step) {
+    const int n = t / a.tiles_img, tt = t - n * a.tiles_img;
+    const int ty0 = (tt / a.tiles_w) * STH, tx0 = (tt - (tt / a.tiles_w) * a.tiles_w) * STW;
+    const int8_t *const xn = a.x + (size_t)n * a.H * a.W * C;
+    // x chunks: run `e` of the 8 KP 16-byte runs of each halo pixel, clamped into
+    // the image (what lies outside only feeds y1 values that are zeroed)
+    int xoff[XR], xdst[XR], xkb[XR];
+#pragma unroll
+    for (int j = 0; j < XR; ++j) {
+      const int e = min(opaque(tid) + SNT * j, SHP * 8 * KP - 1), hp = e / (8 * KP), hy = hp / SHW, hx = hp - hy * SHW;
+      const int iy = min(max(ty0 + hy - 1, 0), a.H - 1), ix = min(max(tx0 + hx - 1, 0), a.W - 1);
+      xkb[j] = (e - hp * 8 * KP) * 16;
+      xoff[j] = (iy * a.W + ix) * C;
+      xdst[j] = hp * XS + xkb[j];
+    }
+    u32x4 xr0[XR], xr1[XR];
+    auto xfetch = [&](int k, u32x4 (&xr)[XR]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < XR; ++j) {
+        const int kb = k * 128 * KP + xkb[j];
+        xr[j] = *reinterpret_cast<const u32x4 *>(xn + (xoff[j] + (kb < C ? kb : 0)));
+      }
+    };
+    auto xcommit = [&](int buf, const u32x4 (&xr)[XR]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < XR; ++j) *reinterpret_cast<u32x4 *>(xbuf + buf * S::XBUF + xdst[j]) = xr[j];
+    };
+    fetch_start();
+    fetch_next(fr0);
+    xfetch(0, xr0);
+    fetch_next(fr1);
+    xfetch(1, xr1);
+    commit(0, fr0);
+    xcommit(0, xr0);
+    fetch_next(fr0);
+    xfetch(kc1 > 2 ? 2 : 0, xr0);
+    __syncthreads();
+
+    // ---- conv1 on the halo: requant + ReLU clamp into y1, zero outside the image
+    {
+      // recomputed per tile: hoisted out of the tile loop, every phase's
+      // addresses would be held at once
+      const int ol = opaque(lane), r = ol & 15, q = ol >> 4;
+      constexpr int FGW = KP == 1 ? 8 : 4;  // waves along the filters
+      const int fw = wave % FGW * 16 * NF1, pw = wave / FGW * NP1;
+      int px[NP1];
+#pragma unroll
+      for (int p = 0; p < NP1; ++p) px[p] = min((pw + p) * 16 + r, SHP - 1) * XS + 16 * q;
+      for (int g = 0; g < rg; ++g) {
+        i32x4 acc[NF1][NP1] = {};
+        auto chunk = [&](int k, auto odd) __attribute__((always_inline)) {
+          constexpr bool ODD = decltype(odd)::value;
+          constexpr int buf = ODD;
+          // the next chunk to LDS, the one three ahead on its way
+          commit(buf ^ 1, ODD ? fr0 : fr1);
+          fetch_next(ODD ? fr0 : fr1);
+          xcommit(buf ^ 1, ODD ? xr0 : xr1);
+          // chunk (k + 3) mod kc1 of this row group or the next (kc1 >= 2)
+          xfetch(k + 3 < kc1 ? k + 3 : k + 3 < 2 * kc1 ? k + 3 - kc1 : k + 3 - 2 * kc1, ODD ? xr0 : xr1);
+          const int steps = min(2 * KP, C / 64 - k * 2 * KP);
+#pragma unroll
+          for (int s = 0; s < 2 * KP; ++s)
+            if (s < steps) {  // uniform
+              Frag16 f[NF1];
+#pragma unroll
+              for (int b = 0; b < NF1; ++b) f[b] = ffrag(buf, (s >> 1) * R + fw + 16 * b + r, s & 1);
+#pragma unroll
+              for (int p = 0; p < NP1; ++p) {
+                const Frag16 v = load16(xbuf + buf * S::XBUF + px[p] + s * 64);
+#pragma unroll
+                for (int b = 0; b < NF1; ++b) MfmaI8::mma(acc[b][p], f[b], v);
+              }
+            }
+          if constexpr (ODD) {
+           if (k + 1 == kc1) {
+#pragma unroll
+            for (int b = 0; b < NF1; ++b) {
+              const int f0 = g * R + fw + 16 * b;
+              const Scale4 s4 = scale(load_params(a.m1, a.s1, min(f0, M1 - 16) + 4 * q));
+#pragma unroll
+              for (int p = 0; p < NP1; ++p) {
+                const int hp = (pw + p) * 16 + r, hy = hp / SHW, hx = hp - hy * SHW;
+                const bool inside = (unsigned)(ty0 + hy - 1) < (unsigned)a.H && (unsigned)(tx0 + hx - 1) < (unsigned)a.W;
+                const uint32_t v = requant4(acc[b][p], s4);
+                if (hp < SHP && fw + 16 * b < R && f0 < M1)
+                  *reinterpret_cast<uint32_t *>(y1 + hp * YS + f0 + 4 * q) = inside ? v : 0u;
+                __builtin_amdgcn_sched_barrier(0);  // one block's 64-bit values at a time
+              }
+            }
+          }
+          }
+          __syncthreads();
+        };
+        for (int k = 0; k < kc1; k += 2) {
+          chunk(k, std::false_type{});
+          chunk(k + 1, std::true_type{});
+        }
+      }
+    }
+
+    // the residual's tile of 256 channels, one group ahead: this thread's
+    // 16-byte run, its place in the tile and in the image (recomputed at each use)
+    u32x4 rr;
+    auto rplace = [&](int &lds, int &off, int &c) __attribute__((always_inline)) {
+      const int rt = opaque(tid), o = min(rt >> 4, SOP - 1), oy = o / STW, ox = o - oy * STW;
+      c = (rt & 15) * 16;
+      lds = o * SOS + c;
+      const bool in = rt < SOP * 16 && ty0 + oy < a.H && tx0 + ox < a.W;
+      off = in ? ((ty0 + oy) * a.W + tx0 + ox) * C : 0;
+      return in;
+    };
+    auto rfetch = [&](int g) __attribute__((always_inline)) {
+      int lds, off, c;
+      rplace(lds, off, c);
+      c += g * SROWS;
+      rr = *reinterpret_cast<const u32x4 *>(xn + (off + (c < C ? c : 0)));
+    };
+    auto rcommit = [&](int g) __attribute__((always_inline)) {
+      int lds, off, c;
+      rplace(lds, off, c);
+      if (tid < SOP * 16) *reinterpret_cast<u32x4 *>(xbuf + (g % S::NOB) * SOP * SOS + lds) = rr;
+    };
+
+    // ---- conv2 (3x3) on the output pixels, k steps tap by tap
+    {
+      const int ol = opaque(lane), r = ol & 15, q = ol >> 4;
+      constexpr int FGW = 8;
+      const int fw = wave % FGW * 16 * NF2, pw = wave / FGW;
+      const int o = min(pw * 16 + r, SOP - 1), oy = o / STW;
+      const int px = (oy * SHW + o - oy * STW) * YS + 16 * q;
+      const bool on = fw < R;  // uniform
+      for (int g = 0; g < rg; ++g) {
+        i32x4 acc[NF2] = {};
+        Mul4 sc[NF2];
+#pragma unroll
+        for (int b = 0; b < NF2; ++b) sc[b] = load_params(a.m2, a.s2, min(g * R + fw + 16 * b, M1 - 16) + 4 * q);
+        auto chunk = [&](int k, auto odd) __attribute__((always_inline)) {
+          constexpr bool ODD = decltype(odd)::value;
+          constexpr int buf = ODD;
+          commit(buf ^ 1, ODD ? fr0 : fr1);
+          fetch_next(ODD ? fr0 : fr1);
+          if (g + 1 == rg && k + (ODD ? 1 : 2) == kc2) {  // the last pair
+            if constexpr (ODD) rcommit(0);
+            rfetch(ODD && rg3 > 1 ? 1 : 0);
+          }
+          const int ks = k * 2 * KP, steps = on ? min(2 * KP, 9 * mk - ks) : 0;
+#pragma unroll
+          for (int s = 0; s < 2 * KP; ++s)
+            if (s < steps) {
+              const int tap = a.by_mk.div(ks + s), kh = tap / 3;
+              const Frag16 v = load16(y1 + px + (kh * SHW + tap - 3 * kh) * YS + (ks + s - tap * mk) * 64);
+#pragma unroll
+              for (int b = 0; b < NF2; ++b)
+                MfmaI8::mma(acc[b], ffrag(buf, (s >> 1) * R + fw + 16 * b + r, s & 1), v);
+            }
+          if constexpr (ODD) {
+            if (k + 1 == kc2 && on) {
+#pragma unroll
+              for (int b = 0; b < NF2; ++b)
+                if (fw + 16 * b < R && g * R + fw + 16 * b < M1)
+                  *reinterpret_cast<uint32_t *>(y2 + (pw * 16 + r) * YS + g * R + fw + 16 * b + 4 * q) =
+                      requant4(acc[b], scale(sc[b]));
+            }
+          }
+          __syncthreads();
+        };
+        for (int k = 0; k < kc2; k += 2) {
+          chunk(k, std::false_type{});
+          chunk(k + 1, std::true_type{});
+        }
+      }
+    }
+
+    // ---- conv3 + requant + residual + clamp, 256 channels at a time
+    {
+      const int ol = opaque(lane), r = ol & 15, q = ol >> 4;
+      const int fw = wave % 8 * 32, pw = wave / 8, o = pw * 16 + r;
+      const int px = o * YS + 16 * q;
+      auto store = [&](int g) __attribute__((always_inline)) {
+        int lds, off, c;
+        const bool in = rplace(lds, off, c);
+        if (in && g * SROWS + c < C)
+          *reinterpret_cast<u32x4 *>(a.out + (size_t)n * a.H * a.W * C + (off + g * SROWS + c)) =
+              *reinterpret_cast<const u32x4 *>(xbuf + (g % S::NOB) * SOP * SOS + lds);
+      };
+      for (int g = 0; g < rg3; ++g) {
+        i32x4 acc[2] = {};
+        Mul4 sc[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) sc[b] = load_params(a.m3, a.s3, min(g * SROWS + fw + 16 * b, C - 16) + 4 * q);
+        auto chunk = [&](int k, auto odd) __attribute__((always_inline)) {
+          constexpr bool ODD = decltype(odd)::value;
+          constexpr int buf = ODD;
+          commit(buf ^ 1, ODD ? fr0 : fr1);
+          fetch_next(ODD ? fr0 : fr1);
+          if (k == 0 && g > 0) store(g - 1);
+          const int steps = min(2, mk - 2 * k);
+#pragma unroll
+          for (int s = 0; s < 2; ++s)
+            if (s < steps) {
+              const Frag16 v = load16(y2 + px + (2 * k + s) * 64);
+#pragma unroll
+              for (int b = 0; b < 2; ++b) MfmaI8::mma(acc[b], ffrag(buf, fw + 16 * b + r, s), v);
+            }
+          if constexpr (ODD) {
+           if (k + 1 == kc3) {
+            int8_t *const ob = xbuf + (g % S::NOB) * SOP * SOS + o * SOS;
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+              if (o < SOP) {
+                const Scale4 s4 = scale(sc[b]);
+                uint32_t *slot = reinterpret_cast<uint32_t *>(ob + fw + 16 * b + 4 * q);
+                const uint32_t res = *slot;
+                uint32_t packed = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  const int v = requant(acc[b][e], s4.m[e], s4.r[e], s4.s[e]) + (int)(int8_t)(res >> (8 * e));
+                  packed |= (uint32_t)clamp_i(v, 0, 127) << (8 * e);
+                }
+                *slot = packed;
+              }
+            }
+            if (g + 1 < rg3) {
+              rcommit(g + 1);
+              if (g + 2 < rg3) rfetch(g + 2);
+            }
+          }
+          }
+          __syncthreads();
+        };
+        for (int k = 0; k < kc3; k += 2) {
+          chunk(k, std::false_type{});
+          chunk(k + 1, std::true_type{});
+        }
+      }
+      store(rg3 - 1);
+    }
+    __syncthreads();  // the buffers are the next tile's
+  }
+}
+
+template <int KP>
+hipError_t launch_qb_stream(const QBottleneckArgs &c, hipStream_t s) {
+  using S = QStreamShape<KP>;
+  auto kern = qb_stream_kernel<KP>;
+  QStreamArgs a{c.x, c.w1, c.w2, c.w3, c.m1, c.s1, c.m2, c.s2, c.m3, c.s3, c.out, c.H, c.W, c.C, c.M1,
+                (c.W + STW - 1) / STW, 0, 0, FastDiv(c.M1 / 64)};
+  a.tiles_img = a.tiles_w * ((c.H + STH - 1) / STH);
+  a.ntiles = c.N * a.tiles_img;
+  const size_t lds = S::lds(c.M1);
+  if (lds > 160 * 1024) return hipErrorInvalidValue;
+  const int cus = cached_per_kernel(reinterpret_cast<const void *>(kern), [&](int dev) {
+    int n = 0;
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess &&
+                   hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess
+               ? n : 0;
+  });
+  if (cus <= 0) return hipErrorInvalidValue;
+  const int full = cus / kXcds * kXcds;  // one workgroup per CU: its LDS
+  const int grid = a.ntiles < full ? (a.ntiles + kXcds - 1) / kXcds * kXcds : full;
+  {
+    npu_launch_plan p = make_plan("int8_bottleneck_stream", grid, 4, a.ntiles, 8);
+    p.unit_waves = 16;
+    p.load_phases = 1;  // the first chunk; later ones are in flight ahead of their use
+    const double wbytes = 2.0 * c.M1 * c.C + 9.0 * c.M1 * c.M1;
+    p.tile_macs = 64.0 * c.M1 * c.C + 32.0 * 9 * c.M1 * c.M1 + 32.0 * c.C * c.M1;
+    p.tile_valu = 16.0 * (60.0 + 30.0 * wbytes / 32768 + 20.0 * (64.0 * c.M1 + 32.0 * c.M1 + 32.0 * c.C) / 16 / 64 / 4);
+    p.tile_lds_bytes = wbytes + 2.0 * SHP * c.C + 2.0 * p.tile_macs / 16.0 / 16.0 / 64.0 * 1024;
+    p.tile_load_bytes = (double)(SHP + SOP) * c.C + wbytes;
+    p.tile_store_bytes = (double)SOP * c.C;
+    p.hbm_bytes = 2.0 * c.N * c.H * c.W * c.C + wbytes + 4.0 * 2 * (2 * c.M1 + c.C);
+    plans_add(p);
+  }
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(SNT), lds, s, a);
+  return hipGetLastError();
+}
+
+// Small filters that the tuned instances above do not cover (M1 = 64, or
+// M1 = 128 with few channels): every filter block is read from L2 where it is
+// used, so nothing scales the registers with the channel counts.  A workgroup
+// walks 4 x 4 output tiles; per tile: the x halo (6 x 6 pixels, all C channels,
+// zero outside the image) to LDS; conv1 on the halo, one unit = 16 output
+// channels x 16 halo pixels, requant + ReLU clamp into y1 (zero outside the
+// image: the pad before conv2); conv2, one unit = 16 channels of the 16 output
+// pixels, into y2; conv3, one unit = 16 output channels, with requant, the
+// residual from the halo and the clamp, stored.  The units of a phase are dealt
+// round-robin over the four waves, one barrier per phase.
+__global__ __launch_bounds__(256, 1) void qb_direct_kernel(
     const int8_t *__restrict__ x, const int8_t *__restrict__ w1, const int8_t *__restrict__ w2,
     const int8_t *__restrict__ w3, const int32_t *__restrict__ m1, const int32_t *__restrict__ s1,
     const int32_t *__restrict__ m2, const int32_t *__restrict__ s2,
     const int32_t *__restrict__ m3, const int32_t *__restrict__ s3, int8_t *__restrict__ out,
     int H, int W, int C, int M1, int tiles_w, int tiles_img, int ntiles) {
-  constexpr int SHW = 6, SHP = 36, SHPB = 3, CMAX = 2048, MMAX = 512;
+  constexpr int SHW = 6, SHP = 36, SHPB = 3, CMAX = 2048, MMAX = 128;
   __shared__ __attribute__((aligned(16))) int8_t xs[SHP * (CMAX + 32)];
   __shared__ __attribute__((aligned(16))) int8_t y1[SHPB * 16 * (MMAX + 32)];
   __shared__ __attribute__((aligned(16))) int8_t y2[16 * (MMAX + 32)];
@@ -393,13 +796,13 @@ __global__ __launch_bounds__(256, 1) void qb_stream_kernel(
   }
 }
 
-hipError_t launch_qb_stream(const QBottleneckArgs &a, hipStream_t s) {
+hipError_t launch_qb_direct(const QBottleneckArgs &a, hipStream_t s) {
   const int tiles_w = (a.W + 3) / 4, tiles_img = tiles_w * ((a.H + 3) / 4), ntiles = a.N * tiles_img;
-  const int full = persistent_grid(qb_stream_kernel);
+  const int full = persistent_grid(qb_direct_kernel);
   if (full <= 0) return hipErrorInvalidValue;
   const int grid = ntiles < full ? (ntiles + kXcds - 1) / kXcds * kXcds : full;
   {
-    npu_launch_plan p = make_plan("int8_bottleneck_stream", grid, wg_per_cu(qb_stream_kernel), ntiles, 8);
+    npu_launch_plan p = make_plan("int8_bottleneck_direct", grid, wg_per_cu(qb_direct_kernel), ntiles, 8);
     p.load_phases = 4;  // the halo, then each phase's filters from L2
     p.tile_macs = 48.0 * a.M1 * a.C + 16.0 * 9 * a.M1 * a.M1 + 16.0 * a.C * a.M1;
     p.tile_valu = 4.0 * (40.0 + 30.0 * (3 * a.M1 / 16 + a.M1 / 16 + a.C / 16) / 4.0);
@@ -411,7 +814,7 @@ hipError_t launch_qb_stream(const QBottleneckArgs &a, hipStream_t s) {
                   4.0 * 2 * (2 * a.M1 + a.C);
     plans_add(p);
   }
-  hipLaunchKernelGGL(qb_stream_kernel, dim3(grid), dim3(256), 0, s, a.x, a.w1, a.w2, a.w3, a.m1,
+  hipLaunchKernelGGL(qb_direct_kernel, dim3(grid), dim3(256), 0, s, a.x, a.w1, a.w2, a.w3, a.m1,
                      a.s1, a.m2, a.s2, a.m3, a.s3, a.out, a.H, a.W, a.C, a.M1, tiles_w, tiles_img,
                      ntiles);
   return hipGetLastError();
@@ -432,7 +835,13 @@ hipError_t launch_qbottleneck_i8(const QBottleneckArgs &a, hipStream_t s) {
   if (a.C == 128 && a.M1 == 64) return launch_qb<128, 64>(a, s);
   if (a.C == 64 && a.M1 == 64) return launch_qb<64, 64>(a, s);
   if (!qbottleneck_supported(a.C, a.M1)) return hipErrorInvalidValue;
-  return launch_qb_stream(a, s);
+  // Filters streamed through LDS from 256 KB on.  Measured, us, streamed / read
+  // from L2: 512/128 (279 KB) one 14x14 image 17.7 / 20.4, batch 32 of 7x7
+  // 18.1 / 20.5; 192/192 (406 KB) 17.9 / 19.7; 1024/256 (1.1 MB) one 7x7 image
+  // 30.7 / 59.6; 320/128 (229 KB) 17.5 / 15.3; 320/64 (78 KB) 14.4 / 9.2.
+  if (a.M1 >= 128 && 2 * a.M1 * a.C + 9 * a.M1 * a.M1 >= 256 * 1024)
+    return a.M1 >= 192 ? launch_qb_stream<1>(a, s) : launch_qb_stream<2>(a, s);
+  return launch_qb_direct(a, s);
 }
 
 }  // namespace npu

@@ -481,9 +481,9 @@ def _qb_wide_inputs(N, H, W, C, M1, seed):
     (8, 20, 20, 64, 192),    # more tiles than resident workgroups
 ])
 def test_c4_qbottleneck_any_channels(cuda, N, H, W, C, M1):
-    """(C, M1) outside the tuned instances run on the kernel that reads its
-    filter blocks from L2 where they are used: bit for bit against the
-    oracle, with most requantized values off the clamp bounds."""
+    """(C, M1) outside the tuned instances, whose filters stream through LDS
+    or are read from L2 where they are used: bit for bit against the oracle,
+    with most requantized values off the clamp bounds."""
     inp = _qb_wide_inputs(N, H, W, C, M1, 90 + C // 64)
     print(f"qbottleneck stream {N}x{H}x{W}x{C}/{M1}", flush=True)
     ref = oracle.block_qbottleneck(**inp)
@@ -508,6 +508,23 @@ def test_c3_irb_config_n32(cuda):
         ref, mag = refs.reference(w.name, arrs)["out"]
     check_bound(out["out"], ref, mag, RTOL_F32, what=w.name)
     assert np.isfinite(out["out"]).all()
+
+
+@pytest.mark.parametrize("N,H,W,C,M1", [
+    (1, 2, 3, 448, 128),     # two runs per filter row, an image inside one tile, C off 256
+    (2, 9, 15, 704, 128),    # ragged tiles, the last conv1 chunk partial, C % 256 = 192
+    (1, 5, 8, 256, 192),     # one run per row, 192 of 256 rows, an odd count of conv3 chunks
+    (1, 6, 7, 64, 320),      # two row groups, the second of 64 rows; one conv1 step
+    (1, 4, 14, 2048, 512),   # the largest channel counts
+    (10, 28, 28, 512, 128),  # more tiles than CUs: a second tile per workgroup
+])
+def test_c4_qbottleneck_streamed_filters(cuda, N, H, W, C, M1):
+    """The int8 bottleneck whose filters stream through LDS: bit-exact at the
+    edges of its tiles, chunks and row groups."""
+    inp = _qb_wide_inputs(N, H, W, C, M1, 110 + C // 64)
+    with oracle.threaded():
+        ref = oracle.block_qbottleneck(**inp)
+    assert np.array_equal(_qb_run(inp), ref)
 
 
 @pytest.mark.parametrize("N,H,W,C,E", [
