@@ -389,6 +389,184 @@ __global__ __launch_bounds__(GT) void llama_gemm_kernel(const LlamaGemmArgs a, i
   }
 }
 
+// ---- long sequences: BM x BN tiles of 2 x 2 waves, K in steps of 64 -------------
+//
+// The shapes above give a tile to 16 waves and, for the RMSNorm GEMMs, keep its
+// whole A panel in LDS: right for one tile per CU, but at S = 2048 they reached
+// 134 TFLOP/s.  Here a wave holds a (BM / 2) x (BN / 2) part of the tile (per
+// weight), A and B stream through two LDS buffers, one barrier per step, the
+// next step's loads in flight, two workgroups per CU.  The RMSNorm is folded in
+// without a pass of its own: A is staged as bf16(x g) -- one rounding, as
+// bf16(x inv g) has -- while the same registers feed the row's sum of squares,
+// and the accumulator is scaled by the row's inv in f32 at the end.
+template <int EPI, int BM, int BN>
+struct TileShape {
+  static constexpr int NB = EPI == kEpiSwiglu ? 2 : 1, KC = 64;
+  static constexpr int TM = BM / 32, TN = BN / 32;               // MFMA blocks of a wave (per weight)
+  static constexpr int AREC = KC * 2 + 32, SB = KC * 32 + 32;    // A row, B strip (bytes)
+  static constexpr int STRIPS = BN / 16, ABYTES = BM * AREC;
+  static constexpr int BUF = ABYTES + NB * STRIPS * SB;
+  static constexpr int AR = BM / 32, BR = NB * BN / 32;          // 16-byte runs per thread and step
+};
+
+template <int PRO, int EPI, int BM, int BN>
+__global__ __launch_bounds__(256, 2) void llama_tile_kernel(const LlamaGemmArgs a, int tiles_m,
+                                                            int tiles_n, int xm) {
+  using S = TileShape<EPI, BM, BN>;
+  constexpr int NB = S::NB, TM = S::TM, TN = S::TN, KC = S::KC, AR = S::AR, BR = S::BR;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ float inv_s[PRO == kProRmsnorm ? BM : 1];
+  int tm, tn;
+  if (!xcd_tile(tiles_m, tiles_n, xm, tm, tn)) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int M = a.M, K = a.K, Np = a.Npart;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int wr = wave & 1, wc = wave >> 1;
+  const int ml = lane & 15, ng = 4 * (lane >> 4);
+
+  // A: run `seg` of rows row0 + 32 i; rows past M read row M - 1
+  const int seg = tid & 7, row0 = tid >> 3;
+  const uint16_t *ap[AR];
+#pragma unroll
+  for (int i = 0; i < AR; ++i) ap[i] = a.A + (size_t)min(m0 + row0 + 32 * i, M - 1) * K + seg * 8;
+  unsigned char *const adst = smem + row0 * S::AREC + seg * 16;
+  // B: 16-byte pieces, NB BN / 8 per k row
+  const uint16_t *bp[BR];
+  int bdst[BR];
+#pragma unroll
+  for (int i = 0; i < BR; ++i) {
+    constexpr int CPR = NB * BN / 8;
+    const int it = tid + 256 * i, k = it / CPR, c = it % CPR;
+    const int nb = c / (BN / 8), cc = c % (BN / 8), gc = n0 + cc * 8;
+    const int part = EPI == kEpiQkvRope ? gc / Np : nb, col = EPI == kEpiQkvRope ? gc % Np : gc;
+    bp[i] = a.B[part] + (size_t)k * Np + col;
+    bdst[i] = S::ABYTES + (nb * S::STRIPS + cc / 2) * S::SB + strip_row(k) * 32 + (cc & 1) * 16;
+  }
+  u32x4 av[AR], bv[BR];
+  f32x4 g0, g1;
+  auto fetch = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < AR; ++i) av[i] = *reinterpret_cast<const u32x4 *>(ap[i] + k0);
+    if constexpr (PRO == kProRmsnorm) {
+      g0 = *reinterpret_cast<const f32x4 *>(a.gamma + k0 + seg * 8);
+      g1 = *reinterpret_cast<const f32x4 *>(a.gamma + k0 + seg * 8 + 4);
+    }
+#pragma unroll
+    for (int i = 0; i < BR; ++i) bv[i] = *reinterpret_cast<const u32x4 *>(bp[i] + (size_t)k0 * Np);
+  };
+  float ss[AR];
+#pragma unroll
+  for (int i = 0; i < AR; ++i) ss[i] = 0.0f;
+  auto commit = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < AR; ++i) {
+      u32x4 o = av[i];
+      if constexpr (PRO == kProRmsnorm) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = bf_lo(av[i][e]), hi = bf_hi(av[i][e]);
+          ss[i] = fmaf(hi, hi, fmaf(lo, lo, ss[i]));
+          o[e] = cvt_pk_bf16(lo * (e < 2 ? g0[2 * e] : g1[2 * e - 4]), hi * (e < 2 ? g0[2 * e + 1] : g1[2 * e - 3]));
+        }
+      }
+      *reinterpret_cast<u32x4 *>(adst + buf * S::BUF + 32 * i * S::AREC) = o;
+    }
+#pragma unroll
+    for (int i = 0; i < BR; ++i) *reinterpret_cast<u32x4 *>(smem + buf * S::BUF + bdst[i]) = bv[i];
+  };
+
+  f32x4 acc[NB][TM][TN];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const unsigned char *const arow = smem + (wr * (BM / 2) + ml) * S::AREC + (lane >> 4) * 16;
+  const int steps = K / KC;
+  fetch(0);
+  commit(0);
+  fetch(min(KC, K - KC));
+  __syncthreads();
+  for (int s = 0; s < steps; ++s) {
+    const int off = (s & 1) * S::BUF;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      Frag16 xf[TM], wf[NB][TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) xf[i].u = *reinterpret_cast<const u32x4 *>(arow + off + 16 * i * S::AREC + 64 * h);
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          wf[b][j] = read_wfrag(smem + off + S::ABYTES + (b * S::STRIPS + wc * TN + j) * S::SB, h, lane);
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            acc[b][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[b][j].h, xf[i].h, acc[b][i][j], 0, 0, 0);
+    }
+    if (s + 1 < steps) {
+      commit((s + 1) & 1);
+      fetch(min((s + 2) * KC, K - KC));
+    }
+    __syncthreads();
+  }
+  if constexpr (PRO == kProRmsnorm) {
+    // the eight lanes of a row: xor 1, 2 (quad permutes), then the half-row mirror
+#pragma unroll
+    for (int i = 0; i < AR; ++i) {
+      float v = ss[i];
+      v += dpp_mov<0xb1>(v);
+      v += dpp_mov<0x4e>(v);
+      v += dpp_mov<0x141>(v);
+      if (seg == 0) inv_s[row0 + 32 * i] = __builtin_amdgcn_rsqf(v * (1.0f / (float)K) + a.eps);
+    }
+    __syncthreads();
+  }
+
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int row = wr * (BM / 2) + 16 * i + ml, m = m0 + row;
+    const float inv = PRO == kProRmsnorm ? inv_s[row] : 1.0f;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + wc * (BN / 2) + 16 * j + ng;
+      f32x4 v = acc[0][i][j];
+      if constexpr (PRO == kProRmsnorm) v *= inv;
+      uint2 o;
+      uint16_t *dst;
+      if constexpr (EPI == kEpiQkvRope) {
+        const int part = n / Np, c = n % Np;
+        dst = a.out[part] + (size_t)m * Np + c;
+        if (part < 2) {  // (2t, 2t+1) -> (x0 c - x1 s, x0 s + x1 c)
+          const size_t t = (size_t)m * (a.Dh / 2) + (c % a.Dh) / 2;
+          const float2 cc = *reinterpret_cast<const float2 *>(a.cos_t + t);
+          const float2 sn = *reinterpret_cast<const float2 *>(a.sin_t + t);
+          o = pack4_bf16(v[0] * cc.x - v[1] * sn.x, v[0] * sn.x + v[1] * cc.x,
+                         v[2] * cc.y - v[3] * sn.y, v[2] * sn.y + v[3] * cc.y);
+        } else {
+          o = pack4_bf16(v[0], v[1], v[2], v[3]);
+        }
+      } else if constexpr (EPI == kEpiResidual) {
+        const uint2 r = *reinterpret_cast<const uint2 *>(a.res + (size_t)m * Np + n);
+        dst = a.out[0] + (size_t)m * Np + n;
+        o = pack4_bf16(bf_lo(r.x) + v[0], bf_hi(r.x) + v[1], bf_lo(r.y) + v[2], bf_hi(r.y) + v[3]);
+      } else {
+        f32x4 u = acc[NB - 1][i][j];
+        if constexpr (PRO == kProRmsnorm) u *= inv;
+        dst = a.out[0] + (size_t)m * Np + n;
+        o = pack4_bf16(silu_fast(v[0]) * u[0], silu_fast(v[1]) * u[1], silu_fast(v[2]) * u[2],
+                       silu_fast(v[3]) * u[3]);
+      }
+      *reinterpret_cast<uint2 *>(dst) = o;
+    }
+  }
+}
+
 // ---- attention ----------------------------------------------------------------
 constexpr int AQ = 16;    // queries per workgroup
 constexpr int AKB = 32;   // keys per block
@@ -593,6 +771,170 @@ __global__ __launch_bounds__(256) void llama_attention_kernel(const uint16_t *__
   }
 }
 
+// Long sequences: 64 queries per workgroup, 16 per wave, in two groups of four
+// waves that take the even and the odd key blocks of 64 and merge at the end.
+// A pair of blocks is staged in LDS for all eight waves, the next pair's loads
+// in flight: a quarter of the K and V traffic of the kernel above.  Workgroups
+// are dealt longest first (the last query blocks), so the short ones fill in
+// behind them.
+// What bounds it: one wave's chain per block (scores, maximum, exponentials,
+// products: about 1 800 clocks alone on its SIMD), which is why the keys are
+// split.
+constexpr int TQ = 64, TKB = 64, TGR = 2;
+
+template <int DH>
+__global__ __launch_bounds__(256 * TGR, 4) void llama_attention_tile_kernel(const uint16_t *__restrict__ Q,
+                                                                   const uint16_t *__restrict__ Kg,
+                                                                   const uint16_t *__restrict__ V,
+                                                                   uint16_t *__restrict__ O, int S,
+                                                                   int H, float scale) {
+  using Sh = AttnShape<DH>;
+  constexpr int NQF = Sh::NQF, LD = Sh::VLD, PPR = Sh::PPR, NDT = Sh::NDT, NT = TKB / 16;
+  constexpr int NR = TKB * PPR / 256;  // 16-byte pieces of K (and of V) per thread and block
+  // one pair of blocks; after the walk, the odd group's states
+  __shared__ __attribute__((aligned(16))) uint16_t kvbuf[2 * TGR][TKB * LD];
+  const int nqb = (S + TQ - 1) / TQ;
+  const int qb = nqb - 1 - blockIdx.x / H, h = blockIdx.x % H;
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+  const int gr = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);  // this wave's group
+  const int g = lane >> 4, ql = lane & 15;
+  const int D = H * DH;
+  const int q0 = qb * TQ + 16 * wave;  // this wave's queries
+  const float kscale = scale * 1.4426950408889634f;  // exp(x * scale) = exp2(x * kscale)
+
+  // Rows past S are read from row S - 1, as above: such keys lie above every
+  // stored query's diagonal, and such queries are not stored.
+  Frag16 qf[NQF];
+  {
+    const uint16_t *qp = Q + (size_t)min(q0 + ql, S - 1) * D + h * DH + 8 * g;
+#pragma unroll
+    for (int k = 0; k < NQF; ++k) qf[k] = load16(qp + 32 * k);
+  }
+  u32x4 kr[NR], vr[NR];
+  auto fetch = [&](int kb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int item = tid + 256 * i;  // key item / PPR, dh 8 (item % PPR)
+      const size_t o = (size_t)min(kb * TKB + item / PPR, S - 1) * D + h * DH + (item % PPR) * 8;
+      kr[i] = *reinterpret_cast<const u32x4 *>(Kg + o);
+      vr[i] = *reinterpret_cast<const u32x4 *>(V + o);
+    }
+  };
+  auto commit = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int item = tid + 256 * i, o = (item / PPR) * LD + (item % PPR) * 8;
+      *reinterpret_cast<u32x4 *>(kvbuf[gr] + o) = kr[i];
+      *reinterpret_cast<u32x4 *>(kvbuf[TGR + gr] + o) = vr[i];
+    }
+  };
+  float m_run = -__builtin_inff(), l_run = 0.0f;
+  f32x4 o[NDT];
+#pragma unroll
+  for (int d = 0; d < NDT; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const uint16_t *const ks = kvbuf[gr], *const vs = kvbuf[TGR + gr];
+  fetch(min(gr, qb));
+  for (int kb0 = 0; kb0 <= qb; kb0 += TGR) {
+    const int kb = kb0 + gr;
+    if (kb0 > 0) __syncthreads();  // every wave is done with the last pair
+    commit();
+    __syncthreads();
+    fetch(min(kb + TGR, qb));
+    if (kb > qb) break;  // the odd group's last pair has no block for it
+    // S^T = K Q^T: four 16-key tiles
+    f32x4 s[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < NQF; ++k)
+        s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load16(ks + (16 * t + ql) * LD + 32 * k + 8 * g).h,
+                                                       qf[k].h, s[t], 0, 0, 0);
+    }
+    if (kb == qb) {  // the diagonal block: key > query
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * t + 4 * g + r > 16 * wave + ql) s[t][r] = -__builtin_inff();
+    }
+    float mx = fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3]));
+#pragma unroll
+    for (int t = 1; t < NT; ++t)
+      mx = fmaxf(mx, fmaxf(fmaxf(s[t][0], s[t][1]), fmaxf(s[t][2], s[t][3])));
+    const LanePair p16 = lane_pair16(mx);
+    mx = fmaxf(p16.lo, p16.hi);
+    const LanePair p32 = lane_pair32(mx);
+    mx = fmaxf(p32.lo, p32.hi);
+    const float m_new = fmaxf(m_run, mx);
+    const float m_use = m_new == -__builtin_inff() ? 0.0f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * kscale);
+    const float bias = -m_use * kscale;
+    // P^T as bf16, keys 4g + r of each tile.  The normaliser sums the rounded
+    // values, so the weights that V is multiplied by add up to one (relative
+    // error of the output at 2048x12x64 0.00332, as the kernel above has; with
+    // the sum of the unrounded ones 0.00334).
+    uint2 pk[NT];
+    float psum = 0.0f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      float p[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(s[t][r], kscale, bias));
+      pk[t] = pack4_bf16(p[0], p[1], p[2], p[3]);
+      psum += (bf_lo(pk[t].x) + bf_hi(pk[t].x)) + (bf_lo(pk[t].y) + bf_hi(pk[t].y));
+    }
+    l_run = l_run * alpha + psum;
+    m_run = m_new;
+#pragma unroll
+    for (int d = 0; d < NDT; ++d) o[d] *= alpha;
+#pragma unroll
+    for (int b = 0; b < NT / 2; ++b) {
+      Frag16 pf;  // k slots: keys 4g + r of tiles 2b and 2b + 1
+      pf.u = u32x4{pk[2 * b].x, pk[2 * b].y, pk[2 * b + 1].x, pk[2 * b + 1].y};
+#pragma unroll
+      for (int d = 0; d < NDT; ++d) {
+        const Frag16 vf = read_vfrag<LD>(vs + 32 * b * LD, d, lane);
+        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.h, pf.h, o[d], 0, 0, 0);
+      }
+    }
+  }
+  const LanePair a16 = lane_pair16(l_run);
+  const float l16 = a16.lo + a16.hi;
+  const LanePair a32 = lane_pair32(l16);
+  l_run = a32.lo + a32.hi;
+  // the odd group's state to LDS, lane by lane; the even group merges it
+  float *const st = reinterpret_cast<float *>(kvbuf) + tid;
+  __syncthreads();
+  constexpr int SS = 256;  // words between a lane's values
+  static_assert((4 * NDT + 2) * SS * 4 <= (int)sizeof kvbuf, "states fit");
+  if (gr == 1) {
+    st[0] = m_run;
+    st[SS] = l_run;
+#pragma unroll
+    for (int d = 0; d < NDT; ++d)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) st[(2 + 4 * d + e) * SS] = o[d][e];
+  }
+  __syncthreads();
+  if (gr == 1) return;
+  const float m1 = st[0], l1 = st[SS], m = fmaxf(m_run, m1);
+  const float m_use = m == -__builtin_inff() ? 0.0f : m;
+  const float f0 = __builtin_amdgcn_exp2f((m_run - m_use) * kscale), f1 = __builtin_amdgcn_exp2f((m1 - m_use) * kscale);
+  const float invl = 1.0f / (l_run * f0 + l1 * f1);
+  if (q0 + ql < S) {
+    uint16_t *const op = O + (size_t)(q0 + ql) * D + h * DH + 4 * g;
+#pragma unroll
+    for (int d = 0; d < NDT; ++d) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (o[d][e] * f0 + st[(2 + 4 * d + e) * SS] * f1) * invl;
+      *reinterpret_cast<uint2 *>(op + 16 * d) = pack4_bf16(v[0], v[1], v[2], v[3]);
+    }
+  }
+}
+
 // ---- launch plans ---------------------------------------------------------------
 // Per-tile work of a GEMM launch, from the kernel's own loops.
 template <class Sh, class Kern>
@@ -662,6 +1004,41 @@ hipError_t run_gemm(const char *name, const LlamaGemmArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <int PRO, int EPI, int BM, int BN>
+hipError_t run_tile(const char *name, const LlamaGemmArgs &a, hipStream_t s) {
+  using S = TileShape<EPI, BM, BN>;
+  auto kern = llama_tile_kernel<PRO, EPI, BM, BN>;
+  const int ncols = a.Npart * (EPI == kEpiQkvRope ? a.nparts : 1);
+  if (ncols % BN != 0 || a.Npart % 8 != 0 || a.K % S::KC != 0) return hipErrorInvalidValue;
+  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = ncols / BN;
+  const int G = tiles_m * tiles_n, grid = (G + 7) / 8 * 8;
+  const int ok = cached_per_kernel(reinterpret_cast<const void *>(kern), [&](int) {
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, 2 * S::BUF) == hipSuccess
+               ? 1 : 0;
+  });
+  if (!ok) return hipErrorInvalidValue;
+  {
+    const double steps = a.K / S::KC;
+    npu_launch_plan p = make_plan(name, G, wg_per_cu(kern, 256), G, 16);
+    p.tile_macs = (double)BM * BN * S::NB * a.K;
+    p.tile_valu = 4.0 * (steps * ((PRO == kProRmsnorm ? 32.0 : 2.0) * S::AR + 3.0 * S::BR + 20.0) +
+                         24.0 * S::TM * S::TN * S::NB + 120.0);
+    p.tile_lds_bytes = steps * (S::BUF + 4.0 * 2 * 1024 * (S::TM + S::NB * S::TN));
+    p.tile_load_bytes = 2.0 * a.K * (BM + S::NB * BN);
+    p.tile_store_bytes = 2.0 * BM * BN;
+    const double parts = EPI == kEpiQkvRope ? a.nparts : S::NB;
+    p.hbm_bytes = 2.0 * ((double)a.M * a.K + parts * a.K * a.Npart +
+                         (double)a.M * a.Npart * (EPI == kEpiQkvRope ? a.nparts : 1) +
+                         (EPI == kEpiResidual ? (double)a.M * a.Npart : 0.0)) +
+                  (PRO == kProRmsnorm ? 4.0 * a.K : 0.0) + (EPI == kEpiQkvRope ? 2.0 * 4 * a.M * a.Dh / 2 : 0.0);
+    plans_add(p);
+  }
+  const int xm = xcd_block_grid(tiles_m, tiles_n, BM, BN * S::NB, true);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 2 * S::BUF, s, a, tiles_m, tiles_n, xm);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 // Tiles (16 waves each).  At d_model <= 512 the RMSNorm GEMMs give each wave
@@ -673,6 +1050,33 @@ hipError_t run_gemm(const char *name, const LlamaGemmArgs &a, hipStream_t s) {
 // workgroups; K in chunks of 512, the down projection's 1408 in three, at
 // most 2048).  Chunk sizes keep two chunk buffers within the 160 KiB of LDS.
 hipError_t launch_llama_gemm(const LlamaGemmArgs &a, int pro, int epi, hipStream_t s) {
+  // Long sequences (see llama_tile_kernel), where their tiles outnumber what
+  // the 16-wave shapes are made for.  Measured, us, 16 waves / tiles (count):
+  //   QKV S x D: 2048x768 54.8 / 25.8 (1152), 1024x512 12.7 / 10.3 (384),
+  //     512x768 18.2 / 12.1 (288), 300x768 10.4 / 9.9 (180), 512x512 6.9 / 8.1 (192);
+  //   SwiGLU S x D x F: 2048x768x2048 61.8 / 23.9 (512 of 128 x 64; of 64 x 64
+  //     29.2), 1024x768x2048 31.9 / 16.1, 300x768x2048 16.1 / 10.7 (160 of 64 x
+  //     64), 512x512x1408 8.3 / 8.5 (176);
+  //   residual S x K x N: 2048x2048x768 49.5 / 19.6 (384 of 64 x 64),
+  //     1024x1408x512 12.4 / 8.2 (256 of 32 x 64), 512x768x768 8.7 / 5.7 (192),
+  //     512x512x512 4.1 / 4.6 (128), 300x2048x768 8.9 / 9.9 (120).
+  const auto tiles = [&](int bm, int bn, int cols) { return (long long)((a.M + bm - 1) / bm) * (cols / bn); };
+  if (pro == kProRmsnorm && a.K <= 1024) {
+    const int cols = a.Npart * (epi == kEpiQkvRope ? a.nparts : 1);
+    const bool many = tiles(64, 64, cols) >= (a.K <= 512 ? 256 : 160);
+    if (epi == kEpiQkvRope && many)
+      return run_tile<kProRmsnorm, kEpiQkvRope, 64, 64>("llama_rmsnorm_qkv_rope", a, s);
+    if (epi == kEpiSwiglu && tiles(128, 64, cols) >= 320)
+      return run_tile<kProRmsnorm, kEpiSwiglu, 128, 64>("llama_rmsnorm_swiglu", a, s);
+    if (epi == kEpiSwiglu && many)
+      return run_tile<kProRmsnorm, kEpiSwiglu, 64, 64>("llama_rmsnorm_swiglu", a, s);
+  }
+  if (pro == kProPlain && epi == kEpiResidual && a.K <= 2048) {
+    if (tiles(64, 64, a.Npart) >= 256)
+      return run_tile<kProPlain, kEpiResidual, 64, 64>("llama_matmul_residual", a, s);
+    if (tiles(32, 64, a.Npart) >= 160)
+      return run_tile<kProPlain, kEpiResidual, 32, 64>("llama_matmul_residual", a, s);
+  }
   if (pro == kProRmsnorm && epi == kEpiQkvRope) {
     if (a.K <= 512)
       return run_gemm<kProRmsnorm, kEpiQkvRope, 64, 64, 4, 4, 1, 512, 1, 512>("llama_rmsnorm_qkv_rope", a, s);
@@ -692,8 +1096,37 @@ hipError_t launch_llama_gemm(const LlamaGemmArgs &a, int pro, int epi, hipStream
 }
 
 template <int DH>
+hipError_t launch_attention_tiles(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
+                                  uint16_t *O, int S, int H, float scale, hipStream_t s) {
+  auto kern = llama_attention_tile_kernel<DH>;
+  const int nqb = (S + TQ - 1) / TQ, grid = nqb * H;
+  {
+    // per wave and key block: 8 DH / 64 x 2 MFMAs, the softmax of 16 scores
+    // per lane; the plan's tile is the longest workgroup's (the last query block)
+    const double kblocks = nqb;
+    npu_launch_plan p = make_plan("llama_causal_attention", grid, wg_per_cu(kern, 256 * TGR), grid, 16);
+    p.unit_waves = 4 * TGR;
+    p.load_phases = 1;
+    p.tile_macs = kblocks * 2.0 * TQ * TKB * DH;
+    p.tile_valu = 4.0 * (100.0 + 190.0 * kblocks) * (DH / 64);
+    p.tile_lds_bytes = kblocks * (2.0 * TKB * DH * 2 + 4.0 * 2.0 * TKB * DH * 2);
+    p.tile_load_bytes = kblocks * 2.0 * TKB * DH * 2 + TQ * DH * 2.0;
+    p.tile_store_bytes = TQ * DH * 2.0;
+    p.hbm_bytes = 4.0 * S * H * DH * 2;  // Q, K, V in, O out
+    plans_add(p);
+  }
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256 * TGR), 0, s, Q, K, V, O, S, H, scale);
+  return hipGetLastError();
+}
+
+template <int DH>
 hipError_t launch_attention_dh(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
                                uint16_t *O, int S, int H, float scale, hipStream_t s) {
+  // 64-query workgroups from 160 of them on; measured, us, 16 queries / 64
+  // (workgroups of 64): S x heads x dim 2048x12x64 49.5 / 24.4 (384), 2048x6x128
+  // 55.8 / 35.3 (192), 1024x12x64 16.7 / 12.2 (192), 1024x8x64 10.2 / 11.3 (128),
+  // 1500x4x64 14.2 / 15.1 (96), 512x8x64 5.4 / 7.0 (64).
+  if ((long long)((S + TQ - 1) / TQ) * H >= 160) return launch_attention_tiles<DH>(Q, K, V, O, S, H, scale, s);
   auto kern = llama_attention_kernel<DH>;
   const int G = (S + AQ - 1) / AQ * H, grid = (G + 7) / 8 * 8;
   {

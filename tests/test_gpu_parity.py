@@ -737,6 +737,59 @@ def test_c5_layer_small_shapes(cuda, S, D, H, F):
         check_bound(bf16(_host(o[name])), bf16(ref), mag, RTOL_BF16, what=f"layer {name}")
 
 
+@pytest.mark.parametrize("S,D,H,F", [
+    (1400, 256, 4, 896),   # QKV and SwiGLU 64x64, residual 32x64; S a row block of 56 past a tile
+    (330, 576, 9, 1920),   # K past 512: QKV and SwiGLU 64x64
+    (2100, 512, 8, 1280),  # SwiGLU 128x64, residual 64x64, 64-query attention; 52 rows past a tile
+])
+def test_c5_stages_long_sequences(cuda, S, D, H, F):
+    """Every stage on the tiles for long sequences, against the stage in
+    float64 on the oracle's inputs under the configuration's bounds."""
+    inp = configs.llama_layer(S=S, D=D, H=H, F=F, seed=171 + S).make_inputs()
+    with oracle.threaded():
+        st = refs.llama_stages(inp, H, LL_EPS)
+    ex = refs.llama_stage_exact(inp, st, H, LL_EPS)
+    d = configs.to_device(inp)
+    sd = configs.to_device({k: st[k] for k in ("Q", "K", "V", "A", "h", "act")})
+    Q, K, V, A, h, out = (_bf_dev((S, D)) for _ in range(6))
+    act = _bf_dev((S, F))
+    groups.fused_llama_qkv_rope(d["x"], d["g1"], d["wq"], d["wk"], d["wv"], d["cos_t"],
+                                d["sin_t"], Q, K, V, LL_EPS)
+    groups.fused_llama_attention(sd["Q"], sd["K"], sd["V"], A, H, (D // H) ** -0.5)
+    groups.fused_llama_matmul_residual(sd["A"], d["wo"], d["x"], h)
+    groups.fused_llama_rmsnorm_swiglu(sd["h"], d["g2"], d["wg"], d["wu"], act, LL_EPS)
+    groups.fused_llama_matmul_residual(sd["act"], d["wd"], sd["h"], out)
+    torch.cuda.synchronize()
+    xn, hn = refs.normed_bf16(inp["x"], inp["g1"], LL_EPS), refs.normed_bf16(st["h"], inp["g2"], LL_EPS)
+    for name, t, wname, rope in (("Q", Q, "wq", True), ("K", K, "wk", True), ("V", V, "wv", False)):
+        mag = refs.mag_qkv(xn, inp[wname], inp["cos_t"], inp["sin_t"], rope)
+        check_bf16_stage(_host(t), ex[name], mag, D + 2, what=name)
+    check_bf16_stage(_host(A), ex["A"], refs.mag_attention(st["Q"], st["K"], st["V"], H), S + D // H,
+                     what="attention")
+    check_bf16_rounded(_host(h), ex["h"], refs.mag_residual(st["A"], inp["wo"], inp["x"]), D + 1, what="h")
+    check_bf16_stage(_host(act), ex["act"], refs.mag_swiglu(hn, inp["wg"], inp["wu"]), D + 4, what="act")
+    check_bf16_rounded(_host(out), ex["out"], refs.mag_residual(st["act"], inp["wd"], st["h"]), F + 1,
+                       what="out")
+
+
+@pytest.mark.parametrize("S,H,dh", [(641, 15, 128), (64, 160, 64), (129, 64, 64), (193, 40, 128)])
+def test_c5_attention_64_queries(cuda, S, H, dh):
+    """The 64-query attention at its block edges: one query past a block, a
+    single block, an odd and an even number of key blocks, heads of 128."""
+    q, k, v = (rng.to_bf16_bits(rng.normal(181 + S, i, (S, H * dh), 0.0, 1.0)) for i in range(3))
+    A = _bf_dev((S, H * dh))
+    groups.fused_llama_attention(_dev(q), _dev(k), _dev(v), A, H, dh ** -0.5)
+    torch.cuda.synchronize()
+    heads = lambda b: torch.from_numpy(np.ascontiguousarray(bf16(b))).double().reshape(S, H, dh).transpose(0, 1)
+    Q, K, V = heads(q), heads(k), heads(v)
+    sc = torch.matmul(Q, K.transpose(1, 2).contiguous()) * dh ** -0.5
+    P = torch.softmax(sc.masked_fill(torch.ones(S, S, dtype=torch.bool).triu(1), float("-inf")), 2)
+    back = lambda t: t.transpose(0, 1).reshape(S, H * dh).numpy()
+    check_bf16_stage(_host(A), back(torch.matmul(P, V)), back(torch.matmul(P, V.abs())), S + dh,
+                     what=f"attention S={S} H={H} dh={dh}")
+    assert np.array_equal(_host(A)[0], v[0])
+
+
 # ------------------------------------------------------------------ SRAM plan as LDS layout
 def _planned_case(M, K, N, seed, bias=True):
     from npu_amd import tileplan
