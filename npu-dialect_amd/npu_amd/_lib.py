@@ -8,6 +8,7 @@ silently execute anything but the HIP path.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import os
 import subprocess
 
@@ -57,9 +58,12 @@ class NpuLaunchPlan(C.Structure):
         ("wg_setup_valu", C.c_double),
     ]
 
+
+@functools.lru_cache(maxsize=None)
 def strided_memref_type(rank: int):
     """MLIR's StridedMemRefType<T, rank> layout: {allocated, aligned, offset,
-    sizes[rank], strides[rank]} (include/npu_amd.h NPU_STRIDED_MEMREF)."""
+    sizes[rank], strides[rank]} (include/npu_amd.h NPU_STRIDED_MEMREF).  One
+    class per rank: making it anew for each argument took 5 us."""
     class StridedMemref(C.Structure):
         _fields_ = [("allocated", C.c_void_p), ("aligned", C.c_void_p), ("offset", C.c_int64),
                     ("sizes", C.c_int64 * rank), ("strides", C.c_int64 * rank)]

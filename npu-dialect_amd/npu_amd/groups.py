@@ -10,10 +10,12 @@ The group names follow the op chains the reference's outliner groups
 """
 from __future__ import annotations
 
+import array
 import ctypes as C
+import struct
 
 from . import _lib
-from .memref import absent, from_tensor, ref
+from .memref import absent, from_tensor, ref, tensor_dtype
 from .names import OUTLINED_NAMES  # noqa: F401  (re-exported)
 
 ACT = {"none": 0, "relu": 1, "relu6": 2}
@@ -30,7 +32,8 @@ class NpuError(RuntimeError):
 def _stream(stream):
     if stream is None:
         import torch
-        return torch.cuda.current_stream().cuda_stream
+        # the raw handle of torch.cuda.current_stream(), without the Stream object
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     return getattr(stream, "cuda_stream", stream)
 
 
@@ -211,32 +214,37 @@ class Empty:
 _DT = {"f32": 0, "bf16": 1, "i8": 2, "i32": 3}
 
 
-def _group_arg(x, keep):
-    """One npu_arg for a tensor, an Empty or a scalar fill value."""
-    a = _lib.NpuArg()
+_ARG_PACK = struct.Struct("<qQiid")  # npu_arg: rank, descriptor, dtype, kind, scalar
+assert _ARG_PACK.size == C.sizeof(_lib.NpuArg)
+
+
+def _group_arg(x, keep) -> bytes:
+    """One packed npu_arg for a tensor, an Empty or a scalar fill value; the
+    memref descriptor it points at is appended to `keep`."""
     if isinstance(x, (int, float)):
-        a.kind, a.dtype, a.scalar, a.rank = 1, _DT["f32"], float(x), 0
-        return a
+        return _ARG_PACK.pack(0, 0, _DT["f32"], 1, x)
     if isinstance(x, Empty):
         if x.tensor is not None:
             return _group_arg(x.tensor, keep)
-        shape, dtype, ptr, offset, strides = x.shape, _DT[x.dtype], 0, 0, None
-    else:
-        m = from_tensor(x)
-        shape, dtype, ptr, offset = list(x.shape), m.dtype, m.aligned, m.offset
-        strides = list(x.stride())
-    if strides is None:
+        shape, dtype, ptr, offset = x.shape, _DT[x.dtype], 0, 0
         strides = [1] * len(shape)
         for i in range(len(shape) - 2, -1, -1):
             strides[i] = strides[i + 1] * shape[i + 1]
-    d = _lib.strided_memref_type(len(shape))()
-    d.allocated = d.aligned = ptr
-    d.offset = offset
-    for i, (sz, st) in enumerate(zip(shape, strides)):
-        d.sizes[i], d.strides[i] = sz, st
+    else:
+        dtype = tensor_dtype(x)
+        shape, strides, offset = x.shape, x.stride(), x.storage_offset()
+        ptr = x.untyped_storage().data_ptr()
+    # StridedMemRefType's words in order: the two pointers, the offset, the
+    # sizes, the strides
+    d = array.array("q", (ptr, ptr, offset, *shape, *strides))
     keep.append(d)
-    a.rank, a.descriptor, a.dtype, a.kind = len(shape), C.addressof(d), dtype, 0
-    return a
+    return _ARG_PACK.pack(len(shape), d.buffer_info()[0], dtype, 0, 0.0)
+
+
+def _arg_list(xs, keep):
+    n = max(len(xs), 1)
+    raw = b"".join([_group_arg(x, keep) for x in xs]).ljust(n * _ARG_PACK.size, b"\0")
+    return (_lib.NpuArg * n).from_buffer_copy(raw)
 
 
 def group_launch(outlined_name, ins, outs, act=("none",), pad=0, n_heads=0, eps=0.0, scale=0.0,
@@ -247,8 +255,7 @@ def group_launch(outlined_name, ins, outs, act=("none",), pad=0, n_heads=0, eps=
     result tensors.  ``res_arg``: the index in ``ins`` of a conv group's
     residual operand (0: none named)."""
     keep = []
-    ia = (_lib.NpuArg * max(len(ins), 1))(*[_group_arg(x, keep) for x in ins])
-    oa = (_lib.NpuArg * max(len(outs), 1))(*[_group_arg(x, keep) for x in outs])
+    ia, oa = _arg_list(ins, keep), _arg_list(outs, keep)
     at = _lib.NpuGroupAttrs()
     for i, a in enumerate(act):
         at.act[i] = ACT[a]

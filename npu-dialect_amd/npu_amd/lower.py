@@ -752,6 +752,7 @@ class Program:
         self.func = func
         self.calls = calls
         self.launches = list(launches)
+        self._producer = {r: op for op in func.ops for r in op.results}
 
     @property
     def entry_points(self):
@@ -795,10 +796,9 @@ class Program:
             outs = [vals[v] for v in L.outs]
             getattr(groups, L.entry)(*ins, *outs, **L.params, stream=stream)
             return
-        prod = {r: op for op in self.func.ops for r in op.results}
         ins = []
         for v in L.ins:
-            op = prod.get(v)
+            op = self._producer.get(v)
             if v == L.padded:
                 ins.append(vals[L.pad_source])
             elif v in vals:
@@ -823,7 +823,11 @@ class Program:
         """inputs: argument name (with or without %) -> tensor.  Runs every
         launch through npu_group_launch and returns the function's results by
         SSA name."""
+        from . import groups
+
         vals = self.check_inputs(inputs)
+        if self.launches:
+            stream = groups._stream(stream)  # looked up once for all launches
         for i in range(len(self.launches)):
             self.run_launch(i, vals, stream)
         ret = [op for op in self.func.ops if op.name == "func.return"]

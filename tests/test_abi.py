@@ -225,3 +225,29 @@ def test_zero_sized_dimensions_are_rejected_before_launch():
                  (_mr([8, 0]), _mr([0, 4]), b, o)):
         assert call(*args, 1) == 1
         assert "must be positive" in _err()
+
+
+@pytest.mark.parametrize("rank", range(1, 5))
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "int8", "int32"])
+def test_descriptors_hold_pointer_offset_sizes_and_strides(rank, dtype):
+    """npu_memref and npu_arg descriptors of a transposed view inside a larger
+    buffer, field by field: what the packed layouts put where."""
+    import torch
+    from npu_amd import groups, memref
+
+    t = torch.zeros([3, 4, 5, 6][:rank], dtype=getattr(torch, dtype))[1:].transpose(0, rank - 1)
+    m = memref.from_tensor(t)
+    base, code = t.untyped_storage().data_ptr(), memref.tensor_dtype(t)
+    assert (m.allocated, m.aligned, m.offset, m.rank, m.dtype) == \
+        (base, base, t.storage_offset(), rank, code) and m.offset > 0
+    assert list(m.sizes) == list(t.shape) + [0] * (4 - rank)
+    assert list(m.strides) == list(t.stride()) + [0] * (4 - rank)
+    keep = []
+    a = groups._arg_list([t, 0.5, groups.Empty([2] * rank, "bf16")], keep)
+    assert [(x.kind, x.rank, x.dtype, x.scalar) for x in a] == \
+        [(0, rank, code, 0.0), (1, 0, 0, 0.5), (0, rank, 1, 0.0)]
+    for x, want in ((a[0], (base, t.storage_offset(), list(t.shape), list(t.stride()))),
+                    (a[2], (None, 0, [2] * rank, [2 ** (rank - 1 - i) for i in range(rank)]))):
+        d = _lib.strided_memref_type(rank).from_address(x.descriptor)
+        assert (d.allocated, d.offset, list(d.sizes), list(d.strides)) == want
+        assert d.aligned == d.allocated
