@@ -363,70 +363,153 @@ hipError_t launch_irb_t(const IrbArgs &a, hipStream_t s) {
 // Any (C, E) with C % 4 == 0, C <= 16 CB and E % 16 == 0, for the channel
 // counts the tuned instances above do not cover: the expanded channels are
 // streamed in chunks of 16, so neither the filters nor the expanded tile
-// need to fit in registers or LDS.  A workgroup walks 4 x 4 output tiles;
-// per tile the x halo (6 x 6 pixels, all C channels, zero outside the image
-// and past C) goes to LDS, then wave w takes chunks w, w + 4, ... of E / 16:
-// the expand of the chunk on the halo (its 16 filters as the A operand, from
-// L2), ReLU6 and the zero padding into the wave's own LDS slot, the
-// depthwise of the 16 output pixels in the project MFMA's B layout, and the
-// project of the chunk into the wave's CB accumulator blocks (its columns of
-// wp as the A operand).  Waves 1..3 leave their partial projections in LDS
-// and wave 0 adds them in wave order, then the residual, and stores.
-template <int CB>
-__global__ __launch_bounds__(256, 1) void irb_stream_kernel(
+// need to fit in registers or LDS.  A workgroup of NW waves walks TH x TW
+// output tiles; per tile the x halo (all C channels, zero outside the image
+// and past C) is in LDS, then wave w takes chunks w, w + NW, ... of E / 16:
+// the expand of the chunk on the halo (its 16 filters as the A operand),
+// ReLU6 and the zero padding into the wave's own LDS slot, the depthwise of
+// the output pixels in the project MFMA's B layout, and the project of the
+// chunk into the wave's CB x OPB accumulators (its columns of wp as the A
+// operand).  The waves' partial projections meet in LDS, 16 pixels at a
+// time, and all threads add them in wave order, then the residual.
+//
+// What bounds it: the f32 MFMAs, once the filters' loads are off the chain.
+// A chunk's filters come from L2 into registers that are reloaded for the
+// wave's next chunk right where they were last used, and the next tile's
+// halo is in flight during this one.  Before, with four waves, 4 x 4 tiles
+// and every filter loaded where it was used, a wave waited for L2 five times
+// a chunk.  us, before -> now: 14x14x64/384 batch 32 25.4 -> 17.9 (7.7 of it
+// f32 MFMAs), 96/576 50 -> 32, 7x7x160/960 105 -> 54, batch 1 14x14x64/384
+// 19.0 -> 12.3, 7x7x320/1920 batch 2 565 -> 213.
+template <int CB, int TH, int TW, int NW>
+__global__ __launch_bounds__(64 * NW, NW / 4) void irb_stream_kernel(
     const float *__restrict__ x, const float *__restrict__ we, const float *__restrict__ wdw,
     const float *__restrict__ wp, float *__restrict__ out, int H, int W, int C, int E,
     int tiles_w, int tiles_per_image, int ntiles) {
-  constexpr int TW = 4, HW = 6, HP = 36, HPB = 3;
-  constexpr int ESS = 24;  // a wave's expanded chunk: 16 channels per pixel + 8 (32 mod 64 bytes)
-  __shared__ __attribute__((aligned(16))) float xs[HP * (16 * CB + 8)];
-  __shared__ __attribute__((aligned(16))) float esw[4][HPB * 16 * ESS];
-  __shared__ __attribute__((aligned(16))) float part[3 * 16 * CB * 16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int NT = 64 * NW, HW = TW + 2, HP = HW * (TH + 2), HPB = (HP + 15) / 16;
+  constexpr int OP = TH * TW, OPB = (OP + 15) / 16;
+  // LDS strides of 32 mod 64 bytes: an x row, a pixel of a wave's expanded
+  // chunk, a pixel of the partial projections
+  constexpr int XS = 16 * CB + 8, ESS = 24, PS = 16 * CB + 8;
+  constexpr int XV = 4 * CB, XSEG = HP * XV, NS = (XSEG + NT - 1) / NT;
+  __shared__ __attribute__((aligned(16))) float xs[HP * XS];
+  __shared__ __attribute__((aligned(16))) float esw[NW][HP * ESS];
+  __shared__ __attribute__((aligned(16))) float part[NW * 16 * PS];
+  static_assert(sizeof(xs) + sizeof(esw) + sizeof(part) <= 160 * 1024, "LDS");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
-  const int KC1 = (C + 15) / 16, XV = KC1 * 4, XS = KC1 * 16 + 8;  // x row: 32 mod 64 bytes
-  const int py = r / TW, px = r - py * TW, hbase = py * HW + px;
   float *const ew = esw[wave];
   const TileWalk walk = tile_walk(ntiles);
-  for (int t = walk.first; t < walk.end; t += walk.step) {
-    const int n = t / tiles_per_image, tt = t - n * tiles_per_image;
-    const int ty0 = (tt / tiles_w) * 4, tx0 = (tt - (tt / tiles_w) * tiles_w) * TW;
-    for (int idx = tid; idx < HP * XV; idx += 256) {
-      const int hp = idx / XV, cv = idx - hp * XV, hy = hp / HW, hx = hp - hy * HW;
-      const int iy = ty0 + hy - 1, ix = tx0 + hx - 1;
-      const bool inside = (unsigned)iy < (unsigned)H && (unsigned)ix < (unsigned)W && 4 * cv < C;
-      const float *src = x + ((size_t)(n * H + (inside ? iy : 0)) * W + (inside ? ix : 0)) * C +
-                         (inside ? 4 * cv : 0);
-      *reinterpret_cast<u32x4 *>(xs + hp * XS + 4 * cv) = masked(*reinterpret_cast<const u32x4 *>(src), inside);
-    }
-    __syncthreads();
-    f32x4 acc2[CB];
+  if (walk.first >= walk.end) return;  // uniform over the workgroup
+
+  // ---- x halo: raw loads (the tile origin for runs outside the image or
+  //      past C), zeroed when written to LDS
+  int xrel[NS], xhyx[NS];
 #pragma unroll
-    for (int ob = 0; ob < CB; ++ob) acc2[ob] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k = wave; k < E / 16; k += 4) {
-      const int e0 = k * 16;
-      // expand: filters e0 + r (A), halo pixels pb*16 + r (B), channels kc*16 + 4q + s
+  for (int s = 0; s < NS; ++s) {
+    const int idx = min(tid + NT * s, XSEG - 1), hp = idx / XV, c = (idx - hp * XV) * 4;
+    const int hy = hp / HW, hx = hp - hy * HW;
+    xhyx[s] = hy | hx << 8 | (c < C ? 0 : 1 << 16);
+    xrel[s] = ((hy - 1) * W + hx - 1) * C + min(c, C - 4);
+  }
+  auto tile_origin = [&](int t, int &n, int &ty0, int &tx0) {
+    n = t / tiles_per_image;
+    const int tt = t - n * tiles_per_image;
+    ty0 = (tt / tiles_w) * TH;
+    tx0 = (tt - (tt / tiles_w) * tiles_w) * TW;
+  };
+  u32x4 st[NS];
+  uint32_t inside_bits = 0;
+  auto fetch = [&](int t) __attribute__((always_inline)) {
+    int n, ty0, tx0;
+    tile_origin(t, n, ty0, tx0);
+    const float *base = x + ((size_t)(n * H + ty0) * W + tx0) * C;
+    inside_bits = 0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const bool inside = !(xhyx[s] >> 16) && (unsigned)(ty0 + (xhyx[s] & 0xff) - 1) < (unsigned)H &&
+                          (unsigned)(tx0 + (xhyx[s] >> 8 & 0xff) - 1) < (unsigned)W;
+      st[s] = *reinterpret_cast<const u32x4 *>(base + (inside ? xrel[s] : 0));
+      inside_bits |= (uint32_t)inside << s;
+    }
+  };
+  auto commit = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int idx = tid + NT * s;
+      if ((s + 1) * NT <= XSEG || idx < XSEG)
+        *reinterpret_cast<u32x4 *>(xs + (idx / XV) * XS + (idx % XV) * 4) =
+            masked(st[s], (inside_bits >> s) & 1u);
+    }
+  };
+
+  // ---- a chunk's filters (expand: filter e0 + r, channels kc*16 + 4q .. +3;
+  //      depthwise taps: channels e0 + 4q .. +3; project: output channel
+  //      ob*16 + r, channels e0 + 4q .. +3).  Past C the loads repeat the
+  //      last channel: the expand's are zeroed where they are used, the
+  //      project's rows are not stored.
+  const int nch = E / 16;
+  Frag16 fe[CB], fp[CB];
+  f32x4 fd[9];
+  auto load_e = [&](int k, int kc) __attribute__((always_inline)) {
+    fe[kc] = load16(we + (uint32_t)((k * 16 + opaque(r)) * C + min(kc * 16 + 4 * q, C - 4)));
+  };
+  auto load_d = [&](int k, int tap) __attribute__((always_inline)) {
+    fd[tap] = *reinterpret_cast<const f32x4 *>(wdw + (uint32_t)(tap * E + k * 16 + 4 * q));
+  };
+  auto load_p = [&](int k, int ob) __attribute__((always_inline)) {
+    fp[ob] = load16(wp + (uint32_t)(min(ob * 16 + opaque(r), C - 1) * E + k * 16 + 4 * q));
+  };
+  fetch(walk.first);
+  const int kfirst = min(wave, nch - 1);
+#pragma unroll
+  for (int kc = 0; kc < CB; ++kc) load_e(kfirst, kc);
+#pragma unroll
+  for (int tap = 0; tap < 9; ++tap) load_d(kfirst, tap);
+#pragma unroll
+  for (int ob = 0; ob < CB; ++ob) load_p(kfirst, ob);
+  commit();
+  __syncthreads();
+
+  int hbase[OPB];  // top left halo pixel of this lane's output pixel (past OP: of the last)
+#pragma unroll
+  for (int b = 0; b < OPB; ++b) {
+    const int p = min(b * 16 + r, OP - 1), py = p / TW;
+    hbase[b] = py * HW + p - py * TW;
+  }
+  for (int t = walk.first; t < walk.end; t += walk.step) {
+    int n, ty0, tx0;
+    tile_origin(t, n, ty0, tx0);
+    fetch(t + walk.step < walk.end ? t + walk.step : t);
+    f32x4 acc2[OPB][CB];
+#pragma unroll
+    for (int b = 0; b < OPB; ++b)
+#pragma unroll
+      for (int ob = 0; ob < CB; ++ob) acc2[b][ob] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k = wave; k < nch; k += NW) {
+      const int kn = k + NW < nch ? k + NW : kfirst;  // the wave's next chunk, this tile's or the next's
       f32x4 acc[HPB];
 #pragma unroll
       for (int pb = 0; pb < HPB; ++pb) acc[pb] = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int kc = 0; kc < KC1; ++kc) {
+#pragma unroll
+      for (int kc = 0; kc < CB; ++kc) {
         const int c = kc * 16 + 4 * q;
-        Frag16 a = load16(we + (size_t)(e0 + r) * C + min(c, C - 4));
+        Frag16 a = fe[kc], bx[HPB];
         a.u = masked(a.u, c < C);
-        Frag16 bx[HPB];
 #pragma unroll
         for (int pb = 0; pb < HPB; ++pb) bx[pb] = load16(xs + min(pb * 16 + r, HP - 1) * XS + c);
 #pragma unroll
         for (int s2 = 0; s2 < 4; ++s2)
 #pragma unroll
           for (int pb = 0; pb < HPB; ++pb) MfmaF32::step(acc[pb], a, bx[pb], s2);
+        load_e(kn, kc);
       }
       // ReLU6, then the zero padding of the expanded tensor outside the image
 #pragma unroll
       for (int pb = 0; pb < HPB; ++pb) {
         const int hp = pb * 16 + r, hy = hp / HW, hx = hp - hy * HW;
         const bool inside = (unsigned)(ty0 + hy - 1) < (unsigned)H && (unsigned)(tx0 + hx - 1) < (unsigned)W;
-        if (hp < HP) {
+        if (pb * 16 + 15 < HP || hp < HP) {
           f32x4 v;
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = inside ? relu6(acc[pb][e]) : 0.0f;
@@ -435,77 +518,94 @@ __global__ __launch_bounds__(256, 1) void irb_stream_kernel(
       }
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      // depthwise: output pixel r, channels e0 + 4q .. +3
-      f32x4 d = {0.f, 0.f, 0.f, 0.f};
+      // depthwise: the lane's output pixels, channels e0 + 4q .. +3
+      Frag16 bd[OPB];
 #pragma unroll
-      for (int tap = 0; tap < 9; ++tap)
-        d += *reinterpret_cast<const f32x4 *>(ew + (hbase + (tap / 3) * HW + (tap % 3)) * ESS + 4 * q) *
-             *reinterpret_cast<const f32x4 *>(wdw + tap * E + e0 + 4 * q);
-      Frag16 bd;
-      bd.f = f32x4{relu6(d[0]), relu6(d[1]), relu6(d[2]), relu6(d[3])};
-      // project: output channels ob*16 + r (A: wp rows), the chunk's channels
+      for (int b = 0; b < OPB; ++b) {
+        f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap)
+          d += *reinterpret_cast<const f32x4 *>(ew + (hbase[b] + (tap / 3) * HW + (tap % 3)) * ESS + 4 * q) * fd[tap];
+        bd[b].f = f32x4{relu6(d[0]), relu6(d[1]), relu6(d[2]), relu6(d[3])};
+      }
+#pragma unroll
+      for (int tap = 0; tap < 9; ++tap) load_d(kn, tap);
 #pragma unroll
       for (int ob = 0; ob < CB; ++ob) {
-        if (ob * 16 < C) {
-          const int co = ob * 16 + r;
-          Frag16 a = load16(wp + (size_t)min(co, C - 1) * E + e0 + 4 * q);
-          a.u = masked(a.u, co < C);
-          MfmaF32::mma(acc2[ob], a, bd);
-        }
+#pragma unroll
+        for (int b = 0; b < OPB; ++b) MfmaF32::mma(acc2[b][ob], fp[ob], bd[b]);
+        load_p(kn, ob);
       }
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    if (wave > 0) {
+    float *const ot = out + ((size_t)(n * H + ty0) * W + tx0) * C;
+#pragma unroll
+    for (int b = 0; b < OPB; ++b) {
+      if (b > 0) __syncthreads();  // part is read out
 #pragma unroll
       for (int ob = 0; ob < CB; ++ob)
-        if (ob * 16 < C)
-          *reinterpret_cast<f32x4 *>(part + ((wave - 1) * 16 + r) * CB * 16 + ob * 16 + 4 * q) = acc2[ob];
-    }
-    __syncthreads();
-    if (wave == 0 && ty0 + py < H && tx0 + px < W) {
-      float *o = out + ((size_t)(n * H + ty0 + py) * W + tx0 + px) * C;
+        *reinterpret_cast<f32x4 *>(part + (wave * 16 + r) * PS + ob * 16 + 4 * q) = acc2[b][ob];
+      __syncthreads();
+      for (int i = tid; i < 16 * XV; i += NT) {
+        const int pl = i / XV, c = (i - pl * XV) * 4, p = b * 16 + pl, py = p / TW, px = p - py * TW;
+        if (p < OP && c < C && ty0 + py < H && tx0 + px < W) {
+          f32x4 v = *reinterpret_cast<const f32x4 *>(part + pl * PS + c);
 #pragma unroll
-      for (int ob = 0; ob < CB; ++ob) {
-        const int c = ob * 16 + 4 * q;
-        if (ob * 16 < C) {
-          f32x4 v = acc2[ob];
-#pragma unroll
-          for (int w2 = 0; w2 < 3; ++w2)
-            v += *reinterpret_cast<const f32x4 *>(part + (w2 * 16 + r) * CB * 16 + ob * 16 + 4 * q);
-          v += *reinterpret_cast<const f32x4 *>(xs + (hbase + HW + 1) * XS + c);
-          if (c < C) *reinterpret_cast<f32x4 *>(o + c) = v;
+          for (int w2 = 1; w2 < NW; ++w2)
+            v += *reinterpret_cast<const f32x4 *>(part + (w2 * 16 + pl) * PS + c);
+          v += *reinterpret_cast<const f32x4 *>(xs + ((py + 1) * HW + px + 1) * XS + c);
+          *reinterpret_cast<f32x4 *>(ot + ((size_t)py * W + px) * C + c) = v;
         }
       }
     }
     __syncthreads();  // xs and part are the next tile's
+    commit();
+    __syncthreads();
   }
 }
 
-template <int CB>
+template <int CB, int TH, int TW, int NW>
 hipError_t launch_irb_stream(const IrbArgs &a, hipStream_t s) {
-  auto kern = irb_stream_kernel<CB>;
-  const int tiles_w = (a.W + 3) / 4, tiles_h = (a.H + 3) / 4;
+  auto kern = irb_stream_kernel<CB, TH, TW, NW>;
+  constexpr int HP = (TH + 2) * (TW + 2), HPB = (HP + 15) / 16, OPB = (TH * TW + 15) / 16;
+  const int tiles_w = (a.W + TW - 1) / TW, tiles_h = (a.H + TH - 1) / TH;
   const int per_image = tiles_w * tiles_h, ntiles = a.N * per_image;
-  const int full = persistent_grid(kern);
+  const int full = persistent_grid(kern, 64 * NW);
   if (full == 0) return hipErrorInvalidDeviceFunction;
   const int g = ntiles < full ? (ntiles + kXcds - 1) / kXcds * kXcds : full;
   {
-    const int KC1 = (a.C + 15) / 16, CBr = (a.C + 15) / 16, chunks = a.E / 16;
-    npu_launch_plan p = make_plan("mbv2_inverted_residual_stream", g, wg_per_cu(kern), ntiles, 32);
-    p.load_phases = 1 + (chunks + 3) / 4;  // the halo, then each chunk's filters from L2
-    p.tile_macs = (double)a.E * 48 * KC1 * 16 + 16.0 * CBr * 16 * a.E;
-    p.tile_valu = 4.0 * (40.0 + (chunks + 3) / 4 * (30.0 + 12.0 * KC1 + 8.0 * CBr));
-    p.tile_lds_bytes = 36.0 * KC1 * 16 * 4 * 2 + chunks * (48.0 * 16 * 4 * KC1 + 36.0 * 16 * 4 + 9.0 * 16 * 16 * 4) +
-                       3.0 * 16 * CBr * 16 * 4 * 2;
-    p.tile_load_bytes = 36.0 * a.C * 4 + chunks * 4.0 * (16.0 * a.C + 9.0 * 16 + 16.0 * a.C);
-    p.tile_store_bytes = 16.0 * a.C * 4;
+    // in units of four waves, as the launch model counts workgroups
+    const double units = NW / 4.0, chunks = a.E / 16, per_wave = (a.E / 16 + NW - 1) / NW;
+    npu_launch_plan p = make_plan("mbv2_inverted_residual_stream", (int)(g * units),
+                                  wg_per_cu(kern, 64 * NW), (int)(ntiles * units), 32);
+    p.load_phases = 1;  // the first halo; the filters and later halos are fetched ahead
+    p.tile_macs = ((double)a.E * HPB * 16 * CB * 16 + OPB * 16.0 * CB * 16 * a.E) / units;
+    p.tile_valu = 4.0 * (60.0 + per_wave * (8.0 * CB + 14.0 * HPB + 60.0 * OPB));
+    p.tile_lds_bytes = (HP * CB * 16 * 4.0 * 2 +
+                        chunks * (HPB * 16.0 * 16 * 4 * CB + HP * 16 * 4.0 + OPB * 9.0 * 16 * 16 * 4) +
+                        2.0 * NW * OPB * 16 * CB * 16 * 4) / units;
+    p.tile_load_bytes = (HP * a.C * 4.0 + chunks * 4.0 * (32.0 * a.C + 9.0 * 16)) / units;
+    p.tile_store_bytes = TH * TW * a.C * 4.0 / units;
     p.hbm_bytes = 4.0 * (2.0 * a.N * a.H * a.W * a.C + 2.0 * a.C * a.E + 9.0 * a.E);
     plans_add(p);
   }
-  hipLaunchKernelGGL(kern, dim3(g), dim3(256), 0, s, a.x, a.we, a.wdw, a.wp, a.out, a.H, a.W, a.C,
+  hipLaunchKernelGGL(kern, dim3(g), dim3(64 * NW), 0, s, a.x, a.we, a.wdw, a.wp, a.out, a.H, a.W, a.C,
                      a.E, tiles_w, per_image, ntiles);
   return hipGetLastError();
+}
+
+// 4 x 7 tiles (4 blocks of halo pixels and 2 of output pixels) or 4 x 4 (3 and
+// 1), whichever takes the busiest CU fewer blocks: 4 x 7 at 14x14 and batch
+// 32 (256 tiles, one per CU, against 512), 4 x 4 for small batches.
+template <int CB, int NW>
+hipError_t launch_irb_stream_t(const IrbArgs &a, hipStream_t s) {
+  auto rounds = [&](int tw) {
+    const long long tiles = (long long)a.N * ((a.H + 3) / 4) * ((a.W + tw - 1) / tw);
+    return (tiles + 255) / 256;
+  };
+  if (6 * rounds(7) < 4 * rounds(4)) return launch_irb_stream<CB, 4, 7, NW>(a, s);
+  return launch_irb_stream<CB, 4, 4, NW>(a, s);
 }
 
 bool irb_tuned(int C, int E) {
@@ -523,10 +623,17 @@ hipError_t launch_irb_f32(const IrbArgs &a, hipStream_t s) {
   if (a.C == 16 && a.E == 96) return launch_irb_t<16, 96>(a, s);
   if (a.C == 32 && a.E == 192) return launch_irb_t<32, 192>(a, s);
   if (!irb_supported(a.C, a.E)) return hipErrorInvalidValue;
-  if (a.C <= 32) return launch_irb_stream<2>(a, s);
-  if (a.C <= 64) return launch_irb_stream<4>(a, s);
-  if (a.C <= 128) return launch_irb_stream<8>(a, s);
-  return launch_irb_stream<20>(a, s);
+  // eight waves where E has a chunk for each (up to 32 channels four are
+  // enough: 32x28x29x20/112 15.8 us against 17.4); past 160 channels the
+  // registers and LDS of eight do not hold a pixel block's sums
+  const bool wide = a.E >= 128;
+  if (a.C <= 16) return launch_irb_stream_t<1, 4>(a, s);
+  if (a.C <= 32) return launch_irb_stream_t<2, 4>(a, s);
+  if (a.C <= 64) return wide ? launch_irb_stream_t<4, 8>(a, s) : launch_irb_stream_t<4, 4>(a, s);
+  if (a.C <= 96) return wide ? launch_irb_stream_t<6, 8>(a, s) : launch_irb_stream_t<6, 4>(a, s);
+  if (a.C <= 128) return wide ? launch_irb_stream<8, 4, 4, 8>(a, s) : launch_irb_stream<8, 4, 4, 4>(a, s);
+  if (a.C <= 160) return wide ? launch_irb_stream<10, 4, 4, 8>(a, s) : launch_irb_stream<10, 4, 4, 4>(a, s);
+  return launch_irb_stream<20, 4, 4, 4>(a, s);
 }
 
 }  // namespace npu

@@ -21,8 +21,8 @@ def _codes():
 
 
 # NpuMemref's layout by rank, the sizes and strides past the rank left zero.
-# Packing a descriptor in one call takes 2.9 us where assigning its fields one
-# by one took 6.3 (every group call builds four to eleven of them
+# Packing a descriptor in one call takes 1.8 us where assigning its fields one
+# by one took 6.3; every group call builds four to eleven of them.
 _PACK = [struct.Struct(f"<QQq{r}q{8 * (4 - r)}x{r}q{8 * (4 - r)}xii") for r in range(5)]
 assert all(p.size == C.sizeof(NpuMemref) for p in _PACK)
 

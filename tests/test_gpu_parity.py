@@ -560,6 +560,12 @@ def test_c3_irb_shapes(cuda, N, H, W, C, E):
     (2, 5, 6, 8, 16),       # fewer chunks than waves
     (1, 6, 5, 320, 1280),   # the largest C
     (4, 30, 31, 24, 96),    # more tiles than resident workgroups
+    (32, 10, 13, 64, 48),   # 4 x 7 tiles: ragged rows and columns, fewer chunks than waves
+    (32, 9, 12, 96, 144),   # more chunks than waves, the last round partly idle
+    (80, 10, 14, 40, 64),   # several tiles per workgroup
+    (33, 10, 14, 28, 80),   # four waves
+    (2, 9, 10, 12, 64),     # one channel block
+    (2, 7, 9, 124, 112), (2, 7, 9, 112, 144), (2, 7, 9, 144, 96), (2, 7, 9, 80, 64),
 ])
 def test_c3_irb_any_channels(cuda, N, H, W, C, E):
     """(C, E) outside the tuned instances run on the kernel that streams the
