@@ -143,6 +143,31 @@ void conv2d_nchw_split_kernel(const NchwArgs a) {
   };
   stage(0);
 
+  // ---- the outputs this thread finishes, and their bias and residual: with
+  //      few of them they are loaded here, so that the epilogue does not wait
+  //      for memory once per output.  Outputs that do not exist, and operands
+  //      that are absent, load the input's first word instead.
+  constexpr int NE = (16 * WF * PX + NT - 1) / NT;  // outputs per thread
+  constexpr bool PRE = NE <= 4;
+  // output e (filter e / PX of the workgroup's, pixel e % PX): its index, or -1
+  auto out_at = [&](int e, int &f) __attribute__((always_inline)) {
+    const int px = e % PX, p = p0 + px, oy = a.by_tw.div(p), ox = p - oy * a.tw;
+    f = fb * WF * 16 + e / PX;
+    const bool ok = e < 16 * WF * PX && oy < a.Ho && ox < tw && f < a.F;
+    return ok ? ((n * a.F + f) * a.Ho + oy) * a.Wo + ox0 + ox : -1;
+  };
+  float rv[PRE ? NE : 1], bv[PRE ? NE : 1];
+  if constexpr (PRE) {
+    const float *const rp = a.res ? a.res : a.x, *const bp = a.bias ? a.bias : a.x;
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+      int f;
+      const int o = out_at(tid + NT * i, f);
+      rv[i] = rp[o >= 0 && a.res ? o : 0];
+      bv[i] = bp[o >= 0 && a.bias ? f : 0];
+    }
+  }
+
   // ---- where k lies in the patches
   for (int k = tid; k < KT; k += NT) {
     const int c = a.by_t.div(k), t = k - c * a.T, kh = a.by_kw.div(t), kw = t - kh * (int)a.by_kw.d;
@@ -225,16 +250,17 @@ void conv2d_nchw_split_kernel(const NchwArgs a) {
     *reinterpret_cast<f32x4 *>(red + ((size_t)wave * 16 + r) * RS + 16 * i + 4 * q) = acc[i];
   __syncthreads();
   const ActBounds ab = act_bounds(a.act);
-  for (int e = tid; e < 16 * WF * PX; e += NT) {
-    const int px = e % PX, fl = e / PX;  // filter fl: wave fl / 16's block, row fl % 16
-    float v = 0.0f;
 #pragma unroll
-    for (int k = 0; k < WK; ++k) v += red[((size_t)(k * WF) * 16 + fl) * RS + px];
-    const int p = p0 + px, oy = a.by_tw.div(p), ox = p - oy * a.tw, f = fb * WF * 16 + fl;
-    if (oy < a.Ho && ox < tw && f < a.F) {
-      const size_t o = ((size_t)(n * a.F + f) * a.Ho + oy) * a.Wo + ox0 + ox;
-      if (a.bias) v += a.bias[f];
-      if (a.res) v += a.res[o];
+  for (int i = 0; i < NE; ++i) {
+    const int e = tid + NT * i, px = e % PX, fl = e / PX;  // filter fl: wave fl / 16's block, row fl % 16
+    int f;
+    const int o = out_at(e, f);
+    if (o >= 0) {
+      float v = 0.0f;
+#pragma unroll
+      for (int k = 0; k < WK; ++k) v += red[((size_t)(k * WF) * 16 + fl) * RS + px];
+      if (a.bias) v += PRE ? bv[PRE ? i : 0] : a.bias[f];
+      if (a.res) v += PRE ? rv[PRE ? i : 0] : a.res[o];
       a.out[o] = act_clamp(v, ab);
     }
   }
