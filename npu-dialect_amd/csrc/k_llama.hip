@@ -395,7 +395,8 @@ __global__ __launch_bounds__(GT) void llama_gemm_kernel(const LlamaGemmArgs a, i
 // whole A panel in LDS: right for one tile per CU, but at S = 2048 they reached
 // 134 TFLOP/s.  Here a wave holds a (BM / 2) x (BN / 2) part of the tile (per
 // weight), A and B stream through two LDS buffers, one barrier per step, the
-// next step's loads in flight, two workgroups per CU.  The RMSNorm is folded in
+// next one or two steps' loads in flight, two workgroups per CU; what bounds it
+// is the fragments' LDS reads (twice the MFMAs' time at 64 x 64).  The RMSNorm is folded in
 // without a pass of its own: A is staged as bf16(x g) -- one rounding, as
 // bf16(x inv g) has -- while the same registers feed the row's sum of squares,
 // and the accumulator is scaled by the row's inv in f32 at the end.
@@ -442,37 +443,47 @@ __global__ __launch_bounds__(256, 2) void llama_tile_kernel(const LlamaGemmArgs 
     bp[i] = a.B[part] + (size_t)k * Np + col;
     bdst[i] = S::ABYTES + (nb * S::STRIPS + cc / 2) * S::SB + strip_row(k) * 32 + (cc & 1) * 16;
   }
-  u32x4 av[AR], bv[BR];
-  f32x4 g0, g1;
-  auto fetch = [&](int k0) __attribute__((always_inline)) {
+  // Register sets of staged runs: a step is 128 to 256 clocks of MFMAs per
+  // wave, less than a load from L2 takes, so each step's loads are issued DEP
+  // steps before they are committed.  us with one / two: down projection
+  // 2048x2048x768 18.1 / 17.5, 512x2048x768 9.8 / 8.5, 1024x1408x512 7.7 / 6.8;
+  // SwiGLU 2048x768x2048 23.0 / 21.8, 300x768x2048 10.4 / 9.8; QKV 1024x512
+  // 9.2 / 9.9, 512x768 11.2 / 12.1 (registers of the RMSNorm's staging), so one.
+  constexpr int DEP = EPI == kEpiQkvRope ? 1 : 2;
+  u32x4 av[DEP][AR], bv[DEP][BR];
+  f32x4 gv[DEP][2];
+  auto fetch = [&](int set, int k0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < AR; ++i) av[i] = *reinterpret_cast<const u32x4 *>(ap[i] + k0);
+    for (int i = 0; i < AR; ++i) av[set][i] = *reinterpret_cast<const u32x4 *>(ap[i] + k0);
     if constexpr (PRO == kProRmsnorm) {
-      g0 = *reinterpret_cast<const f32x4 *>(a.gamma + k0 + seg * 8);
-      g1 = *reinterpret_cast<const f32x4 *>(a.gamma + k0 + seg * 8 + 4);
+      gv[set][0] = *reinterpret_cast<const f32x4 *>(a.gamma + k0 + seg * 8);
+      gv[set][1] = *reinterpret_cast<const f32x4 *>(a.gamma + k0 + seg * 8 + 4);
     }
 #pragma unroll
-    for (int i = 0; i < BR; ++i) bv[i] = *reinterpret_cast<const u32x4 *>(bp[i] + (size_t)k0 * Np);
+    for (int i = 0; i < BR; ++i) bv[set][i] = *reinterpret_cast<const u32x4 *>(bp[i] + (size_t)k0 * Np);
   };
   float ss[AR];
 #pragma unroll
   for (int i = 0; i < AR; ++i) ss[i] = 0.0f;
+  // a register set to LDS buffer `buf`
   auto commit = [&](int buf) __attribute__((always_inline)) {
+    const int set = buf % DEP;
 #pragma unroll
     for (int i = 0; i < AR; ++i) {
-      u32x4 o = av[i];
+      u32x4 o = av[set][i];
       if constexpr (PRO == kProRmsnorm) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float lo = bf_lo(av[i][e]), hi = bf_hi(av[i][e]);
+          const float lo = bf_lo(o[e]), hi = bf_hi(o[e]);
+          const f32x4 g = gv[set][e / 2];
           ss[i] = fmaf(hi, hi, fmaf(lo, lo, ss[i]));
-          o[e] = cvt_pk_bf16(lo * (e < 2 ? g0[2 * e] : g1[2 * e - 4]), hi * (e < 2 ? g0[2 * e + 1] : g1[2 * e - 3]));
+          o[e] = cvt_pk_bf16(lo * g[2 * (e & 1)], hi * g[2 * (e & 1) + 1]);
         }
       }
       *reinterpret_cast<u32x4 *>(adst + buf * S::BUF + 32 * i * S::AREC) = o;
     }
 #pragma unroll
-    for (int i = 0; i < BR; ++i) *reinterpret_cast<u32x4 *>(smem + buf * S::BUF + bdst[i]) = bv[i];
+    for (int i = 0; i < BR; ++i) *reinterpret_cast<u32x4 *>(smem + buf * S::BUF + bdst[i]) = bv[set][i];
   };
 
   f32x4 acc[NB][TM][TN];
@@ -483,13 +494,8 @@ __global__ __launch_bounds__(256, 2) void llama_tile_kernel(const LlamaGemmArgs 
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const unsigned char *const arow = smem + (wr * (BM / 2) + ml) * S::AREC + (lane >> 4) * 16;
-  const int steps = K / KC;
-  fetch(0);
-  commit(0);
-  fetch(min(KC, K - KC));
-  __syncthreads();
-  for (int s = 0; s < steps; ++s) {
-    const int off = (s & 1) * S::BUF;
+  auto multiply = [&](int buf) __attribute__((always_inline)) {
+    const int off = buf * S::BUF;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       Frag16 xf[TM], wf[NB][TN];
@@ -508,11 +514,32 @@ __global__ __launch_bounds__(256, 2) void llama_tile_kernel(const LlamaGemmArgs 
           for (int j = 0; j < TN; ++j)
             acc[b][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[b][j].h, xf[i].h, acc[b][i][j], 0, 0, 0);
     }
-    if (s + 1 < steps) {
-      commit((s + 1) & 1);
-      fetch(min((s + 2) * KC, K - KC));
-    }
+  };
+  // Step s is in buffer s % 2 and passed through register set s % DEP.  Past
+  // the last step the loads repeat it and are never committed (a condition on
+  // them would make the wave wait for them at once).
+  const int steps = K / KC, klast = K - KC;
+  fetch(0, 0);
+  if constexpr (DEP == 2) fetch(1, min(KC, klast));
+  commit(0);
+  fetch(0, min(DEP * KC, klast));
+  __syncthreads();
+  int s = 0;
+  for (; s + 2 < steps; s += 2) {
+    multiply(0);
+    commit(1);
+    fetch(1 % DEP, min((s + 1 + DEP) * KC, klast));
     __syncthreads();
+    multiply(1);
+    commit(0);
+    fetch(0, min((s + 2 + DEP) * KC, klast));
+    __syncthreads();
+  }
+  multiply(0);
+  if (s + 1 < steps) {
+    commit(1);
+    __syncthreads();
+    multiply(1);
   }
   if constexpr (PRO == kProRmsnorm) {
     // the eight lanes of a row: xor 1, 2 (quad permutes), then the half-row mirror
