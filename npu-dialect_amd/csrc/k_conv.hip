@@ -12,8 +12,8 @@
 // A workgroup of 2 x 2 waves owns BM pixels x BN filters.  The reduction walks
 // the taps and, within a tap, chunks of 128 bytes of channels; per step the
 // pixels' runs (zero outside the image and past C) and the filters' runs are
-// staged in LDS, double-buffered, the next step's loads in flight while the
-// current one is multiplied, one barrier per step.  The filter fragment is the
+// staged in LDS, double-buffered, the next two steps' loads in flight while
+// the current one is multiplied, one barrier per step.  The filter fragment is the
 // MFMA's first operand, so a lane ends with four consecutive filters of one
 // pixel: the epilogue (bias add, residual add, act, and the bf16 rounding of
 // the bf16 variant) runs on the accumulators and stores 8 or 16 bytes.
@@ -71,32 +71,32 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
   for (int i = 0; i < BR; ++i) bbase[i] = min(f0 + row0 + 32 * i, a.F - 1) * a.taps * a.C;
   // Loads from clamped addresses now, zeros chosen when the runs are written
   // (a select on a loaded value would make the wave wait for it there).
-  u32x4 av[AR], bv[BR];
-  uint32_t keep = 0;
-  auto fetch = [&](int kh, int kw, int c0) __attribute__((always_inline)) {
+  u32x4 av[2][AR], bv[2][BR];
+  uint32_t keep[2];
+  auto fetch = [&](int set, int kh, int kw, int c0) __attribute__((always_inline)) {
     const int c = c0 + seg * RUN;
     const bool cin = c < a.C;
     const int cc = cin ? c : 0;
-    keep = (uint32_t)cin << AR;
+    keep[set] = (uint32_t)cin << AR;
 #pragma unroll
     for (int i = 0; i < AR; ++i) {
       const int ih = aoh[i] + kh, iw = aow[i] + kw;
       const bool in = (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
-      av[i] = *reinterpret_cast<const u32x4 *>(x + (size_t)(abase[i] + (in ? ih * a.W + iw : 0)) * a.C + cc);
-      keep |= (uint32_t)(in && cin) << i;
+      av[set][i] = *reinterpret_cast<const u32x4 *>(x + (size_t)(abase[i] + (in ? ih * a.W + iw : 0)) * a.C + cc);
+      keep[set] |= (uint32_t)(in && cin) << i;
     }
     const int tap = (kh * a.KW + kw) * a.C + cc;
 #pragma unroll
-    for (int i = 0; i < BR; ++i) bv[i] = *reinterpret_cast<const u32x4 *>(w + (size_t)(bbase[i] + tap));
+    for (int i = 0; i < BR; ++i) bv[set][i] = *reinterpret_cast<const u32x4 *>(w + (size_t)(bbase[i] + tap));
   };
   unsigned char *const dst = lds + row0 * REC + seg * 16;
   auto commit = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < AR; ++i)
-      *reinterpret_cast<u32x4 *>(dst + buf * BUF + 32 * i * REC) = masked(av[i], (keep >> i) & 1u);
+      *reinterpret_cast<u32x4 *>(dst + buf * BUF + 32 * i * REC) = masked(av[buf][i], (keep[buf] >> i) & 1u);
 #pragma unroll
     for (int i = 0; i < BR; ++i)
-      *reinterpret_cast<u32x4 *>(dst + buf * BUF + (BM + 32 * i) * REC) = masked(bv[i], (keep >> AR) & 1u);
+      *reinterpret_cast<u32x4 *>(dst + buf * BUF + (BM + 32 * i) * REC) = masked(bv[buf][i], (keep[buf] >> AR) & 1u);
   };
 
   typename MM::acc_t acc[TM][TN];
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
     for (int j = 0; j < TN; ++j) acc[i][j] = typename MM::acc_t{0, 0, 0, 0};
 
   // steps in order (kh, kw, channel chunk); the coordinates of the step being
-  // fetched run one ahead, and stay on the last step past the end
+  // fetched run ahead, and stay in the last filter row past the end
   const int chunks = (a.C + KC - 1) / KC, steps = a.taps * chunks, KH = a.taps / a.KW;
   int kh = 0, kw = 0, ch = 0;
   auto advance = [&]() __attribute__((always_inline)) {
@@ -115,16 +115,11 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
       if (++kw == a.KW) kw = 0, kh = min(kh + 1, KH - 1);
     }
   };
-  fetch(0, 0, 0);
-  commit(0);
-  advance();
-  fetch(kh, kw, ch * KC);
-  __syncthreads();
   const unsigned char *const arow = lds + (wp * (BM / 2) + r) * REC + q * 16;
   const unsigned char *const brow = lds + (BM + wf * (BN / 2) + r) * REC + q * 16;
   int mch = 0;  // channel chunk of the step being multiplied
-  for (int s = 0; s < steps; ++s) {
-    const int off = (s & 1) * BUF;
+  auto multiply = [&](int buf) __attribute__((always_inline)) {
+    const int off = buf * BUF;
     const int frags = min(2, (a.C - mch * KC + KC / 2 - 1) / (KC / 2));
     if (++mch == chunks) mch = 0;
 #pragma unroll
@@ -143,12 +138,39 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
             for (int j = 0; j < TN; ++j) MM::step(acc[i][j], bf[j], af[i], st);
       }
     }
-    if (s + 1 < steps) {
-      commit((s + 1) & 1);
-      advance();
-      fetch(kh, kw, ch * KC);
-    }
+  };
+  auto fetch_next = [&](int set) __attribute__((always_inline)) {
+    fetch(set, kh, kw, ch * KC);
+    advance();
+  };
+  // Step s is in buffer s % 2 and passed through register set s % 2: its loads
+  // are issued two steps before they are committed (a step's MFMAs take less
+  // time than a load from L2; us with one step / two: bf16 7x7x512 batch 32
+  // 35.5 / 33.4, 28x28x128 batch 4 8.6 / 8.05, 5x5 30x30x64 batch 2 10.4 /
+  // 9.55, f32 14x14x256 97 / 90; with more workgroups per CU, 28x28x128 batch
+  // 32, the fragments' LDS reads bound it and it stays at 21.8).  Past the last step the
+  // loads stay inside the filter's last row and are never committed.
+  fetch_next(0);
+  fetch_next(1);
+  commit(0);
+  fetch_next(0);
+  __syncthreads();
+  int s = 0;
+  for (; s + 2 < steps; s += 2) {
+    multiply(0);
+    commit(1);
+    fetch_next(1);
     __syncthreads();
+    multiply(1);
+    commit(0);
+    fetch_next(0);
+    __syncthreads();
+  }
+  multiply(0);
+  if (s + 1 < steps) {
+    commit(1);
+    __syncthreads();
+    multiply(1);
   }
 
   // Epilogue: pixel r of each block, its filters 4q .. +3.
@@ -216,7 +238,7 @@ hipError_t launch_tile(const ConvArgs &c, hipStream_t s) {
   const int G = a.npt * a.nft, grid = (G + kXcds - 1) / kXcds * kXcds;
   const double steps = (double)a.taps * ((a.C + 128 / sizeof(T) - 1) / (128 / sizeof(T)));
   npu_launch_plan p = make_plan("conv2d_nhwc", G, wg_per_cu(kern), G, 8 * sizeof(T));
-  p.load_phases = 1;  // a step's loads are in flight during the step before
+  p.load_phases = 1;  // a step's loads are in flight during the two before
   p.tile_macs = (double)BM * BN * steps * 128 / sizeof(T);
   p.tile_valu = 4.0 * (steps * (10.0 * (BM + BN) / 32 + 20.0) + 12.0 * BM * BN / 1024 + 120.0);
   p.tile_lds_bytes = steps * (128.0 * (BM + BN) + 4.0 * 2 * 1024 * (BM + BN) / 32);
