@@ -26,8 +26,8 @@ namespace npu {
 
 namespace {
 
-// Output tile TH x TW: 8 x 8 when the batch has tiles enough for every CU,
-// 4 x 4 below that (more workgroups, each with a shorter serial chain; the
+// Output tile TH x TW: 8 x 8 or 8 x 7 when the batch has tiles enough for every
+// CU (8 x 7 has 90 halo pixels, 6 MFMA blocks against 7), 4 x 4 below that (more workgroups, each with a shorter serial chain; the
 // expand conv is recomputed on 36 halo pixels for 16 outputs instead of 100
 // for 64, which idle CUs pay for).
 template <int TH, int TW>
@@ -36,11 +36,11 @@ struct IrbTile {
   static constexpr int HP = HW * (TH + 2);    // halo pixels (100 for 8 x 8)
   static constexpr int HPB = (HP + 15) / 16;  // blocks of 16 halo pixels
   static constexpr int OP = TH * TW;          // output pixels
-  static constexpr int OPB = OP / 16;         // blocks of 16 output pixels
+  static constexpr int OPB = (OP + 15) / 16;  // blocks of 16 output pixels
   // the depthwise/project stage: wave w takes output block w % OPB and
   // channel group w / OPB of CS (CS > 1: partial projections summed in LDS)
   static constexpr int CS = 4 / OPB;
-  static_assert(OP % 16 == 0 && 4 % OPB == 0, "one to four output blocks");
+  static_assert(4 % OPB == 0, "one, two or four output blocks");
 };
 
 __device__ __forceinline__ float relu6(float v) { return act_clamp(v, ActBounds{0.0f, 6.0f}); }
@@ -180,7 +180,9 @@ __global__ __launch_bounds__(256, E >= 192 ? 1 : 2) void irb_kernel(const float 
     for (int fb = 0; fb < FB2; ++fb) settle(bp[j][fb].u);
   __syncthreads();
 
-  const int p = ob * 16 + r, py = p / TW, px = p - py * TW;
+  // past the tile's pixels (the last block of 8 x 7): the last one, not stored
+  const int p = min(ob * 16 + r, TH * TW - 1), py = p / TW, px = p - py * TW;
+  const bool own = ob * 16 + r < TH * TW;
   const int hbase = py * HW + px;
   const uint32_t ooff = (uint32_t)(((py * W + px) * C + 4 * q) * 4);
 
@@ -294,7 +296,7 @@ __global__ __launch_bounds__(256, E >= 192 ? 1 : 2) void irb_kernel(const float 
     }
     commit();
     fetch(next_of(next_of(t)));
-    if ((CS == 1 || cg == 0) && ty0 + py < H && tx0 + px < W) {
+    if ((CS == 1 || cg == 0) && own && ty0 + py < H && tx0 + px < W) {
       char *ob = reinterpret_cast<char *>(out) + ((size_t)(n * H + ty0) * W + tx0) * C * 4;
 #pragma unroll
       for (int fb = 0; fb < FB2; ++fb)
@@ -308,7 +310,7 @@ __global__ __launch_bounds__(256, E >= 192 ? 1 : 2) void irb_kernel(const float 
 template <int C, int E, int TH, int TW>
 hipError_t launch_irb_tile(const IrbArgs &a, hipStream_t s) {
   using Tl = IrbTile<TH, TW>;
-  constexpr int HP = Tl::HP, HPB = Tl::HPB, OP = Tl::OP;
+  constexpr int HP = Tl::HP, HPB = Tl::HPB, OPB = Tl::OPB, OP = Tl::OP;
   auto kern = irb_kernel<C, E, TH, TW>;
   const int tiles_w = (a.W + TW - 1) / TW, tiles_h = (a.H + TH - 1) / TH;
   const int per_image = tiles_w * tiles_h, ntiles = a.N * per_image;
@@ -321,7 +323,7 @@ hipError_t launch_irb_tile(const IrbArgs &a, hipStream_t s) {
     constexpr int KC1 = (C + 15) / 16, FB2 = (C + 15) / 16, FB1 = E / 16;
     npu_launch_plan p = make_plan("mbv2_inverted_residual", g, wg_per_cu(kern), ntiles, 32);
     p.load_phases = 0;  // the next tile's halo is fetched during this tile
-    p.tile_macs = (double)E * HPB * 16 * KC1 * 16 + (double)OP * FB2 * 16 * E;
+    p.tile_macs = (double)E * HPB * 16 * KC1 * 16 + (double)OPB * 16 * FB2 * 16 * E;
     // Vector instructions per wave and tile, counted in the compiled code
     // (gfx950 assembly, <24, 144, 8, 8>): 81 for the tile (halo commit and
     // fetch addresses, residual, stores, loop control); 13.4 per expand unit
@@ -331,12 +333,12 @@ hipError_t launch_irb_tile(const IrbArgs &a, hipStream_t s) {
     // OP / 16 blocks over four waves: 706 per 8 x 8 tile at E = 144.
     // Set-up: 330 (the filter staging and the first halo's addresses; 254
     // for the 4 x 4 tile's 36-pixel halo, <24, 144, 4, 4>).
-    p.tile_valu = 4.0 * (81.0 + FB1 * HPB / 4.0 * 13.4 + 46.0 * (E / 16) * (OP / 16) / 4.0);
+    p.tile_valu = 4.0 * (81.0 + FB1 * HPB / 4.0 * 13.4 + 46.0 * (E / 16) * OPB / 4.0);
     p.wg_setup_valu = 4.0 * (TH == 4 ? 254.0 : 330.0);
     p.tile_lds_bytes = HP * (KC1 * 16 + 8) * 4.0 +                // halo written
                        (E / 16.0) * KC1 * HPB * 1024 +            // expand A read
                        HP * E * 4.0 +                             // expanded tile written
-                       2.0 * (OP / 16) * (E / 16) * 9 * 1024 +    // depthwise taps and weights read
+                       2.0 * OPB * (E / 16) * 9 * 1024 +    // depthwise taps and weights read
                        OP * C * 4.0;                              // residual
     p.tile_load_bytes = HP * C * 4.0;
     p.tile_store_bytes = OP * C * 4.0;
@@ -349,14 +351,22 @@ hipError_t launch_irb_tile(const IrbArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// 8 x 8 tiles when there are at least as many as CUs, else 4 x 4.
+// 4 x 4 tiles when there are fewer of 8 x 8 than CUs; else 8 x 8 or 8 x 7,
+// whichever takes the busiest CU fewer MFMAs: at 56x56 and batch 32 both give
+// it seven tiles, of 792 and 720 (24/144).  us, 8 x 8 / 8 x 7: that 38.9 / 36.1,
+// 16/96 21.5 / 19.3, 32/192 66.1 / 61.4, batch 16 24/144 25.6 / 24.5.
 template <int C, int E>
 hipError_t launch_irb_t(const IrbArgs &a, hipStream_t s) {
-  const long long tiles8 = (long long)a.N * ((a.H + 7) / 8) * ((a.W + 7) / 8);
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (tiles8 < cus) return launch_irb_tile<C, E, 4, 4>(a, s);
+  auto tiles = [&](int tw) { return (long long)a.N * ((a.H + 7) / 8) * ((a.W + tw - 1) / tw); };
+  if (tiles(8) < cus) return launch_irb_tile<C, E, 4, 4>(a, s);
+  auto busiest = [&](int tw, int hpb) {  // MFMAs / 4: expand on hpb blocks, project on four
+    constexpr int CB = (C + 15) / 16;
+    return (tiles(tw) + cus - 1) / cus * (E / 16) * CB * (hpb + 4);
+  };
+  if (busiest(7, IrbTile<8, 7>::HPB) < busiest(8, IrbTile<8, 8>::HPB)) return launch_irb_tile<C, E, 8, 7>(a, s);
   return launch_irb_tile<C, E, 8, 8>(a, s);
 }
 

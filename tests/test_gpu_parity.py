@@ -537,6 +537,8 @@ def test_c4_qbottleneck_streamed_filters(cuda, N, H, W, C, M1):
     (16, 30, 30, 24, 144),  # 8 x 8 tiles (256 of them), ragged at the image edge
     (8, 44, 50, 16, 96),
     (20, 31, 30, 32, 192),
+    (21, 29, 27, 24, 144),  # 8 x 7 tiles (336, as of 8 x 8), ragged rows and columns
+    (16, 30, 30, 32, 192), (16, 30, 30, 16, 96),
 ])
 def test_c3_irb_shapes(cuda, N, H, W, C, E):
     x = rng.uniform(31, 0, (N, H, W, C), 0, 1)
