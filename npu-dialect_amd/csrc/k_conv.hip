@@ -55,7 +55,12 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
   const T *const x = static_cast<const T *>(a.x);
   const T *const w = static_cast<const T *>(a.w);
 
-  // staging: this thread's 16-byte run `seg` of rows tid / 8 + 32 i
+  // staging: this thread's 16-byte run `seg` of rows tid / 8 + 32 i.  Offsets
+  // are 32-bit words from the tensors' bases (an operand has less than 2^31
+  // elements): a lane part that is fixed for the launch plus a step part that
+  // is uniform, so a load's address is one vector addition.  us, with 64-bit
+  // products of the coordinates instead / so: bf16 28x28x128 batch 32 21.8 /
+  // 21.1, 7x7x512 33.9 / 32.2, 5x5 30x30x64 batch 2 9.56 / 9.27.
   const int seg = tid & 7, row0 = tid >> 3;
   int abase[AR], aoh[AR], aow[AR], bbase[BR];
 #pragma unroll
@@ -65,7 +70,7 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
     const int oh = rem / a.Wo;
     aoh[i] = oh - a.pad;
     aow[i] = rem - oh * a.Wo - a.pad;
-    abase[i] = n * a.H * a.W;
+    abase[i] = ((n * a.H + aoh[i]) * a.W + aow[i]) * a.C;
   }
 #pragma unroll
   for (int i = 0; i < BR; ++i) bbase[i] = min(f0 + row0 + 32 * i, a.F - 1) * a.taps * a.C;
@@ -74,20 +79,19 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
   u32x4 av[2][AR], bv[2][BR];
   uint32_t keep[2];
   auto fetch = [&](int set, int kh, int kw, int c0) __attribute__((always_inline)) {
-    const int c = c0 + seg * RUN;
-    const bool cin = c < a.C;
-    const int cc = cin ? c : 0;
+    const bool cin = c0 + seg * RUN < a.C;
+    const int lc = cin ? seg * RUN : 0;
+    const int xoff = (kh * a.W + kw) * a.C + c0, woff = (kh * a.KW + kw) * a.C + c0;
     keep[set] = (uint32_t)cin << AR;
 #pragma unroll
     for (int i = 0; i < AR; ++i) {
-      const int ih = aoh[i] + kh, iw = aow[i] + kw;
-      const bool in = (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
-      av[set][i] = *reinterpret_cast<const u32x4 *>(x + (size_t)(abase[i] + (in ? ih * a.W + iw : 0)) * a.C + cc);
+      const bool in = (unsigned)(aoh[i] + kh) < (unsigned)a.H && (unsigned)(aow[i] + kw) < (unsigned)a.W;
+      av[set][i] = *reinterpret_cast<const u32x4 *>(x + (uint32_t)(in ? abase[i] + xoff + lc : 0));
       keep[set] |= (uint32_t)(in && cin) << i;
     }
-    const int tap = (kh * a.KW + kw) * a.C + cc;
 #pragma unroll
-    for (int i = 0; i < BR; ++i) bv[set][i] = *reinterpret_cast<const u32x4 *>(w + (size_t)(bbase[i] + tap));
+    for (int i = 0; i < BR; ++i)
+      bv[set][i] = *reinterpret_cast<const u32x4 *>(w + (uint32_t)(bbase[i] + woff + lc));
   };
   unsigned char *const dst = lds + row0 * REC + seg * 16;
   auto commit = [&](int buf) __attribute__((always_inline)) {
