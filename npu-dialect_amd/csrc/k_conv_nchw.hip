@@ -277,7 +277,9 @@ bool split_shape(const ConvArgs &c, NchwArgs &a, size_t &lds) {
   a.tw = (c.Wo + a.nstrips - 1) / a.nstrips;
   a.nstrips = (c.Wo + a.tw - 1) / a.tw;
   const long long npx = (long long)a.tw * c.Ho;
-  if (npx + PX >= 65536) return false;
+  // by_tw's range (tw <= 16); 3x3 16 -> 16 at 4200x600 495 us (the direct
+  // kernel, where taller images would go, reads each input word nine times)
+  if (npx + PX >= 1 << 28) return false;
   a.tiles = (int)((npx + PX - 1) / PX);
   const long long npt = (long long)c.N * a.nstrips * a.tiles, grid = npt * ((c.F + 16 * WF - 1) / (16 * WF));
   if (grid > 0x7fffffff - kXcds) return false;

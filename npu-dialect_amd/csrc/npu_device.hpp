@@ -134,9 +134,10 @@ __device__ __forceinline__ float act_clamp(float v, ActBounds b) {
   return __builtin_elementwise_minimum(__builtin_elementwise_maximum(v, b.lo), b.hi);
 }
 
-// Division of v < 2^16 by d < 2^16 as a multiply: q = (v * m) >> 32 with
-// m = ceil(2^32 / d) (the error v * (m d - 2^32) / (d 2^32) < 2^-16 cannot
-// carry past the next multiple); d = 1 takes v itself.
+// Division as a multiply: q = (v * m) >> 32 with m = ceil(2^32 / d).  Since
+// m d - 2^32 < d, the quotient's error is below v / 2^32, and it cannot carry
+// past the next multiple, 1 / d away at least, while v d <= 2^32 (v and d
+// below 2^16, or v below 2^28 for d <= 16); d = 1 takes v itself.
 struct FastDiv {
   uint32_t d, m;
   explicit FastDiv(int dv = 1) : d((uint32_t)dv), m(dv > 1 ? (uint32_t)(((1ULL << 32) + dv - 1) / dv) : 0u) {}

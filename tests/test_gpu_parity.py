@@ -1113,6 +1113,7 @@ def test_nchw_conv_shapes(cuda, N, C, H, W, F, K, pad, st, act, bias, res):
     (1, 2, 60, 60, 8, 11, 11, 2, 4, True, False),  # stride 4, 11x11: patches of 16 loads
     (1, 2, 70, 70, 4, 15, 15, 0, 9, False, False),  # a patch past 1024 words: the direct kernel
     (2, 520, 4, 4, 24, 1, 1, 0, 1, False, False),  # 1x1 over several chunks
+    (1, 3, 6600, 20, 8, 3, 3, 1, 1, True, False),  # strips of 66000 pixels
     (1, 7, 3, 5, 9, 3, 5, 0, 1, True, True),       # window = input, K = 105 (word loads)
     (2, 36, 4, 4, 130, 4, 4, 0, 1, True, False),   # window = input, two of eight images
     (11, 8, 2, 2, 5, 2, 2, 0, 3, False, True),     # window = input, two image groups
