@@ -586,6 +586,18 @@ namespace {
 // (56x56x64 at batch 8 33.2 against 32.2 us, 28x28x128 at batch 16 56.8 against
 // 57.4) and every sum runs in k order.
 constexpr long long kMinWgs = 160;
+
+// A whole-window conv of filters up to kDotShort long takes the direct kernel
+// past kDotOutputs images x filters: the dot kernel's time grows with the
+// images (its filters are read once per eight), the direct kernel's first
+// with the filter's length only.  Measured, us, 1000 filters: of 512 words, dot
+// 66 at 256 images, 128 at 512, 502 at 2048, direct 138 at 300, 141 at 512,
+// 166 at 2048; of 1024, dot 69 at 256, direct 155 at 300, 159 at 1024; of
+// 2048, dot 205 at 512, 388 at 1024, direct 677 at 2200; of 25088, dot 1375 at
+// 512, 5469 at 2048, direct 3503 and 5449: there the two end at the same rate.
+// kDotImages: the launch's y range.
+constexpr long long kDotOutputs = 1 << 19, kDotShort = 2048;
+constexpr int kDotImages = 8 * 65535;
 template <int NB, int WF, int WK>
 bool try_split(const ConvArgs &a, long long min_wgs, hipStream_t s, hipError_t &e) {
   NchwArgs n;
@@ -609,6 +621,7 @@ bool try_split(const ConvArgs &a, long long min_wgs, hipStream_t s, hipError_t &
 hipError_t launch_conv2d_nchw_f32(const ConvArgs &a, hipStream_t s) {
   const long long K = (long long)a.C * a.KH * a.KW;
   if (a.Ho == 1 && a.Wo == 1 && a.pad == 0 && a.KH == a.H && a.KW == a.W && K < (1 << 30)) {
+    if (a.N > kDotImages || (K <= kDotShort && (long long)a.N * a.F > kDotOutputs)) return launch_nchw_direct(a, s);
     if (K % 4 == 0) return a.N == 1 ? launch_dot<4, 1, true>(a, (int)K, s) : launch_dot<4, 8, true>(a, (int)K, s);
     return launch_dot<4, 8, false>(a, (int)K, s);
   }

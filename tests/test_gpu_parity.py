@@ -1117,6 +1117,8 @@ def test_nchw_conv_shapes(cuda, N, C, H, W, F, K, pad, st, act, bias, res):
     (1, 7, 3, 5, 9, 3, 5, 0, 1, True, True),       # window = input, K = 105 (word loads)
     (2, 36, 4, 4, 130, 4, 4, 0, 1, True, False),   # window = input, two of eight images
     (11, 8, 2, 2, 5, 2, 2, 0, 3, False, True),     # window = input, two image groups
+    (1024, 3, 2, 2, 512, 2, 2, 0, 1, True, False),  # window = input, the most outputs on the dot kernel
+    (1025, 3, 2, 2, 512, 2, 2, 0, 1, True, True),   # and one image more: the direct kernel
 ])
 def test_nchw_conv_tiles(cuda, N, C, H, W, F, KH, KW, pad, st, bias, res):
     """Edges of the split-K kernel's tiles, chunks and filter runs, of the
