@@ -14,7 +14,7 @@
 // pixels' runs (zero outside the image and past C) and the filters' runs are
 // staged in LDS, double-buffered, the next two steps' loads in flight while
 // the current one is multiplied, one barrier per step.  The filter fragment is the
-// MFMA's first operand, so a lane ends with four consecutive filters of one
+// MFMA's first operand where F is a multiple of 4, so a lane ends with four consecutive filters of one
 // pixel: the epilogue (bias add, residual add, act, and the bf16 rounding of
 // the bf16 variant) runs on the accumulators and stores 8 or 16 bytes.
 // C need not be a multiple of an MFMA fragment's 16 (f32) or 32 (bf16)
@@ -36,7 +36,7 @@ struct ConvTileArgs {
   int H, W, C, F, KW, taps, pad, Ho, Wo, act, P, npt, nft;
 };
 
-template <class MM, typename T, int BM, int BN>
+template <class MM, typename T, int BM, int BN, bool VEC>
 __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs a) {
   constexpr int ES = sizeof(T), RUN = 16 / ES;        // elements of a 16-byte run
   constexpr int KC = 128 / ES;                        // channels of a step
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
 #pragma unroll
           for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) MM::step(acc[i][j], bf[j], af[i], st);
+            for (int j = 0; j < TN; ++j) VEC ? MM::step(acc[i][j], bf[j], af[i], st) : MM::step(acc[i][j], af[i], bf[j], st);
       }
     }
   };
@@ -181,7 +181,29 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
   const ActBounds ab = act_bounds(a.act);
   const T *const res = static_cast<const T *>(a.res);
   T *const out = static_cast<T *>(a.out);
-  const bool vec = a.F % 4 == 0;
+  if constexpr (!VEC) {
+    // pixels 4q .. +3 of each block, its filter r: sixteen lanes on
+    // consecutive filters.  us, lanes on four filters of a pixel / so: bf16
+    // 1x1 34x35x16 -> 481 with residual at batch 13 27.2 / 17.4.
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int f = f0 + wf * (BN / 2) + 16 * j + r;
+      if (f >= a.F) continue;
+      const float bj = a.bias ? a.bias[f] : 0.0f;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int p = p0 + wp * (BM / 2) + 16 * i + 4 * q + e;
+          if (p >= a.P) continue;
+          const size_t o = (size_t)p * a.F + f;
+          const float v = acc[i][j][e] + bj;
+          if constexpr (sizeof(T) == 4) out[o] = act_clamp(res ? v + res[o] : v, ab);
+          else out[o] = f32_to_bf16(act_clamp(res ? v + bf16_to_f32(res[o]) : v, ab));
+        }
+    }
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int f = f0 + wf * (BN / 2) + 16 * j + 4 * q;
@@ -199,42 +221,29 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] + bj[e];
       if constexpr (sizeof(T) == 4) {
-        if (vec) {
-          if (res) v += *reinterpret_cast<const f32x4 *>(res + o);
+        if (res) v += *reinterpret_cast<const f32x4 *>(res + o);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = act_clamp(v[e], ab);
-          *reinterpret_cast<f32x4 *>(out + o) = v;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (f + e < a.F) out[o + e] = act_clamp(res ? v[e] + res[o + e] : v[e], ab);
-        }
+        for (int e = 0; e < 4; ++e) v[e] = act_clamp(v[e], ab);
+        *reinterpret_cast<f32x4 *>(out + o) = v;
       } else {
-        if (vec) {
-          if (res) {
-            const uint2 u = *reinterpret_cast<const uint2 *>(res + o);
-            v[0] += __uint_as_float(u.x << 16);
-            v[1] += __uint_as_float(u.x & 0xffff0000u);
-            v[2] += __uint_as_float(u.y << 16);
-            v[3] += __uint_as_float(u.y & 0xffff0000u);
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = act_clamp(v[e], ab);
-          *reinterpret_cast<uint2 *>(out + o) = make_uint2(cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]));
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (f + e < a.F)
-              out[o + e] = f32_to_bf16(act_clamp(res ? v[e] + bf16_to_f32(res[o + e]) : v[e], ab));
+        if (res) {
+          const uint2 u = *reinterpret_cast<const uint2 *>(res + o);
+          v[0] += __uint_as_float(u.x << 16);
+          v[1] += __uint_as_float(u.x & 0xffff0000u);
+          v[2] += __uint_as_float(u.y << 16);
+          v[3] += __uint_as_float(u.y & 0xffff0000u);
         }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = act_clamp(v[e], ab);
+        *reinterpret_cast<uint2 *>(out + o) = make_uint2(cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]));
       }
     }
   }
 }
 
-template <class MM, typename T, int BM, int BN>
+template <class MM, typename T, int BM, int BN, bool VEC>
 hipError_t launch_tile(const ConvArgs &c, hipStream_t s) {
-  auto kern = conv2d_nhwc_kernel<MM, T, BM, BN>;
+  auto kern = conv2d_nhwc_kernel<MM, T, BM, BN, VEC>;
   ConvTileArgs a{c.x, c.w, c.res, c.bias, c.out, c.H, c.W, c.C, c.F, c.KW, c.KH * c.KW, c.pad, c.Ho, c.Wo, c.act,
                  c.N * c.Ho * c.Wo, 0, 0};
   a.npt = (a.P + BM - 1) / BM;
@@ -253,6 +262,11 @@ hipError_t launch_tile(const ConvArgs &c, hipStream_t s) {
   plans_add(p);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, a);
   return hipGetLastError();
+}
+
+template <class MM, typename T, int BM, int BN>
+hipError_t launch_tile(const ConvArgs &c, hipStream_t s) {
+  return c.F % 4 == 0 ? launch_tile<MM, T, BM, BN, true>(c, s) : launch_tile<MM, T, BM, BN, false>(c, s);
 }
 
 // Tiles of 64 pixels x 64 filters when there are enough to keep more than one
