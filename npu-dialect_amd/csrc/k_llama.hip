@@ -101,6 +101,13 @@ struct GemmShape {
   }
 };
 
+// RoPE of two pairs: (2t, 2t+1) -> (x0 c - x1 s, x0 s + x1 c), the roundings
+// spelled out (which product is fused would be the compiler's choice).
+__device__ __forceinline__ uint2 rope4(const f32x4 &v, float2 c, float2 s) {
+  return pack4_bf16(fmaf(v[0], c.x, -(v[1] * s.x)), fmaf(v[0], s.x, v[1] * c.x),
+                    fmaf(v[2], c.y, -(v[3] * s.y)), fmaf(v[2], s.y, v[3] * c.y));
+}
+
 // SiLU with the hardware exp2 and reciprocal (v_exp_f32, v_rcp_f32).
 __device__ __forceinline__ float silu_fast(float g) {
   return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g));
@@ -368,10 +375,8 @@ __global__ __launch_bounds__(GT) void llama_gemm_kernel(const LlamaGemmArgs a, i
     if constexpr (EPI == kEpiQkvRope) {
       const int part = n / Np, c = n % Np;
       if (part < 2) {
-        // (2t, 2t+1) -> (x0 c - x1 s, x0 s + x1 c)
         const float2 cc = cs[e], ss = sn[e];
-        o = pack4_bf16(v[0] * cc.x - v[1] * ss.x, v[0] * ss.x + v[1] * cc.x,
-                       v[2] * cc.y - v[3] * ss.y, v[2] * ss.y + v[3] * cc.y);
+        o = rope4(v, cc, ss);
       } else {
         o = pack4_bf16(v[0], v[1], v[2], v[3]);
       }
@@ -389,32 +394,42 @@ __global__ __launch_bounds__(GT) void llama_gemm_kernel(const LlamaGemmArgs a, i
   }
 }
 
-// ---- long sequences: BM x BN tiles of 2 x 2 waves, K in steps of 64 -------------
+// ---- long sequences: BM x BN tiles of WR x WC waves, K in steps of 64 ------------
 //
 // The shapes above give a tile to 16 waves and, for the RMSNorm GEMMs, keep its
 // whole A panel in LDS: right for one tile per CU, but at S = 2048 they reached
-// 134 TFLOP/s.  Here a wave holds a (BM / 2) x (BN / 2) part of the tile (per
+// 134 TFLOP/s.  Here a wave holds a 32 x 16 to 32 x 48 part of the tile (per
 // weight), A and B stream through two LDS buffers, one barrier per step, the
-// next one or two steps' loads in flight, two workgroups per CU; what bounds it
-// is the fragments' LDS reads (twice the MFMAs' time at 64 x 64).  The RMSNorm is folded in
-// without a pass of its own: A is staged as bf16(x g) -- one rounding, as
-// bf16(x inv g) has -- while the same registers feed the row's sum of squares,
-// and the accumulator is scaled by the row's inv in f32 at the end.
-template <int EPI, int BM, int BN>
+// next DEP steps' loads in flight (two for the residual GEMMs: a step's MFMAs
+// take less time than a load from L2; 2048x2048x768 18.1 / 17.5 us with one /
+// two).  What bounds it is the fragments' LDS reads (twice the MFMAs' time at
+// 32 x 32) and, with the RMSNorm, its vector work: the row sums once per tile
+// (about 5 of 31 us at 2048x768) and the normalisation of each staged run,
+// which is why those tiles are 128 or 192 columns wide.
+//
+// A row's result is the same bits whichever kernel computes it: a prompt's
+// length chooses the kernel, not the numbers.  So the RMSNorm's row sums go
+// over the lanes as above, A is staged as bf16((x inv) g), and where the shapes
+// above split K over four waves (PARTS = 4: k steps of 32 dealt round-robin),
+// the wave keeps the four parts' sums apart and adds them in the same order.
+template <int EPI, int BM, int BN, int WR, int WC>
 struct TileShape {
-  static constexpr int NB = EPI == kEpiSwiglu ? 2 : 1, KC = 64;
-  static constexpr int TM = BM / 32, TN = BN / 32;               // MFMA blocks of a wave (per weight)
+  static constexpr int NB = EPI == kEpiSwiglu ? 2 : 1, KC = 64, NT = 64 * WR * WC;
+  static constexpr int TM = BM / WR / 16, TN = BN / WC / 16;     // MFMA blocks of a wave (per weight)
   static constexpr int AREC = KC * 2 + 32, SB = KC * 32 + 32;    // A row, B strip (bytes)
   static constexpr int STRIPS = BN / 16, ABYTES = BM * AREC;
   static constexpr int BUF = ABYTES + NB * STRIPS * SB;
-  static constexpr int AR = BM / 32, BR = NB * BN / 32;          // 16-byte runs per thread and step
+  // 16-byte runs per thread and step (A: of the first BM * 8 threads)
+  static constexpr int AR = (BM * 8 + NT - 1) / NT, BR = NB * BN * 8 / NT;
+  static_assert((AR == 1 || AR * NT == BM * 8) && BR * NT == NB * BN * 8, "whole runs");
 };
 
-template <int PRO, int EPI, int BM, int BN>
-__global__ __launch_bounds__(256, 2) void llama_tile_kernel(const LlamaGemmArgs a, int tiles_m,
-                                                            int tiles_n, int xm) {
-  using S = TileShape<EPI, BM, BN>;
-  constexpr int NB = S::NB, TM = S::TM, TN = S::TN, KC = S::KC, AR = S::AR, BR = S::BR;
+template <int PRO, int EPI, int BM, int BN, int WR, int WC, int PARTS, int OCC, int DEP>
+__global__ __launch_bounds__(64 * WR * WC, OCC) void llama_tile_kernel(const LlamaGemmArgs a, int tiles_m,
+                                                                       int tiles_n, int xm) {
+  using S = TileShape<EPI, BM, BN, WR, WC>;
+  constexpr int NB = S::NB, TM = S::TM, TN = S::TN, KC = S::KC, AR = S::AR, BR = S::BR, NT = S::NT;
+  constexpr int ROWS = NT / 8;  // A rows a pass of the threads stages
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float inv_s[PRO == kProRmsnorm ? BM : 1];
   int tm, tn;
@@ -422,14 +437,14 @@ __global__ __launch_bounds__(256, 2) void llama_tile_kernel(const LlamaGemmArgs 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int M = a.M, K = a.K, Np = a.Npart;
   const int m0 = tm * BM, n0 = tn * BN;
-  const int wr = wave & 1, wc = wave >> 1;
+  const int wr = wave % WR, wc = wave / WR;
   const int ml = lane & 15, ng = 4 * (lane >> 4);
 
-  // A: run `seg` of rows row0 + 32 i; rows past M read row M - 1
+  // A: run `seg` of rows row0 + ROWS i; rows past M read row M - 1
   const int seg = tid & 7, row0 = tid >> 3;
   const uint16_t *ap[AR];
 #pragma unroll
-  for (int i = 0; i < AR; ++i) ap[i] = a.A + (size_t)min(m0 + row0 + 32 * i, M - 1) * K + seg * 8;
+  for (int i = 0; i < AR; ++i) ap[i] = a.A + (size_t)min(m0 + row0 + ROWS * i, M - 1) * K + seg * 8;
   unsigned char *const adst = smem + row0 * S::AREC + seg * 16;
   // B: 16-byte pieces, NB BN / 8 per k row
   const uint16_t *bp[BR];
@@ -437,19 +452,14 @@ __global__ __launch_bounds__(256, 2) void llama_tile_kernel(const LlamaGemmArgs 
 #pragma unroll
   for (int i = 0; i < BR; ++i) {
     constexpr int CPR = NB * BN / 8;
-    const int it = tid + 256 * i, k = it / CPR, c = it % CPR;
+    const int it = tid + NT * i, k = it / CPR, c = it % CPR;
     const int nb = c / (BN / 8), cc = c % (BN / 8), gc = n0 + cc * 8;
     const int part = EPI == kEpiQkvRope ? gc / Np : nb, col = EPI == kEpiQkvRope ? gc % Np : gc;
     bp[i] = a.B[part] + (size_t)k * Np + col;
     bdst[i] = S::ABYTES + (nb * S::STRIPS + cc / 2) * S::SB + strip_row(k) * 32 + (cc & 1) * 16;
   }
-  // Register sets of staged runs: a step is 128 to 256 clocks of MFMAs per
-  // wave, less than a load from L2 takes, so each step's loads are issued DEP
-  // steps before they are committed.  us with one / two: down projection
-  // 2048x2048x768 18.1 / 17.5, 512x2048x768 9.8 / 8.5, 1024x1408x512 7.7 / 6.8;
-  // SwiGLU 2048x768x2048 23.0 / 21.8, 300x768x2048 10.4 / 9.8; QKV 1024x512
-  // 9.2 / 9.9, 512x768 11.2 / 12.1 (registers of the RMSNorm's staging), so one.
-  constexpr int DEP = EPI == kEpiQkvRope ? 1 : 2;
+  // Register sets of staged runs: each step's loads are issued DEP steps before
+  // they are committed.
   u32x4 av[DEP][AR], bv[DEP][BR];
   f32x4 gv[DEP][2];
   auto fetch = [&](int set, int k0) __attribute__((always_inline)) {
@@ -462,9 +472,50 @@ __global__ __launch_bounds__(256, 2) void llama_tile_kernel(const LlamaGemmArgs 
 #pragma unroll
     for (int i = 0; i < BR; ++i) bv[set][i] = *reinterpret_cast<const u32x4 *>(bp[i] + (size_t)k0 * Np);
   };
-  float ss[AR];
+  const int steps = K / KC, klast = K - KC;
+  fetch(0, 0);
+  if constexpr (DEP == 2) fetch(1, min(KC, klast));
+
+  // ---- 1 / rms of the tile's rows, summed as the RMSNorm prologue above sums
+  //      them: lane l takes the 8-element pieces l and l + 64
+  float inv[AR];
+  if constexpr (PRO == kProRmsnorm) {
+    constexpr int RPW = BM / (NT / 64), RB = OCC >= 4 ? 4 : 8;  // rows per wave, per batch of loads
+    constexpr int PPL = PARTS == 1 ? 1 : 2;                     // pieces per lane: K <= 512, <= 1024
+    static_assert(RPW % RB == 0 && RPW * (NT / 64) == BM, "whole batches");
+    const int pieces = K / 8;
+    const float invk = 1.0f / (float)K;
+#pragma unroll 1
+    for (int b = 0; b < RPW; b += RB) {
+      u32x4 x[RB][PPL];
 #pragma unroll
-  for (int i = 0; i < AR; ++i) ss[i] = 0.0f;
+      for (int rr = 0; rr < RB; ++rr)
+#pragma unroll
+        for (int p = 0; p < PPL; ++p)
+          x[rr][p] = *reinterpret_cast<const u32x4 *>(a.A + (size_t)min(m0 + wave * RPW + b + rr, M - 1) * K +
+                                                      min(lane + 64 * p, pieces - 1) * 8);
+#pragma unroll
+      for (int rr = 0; rr < RB; ++rr) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int p = 0; p < PPL; ++p) {
+          float part = 0.0f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float lo = bf_lo(x[rr][p][e]), hi = bf_hi(x[rr][p][e]);
+            part = fmaf(lo, lo, part);
+            part = fmaf(hi, hi, part);
+          }
+          ss += lane + 64 * p < pieces ? part : 0.0f;
+        }
+        const float v = __builtin_amdgcn_rsqf(wave_sum(ss) * invk + a.eps);
+        if (lane == 0) inv_s[wave * RPW + b + rr] = v;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < AR; ++i) inv[i] = inv_s[min(row0 + ROWS * i, BM - 1)];
+  }
   // a register set to LDS buffer `buf`
   auto commit = [&](int buf) __attribute__((always_inline)) {
     const int set = buf % DEP;
@@ -474,30 +525,32 @@ __global__ __launch_bounds__(256, 2) void llama_tile_kernel(const LlamaGemmArgs 
       if constexpr (PRO == kProRmsnorm) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float lo = bf_lo(o[e]), hi = bf_hi(o[e]);
           const f32x4 g = gv[set][e / 2];
-          ss[i] = fmaf(hi, hi, fmaf(lo, lo, ss[i]));
-          o[e] = cvt_pk_bf16(lo * g[2 * (e & 1)], hi * g[2 * (e & 1) + 1]);
+          o[e] = cvt_pk_bf16((bf_lo(o[e]) * inv[i]) * g[2 * (e & 1)], (bf_hi(o[e]) * inv[i]) * g[2 * (e & 1) + 1]);
         }
       }
-      *reinterpret_cast<u32x4 *>(adst + buf * S::BUF + 32 * i * S::AREC) = o;
+      if (BM * 8 >= NT || tid < BM * 8) *reinterpret_cast<u32x4 *>(adst + buf * S::BUF + ROWS * i * S::AREC) = o;
     }
 #pragma unroll
     for (int i = 0; i < BR; ++i) *reinterpret_cast<u32x4 *>(smem + buf * S::BUF + bdst[i]) = bv[set][i];
   };
 
-  f32x4 acc[NB][TM][TN];
+  f32x4 acc[PARTS][NB][TM][TN];
 #pragma unroll
-  for (int b = 0; b < NB; ++b)
+  for (int p = 0; p < PARTS; ++p)
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const unsigned char *const arow = smem + (wr * (BM / 2) + ml) * S::AREC + (lane >> 4) * 16;
-  auto multiply = [&](int buf) __attribute__((always_inline)) {
-    const int off = buf * S::BUF;
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[p][b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const unsigned char *const arow = smem + (wr * (BM / WR) + ml) * S::AREC + (lane >> 4) * 16;
+  // step s holds k steps 2 s and 2 s + 1 of 32, of parts 2 (s % 2) and that + 1
+  auto multiply = [&](auto par) __attribute__((always_inline)) {
+    constexpr int buf = decltype(par)::value, off = buf * S::BUF;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      const int p = PARTS == 4 ? 2 * buf + h : 0;
       Frag16 xf[TM], wf[NB][TN];
 #pragma unroll
       for (int i = 0; i < TM; ++i) xf[i].u = *reinterpret_cast<const u32x4 *>(arow + off + 16 * i * S::AREC + 64 * h);
@@ -512,69 +565,61 @@ __global__ __launch_bounds__(256, 2) void llama_tile_kernel(const LlamaGemmArgs 
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < TN; ++j)
-            acc[b][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[b][j].h, xf[i].h, acc[b][i][j], 0, 0, 0);
+            acc[p][b][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[b][j].h, xf[i].h, acc[p][b][i][j], 0, 0, 0);
     }
   };
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
   // Step s is in buffer s % 2 and passed through register set s % DEP.  Past
   // the last step the loads repeat it and are never committed (a condition on
   // them would make the wave wait for them at once).
-  const int steps = K / KC, klast = K - KC;
-  fetch(0, 0);
-  if constexpr (DEP == 2) fetch(1, min(KC, klast));
   commit(0);
   fetch(0, min(DEP * KC, klast));
   __syncthreads();
   int s = 0;
   for (; s + 2 < steps; s += 2) {
-    multiply(0);
+    multiply(even);
     commit(1);
     fetch(1 % DEP, min((s + 1 + DEP) * KC, klast));
     __syncthreads();
-    multiply(1);
+    multiply(odd);
     commit(0);
     fetch(0, min((s + 2 + DEP) * KC, klast));
     __syncthreads();
   }
-  multiply(0);
+  multiply(even);
   if (s + 1 < steps) {
     commit(1);
     __syncthreads();
-    multiply(1);
-  }
-  if constexpr (PRO == kProRmsnorm) {
-    // the eight lanes of a row: xor 1, 2 (quad permutes), then the half-row mirror
-#pragma unroll
-    for (int i = 0; i < AR; ++i) {
-      float v = ss[i];
-      v += dpp_mov<0xb1>(v);
-      v += dpp_mov<0x4e>(v);
-      v += dpp_mov<0x141>(v);
-      if (seg == 0) inv_s[row0 + 32 * i] = __builtin_amdgcn_rsqf(v * (1.0f / (float)K) + a.eps);
-    }
-    __syncthreads();
+    multiply(odd);
   }
 
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const int row = wr * (BM / 2) + 16 * i + ml, m = m0 + row;
-    const float inv = PRO == kProRmsnorm ? inv_s[row] : 1.0f;
+    const int m = m0 + wr * (BM / WR) + 16 * i + ml;
     if (m >= M) continue;
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const int n = n0 + wc * (BN / 2) + 16 * j + ng;
-      f32x4 v = acc[0][i][j];
-      if constexpr (PRO == kProRmsnorm) v *= inv;
+      const int n = n0 + wc * (BN / WC) + 16 * j + ng;
+      f32x4 v = acc[0][0][i][j], u = acc[0][NB - 1][i][j];
+      if constexpr (PARTS > 1) {
+        v = u = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+          v += acc[p][0][i][j];
+          if constexpr (NB == 2) u += acc[p][NB - 1][i][j];
+        }
+      }
       uint2 o;
       uint16_t *dst;
       if constexpr (EPI == kEpiQkvRope) {
         const int part = n / Np, c = n % Np;
         dst = a.out[part] + (size_t)m * Np + c;
-        if (part < 2) {  // (2t, 2t+1) -> (x0 c - x1 s, x0 s + x1 c)
+        if (part < 2) {
           const size_t t = (size_t)m * (a.Dh / 2) + (c % a.Dh) / 2;
           const float2 cc = *reinterpret_cast<const float2 *>(a.cos_t + t);
           const float2 sn = *reinterpret_cast<const float2 *>(a.sin_t + t);
-          o = pack4_bf16(v[0] * cc.x - v[1] * sn.x, v[0] * sn.x + v[1] * cc.x,
-                         v[2] * cc.y - v[3] * sn.y, v[2] * sn.y + v[3] * cc.y);
+          o = rope4(v, cc, sn);
         } else {
           o = pack4_bf16(v[0], v[1], v[2], v[3]);
         }
@@ -583,8 +628,6 @@ __global__ __launch_bounds__(256, 2) void llama_tile_kernel(const LlamaGemmArgs 
         dst = a.out[0] + (size_t)m * Np + n;
         o = pack4_bf16(bf_lo(r.x) + v[0], bf_hi(r.x) + v[1], bf_lo(r.y) + v[2], bf_hi(r.y) + v[3]);
       } else {
-        f32x4 u = acc[NB - 1][i][j];
-        if constexpr (PRO == kProRmsnorm) u *= inv;
         dst = a.out[0] + (size_t)m * Np + n;
         o = pack4_bf16(silu_fast(v[0]) * u[0], silu_fast(v[1]) * u[1], silu_fast(v[2]) * u[2],
                        silu_fast(v[3]) * u[3]);
@@ -623,6 +666,66 @@ __device__ __forceinline__ Frag16 read_vfrag(const uint16_t *vs, int dtile, int 
   Frag16 f;
   f.u = u32x4{lo.x, lo.y, hi.x, hi.y};
   return f;
+}
+
+// One key block of the online softmax for this lane's query: scores s (two
+// 16-key tiles) to probabilities p, the running maximum and sum updated (the sum
+// over this lane's keys); returns the factor for what was summed before.
+__device__ __forceinline__ float softmax_block(const f32x4 (&s)[2], float kscale, float &m_run, float &l_run,
+                                               float (&p)[2][4]) {
+  float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
+                   fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+  const LanePair p16 = lane_pair16(mx);
+  mx = fmaxf(p16.lo, p16.hi);
+  const LanePair p32 = lane_pair32(mx);
+  mx = fmaxf(p32.lo, p32.hi);
+  const float m_new = fmaxf(m_run, mx);
+  const float m_use = m_new == -__builtin_inff() ? 0.0f : m_new;
+  const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * kscale);
+  const float bias = -m_use * kscale;
+  float psum = 0.0f;
+#pragma unroll
+  for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      p[tt][r] = __builtin_amdgcn_exp2f(fmaf(s[tt][r], kscale, bias));
+      psum += p[tt][r];
+    }
+  l_run = l_run * alpha + psum;
+  m_run = m_new;
+  return alpha;
+}
+// P^T as the MFMA's operand, k slots: keys 4g + r (tile 0), 16 + 4g + r (tile 1).
+__device__ __forceinline__ Frag16 probs_frag(const float (&p)[2][4]) {
+  Frag16 f;
+  f.u = u32x4{cvt_pk_bf16(p[0][0], p[0][1]), cvt_pk_bf16(p[0][2], p[0][3]),
+              cvt_pk_bf16(p[1][0], p[1][1]), cvt_pk_bf16(p[1][2], p[1][3])};
+  return f;
+}
+// A query's sum over its four lane groups.
+__device__ __forceinline__ float group_sum(float l) {
+  const LanePair a16 = lane_pair16(l);
+  const float l16 = a16.lo + a16.hi;
+  const LanePair a32 = lane_pair32(l16);
+  return a32.lo + a32.hi;
+}
+// Query qq's merge of AWAVES waves' states: each wave's factor in f, and the
+// reciprocal of the merged sum.
+__device__ __forceinline__ float merge_factors(const float (*st_m)[AQ], const float (*st_l)[AQ], int qq, float kscale,
+                                               float (&f)[AWAVES]) {
+  float mw[AWAVES], mmax = -__builtin_inff();
+#pragma unroll
+  for (int w = 0; w < AWAVES; ++w) {
+    mw[w] = st_m[w][qq];
+    mmax = fmaxf(mmax, mw[w]);
+  }
+  float L = 0.0f;
+#pragma unroll
+  for (int w = 0; w < AWAVES; ++w) {
+    f[w] = mw[w] == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f((mw[w] - mmax) * kscale);
+    L += st_l[w][qq] * f[w];
+  }
+  return 1.0f / L;
 }
 
 template <int DH>
@@ -715,33 +818,11 @@ __global__ __launch_bounds__(256) void llama_attention_kernel(const uint16_t *__
         for (int r = 0; r < 4; ++r)
           if (k0 + 16 * tt + 4 * g + r > q) s[tt][r] = -__builtin_inff();
     }
-    // online softmax over this block's keys for query q
-    float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
-                     fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
-    const LanePair p16 = lane_pair16(mx);
-    mx = fmaxf(p16.lo, p16.hi);
-    const LanePair p32 = lane_pair32(mx);
-    mx = fmaxf(p32.lo, p32.hi);
-    const float m_new = fmaxf(m_run, mx);
-    const float m_use = m_new == -__builtin_inff() ? 0.0f : m_new;
-    const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * kscale);
-    const float bias = -m_use * kscale;
     float p[2][4];
-    float psum = 0.0f;
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        p[tt][r] = __builtin_amdgcn_exp2f(fmaf(s[tt][r], kscale, bias));
-        psum += p[tt][r];
-      }
-    l_run = l_run * alpha + psum;
-    m_run = m_new;
+    const float alpha = softmax_block(s, kscale, m_run, l_run, p);
 #pragma unroll
     for (int d = 0; d < NDT; ++d) o[d] *= alpha;
-    Frag16 pf;  // P^T, k slots: keys 4g + r (tile 0), 16 + 4g + r (tile 1)
-    pf.u = u32x4{cvt_pk_bf16(p[0][0], p[0][1]), cvt_pk_bf16(p[0][2], p[0][3]),
-                 cvt_pk_bf16(p[1][0], p[1][1]), cvt_pk_bf16(p[1][2], p[1][3])};
+    const Frag16 pf = probs_frag(p);
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
@@ -751,13 +832,7 @@ __global__ __launch_bounds__(256) void llama_attention_kernel(const uint16_t *__
     }
     buf ^= 1;
   }
-  // this wave's state: l summed over its four lane groups
-  {
-    const LanePair a16 = lane_pair16(l_run);
-    const float l16 = a16.lo + a16.hi;
-    const LanePair a32 = lane_pair32(l16);
-    l_run = a32.lo + a32.hi;
-  }
+  l_run = group_sum(l_run);  // this wave's state
   if (g == 0) {
     st_m[wave][ql] = m_run;
     st_l[wave][ql] = l_run;
@@ -771,19 +846,8 @@ __global__ __launch_bounds__(256) void llama_attention_kernel(const uint16_t *__
 #pragma unroll
   for (int pass = 0; pass < DH / 64; ++pass) {
     const int qq = tid >> 4, d0 = 64 * pass + 4 * (tid & 15);
-    float mw[AWAVES], mmax = -__builtin_inff();
-#pragma unroll
-    for (int w = 0; w < AWAVES; ++w) {
-      mw[w] = st_m[w][qq];
-      mmax = fmaxf(mmax, mw[w]);
-    }
-    float L = 0.0f, f[AWAVES];
-#pragma unroll
-    for (int w = 0; w < AWAVES; ++w) {
-      f[w] = mw[w] == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f((mw[w] - mmax) * kscale);
-      L += st_l[w][qq] * f[w];
-    }
-    const float invL = 1.0f / L;
+    float f[AWAVES];
+    const float invL = merge_factors(st_m, st_l, qq, kscale, f);
     float out[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -798,35 +862,46 @@ __global__ __launch_bounds__(256) void llama_attention_kernel(const uint16_t *__
   }
 }
 
-// Long sequences: 64 queries per workgroup, 16 per wave, in two groups of four
-// waves that take the even and the odd key blocks of 64 and merge at the end.
-// A pair of blocks is staged in LDS for all eight waves, the next pair's loads
-// in flight: a quarter of the K and V traffic of the kernel above.  Workgroups
-// are dealt longest first (the last query blocks), so the short ones fill in
-// behind them.
-// What bounds it: one wave's chain per block (scores, maximum, exponentials,
-// products: about 1 800 clocks alone on its SIMD), which is why the keys are
-// split.
-constexpr int TQ = 64, TKB = 64, TGR = 2;
+// Long sequences: 64 queries per workgroup of sixteen waves, wave (qg, w) on
+// queries 16 qg .. +15 and the key blocks w, w + 4, ..., as wave w of the kernel
+// above: the same running maxima, sums and merge, so a query's result is the
+// same bits whichever kernel computes it.  Four key blocks at a time are staged
+// in LDS for all waves, the next four's loads in flight: a quarter of the K and
+// V traffic of the kernel above.  Workgroups are dealt longest first (the last
+// query blocks), so the short ones fill in behind them.
+// What bounds it: the softmax's vector work and the chain of a block (scores,
+// maximum, exponentials, products), four waves per SIMD.
+constexpr int TQ = 64, TKEYS = AWAVES * AKB, TNT = 64 * 4 * AWAVES;
 
 template <int DH>
-__global__ __launch_bounds__(256 * TGR, 4) void llama_attention_tile_kernel(const uint16_t *__restrict__ Q,
-                                                                   const uint16_t *__restrict__ Kg,
-                                                                   const uint16_t *__restrict__ V,
-                                                                   uint16_t *__restrict__ O, int S,
-                                                                   int H, float scale) {
+struct AttnTileShape {
+  static constexpr int KV = 2 * TKEYS * AttnShape<DH>::VLD * 2;  // bytes of the staged K and V
+  static constexpr int ST = 16 * 64 * (DH / 4) * 4;              // of the sixteen waves' outputs
+  static constexpr int LDS = KV > ST ? KV : ST;
+};
+
+template <int DH>
+__global__ __launch_bounds__(TNT, 4) void llama_attention_tile_kernel(const uint16_t *__restrict__ Q,
+                                                                     const uint16_t *__restrict__ Kg,
+                                                                     const uint16_t *__restrict__ V,
+                                                                     uint16_t *__restrict__ O, int S,
+                                                                     int H, float scale) {
   using Sh = AttnShape<DH>;
-  constexpr int NQF = Sh::NQF, LD = Sh::VLD, PPR = Sh::PPR, NDT = Sh::NDT, NT = TKB / 16;
-  constexpr int NR = TKB * PPR / 256;  // 16-byte pieces of K (and of V) per thread and block
-  // one pair of blocks; after the walk, the odd group's states
-  __shared__ __attribute__((aligned(16))) uint16_t kvbuf[2 * TGR][TKB * LD];
+  constexpr int NQF = Sh::NQF, LD = Sh::VLD, PPR = Sh::PPR, NDT = Sh::NDT;
+  constexpr int NR = TKEYS * PPR / TNT;  // 16-byte pieces of K (and of V) per thread
+  // K and V of the four blocks; after the walk, the waves' outputs
+  __shared__ __attribute__((aligned(16))) unsigned char buf[AttnTileShape<DH>::LDS];
+  __shared__ float st_m[4 * AWAVES][AQ], st_l[4 * AWAVES][AQ];
+  uint16_t *const ks = reinterpret_cast<uint16_t *>(buf), *const vs = ks + TKEYS * LD;
   const int nqb = (S + TQ - 1) / TQ;
   const int qb = nqb - 1 - blockIdx.x / H, h = blockIdx.x % H;
-  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
-  const int gr = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);  // this wave's group
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = wave % AWAVES;
   const int g = lane >> 4, ql = lane & 15;
   const int D = H * DH;
-  const int q0 = qb * TQ + 16 * wave;  // this wave's queries
+  const int q0 = qb * TQ + AQ * (wave / AWAVES);  // this wave's queries
+  const int nkb = (q0 + AQ + AKB - 1) / AKB;      // its key blocks: 0 .. nkb - 1
+  const int nsteps = ((qb + 1) * TQ / AKB + AWAVES - 1) / AWAVES;
   const float kscale = scale * 1.4426950408889634f;  // exp(x * scale) = exp2(x * kscale)
 
   // Rows past S are read from row S - 1, as above: such keys lie above every
@@ -838,21 +913,13 @@ __global__ __launch_bounds__(256 * TGR, 4) void llama_attention_tile_kernel(cons
     for (int k = 0; k < NQF; ++k) qf[k] = load16(qp + 32 * k);
   }
   u32x4 kr[NR], vr[NR];
-  auto fetch = [&](int kb) __attribute__((always_inline)) {
+  auto fetch = [&](int step) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
-      const int item = tid + 256 * i;  // key item / PPR, dh 8 (item % PPR)
-      const size_t o = (size_t)min(kb * TKB + item / PPR, S - 1) * D + h * DH + (item % PPR) * 8;
+      const int item = tid + TNT * i;  // key item / PPR, dh 8 (item % PPR)
+      const size_t o = (size_t)min(step * TKEYS + item / PPR, S - 1) * D + h * DH + (item % PPR) * 8;
       kr[i] = *reinterpret_cast<const u32x4 *>(Kg + o);
       vr[i] = *reinterpret_cast<const u32x4 *>(V + o);
-    }
-  };
-  auto commit = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const int item = tid + 256 * i, o = (item / PPR) * LD + (item % PPR) * 8;
-      *reinterpret_cast<u32x4 *>(kvbuf[gr] + o) = kr[i];
-      *reinterpret_cast<u32x4 *>(kvbuf[TGR + gr] + o) = vr[i];
     }
   };
   float m_run = -__builtin_inff(), l_run = 0.0f;
@@ -860,105 +927,78 @@ __global__ __launch_bounds__(256 * TGR, 4) void llama_attention_tile_kernel(cons
 #pragma unroll
   for (int d = 0; d < NDT; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const uint16_t *const ks = kvbuf[gr], *const vs = kvbuf[TGR + gr];
-  fetch(min(gr, qb));
-  for (int kb0 = 0; kb0 <= qb; kb0 += TGR) {
-    const int kb = kb0 + gr;
-    if (kb0 > 0) __syncthreads();  // every wave is done with the last pair
-    commit();
-    __syncthreads();
-    fetch(min(kb + TGR, qb));
-    if (kb > qb) break;  // the odd group's last pair has no block for it
-    // S^T = K Q^T: four 16-key tiles
-    f32x4 s[NT];
+  const uint16_t *const kw = ks + w * AKB * LD, *const vw = vs + w * AKB * LD;  // this wave's block of the four
+  fetch(0);
+  for (int step = 0; step < nsteps; ++step) {
+    if (step > 0) __syncthreads();  // every wave is done with the last blocks
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int k = 0; k < NQF; ++k)
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load16(ks + (16 * t + ql) * LD + 32 * k + 8 * g).h,
-                                                       qf[k].h, s[t], 0, 0, 0);
+    for (int i = 0; i < NR; ++i) {
+      const int item = tid + TNT * i, at = (item / PPR) * LD + (item % PPR) * 8;
+      *reinterpret_cast<u32x4 *>(ks + at) = kr[i];
+      *reinterpret_cast<u32x4 *>(vs + at) = vr[i];
     }
-    if (kb == qb) {  // the diagonal block: key > query
+    __syncthreads();
+    fetch(min(step + 1, nsteps - 1));
+    const int kb = step * AWAVES + w;
+    if (kb >= nkb) continue;  // uniform: only in the last step
+    // S^T = K Q^T: two 16-key tiles
+    f32x4 s[2];
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+    for (int tt = 0; tt < 2; ++tt) {
+      const uint16_t *kp = kw + (16 * tt + ql) * LD + 8 * g;
+      s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load16(kp).h, qf[0].h, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+      for (int k = 1; k < NQF; ++k)
+        s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load16(kp + 32 * k).h, qf[k].h, s[tt], 0, 0, 0);
+    }
+    const int k0 = kb * AKB, q = q0 + ql;
+    if (k0 + AKB - 1 > q0) {  // the block that reaches the diagonal: key > query
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (16 * t + 4 * g + r > 16 * wave + ql) s[t][r] = -__builtin_inff();
+          if (k0 + 16 * tt + 4 * g + r > q) s[tt][r] = -__builtin_inff();
     }
-    float mx = fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3]));
-#pragma unroll
-    for (int t = 1; t < NT; ++t)
-      mx = fmaxf(mx, fmaxf(fmaxf(s[t][0], s[t][1]), fmaxf(s[t][2], s[t][3])));
-    const LanePair p16 = lane_pair16(mx);
-    mx = fmaxf(p16.lo, p16.hi);
-    const LanePair p32 = lane_pair32(mx);
-    mx = fmaxf(p32.lo, p32.hi);
-    const float m_new = fmaxf(m_run, mx);
-    const float m_use = m_new == -__builtin_inff() ? 0.0f : m_new;
-    const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * kscale);
-    const float bias = -m_use * kscale;
-    // P^T as bf16, keys 4g + r of each tile.  The normaliser sums the rounded
-    // values, so the weights that V is multiplied by add up to one (relative
-    // error of the output at 2048x12x64 0.00332, as the kernel above has; with
-    // the sum of the unrounded ones 0.00334).
-    uint2 pk[NT];
-    float psum = 0.0f;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      float p[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(s[t][r], kscale, bias));
-      pk[t] = pack4_bf16(p[0], p[1], p[2], p[3]);
-      psum += (bf_lo(pk[t].x) + bf_hi(pk[t].x)) + (bf_lo(pk[t].y) + bf_hi(pk[t].y));
-    }
-    l_run = l_run * alpha + psum;
-    m_run = m_new;
+    float p[2][4];
+    const float alpha = softmax_block(s, kscale, m_run, l_run, p);
 #pragma unroll
     for (int d = 0; d < NDT; ++d) o[d] *= alpha;
-#pragma unroll
-    for (int b = 0; b < NT / 2; ++b) {
-      Frag16 pf;  // k slots: keys 4g + r of tiles 2b and 2b + 1
-      pf.u = u32x4{pk[2 * b].x, pk[2 * b].y, pk[2 * b + 1].x, pk[2 * b + 1].y};
-#pragma unroll
-      for (int d = 0; d < NDT; ++d) {
-        const Frag16 vf = read_vfrag<LD>(vs + 32 * b * LD, d, lane);
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.h, pf.h, o[d], 0, 0, 0);
-      }
-    }
-  }
-  const LanePair a16 = lane_pair16(l_run);
-  const float l16 = a16.lo + a16.hi;
-  const LanePair a32 = lane_pair32(l16);
-  l_run = a32.lo + a32.hi;
-  // the odd group's state to LDS, lane by lane; the even group merges it
-  float *const st = reinterpret_cast<float *>(kvbuf) + tid;
-  __syncthreads();
-  constexpr int SS = 256;  // words between a lane's values
-  static_assert((4 * NDT + 2) * SS * 4 <= (int)sizeof kvbuf, "states fit");
-  if (gr == 1) {
-    st[0] = m_run;
-    st[SS] = l_run;
-#pragma unroll
-    for (int d = 0; d < NDT; ++d)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) st[(2 + 4 * d + e) * SS] = o[d][e];
-  }
-  __syncthreads();
-  if (gr == 1) return;
-  const float m1 = st[0], l1 = st[SS], m = fmaxf(m_run, m1);
-  const float m_use = m == -__builtin_inff() ? 0.0f : m;
-  const float f0 = __builtin_amdgcn_exp2f((m_run - m_use) * kscale), f1 = __builtin_amdgcn_exp2f((m1 - m_use) * kscale);
-  const float invl = 1.0f / (l_run * f0 + l1 * f1);
-  if (q0 + ql < S) {
-    uint16_t *const op = O + (size_t)(q0 + ql) * D + h * DH + 4 * g;
+    const Frag16 pf = probs_frag(p);
 #pragma unroll
     for (int d = 0; d < NDT; ++d) {
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = (o[d][e] * f0 + st[(2 + 4 * d + e) * SS] * f1) * invl;
-      *reinterpret_cast<uint2 *>(op + 16 * d) = pack4_bf16(v[0], v[1], v[2], v[3]);
+      const Frag16 vf = read_vfrag<LD>(vw, d, lane);
+      o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.h, pf.h, o[d], 0, 0, 0);
     }
+  }
+  l_run = group_sum(l_run);
+  __syncthreads();  // every wave is done with K and V
+  float *const st = reinterpret_cast<float *>(buf) + lane;  // [wave][d][r][lane]
+#pragma unroll
+  for (int d = 0; d < NDT; ++d)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) st[((wave * NDT + d) * 4 + r) * 64] = o[d][r];
+  if (g == 0) {
+    st_m[wave][ql] = m_run;
+    st_l[wave][ql] = l_run;
+  }
+  __syncthreads();
+  // merge: wave w of a query group finishes its 16-wide output tiles w, w + 4, ...
+  const int w0 = wave - w;
+  float f[AWAVES];
+  const float invL = merge_factors(st_m + w0, st_l + w0, ql, kscale, f);
+  if (q0 + ql >= S) return;
+  uint16_t *const op = O + (size_t)(q0 + ql) * D + h * DH + 4 * g;
+#pragma unroll
+  for (int d = w; d < NDT; d += AWAVES) {
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float acc = 0.0f;
+#pragma unroll
+      for (int w2 = 0; w2 < AWAVES; ++w2) acc += st[(((w0 + w2) * NDT + d) * 4 + e) * 64] * f[w2];
+      v[e] = acc * invL;
+    }
+    *reinterpret_cast<uint2 *>(op + 16 * d) = pack4_bf16(v[0], v[1], v[2], v[3]);
   }
 }
 
@@ -1031,12 +1071,14 @@ hipError_t run_gemm(const char *name, const LlamaGemmArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int PRO, int EPI, int BM, int BN>
+template <int PRO, int EPI, int BM, int BN, int WR, int WC, int PARTS, int OCC, int DEP>
 hipError_t run_tile(const char *name, const LlamaGemmArgs &a, hipStream_t s) {
-  using S = TileShape<EPI, BM, BN>;
-  auto kern = llama_tile_kernel<PRO, EPI, BM, BN>;
+  using S = TileShape<EPI, BM, BN, WR, WC>;
+  auto kern = llama_tile_kernel<PRO, EPI, BM, BN, WR, WC, PARTS, OCC, DEP>;
   const int ncols = a.Npart * (EPI == kEpiQkvRope ? a.nparts : 1);
-  if (ncols % BN != 0 || a.Npart % 8 != 0 || a.K % S::KC != 0) return hipErrorInvalidValue;
+  if (ncols % BN != 0 || a.Npart % 8 != 0 || a.K % S::KC != 0 ||
+      (PRO == kProRmsnorm && a.K > 1024))
+    return hipErrorInvalidValue;
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = ncols / BN;
   const int G = tiles_m * tiles_n, grid = (G + 7) / 8 * 8;
   const int ok = cached_per_kernel(reinterpret_cast<const void *>(kern), [&](int) {
@@ -1047,11 +1089,12 @@ hipError_t run_tile(const char *name, const LlamaGemmArgs &a, hipStream_t s) {
   if (!ok) return hipErrorInvalidValue;
   {
     const double steps = a.K / S::KC;
-    npu_launch_plan p = make_plan(name, G, wg_per_cu(kern, 256), G, 16);
+    npu_launch_plan p = make_plan(name, G, wg_per_cu(kern, S::NT), G, 16);
+    p.unit_waves = WR * WC;
     p.tile_macs = (double)BM * BN * S::NB * a.K;
-    p.tile_valu = 4.0 * (steps * ((PRO == kProRmsnorm ? 32.0 : 2.0) * S::AR + 3.0 * S::BR + 20.0) +
+    p.tile_valu = WR * WC * (steps * ((PRO == kProRmsnorm ? 32.0 : 2.0) * S::AR + 3.0 * S::BR + 20.0) +
                          24.0 * S::TM * S::TN * S::NB + 120.0);
-    p.tile_lds_bytes = steps * (S::BUF + 4.0 * 2 * 1024 * (S::TM + S::NB * S::TN));
+    p.tile_lds_bytes = steps * (S::BUF + WR * WC * 2.0 * 1024 * (S::TM + S::NB * S::TN));
     p.tile_load_bytes = 2.0 * a.K * (BM + S::NB * BN);
     p.tile_store_bytes = 2.0 * BM * BN;
     const double parts = EPI == kEpiQkvRope ? a.nparts : S::NB;
@@ -1062,7 +1105,7 @@ hipError_t run_tile(const char *name, const LlamaGemmArgs &a, hipStream_t s) {
     plans_add(p);
   }
   const int xm = xcd_block_grid(tiles_m, tiles_n, BM, BN * S::NB, true);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 2 * S::BUF, s, a, tiles_m, tiles_n, xm);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(S::NT), 2 * S::BUF, s, a, tiles_m, tiles_n, xm);
   return hipGetLastError();
 }
 
@@ -1077,32 +1120,41 @@ hipError_t run_tile(const char *name, const LlamaGemmArgs &a, hipStream_t s) {
 // workgroups; K in chunks of 512, the down projection's 1408 in three, at
 // most 2048).  Chunk sizes keep two chunk buffers within the 160 KiB of LDS.
 hipError_t launch_llama_gemm(const LlamaGemmArgs &a, int pro, int epi, hipStream_t s) {
-  // Long sequences (see llama_tile_kernel), where their tiles outnumber what
-  // the 16-wave shapes are made for.  Measured, us, 16 waves / tiles (count):
-  //   QKV S x D: 2048x768 54.8 / 25.8 (1152), 1024x512 12.7 / 10.3 (384),
-  //     512x768 18.2 / 12.1 (288), 300x768 10.4 / 9.9 (180), 512x512 6.9 / 8.1 (192);
-  //   SwiGLU S x D x F: 2048x768x2048 61.8 / 23.9 (512 of 128 x 64; of 64 x 64
-  //     29.2), 1024x768x2048 31.9 / 16.1, 300x768x2048 16.1 / 10.7 (160 of 64 x
-  //     64), 512x512x1408 8.3 / 8.5 (176);
-  //   residual S x K x N: 2048x2048x768 49.5 / 19.6 (384 of 64 x 64),
-  //     1024x1408x512 12.4 / 8.2 (256 of 32 x 64), 512x768x768 8.7 / 5.7 (192),
-  //     512x512x512 4.1 / 4.6 (128), 300x2048x768 8.9 / 9.9 (120).
+  // Long sequences (see llama_tile_kernel): where the RMSNorm shapes above have
+  // more workgroups than the chip has CUs (a workgroup's A panel leaves no room
+  // for a second).  Measured, us, 16 waves / 64x128 tiles / 32x192 tiles:
+  //   QKV S x D: 2048x768 55.4 / 31.2 / 31.5, 2048x1024 80.9 / 38.9 / 46,
+  //     1024x512 13.1 / 11.4 / 12.5, 2100x512 23.5 / 17.5 / 24.7, 1400x256
+  //     11.4 / 9.0 / 9.8, 700x704 19.2 / - / 14.4, 2047x448 18.8 / - / 15.1,
+  //     600x960 29.6 / - / 22.1; not taken: 300x768 (240 workgroups) 10.6 / 13.1;
+  //   SwiGLU S x D x F, 16 waves / 64x64 tiles: 2048x768x2048 60.0 / 33.0,
+  //     2100x512x1280 22.2 / 18.6, 1024x512x1408 15.1 / 12.8, 300x768x2048
+  //     16.3 / 11.4, 700x704x1024 15.9 / 11.0; not taken: 2048x192x512 (256)
+  //     6.9 / 7.3.
+  // Residual GEMMs, S x K x N, 16 waves / tiles (count): 2048x2048x768 47.3 /
+  //     18.6 (384 of 64 x 64), 1024x1408x512 12.5 / 7.8 (256 of 32 x 64),
+  //     512x768x768 8.8 / 5.8 (192); not taken: 512x512x512 4.1 / 4.6 (128),
+  //     300x2048x768 8.9 / 9.9 (120).
   const auto tiles = [&](int bm, int bn, int cols) { return (long long)((a.M + bm - 1) / bm) * (cols / bn); };
-  if (pro == kProRmsnorm && a.K <= 1024) {
-    const int cols = a.Npart * (epi == kEpiQkvRope ? a.nparts : 1);
-    const bool many = tiles(64, 64, cols) >= (a.K <= 512 ? 256 : 160);
-    if (epi == kEpiQkvRope && many)
-      return run_tile<kProRmsnorm, kEpiQkvRope, 64, 64>("llama_rmsnorm_qkv_rope", a, s);
-    if (epi == kEpiSwiglu && tiles(128, 64, cols) >= 320)
-      return run_tile<kProRmsnorm, kEpiSwiglu, 128, 64>("llama_rmsnorm_swiglu", a, s);
-    if (epi == kEpiSwiglu && many)
-      return run_tile<kProRmsnorm, kEpiSwiglu, 64, 64>("llama_rmsnorm_swiglu", a, s);
+  const int cus = device_cus();
+  if (pro == kProRmsnorm && epi == kEpiQkvRope && a.K <= 1024) {
+    const int cols = a.Npart * a.nparts;
+    if (tiles(64, a.K <= 512 ? 64 : 48, cols) > cus) {
+      if (cols % 128 != 0)
+        return a.K <= 512 ? run_tile<kProRmsnorm, kEpiQkvRope, 32, 192, 1, 4, 1, 2, 1>("llama_rmsnorm_qkv_rope_tiles", a, s)
+                          : run_tile<kProRmsnorm, kEpiQkvRope, 32, 192, 1, 4, 4, 2, 1>("llama_rmsnorm_qkv_rope_tiles", a, s);
+      return a.K <= 512 ? run_tile<kProRmsnorm, kEpiQkvRope, 64, 128, 2, 4, 1, 4, 1>("llama_rmsnorm_qkv_rope_tiles", a, s)
+                        : run_tile<kProRmsnorm, kEpiQkvRope, 64, 128, 2, 4, 4, 4, 1>("llama_rmsnorm_qkv_rope_tiles", a, s);
+    }
   }
+  if (pro == kProRmsnorm && epi == kEpiSwiglu && a.K <= 1024 && tiles(a.K <= 512 ? 64 : 32, 64, a.Npart) > cus)
+    return a.K <= 512 ? run_tile<kProRmsnorm, kEpiSwiglu, 64, 64, 2, 4, 1, 4, 1>("llama_rmsnorm_swiglu_tiles", a, s)
+                      : run_tile<kProRmsnorm, kEpiSwiglu, 64, 64, 2, 4, 4, 4, 1>("llama_rmsnorm_swiglu_tiles", a, s);
   if (pro == kProPlain && epi == kEpiResidual && a.K <= 2048) {
     if (tiles(64, 64, a.Npart) >= 256)
-      return run_tile<kProPlain, kEpiResidual, 64, 64>("llama_matmul_residual", a, s);
+      return run_tile<kProPlain, kEpiResidual, 64, 64, 2, 2, 4, 2, 2>("llama_matmul_residual_tiles", a, s);
     if (tiles(32, 64, a.Npart) >= 160)
-      return run_tile<kProPlain, kEpiResidual, 32, 64>("llama_matmul_residual", a, s);
+      return run_tile<kProPlain, kEpiResidual, 32, 64, 2, 2, 4, 2, 2>("llama_matmul_residual_tiles", a, s);
   }
   if (pro == kProRmsnorm && epi == kEpiQkvRope) {
     if (a.K <= 512)
@@ -1128,21 +1180,21 @@ hipError_t launch_attention_tiles(const uint16_t *Q, const uint16_t *K, const ui
   auto kern = llama_attention_tile_kernel<DH>;
   const int nqb = (S + TQ - 1) / TQ, grid = nqb * H;
   {
-    // per wave and key block: 8 DH / 64 x 2 MFMAs, the softmax of 16 scores
-    // per lane; the plan's tile is the longest workgroup's (the last query block)
-    const double kblocks = nqb;
-    npu_launch_plan p = make_plan("llama_causal_attention", grid, wg_per_cu(kern, 256 * TGR), grid, 16);
-    p.unit_waves = 4 * TGR;
+    // the plan's tile is the longest workgroup's (the last query block): steps
+    // of 128 keys, 139 vector instructions per wave, step and 64 of the head dim
+    const double steps = (nqb * TQ + TKEYS - 1) / TKEYS;
+    npu_launch_plan p = make_plan("llama_causal_attention_tiles", grid, wg_per_cu(kern, TNT), grid, 16);
+    p.unit_waves = TNT / 64;
     p.load_phases = 1;
-    p.tile_macs = kblocks * 2.0 * TQ * TKB * DH;
-    p.tile_valu = 4.0 * (100.0 + 190.0 * kblocks) * (DH / 64);
-    p.tile_lds_bytes = kblocks * (2.0 * TKB * DH * 2 + 4.0 * 2.0 * TKB * DH * 2);
-    p.tile_load_bytes = kblocks * 2.0 * TKB * DH * 2 + TQ * DH * 2.0;
+    p.tile_macs = steps * 2.0 * TQ * TKEYS * DH;
+    p.tile_valu = TNT / 64 * (150.0 + 139.0 * steps) * (DH / 64);
+    p.tile_lds_bytes = steps * (2.0 * TKEYS * DH * 2 + 4.0 * 2.0 * TKEYS * DH * 2) + 2.0 * AttnTileShape<DH>::ST;
+    p.tile_load_bytes = steps * 2.0 * TKEYS * DH * 2 + TQ * DH * 2.0;
     p.tile_store_bytes = TQ * DH * 2.0;
     p.hbm_bytes = 4.0 * S * H * DH * 2;  // Q, K, V in, O out
     plans_add(p);
   }
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256 * TGR), 0, s, Q, K, V, O, S, H, scale);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(TNT), 0, s, Q, K, V, O, S, H, scale);
   return hipGetLastError();
 }
 
@@ -1150,9 +1202,9 @@ template <int DH>
 hipError_t launch_attention_dh(const uint16_t *Q, const uint16_t *K, const uint16_t *V,
                                uint16_t *O, int S, int H, float scale, hipStream_t s) {
   // 64-query workgroups from 160 of them on; measured, us, 16 queries / 64
-  // (workgroups of 64): S x heads x dim 2048x12x64 49.5 / 24.4 (384), 2048x6x128
-  // 55.8 / 35.3 (192), 1024x12x64 16.7 / 12.2 (192), 1024x8x64 10.2 / 11.3 (128),
-  // 1500x4x64 14.2 / 15.1 (96), 512x8x64 5.4 / 7.0 (64).
+  // (workgroups of 64): S x heads x dim 2048x12x64 50.0 / 23.8 (384), 2048x6x128
+  // 55.7 / 30.3 (192), 1024x12x64 16.7 / 12.1 (192), 1024x10x64 13.2 / 12.0 (160),
+  // 1024x8x64 10.5 / 11.9 (128), 1500x4x64 14.7 / 15.7 (96), 512x8x64 5.9 / 8.1 (64).
   if ((long long)((S + TQ - 1) / TQ) * H >= 160) return launch_attention_tiles<DH>(Q, K, V, O, S, H, scale, s);
   auto kern = llama_attention_kernel<DH>;
   const int G = (S + AQ - 1) / AQ * H, grid = (G + 7) / 8 * 8;

@@ -43,6 +43,16 @@ int cached_per_kernel(const void *kernel, F compute) {
   return v;
 }
 
+// CUs of the current device (256 if it cannot be queried).
+inline int device_cus() {
+  static const char key = 0;
+  const int n = cached_per_kernel(&key, [](int dev) {
+    int v = 0;
+    return hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess ? v : 0;
+  });
+  return n > 0 ? n : 256;
+}
+
 // Resident four-wave units per CU for `kernel` launched with `threads`
 // lanes per workgroup (resident workgroups x threads / 256), from the
 // runtime's occupancy calculator (registers and LDS decide it): the waves

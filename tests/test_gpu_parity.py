@@ -15,7 +15,7 @@ import torch
 
 import oracle
 import refs
-from npu_amd import blocks, configs, frontend, groups, lower, mlir
+from npu_amd import _lib, blocks, configs, frontend, groups, lower, mlir
 from npu_amd import inputs as rng
 from tolerance import RTOL_BF16, RTOL_F32, bf16, check_bf16_rounded, check_bf16_stage, check_bound
 
@@ -746,9 +746,10 @@ def test_c5_layer_small_shapes(cuda, S, D, H, F):
 
 
 @pytest.mark.parametrize("S,D,H,F", [
-    (1400, 256, 4, 896),   # QKV and SwiGLU 64x64, residual 32x64; S a row block of 56 past a tile
-    (330, 576, 9, 1920),   # K past 512: QKV and SwiGLU 64x64
-    (2100, 512, 8, 1280),  # SwiGLU 128x64, residual 64x64, 64-query attention; 52 rows past a tile
+    (1400, 256, 4, 896),   # QKV 64x128, residual 32x64; S a row block of 56 past a tile
+    (330, 576, 9, 1920),   # K past 512: SwiGLU
+    (390, 576, 9, 1920),   # K past 512, QKV 32x192: 6 rows past a tile
+    (2100, 512, 8, 1280),  # residual 64x64, 64-query attention; 52 rows past a tile
 ])
 def test_c5_stages_long_sequences(cuda, S, D, H, F):
     """Every stage on the tiles for long sequences, against the stage in
@@ -778,6 +779,69 @@ def test_c5_stages_long_sequences(cuda, S, D, H, F):
     check_bf16_stage(_host(act), ex["act"], refs.mag_swiglu(hn, inp["wg"], inp["wu"]), D + 4, what="act")
     check_bf16_rounded(_host(out), ex["out"], refs.mag_residual(st["act"], inp["wd"], st["h"]), F + 1,
                        what="out")
+
+
+def _plan_name(call):
+    """The kernel an entry point's call launches."""
+    call()
+    (p,) = _lib.last_launch_plans()
+    return p.kernel.decode()
+
+
+@pytest.mark.parametrize("S,D,H,F", [
+    (2048, 768, 12, 2048),  # K past 512: QKV 64x128, SwiGLU, residual 64x64
+    (2100, 512, 8, 1280),   # K of 512, a row block of 52 past a tile
+    (1003, 832, 13, 1024),  # QKV 32x192, 13 k steps of 64 (an odd count)
+    (1500, 320, 5, 1088),   # the same with K up to 512; down projection on 32x64
+    (1300, 1024, 8, 2048),  # the widest, heads of 128
+])
+def test_c5_row_bits_do_not_depend_on_the_sequence_length(cuda, S, D, H, F):
+    """The tiles that long sequences run on give each row the bits that the
+    kernels of short sequences give it: every stage against calls on 64 rows
+    at a time (the attention against a call per head)."""
+    dh = D // H
+    bf = lambda i, shape, sd: _dev(rng.to_bf16_bits(rng.normal(191 + S, i, shape, 0.0, sd)))
+    x, q, k, v = (bf(i, (S, D), 1.0) for i in range(4))
+    a = bf(4, (S, F), 1.0)
+    wq, wk, wv, wo = (bf(5 + i, (D, D), 0.04) for i in range(4))
+    wg, wu, wd = bf(9, (D, F), 0.04), bf(10, (D, F), 0.04), bf(11, (F, D), 0.04)
+    g = _dev(rng.uniform(191 + S, 12, (D,), 0.5, 1.5))
+    cos, sin = (_dev(t) for t in configs.rope_tables(S, dh))
+    Q, K, V, A, h, out = (_bf_dev((S, D)) for _ in range(6))
+    act = _bf_dev((S, F))
+
+    def rows(r):
+        return [("llama_rmsnorm_qkv_rope", lambda: groups.fused_llama_qkv_rope(
+                    x[r], g, wq, wk, wv, cos[r], sin[r], Q[r], K[r], V[r], LL_EPS)),
+                ("llama_matmul_residual", lambda: groups.fused_llama_matmul_residual(v[r], wo, x[r], h[r])),
+                ("llama_rmsnorm_swiglu", lambda: groups.fused_llama_rmsnorm_swiglu(
+                    x[r], g, wg, wu, act[r], LL_EPS)),
+                ("llama_matmul_residual", lambda: groups.fused_llama_matmul_residual(a[r], wd, x[r], out[r]))]
+
+    outs = (Q, K, V, h, act, out)
+    for name, call in rows(slice(None)):
+        assert _plan_name(call) == name + "_tiles"
+    torch.cuda.synchronize()
+    tiles = [t.clone() for t in outs]
+    for t in outs:
+        t.fill_(float("nan"))
+    for r0 in range(0, S, 64):
+        for name, call in rows(slice(r0, r0 + 64)):
+            assert _plan_name(call) == name
+    torch.cuda.synchronize()
+    for n, t, u in zip(("Q", "K", "V", "h", "act", "out"), outs, tiles):
+        assert np.array_equal(_host(t), _host(u)), n
+
+    want = "llama_causal_attention" + ("_tiles" if -(-S // 64) * H >= 160 else "")
+    assert _plan_name(lambda: groups.fused_llama_attention(q, k, v, A, H, dh ** -0.5)) == want
+    for i in range(H):
+        c = slice(i * dh, (i + 1) * dh)
+        one = _bf_dev((S, dh))
+        assert _plan_name(lambda: groups.fused_llama_attention(
+            q[:, c].contiguous(), k[:, c].contiguous(), v[:, c].contiguous(), one, 1, dh ** -0.5)) \
+            == "llama_causal_attention"
+        torch.cuda.synchronize()
+        assert np.array_equal(_host(A[:, c].contiguous()), _host(one)), f"head {i}"
 
 
 @pytest.mark.parametrize("S,H,dh", [(641, 15, 128), (64, 160, 64), (129, 64, 64), (193, 40, 128)])
