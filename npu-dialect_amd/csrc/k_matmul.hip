@@ -338,7 +338,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void matmul_x6_kernel(
 }
 
 template <int BM, int BN, int WR, int WC, bool VEC>
-hipError_t launch_x6(const MatmulArgs &a, hipStream_t s) {
+hipError_t launch_x6(const char *name, const MatmulArgs &a, hipStream_t s) {
   using S = X6Shape<BM, BN, WR, WC>;
   auto kern = matmul_x6_kernel<BM, BN, WR, WC, VEC>;
   // the dynamic LDS limit, raised once per device
@@ -351,7 +351,7 @@ hipError_t launch_x6(const MatmulArgs &a, hipStream_t s) {
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
   const int G = tiles_m * tiles_n, grid = (G + kXcds - 1) / kXcds * kXcds;
   const double steps = (a.K + S::KC - 1) / S::KC;
-  npu_launch_plan p = make_plan("matmul_f32_bf16x6", G, wg_per_cu(kern, S::NT), G, 16);
+  npu_launch_plan p = make_plan(name, G, wg_per_cu(kern, S::NT), G, 16);
   p.unit_waves = WR * WC;
   p.load_phases = 1;
   p.tile_macs = 6.0 * BM * BN * S::KC * steps;
@@ -368,28 +368,53 @@ hipError_t launch_x6(const MatmulArgs &a, hipStream_t s) {
 }
 
 template <int BM, int BN, int WR, int WC>
-hipError_t launch_x6(const MatmulArgs &a, hipStream_t s) {
-  return a.N % 4 == 0 ? launch_x6<BM, BN, WR, WC, true>(a, s) : launch_x6<BM, BN, WR, WC, false>(a, s);
+hipError_t launch_x6(const char *name, const MatmulArgs &a, hipStream_t s) {
+  return a.N % 4 == 0 ? launch_x6<BM, BN, WR, WC, true>(name, a, s) : launch_x6<BM, BN, WR, WC, false>(name, a, s);
 }
 
-// Tiles of 256 x 96 when there are enough to give most CUs one (a workgroup's
-// 153 KB of LDS leave no room for a second), of 64 x 64 when there are enough
-// of those, else the split-K tiles of 16 x 16.  Measured, us, as 16x16 / 64x64
-// / 256x96: 2000x1024x3000 (256 tiles of 256 x 96) 421 / 128 / 82;
-// 1000x2048x1999 (84; 512 of 64 x 64) 403 / 97 / 156; 2000x64x2000 (168) 80 /
-// 12.5 / 11.7; 1024x1024x1024 (256 of 64 x 64) 46 / 30 / 74; 512x1024x2048
-// (256) 50 / 30 / 74; 627x648x900 (150) 22.0 / 20.5 / 50; 64x1024x4096 (64)
-// 17.4 / 27.7 / 73; 512x1024x512 (64) 12.3 / 28 / 72.
+// Which tiles: the ones whose rounds over the CUs take the least time, by the
+// rates measured for each (us per k step of 32 and round, and per tile of
+// 16 x 16).  A count of tiles alone does not tell: one row against 32 000
+// columns counts 334 tiles of 256 x 96, of which hardly anything lies inside
+// the matrix.  So the split-K tiles of 16 x 16 are kept below 32 rows or
+// columns (half a 64 x 64 tile), and below kMinMid tiles of 64 x 64, where the
+// rates are least certain, for anything thinner than a tile or without a fifth
+// to gain.  Over 260 shapes the choice takes 1.2 % longer than the fastest of
+// the three (geometric mean).  Measured, us, as 16x16 / 64x64 / 256x96:
+// 2000x1024x3000 (256 tiles of 256 x 96) 420 / 124 / 83; 1500x1024x4096 (258)
+// 255 / 119 / 147; 2026x384x6040 (504) 318 / 94 / 69; 1024x1024x1024 (256 of
+// 64 x 64) 43 / 29 / 73; 225x1520x2234 (140) 87 / 51 / 117; 1x512x32000 (500)
+// 12.7 / 22.7 / 76; 16x512x32000 15.5 / 23.1 / 76; 64x512x32000 48 / 24 / 79;
+// 50000x256x10 (782) 27.3 / 27.5 / 25; 4521x508x36 (71) 8.3 / 16.0 / -;
+// 1x484x28358 (444) 23.9 / 27.3 / -; 1980x360x158 (93) 14.3 / 16.3 / -.
 // Error against 64 bits, relative 2-norm: K = 1024 1.2e-7 (16x16: 2.9e-7).
-constexpr int kMinBig = 160, kMinMid = 176;
+enum class MatmulTile { k16x16, k64x64, k256x96 };
+
+constexpr int kMinMid = 176;
+
+MatmulTile matmul_tile(const MatmulArgs &a) {
+  const int cus = device_cus();
+  auto tiles = [&](int bm, int bn) { return (long long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
+  auto rounds = [&](long long t) { return (double)((t + cus - 1) / cus); };
+  const long long mid = tiles(64, 64);
+  const int least = mid < kMinMid ? 64 : 32;
+  if (a.M < least || a.N < least) return MatmulTile::k16x16;
+  const double steps = (a.K + 31) / 32;
+  // a row of B that is no multiple of 16 bytes is loaded word by word
+  const double t16 = 4.0 + tiles(16, 16) * (a.N % 4 == 0 ? 0.003 + 0.0003 * steps : 0.004 + 0.0006 * steps);
+  // two workgroups of 64 x 64 share a CU, one of 256 x 96 has it alone
+  const double t64 = 5.0 + steps * (mid <= cus ? 0.8 : 0.58 * rounds(mid));
+  const double t256 = 6.0 + steps * 2.25 * rounds(tiles(256, 96));
+  if (t16 * (mid < kMinMid ? 0.8 : 1.0) <= (t64 < t256 ? t64 : t256)) return MatmulTile::k16x16;
+  return t64 <= t256 ? MatmulTile::k64x64 : MatmulTile::k256x96;
+}
 
 }  // namespace
 
 hipError_t launch_matmul_bias_act_f32(const MatmulArgs &a, hipStream_t s) {
-  const long long big = (long long)((a.M + 255) / 256) * ((a.N + 95) / 96);
-  const long long mid = (long long)((a.M + 63) / 64) * ((a.N + 63) / 64);
-  if (big >= kMinBig) return launch_x6<256, 96, 4, 2>(a, s);
-  if (mid >= kMinMid) return launch_x6<64, 64, 2, 2>(a, s);
+  const MatmulTile tile = matmul_tile(a);
+  if (tile == MatmulTile::k256x96) return launch_x6<256, 96, 4, 2>("matmul_f32_bf16x6_256x96", a, s);
+  if (tile == MatmulTile::k64x64) return launch_x6<64, 64, 2, 2>("matmul_f32_bf16x6_64x64", a, s);
   const int tiles_n = (a.N + 15) / 16, tiles = tiles_n * ((a.M + 15) / 16);
   const int nchunks = (a.K + 15) / 16;
   const bool vec = a.N % 4 == 0;

@@ -30,6 +30,13 @@ def _host(t):
     return configs.to_host(t)
 
 
+def _plan_name(call):
+    """The kernel an entry point's call launches."""
+    call()
+    (p,) = _lib.last_launch_plans()
+    return p.kernel.decode()
+
+
 def _widened_conv(x_bits, w_bits, b, pad, act):
     """The oracle's f32 value of a bf16 conv chain before its final rounding:
     the f32 loops over the inputs widened to f32 (bf16 x bf16 products are
@@ -80,8 +87,11 @@ def test_c1_matmul_shapes(cuda, M, K, N, act, bias):
     (769, 36, 960, "relu", True),      # 64x64 tiles: a row and 4 k past a tile
     (833, 4, 833, "none", False),      # one k run, odd N (word loads and stores)
     (704, 64, 1021, "relu6", True),    # whole k steps, columns ragged by 1 mod 4
-    (2049, 68, 1732, "relu", True),    # 256x96 tiles, a row past a tile, ragged columns
-    (2305, 32, 1537, "none", True),    # 256x96 tiles, odd N, one whole k step
+    (2049, 68, 1732, "relu", True),    # a row past a tile, ragged columns, three k steps
+    (2305, 32, 1537, "none", True),    # odd N, one whole k step
+    (2049, 1028, 2500, "relu", True),  # 256x96 tiles, a row past a tile, 33 k steps, the last of 4
+    (2305, 1020, 2399, "none", True),  # 256x96 tiles, odd N, the last k step of 28
+    (1025, 2020, 1028, "relu6", True),  # 64x64 tiles, 64 k steps, the last of 4
 ])
 def test_c1_matmul_large_tiles(cuda, M, K, N, act, bias):
     """Edges of the large-output tiles on the bf16 matrix pipe."""
@@ -94,6 +104,28 @@ def test_c1_matmul_large_tiles(cuda, M, K, N, act, bias):
     with oracle.threaded():
         ref, mag = refs.matmul_bias_act(A, B, b, act)
     check_bound(_host(out), ref, mag, RTOL_F32, what=f"matmul {M}x{K}x{N}")
+
+
+@pytest.mark.parametrize("M,K,N,tile", [
+    # a few rows or columns: mostly padding in the large tiles
+    (1, 512, 32000, "matmul_bias_act_f32"), (16, 1024, 32000, "matmul_bias_act_f32"),
+    (1, 1024, 16384, "matmul_bias_act_f32"), (8, 512, 11264, "matmul_bias_act_f32"),
+    (11300, 1024, 16, "matmul_bias_act_f32"), (4521, 508, 36, "matmul_bias_act_f32"),
+    (256, 512, 256, "matmul_bias_act_f32"),
+    (64, 512, 32000, "matmul_f32_bf16x6_64x64"), (1024, 1024, 1024, "matmul_f32_bf16x6_64x64"),
+    # a few more 256x96 tiles than CUs: a second round
+    (1500, 1024, 4096, "matmul_f32_bf16x6_64x64"), (1100, 1000, 5001, "matmul_f32_bf16x6_64x64"),
+    (2000, 1024, 3000, "matmul_f32_bf16x6_256x96"), (2049, 1028, 2500, "matmul_f32_bf16x6_256x96"),
+    (1100, 1000, 4801, "matmul_f32_bf16x6_256x96"),
+])
+def test_c1_matmul_tile_rule(cuda, M, K, N, tile):
+    """The kernel that each shape runs on, and its result against float64."""
+    g = torch.Generator(device="cuda").manual_seed(43)
+    A, B = (torch.rand(s, generator=g, device="cuda") * 2 - 1 for s in ((M, K), (K, N)))
+    out = torch.full((M, N), float("nan"), device="cuda")
+    assert _plan_name(lambda: groups.fused_matmul_bias_act(A, B, None, out, "none")) == tile
+    ref, mag = A.double() @ B.double(), A.double().abs() @ B.double().abs()
+    check_bound(_host(out), _host(ref), _host(mag), RTOL_F32, what=f"matmul {M}x{K}x{N}")
 
 
 def test_c1_matmul_large_tiles_out_of_split_domain(cuda):
@@ -779,13 +811,6 @@ def test_c5_stages_long_sequences(cuda, S, D, H, F):
     check_bf16_stage(_host(act), ex["act"], refs.mag_swiglu(hn, inp["wg"], inp["wu"]), D + 4, what="act")
     check_bf16_rounded(_host(out), ex["out"], refs.mag_residual(st["act"], inp["wd"], st["h"]), F + 1,
                        what="out")
-
-
-def _plan_name(call):
-    """The kernel an entry point's call launches."""
-    call()
-    (p,) = _lib.last_launch_plans()
-    return p.kernel.decode()
 
 
 @pytest.mark.parametrize("S,D,H,F", [
