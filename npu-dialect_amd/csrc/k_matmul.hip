@@ -142,14 +142,16 @@ __global__ __launch_bounds__(kWaves * 64) void matmul_bias_act_f32_kernel(
 // ---- large outputs: tiles on the bf16 matrix pipe ------------------------------
 //
 // A BM x BN tile per workgroup of WR x WC waves, K in steps of 32.  Each
-// value is split into its three bf16 parts as it is staged (npu_device.hpp)
-// and a product takes six bf16 MFMAs, 2.7 times the f32 matrix rate, at f32
-// accuracy.  A's rows go to LDS as records of three 64-byte part runs; B's
-// rows as 16-column strips per part, read back as column runs by the
-// transposing LDS read.  The operands are swapped (B's fragment first), so a
-// lane ends with four consecutive columns of one row: 16-byte stores.  Two LDS
-// buffers, one barrier per step: the next step's runs are split and written
-// and the one after's loaded while this one is multiplied.
+// value is split into its three bf16 parts as it is staged (npu_device.hpp; the
+// first part rounded to nearest, as truncating it lost up to two bits of a
+// product: 80.0 us against 78.6 at 2000x1024x3000) and a product takes six bf16
+// MFMAs, 2.7 times the f32 matrix rate, at f32 accuracy.  A's rows go to LDS as
+// records of three 64-byte part runs; B's rows as 16-column strips per part,
+// read back as column runs by the transposing LDS read.  The operands are
+// swapped (B's fragment first), so a lane ends with four consecutive columns of
+// one row: 16-byte stores.  Two LDS buffers, one barrier per step: the next
+// step's runs are split and written and the one after's loaded while this one
+// is multiplied.
 //
 // What bounds it: the MFMAs and the split's vector work (34 instructions per
 // 16-byte run), which two waves per SIMD overlap; the larger the tile, the
@@ -229,7 +231,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void matmul_x6_kernel(
     for (int i = 0; i < S::AR; ++i) {
       const u32x4 v = masked(av[i], k0 + ak < K);
       dom.fold(v);
-      const Parts4 p = split_parts(v);
+      const Parts4 p = split_parts_rn(v);
       *reinterpret_cast<uint2 *>(buf + adst[i]) = p.h;
       *reinterpret_cast<uint2 *>(buf + adst[i] + 64) = p.m;
       *reinterpret_cast<uint2 *>(buf + adst[i] + 128) = p.l;
@@ -238,7 +240,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void matmul_x6_kernel(
     for (int i = 0; i < S::BR; ++i) {
       const u32x4 v = masked(bv[i], k0 + bk[i] < K);
       dom.fold(v);
-      const Parts4 p = split_parts(v);
+      const Parts4 p = split_parts_rn(v);
       if (NT * (i + 1) <= S::BITEMS || tid + NT * i < S::BITEMS) {
         *reinterpret_cast<uint2 *>(buf + bdst[i]) = p.h;
         *reinterpret_cast<uint2 *>(buf + bdst[i] + S::STRIPS * S::SB) = p.m;
@@ -387,7 +389,8 @@ hipError_t launch_x6(const char *name, const MatmulArgs &a, hipStream_t s) {
 // 12.7 / 22.7 / 76; 16x512x32000 15.5 / 23.1 / 76; 64x512x32000 48 / 24 / 79;
 // 50000x256x10 (782) 27.3 / 27.5 / 25; 4521x508x36 (71) 8.3 / 16.0 / -;
 // 1x484x28358 (444) 23.9 / 27.3 / -; 1980x360x158 (93) 14.3 / 16.3 / -.
-// Error against 64 bits, relative 2-norm: K = 1024 1.2e-7 (16x16: 2.9e-7).
+// Error against 64 bits, relative 2-norm, x6 tiles / 16x16: K = 4 2.9e-8 /
+// 4.0e-8, 44 4.4e-8 / 8.0e-8, 256 6.8e-8 / 1.5e-7, 1024 1.1e-7 / 2.9e-7.
 enum class MatmulTile { k16x16, k64x64, k256x96 };
 
 constexpr int kMinMid = 176;

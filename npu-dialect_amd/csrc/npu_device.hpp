@@ -211,7 +211,12 @@ __device__ __forceinline__ Frag16 load16(const void *p) {
 // add up to less than 2^-21 |a b|.  This is the bf16x6 scheme of Henry,
 // Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence
 // Datatype For Higher-Precision Computations" (ARITH 2019), with a
-// truncating first split.  On gfx950 a bf16 MFMA (16 clocks for 16x16x32)
+// truncating first split.  split_parts_rn rounds the first part to nearest
+// even instead, at the same number of instructions: |m| <= 2^-8 |a| and
+// |l| <= 2^-17 |a|, so the products left out stay below 2^-24 |a b|, half a
+// unit in the last place of the f32 product (over all significands 5.9e-8;
+// truncating, 2.35e-7 at 0x3f80ff80).  It cannot round up to Inf inside the
+// split's domain.  On gfx950 a bf16 MFMA (16 clocks for 16x16x32)
 // does the 16x work of an f32 MFMA (32 clocks for 16x16x4), so the six
 // products take 6 * 16 clocks where the f32 instructions take 8 * 32.
 //
@@ -256,6 +261,24 @@ __device__ __forceinline__ Parts4 split_parts(u32x4 v) {
   const float s0 = r[0] - __uint_as_float(p.m.x << 16), s1 = r[1] - __uint_as_float(p.m.x & 0xffff0000u);
   const float s2 = r[2] - __uint_as_float(p.m.y << 16), s3 = r[3] - __uint_as_float(p.m.y & 0xffff0000u);
   p.l = make_uint2(cvt_pk_bf16(s0, s1), cvt_pk_bf16(s2, s3));
+  return p;
+}
+__device__ __forceinline__ Parts4 split_parts_rn(u32x4 v) {
+  float a[4], r[4], s[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) a[e] = __uint_as_float(v[e]);
+  Parts4 p;
+  auto rest = [](const float (&x)[4], uint2 h, float (&y)[4]) {  // x - h, exact
+    y[0] = x[0] - __uint_as_float(h.x << 16);
+    y[1] = x[1] - __uint_as_float(h.x & 0xffff0000u);
+    y[2] = x[2] - __uint_as_float(h.y << 16);
+    y[3] = x[3] - __uint_as_float(h.y & 0xffff0000u);
+  };
+  p.h = make_uint2(cvt_pk_bf16(a[0], a[1]), cvt_pk_bf16(a[2], a[3]));
+  rest(a, p.h, r);
+  p.m = make_uint2(cvt_pk_bf16(r[0], r[1]), cvt_pk_bf16(r[2], r[3]));
+  rest(r, p.m, s);
+  p.l = make_uint2(cvt_pk_bf16(s[0], s[1]), cvt_pk_bf16(s[2], s[3]));
   return p;
 }
 // The domain test, spread over the runs a lane splits: fold() takes a

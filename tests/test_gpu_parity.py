@@ -128,6 +128,27 @@ def test_c1_matmul_tile_rule(cuda, M, K, N, tile):
     check_bound(_host(out), _host(ref), _host(mag), RTOL_F32, what=f"matmul {M}x{K}x{N}")
 
 
+@pytest.mark.parametrize("M,N,tile", [(832, 896, "64x64"), (2560, 2304, "256x96")])
+def test_c1_matmul_large_tiles_single_products(cuda, M, N, tile):
+    """Every output a single product of two f32 values, the significands that
+    a three-part split loses most of among them: off by the products of parts
+    left out (below 2^-24 of it) and one unit in the last place of the sum
+    (the MFMA adds with fewer guard bits than rounding to nearest needs)."""
+    worst = np.array([0x3f80ff80, 0x3f80ffff, 0x3f807f80, 0x3f808080, 0x3f80807f, 0x3f81807f,
+                      0x3f80ff7f, 0x3fff7f7f, 0x3f800001, 0x3fffffff], np.uint32).view(np.float32)
+    K = 4 if tile == "64x64" else 1024  # what the rule gives each tile
+    A, B = np.zeros((M, K), np.float32), np.zeros((K, N), np.float32)
+    A[:, 1], B[1] = rng.uniform(44, 0, (M,), 1, 2), rng.uniform(44, 1, (N,), 1, 2)
+    A[:len(worst), 1] = B[1, :len(worst)] = worst
+    out = torch.empty(M, N, device="cuda")
+    assert _plan_name(lambda: groups.fused_matmul_bias_act(_dev(A), _dev(B), None, out, "none")) \
+        == f"matmul_f32_bf16x6_{tile}"
+    torch.cuda.synchronize()
+    ref = np.outer(A[:, 1].astype(np.float64), B[1].astype(np.float64))
+    # the sum's earlier roundings are at 2^-7 of the product and below
+    assert (np.abs(_host(out) - ref) <= 3 * 2.0 ** -24 * (1 + 2.0 ** -6) * ref).all()
+
+
 def test_c1_matmul_large_tiles_out_of_split_domain(cuda):
     """Values the three-part split does not take (Inf, NaN, magnitudes of 2^60
     and 2^-70, an f32 subnormal) in A or B: their tiles are computed with f32
