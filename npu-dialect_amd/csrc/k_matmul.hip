@@ -157,9 +157,13 @@ __global__ __launch_bounds__(kWaves * 64) void matmul_bias_act_f32_kernel(
 // 16-byte run), which two waves per SIMD overlap; the larger the tile, the
 // fewer splits per product.
 //
-// A value outside the split's domain (Inf, NaN, |v| >= 2^55, 0 < |v| < 2^-55)
-// makes its workgroup compute its tile again with f32 MFMAs straight from
-// memory.
+// A value outside the split's domain (Inf, NaN, |v| >= 2^55, 0 < |v| < 2^-55: the
+// tail of an exponential) makes its workgroup start over, soon after staging it,
+// with f32 MFMAs on the same tiles staged unsplit.  us with such a value in every
+// row's first (middle) k, 16x16 tiles / six products first and the operands then
+// from memory / so: 1024x1024x1024 44 / 94 / 33 (58), 1024x512x1024 24 / 52 / 21
+// (26), 20000x512x64 28 / 88 / 28 (37), 2000x1024x3000 410 / 323 / 117 (182); the
+// tests for it take 2 % where there is none.
 template <int BM, int BN, int WR, int WC>
 struct X6Shape {
   static constexpr int NT = 64 * WR * WC, KC = 32;
@@ -169,6 +173,10 @@ struct X6Shape {
   static constexpr int ABYTES = BM * AREC, BUF = ABYTES + 3 * STRIPS * SB;
   static constexpr int AR = BM * 8 / NT;                      // 16-byte runs per thread and step
   static constexpr int BITEMS = KC * BN / 4, BR = (BITEMS + NT - 1) / NT;
+  // unsplit: A rows 16 bytes past 128, B rows 16 past a multiple of 128 (a lane
+  // group's 16 words of four rows use every bank once)
+  static constexpr int AF = KC * 4 + 16, BF = BN * 4 + 16;
+  static_assert(BM * AF + KC * BF <= BUF, "the unsplit tile fits a buffer");
   static_assert(BM * 8 % NT == 0 && TM >= 1 && TN >= 1, "whole runs, whole blocks");
 };
 
@@ -276,38 +284,73 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void matmul_x6_kernel(
   commit(0, x6mem);
   fetch(KC);
   __syncthreads();
-  for (int s = 0; s < steps; ++s) {
-    multiply(x6mem + (s & 1) * S::BUF);
-    if (s + 1 < steps) {
-      commit((s + 1) * KC, x6mem + ((s + 1) & 1) * S::BUF);
-      fetch((s + 2) * KC);
+  // The domain is tested after 2, 8, 32, ... steps (a test costs about 0.1 us):
+  // data that has such values mostly has them throughout, and one that is
+  // staged later costs the steps done before it.
+  bool out_of_domain = false;
+  for (int s = 0; s < steps && !out_of_domain;) {
+    for (const int end = min(max(2, 4 * s), steps); s < end; ++s) {
+      multiply(x6mem + (s & 1) * S::BUF);
+      if (s + 1 < steps) {
+        commit((s + 1) * KC, x6mem + ((s + 1) & 1) * S::BUF);
+        fetch((s + 2) * KC);
+      }
+      __syncthreads();
     }
+    if (__builtin_amdgcn_ballot_w64(dom.miss()) != 0 && lane == 0) missed = 1;
     __syncthreads();
+    out_of_domain = missed;
   }
-  if (__builtin_amdgcn_ballot_w64(dom.miss()) != 0 && lane == 0) missed = 1;
-  __syncthreads();
-  if (missed) {
-    // f32 MFMAs, k in order, operands from memory (K % 4 == 0)
-    const float *arow[TM], *bp[TN];
+  if (out_of_domain) {
+    // f32 MFMAs: step t of a run of 16 takes k = 4q + t of lane group q
+    // (places in LDS from an opaque lane: none is held through the loop above)
+    const int tid = opaque(threadIdx.x), r = tid & 15, q = (tid >> 4) & 3;
+    auto commit_f32 = [&](int k0, unsigned char *buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) arow[i] = A + (size_t)min(m0 + wr * (BM / WR) + 16 * i + r, M - 1) * K + q;
+      for (int i = 0; i < S::AR; ++i)
+        *reinterpret_cast<u32x4 *>(buf + ((tid + NT * i) >> 3) * S::AF + ak * 4) = masked(av[i], k0 + ak < K);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) bp[j] = B + (size_t)q * N + min(n0 + wc * (BN / WC) + 16 * j + r, N - 1);
+      for (int i = 0; i < S::BR; ++i)
+        if (NT * (i + 1) <= S::BITEMS || tid + NT * i < S::BITEMS)
+          *reinterpret_cast<u32x4 *>(buf + BM * S::AF + (tid + NT * i) / (BN / 4) * S::BF + (tid + NT * i) % (BN / 4) * 16) =
+              masked(bv[i], k0 + bk[i] < K);
+    };
+    auto multiply_f32 = [&](const unsigned char *buf) __attribute__((always_inline)) {
+#pragma unroll
+      for (int run = 0; run < KC / 16; ++run) {
+        Frag16 af[TM], bf[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+          af[i] = load16(buf + (wr * (BM / WR) + 16 * i + r) * S::AF + run * 64 + q * 16);
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            bf[j].f[t] = *reinterpret_cast<const float *>(buf + BM * S::AF + (run * 16 + 4 * q + t) * S::BF +
+                                                          (wc * (BN / WC) + 16 * j + r) * 4);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) MfmaF32::step(acc[i][j], bf[j], af[i], t);
+      }
+    };
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k = 0; k < K; k += 4) {
-      float af[TM], bf[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) af[i] = arow[i][k];
-#pragma unroll
-      for (int j = 0; j < TN; ++j) bf[j] = bp[j][(size_t)k * N];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j], af[i], acc[i][j], 0, 0, 0);
+    fetch(0);
+    commit_f32(0, x6mem);
+    fetch(KC);
+    __syncthreads();
+    for (int s = 0; s < steps; ++s) {
+      multiply_f32(x6mem + (s & 1) * S::BUF);
+      if (s + 1 < steps) {
+        commit_f32((s + 1) * KC, x6mem + ((s + 1) & 1) * S::BUF);
+        fetch((s + 2) * KC);
+      }
+      __syncthreads();
     }
   }
 
@@ -406,8 +449,8 @@ MatmulTile matmul_tile(const MatmulArgs &a) {
   // a row of B that is no multiple of 16 bytes is loaded word by word
   const double t16 = 4.0 + tiles(16, 16) * (a.N % 4 == 0 ? 0.003 + 0.0003 * steps : 0.004 + 0.0006 * steps);
   // two workgroups of 64 x 64 share a CU, one of 256 x 96 has it alone
-  const double t64 = 5.0 + steps * (mid <= cus ? 0.8 : 0.58 * rounds(mid));
-  const double t256 = 6.0 + steps * 2.25 * rounds(tiles(256, 96));
+  const double t64 = 5.0 + steps * (mid <= cus ? 0.88 : 0.58 * rounds(mid));
+  const double t256 = 6.0 + steps * 2.3 * rounds(tiles(256, 96));
   if (t16 * (mid < kMinMid ? 0.8 : 1.0) <= (t64 < t256 ? t64 : t256)) return MatmulTile::k16x16;
   return t64 <= t256 ? MatmulTile::k64x64 : MatmulTile::k256x96;
 }

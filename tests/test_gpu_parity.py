@@ -149,18 +149,23 @@ def test_c1_matmul_large_tiles_single_products(cuda, M, N, tile):
     assert (np.abs(_host(out) - ref) <= 3 * 2.0 ** -24 * (1 + 2.0 ** -6) * ref).all()
 
 
-def test_c1_matmul_large_tiles_out_of_split_domain(cuda):
+@pytest.mark.parametrize("M,K,N,tile", [
+    (769, 40, 960, "64x64"), (705, 1020, 1021, "64x64"),         # vector and word loads
+    (2049, 1028, 2500, "256x96"), (2305, 1020, 2399, "256x96"),
+])
+def test_c1_matmul_large_tiles_out_of_split_domain(cuda, M, K, N, tile):
     """Values the three-part split does not take (Inf, NaN, magnitudes of 2^60
-    and 2^-70, an f32 subnormal) in A or B: their tiles are computed with f32
-    MFMAs, every value and every Inf and NaN where the f32 loops give them."""
-    M, K, N = 769, 40, 960
+    and 2^-70, an f32 subnormal) in A or B, in the first and the last k step
+    and between: their tiles are computed with f32 MFMAs, every value and every
+    Inf and NaN where the f32 loops give them."""
     A = rng.uniform(42, 0, (M, K), -1, 1)
     B = rng.uniform(42, 1, (K, N), -1, 1)
-    A[3, 5], A[70, 39], A[200, 0] = np.inf, np.nan, 2.0 ** 60
+    A[3, 5], A[70, K - 1], A[200, 0] = np.inf, np.nan, 2.0 ** 60
     A[400] = 2.0 ** -70
-    B[7, 130], B[39, 959], B[:, 500] = -np.inf, 2.0 ** -140, 2.0 ** -90
+    B[7, 130], B[K - 1, N - 1], B[:, 500], B[K // 2, 300] = -np.inf, 2.0 ** -140, 2.0 ** -90, 2.0 ** 57
     out = torch.empty(M, N, device="cuda")
-    groups.fused_matmul_bias_act(_dev(A), _dev(B), None, out, "none")
+    assert _plan_name(lambda: groups.fused_matmul_bias_act(_dev(A), _dev(B), None, out, "none")) \
+        == f"matmul_f32_bf16x6_{tile}"
     torch.cuda.synchronize()
     got = _host(out)
     with oracle.threaded():
