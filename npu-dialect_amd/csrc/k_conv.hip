@@ -10,13 +10,15 @@
 // becomes the grid's y dimension; the pixel dimension is the grid's x.
 //
 // A workgroup of 2 x 2 waves owns BM pixels x BN filters.  The reduction walks
-// the taps and, within a tap, chunks of 128 bytes of channels; per step the
+// the taps and, within a tap, chunks of 128 bytes of channels (or, for few
+// channels, the 16-byte runs of all taps one after the other); per step the
 // pixels' runs (zero outside the image and past C) and the filters' runs are
 // staged in LDS, double-buffered, the next two steps' loads in flight while
-// the current one is multiplied, one barrier per step.  The filter fragment is the
-// MFMA's first operand where F is a multiple of 4, so a lane ends with four consecutive filters of one
-// pixel: the epilogue (bias add, residual add, act, and the bf16 rounding of
-// the bf16 variant) runs on the accumulators and stores 8 or 16 bytes.
+// the current one is multiplied, one barrier per step.  The filter fragment is
+// the MFMA's first operand where F is a multiple of 4, so a lane ends with four
+// consecutive filters of one pixel: the epilogue (bias add, residual add, act,
+// and the bf16 rounding of the bf16 variant) runs on the accumulators and stores
+// 8 or 16 bytes.
 // C need not be a multiple of an MFMA fragment's 16 (f32) or 32 (bf16)
 // channels: a 16-byte run past C is staged as zero.  F need not be a multiple
 // of 16 either: filters past F read filter F - 1 and are not stored.
@@ -29,14 +31,22 @@ namespace npu {
 
 namespace {
 
+// How the steps of 128 bytes of a filter walk the reduction: a tap's channels in
+// chunks, the last one zero past C; the 16-byte runs of all taps one after the
+// other; or the runs of one step.
+enum class Walk { kTapChunks, kRuns, kOneStep };
+constexpr const char *kWalkName[] = {"conv2d_nhwc", "conv2d_nhwc_runs", "conv2d_nhwc_one_step"};
+
 struct ConvTileArgs {
   const void *x, *w, *res;
   const float *bias;
   void *out;
   int H, W, C, F, KW, taps, pad, Ho, Wo, act, P, npt, nft;
+  int runs;              // 16-byte runs of a filter
+  FastDiv by_run, by_kw;  // runs of a tap, filter columns
 };
 
-template <class MM, typename T, int BM, int BN, bool VEC>
+template <class MM, typename T, int BM, int BN, bool VEC, Walk WALK>
 __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs a) {
   constexpr int ES = sizeof(T), RUN = 16 / ES;        // elements of a 16-byte run
   constexpr int KC = 128 / ES;                        // channels of a step
@@ -44,7 +54,9 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
   constexpr int TM = BM / 32, TN = BN / 32;           // 16 x 16 blocks of a wave
   constexpr int AR = BM / 32, BR = BN / 32;           // runs per thread and step
   constexpr int BUF = (BM + BN) * REC;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * BUF];
+  constexpr bool FLAT = WALK != Walk::kTapChunks;
+  constexpr int SETS = WALK == Walk::kOneStep ? 1 : 2;  // register sets and LDS buffers
+  __shared__ __attribute__((aligned(16))) unsigned char lds[SETS * BUF];
   const int per = gridDim.x / kXcds, t = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
   if (t >= a.npt * a.nft) return;
   const int pt = t / a.nft, ft = t - pt * a.nft;
@@ -76,8 +88,26 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
   for (int i = 0; i < BR; ++i) bbase[i] = min(f0 + row0 + 32 * i, a.F - 1) * a.taps * a.C;
   // Loads from clamped addresses now, zeros chosen when the runs are written
   // (a select on a loaded value would make the wave wait for it there).
-  u32x4 av[2][AR], bv[2][BR];
-  uint32_t keep[2];
+  u32x4 av[SETS][AR], bv[SETS][BR];
+  uint32_t keep[SETS];
+  // run g of a filter is run g % by_run.d of tap g / by_run.d: the lanes of a
+  // step may be on different taps
+  auto fetch_flat = [&](int set, int step) __attribute__((always_inline)) {
+    const int g = step * 8 + seg;
+    const bool cin = g < a.runs;
+    const int gc = cin ? g : 0, tap = a.by_run.div(gc), kh = a.by_kw.div(tap), kw = tap - kh * a.KW;
+    const int xoff = (kh * a.W + kw) * a.C + (gc - tap * (int)a.by_run.d) * RUN;
+    keep[set] = (uint32_t)cin << AR;
+#pragma unroll
+    for (int i = 0; i < AR; ++i) {
+      const bool in = (unsigned)(aoh[i] + kh) < (unsigned)a.H && (unsigned)(aow[i] + kw) < (unsigned)a.W;
+      av[set][i] = *reinterpret_cast<const u32x4 *>(x + (uint32_t)(in ? abase[i] + xoff : 0));
+      keep[set] |= (uint32_t)(in && cin) << i;
+    }
+#pragma unroll
+    for (int i = 0; i < BR; ++i)
+      bv[set][i] = *reinterpret_cast<const u32x4 *>(w + (uint32_t)(bbase[i] + gc * RUN));
+  };
   auto fetch = [&](int set, int kh, int kw, int c0) __attribute__((always_inline)) {
     const bool cin = c0 + seg * RUN < a.C;
     const int lc = cin ? seg * RUN : 0;
@@ -111,8 +141,9 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
 
   // steps in order (kh, kw, channel chunk); the coordinates of the step being
   // fetched run ahead, and stay in the last filter row past the end
-  const int chunks = (a.C + KC - 1) / KC, steps = a.taps * chunks, KH = a.taps / a.KW;
-  int kh = 0, kw = 0, ch = 0;
+  const int chunks = (a.C + KC - 1) / KC, KH = a.taps / a.KW;
+  const int steps = FLAT ? (a.runs + 7) / 8 : a.taps * chunks;
+  int kh = 0, kw = 0, ch = 0, fstep = 0;
   auto advance = [&]() __attribute__((always_inline)) {
     if (++ch == chunks) {
       ch = 0;
@@ -121,11 +152,11 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
   };
   const unsigned char *const arow = lds + (wp * (BM / 2) + r) * REC + q * 16;
   const unsigned char *const brow = lds + (BM + wf * (BN / 2) + r) * REC + q * 16;
-  int mch = 0;  // channel chunk of the step being multiplied
+  int mch = 0;  // channel chunk (FLAT: index) of the step being multiplied
   auto multiply = [&](int buf) __attribute__((always_inline)) {
     const int off = buf * BUF;
-    const int frags = min(2, (a.C - mch * KC + KC / 2 - 1) / (KC / 2));
-    if (++mch == chunks) mch = 0;
+    const int frags = min(2, FLAT ? (a.runs - mch * 8 + 3) / 4 : (a.C - mch * KC + KC / 2 - 1) / (KC / 2));
+    if (++mch == chunks && !FLAT) mch = 0;
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
       if (f < frags) {  // uniform: the last chunk's second half may lie past C
@@ -144,8 +175,12 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
     }
   };
   auto fetch_next = [&](int set) __attribute__((always_inline)) {
-    fetch(set, kh, kw, ch * KC);
-    advance();
+    if constexpr (FLAT) {
+      fetch_flat(set, fstep++);
+    } else {
+      fetch(set, kh, kw, ch * KC);
+      advance();
+    }
   };
   // Step s is in buffer s % 2 and passed through register set s % 2: its loads
   // are issued two steps before they are committed (a step's MFMAs take less
@@ -154,27 +189,34 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
   // 9.55, f32 14x14x256 97 / 90; with more workgroups per CU, 28x28x128 batch
   // 32, the fragments' LDS reads bound it and it stays at 21.8).  Past the last step the
   // loads stay inside the filter's last row and are never committed.
-  fetch_next(0);
-  fetch_next(1);
-  commit(0);
-  fetch_next(0);
-  __syncthreads();
-  int s = 0;
-  for (; s + 2 < steps; s += 2) {
-    multiply(0);
-    commit(1);
-    fetch_next(1);
+  if constexpr (WALK == Walk::kOneStep) {
+    fetch_next(0);
+    commit(0);
     __syncthreads();
-    multiply(1);
+    multiply(0);
+  } else {
+    fetch_next(0);
+    fetch_next(1);
     commit(0);
     fetch_next(0);
     __syncthreads();
-  }
-  multiply(0);
-  if (s + 1 < steps) {
-    commit(1);
-    __syncthreads();
-    multiply(1);
+    int s = 0;
+    for (; s + 2 < steps; s += 2) {
+      multiply(0);
+      commit(1);
+      fetch_next(1);
+      __syncthreads();
+      multiply(1);
+      commit(0);
+      fetch_next(0);
+      __syncthreads();
+    }
+    multiply(0);
+    if (s + 1 < steps) {
+      commit(1);
+      __syncthreads();
+      multiply(1);
+    }
   }
 
   // Epilogue: pixel r of each block, its filters 4q .. +3.
@@ -241,16 +283,17 @@ __global__ __launch_bounds__(256, 2) void conv2d_nhwc_kernel(const ConvTileArgs 
   }
 }
 
-template <class MM, typename T, int BM, int BN, bool VEC>
+template <class MM, typename T, int BM, int BN, bool VEC, Walk WALK>
 hipError_t launch_tile(const ConvArgs &c, hipStream_t s) {
-  auto kern = conv2d_nhwc_kernel<MM, T, BM, BN, VEC>;
+  auto kern = conv2d_nhwc_kernel<MM, T, BM, BN, VEC, WALK>;
+  constexpr int RUN = 16 / sizeof(T);
   ConvTileArgs a{c.x, c.w, c.res, c.bias, c.out, c.H, c.W, c.C, c.F, c.KW, c.KH * c.KW, c.pad, c.Ho, c.Wo, c.act,
-                 c.N * c.Ho * c.Wo, 0, 0};
+                 c.N * c.Ho * c.Wo, 0, 0, c.KH * c.KW * (c.C / RUN), FastDiv(c.C / RUN), FastDiv(c.KW)};
   a.npt = (a.P + BM - 1) / BM;
   a.nft = (a.F + BN - 1) / BN;
   const int G = a.npt * a.nft, grid = (G + kXcds - 1) / kXcds * kXcds;
-  const double steps = (double)a.taps * ((a.C + 128 / sizeof(T) - 1) / (128 / sizeof(T)));
-  npu_launch_plan p = make_plan("conv2d_nhwc", G, wg_per_cu(kern), G, 8 * sizeof(T));
+  const double steps = WALK != Walk::kTapChunks ? (a.runs + 7) / 8 : (double)a.taps * ((a.C + 8 * RUN - 1) / (8 * RUN));
+  npu_launch_plan p = make_plan(kWalkName[(int)WALK], G, wg_per_cu(kern), G, 8 * sizeof(T));
   p.load_phases = 1;  // a step's loads are in flight during the two before
   p.tile_macs = (double)BM * BN * steps * 128 / sizeof(T);
   p.tile_valu = 4.0 * (steps * (10.0 * (BM + BN) / 32 + 20.0) + 12.0 * BM * BN / 1024 + 120.0);
@@ -264,9 +307,27 @@ hipError_t launch_tile(const ConvArgs &c, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <class MM, typename T, int BM, int BN, Walk WALK>
+hipError_t launch_tile(const ConvArgs &c, hipStream_t s) {
+  return c.F % 4 == 0 ? launch_tile<MM, T, BM, BN, true, WALK>(c, s) : launch_tile<MM, T, BM, BN, false, WALK>(c, s);
+}
+
+// The walk over runs where it saves a quarter of the steps, which are mostly
+// padding for few channels; filters of a single step load and stage it once, in
+// one LDS buffer (twice the workgroups on a CU).  Measured, us, the kernel before
+// the tiles (operands straight from L2) / tap chunks / so: bf16 5x5 34x35x8 ->
+// 267 at batch 13 25.2 / 37.5 / 13.3, 5x5 40x41x16 -> 267 batch 3 15.2 / 17.7 /
+// 8.8, 3x3 34x35x32 -> 481 batch 13 26.9 / 25.9 / 20.6; f32 5x5 34x35x16 -> 64 19.8 /
+// 18.7 / 14.7; one step: bf16 1x1 34x35x16 -> 481 12.1 / 14.2 / 11.0, f32 1x1
+// 34x35x8 -> 267 10.7 / 11.9 / 10.2.
 template <class MM, typename T, int BM, int BN>
 hipError_t launch_tile(const ConvArgs &c, hipStream_t s) {
-  return c.F % 4 == 0 ? launch_tile<MM, T, BM, BN, true>(c, s) : launch_tile<MM, T, BM, BN, false>(c, s);
+  const long long run = c.C * (long long)sizeof(T) / 16, taps = (long long)c.KH * c.KW, runs = taps * run;
+  if (runs <= 8) return launch_tile<MM, T, BM, BN, Walk::kOneStep>(c, s);
+  // (run and runs within FastDiv's range)
+  if (run < 64 && runs < 60000 && 4 * ((runs + 7) / 8) <= 3 * taps * ((run + 7) / 8))
+    return launch_tile<MM, T, BM, BN, Walk::kRuns>(c, s);
+  return launch_tile<MM, T, BM, BN, Walk::kTapChunks>(c, s);
 }
 
 // Tiles of 64 pixels x 64 filters when there are enough to keep more than one

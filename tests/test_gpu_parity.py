@@ -1546,18 +1546,8 @@ def test_model_zoo_block_runs_on_the_gpu(cuda, C, M, final_relu):
                 what=f"model-zoo block C={C} M={M}")
 
 
-@pytest.mark.parametrize("N,H,W,C,F,KH,KW,pad,dtype,res", [
-    (3, 65, 64, 8, 128, 3, 3, 1, "bf16", True),    # 64x64 tiles, one run per tap, ragged pixels
-    (1, 157, 157, 72, 64, 1, 1, 0, "bf16", False),  # 64x64 tiles, a second chunk of one run
-    (2, 80, 81, 40, 70, 3, 3, 0, "bf16", True),    # 64x32 tiles, F % 4 != 0, no pad
-    (4, 80, 80, 20, 96, 3, 3, 1, "f32", True),     # 64x32 tiles, C of five runs
-    (1, 160, 156, 36, 61, 1, 3, 1, "f32", False),  # 64x64 tiles, a 1x3 filter, odd F, 64 + 16 bytes of channels
-    (1, 5, 4, 136, 33, 5, 5, 2, "bf16", True),     # 32x32 tiles, three chunks, 20 pixels
-    (2, 66, 70, 64, 24, 3, 3, 1, "f32", False),    # rows past 64 pixels, two chunks
-])
-def test_conv_tiles(cuda, N, H, W, C, F, KH, KW, pad, dtype, res):
-    """Edges of the NHWC conv's pixel x filter tiles: each tile size, ragged
-    pixels and filters, channel runs past C, vector and scalar epilogues."""
+def _conv_tiles(N, H, W, C, F, KH, KW, pad, dtype, res):
+    """An NHWC conv against float64; returns the kernel it ran on."""
     Ho, Wo = H + 2 * pad - KH + 1, W + 2 * pad - KW + 1
     x = rng.uniform(51, 0, (N, H, W, C), -1, 1)
     w = rng.normal(51, 1, (F, KH, KW, C), 0, math.sqrt(2 / (KH * KW * C)))
@@ -1570,9 +1560,11 @@ def test_conv_tiles(cuda, N, H, W, C, F, KH, KW, pad, dtype, res):
     out = torch.full((N, Ho, Wo, F), float("nan"), dtype=tdt, device="cuda")
     dev = configs.to_device({"x": x, "w": w, "b": b, "r": r})
     if res:
-        groups.fused_conv2d_nhwc_bias_res_act(dev["x"], dev["w"], dev["b"], dev["r"], out, pad, "relu")
+        name = _plan_name(lambda: groups.fused_conv2d_nhwc_bias_res_act(
+            dev["x"], dev["w"], dev["b"], dev["r"], out, pad, "relu"))
     else:
-        groups.fused_conv2d_nhwc_bias_act(dev["x"], dev["w"], dev["b"], out, pad, "relu")
+        name = _plan_name(lambda: groups.fused_conv2d_nhwc_bias_act(
+            dev["x"], dev["w"], dev["b"], out, pad, "relu"))
     torch.cuda.synchronize()
     got = configs.to_host(out)
     if dtype == "bf16":
@@ -1589,6 +1581,41 @@ def test_conv_tiles(cuda, N, H, W, C, F, KH, KW, pad, dtype, res):
         check_bf16_rounded(got, ref, mag, KH * KW * C + 2, what="conv tiles")
     else:
         check_bound(got, ref, mag, RTOL_F32, what="conv tiles")
+    return name
+
+
+@pytest.mark.parametrize("N,H,W,C,F,KH,KW,pad,dtype,res", [
+    (3, 65, 64, 8, 128, 3, 3, 1, "bf16", True),    # 64x64 tiles, one run per tap, ragged pixels
+    (1, 157, 157, 72, 64, 1, 1, 0, "bf16", False),  # 64x64 tiles, a second chunk of one run
+    (2, 80, 81, 40, 70, 3, 3, 0, "bf16", True),    # 64x32 tiles, F % 4 != 0, no pad
+    (4, 80, 80, 20, 96, 3, 3, 1, "f32", True),     # 64x32 tiles, C of five runs
+    (1, 160, 156, 36, 61, 1, 3, 1, "f32", False),  # 64x64 tiles, a 1x3 filter, odd F, 64 + 16 bytes of channels
+    (1, 5, 4, 136, 33, 5, 5, 2, "bf16", True),     # 32x32 tiles, three chunks, 20 pixels
+    (2, 66, 70, 64, 24, 3, 3, 1, "f32", False),    # rows past 64 pixels, two chunks
+])
+def test_conv_tiles(cuda, N, H, W, C, F, KH, KW, pad, dtype, res):
+    """Edges of the NHWC conv's pixel x filter tiles: each tile size, ragged
+    pixels and filters, channel runs past C, vector and scalar epilogues."""
+    assert _conv_tiles(N, H, W, C, F, KH, KW, pad, dtype, res).startswith("conv2d_nhwc")
+
+
+@pytest.mark.parametrize("N,H,W,C,F,KH,KW,pad,dtype,res,walk", [
+    (2, 9, 11, 8, 33, 3, 3, 1, "bf16", False, "runs"),     # a run per tap, one in the last step, odd F
+    (1, 30, 31, 24, 40, 5, 5, 2, "bf16", True, "runs"),    # three runs per tap, steps across taps
+    (2, 12, 9, 4, 20, 3, 3, 0, "f32", False, "runs"),      # nine runs, no pad
+    (1, 7, 7, 16, 24, 7, 5, 3, "f32", True, "runs"),       # an uneven filter, wider than the image
+    (40, 34, 35, 16, 132, 3, 3, 1, "bf16", False, "runs"),  # 64x64 tiles
+    (3, 80, 81, 8, 64, 3, 3, 1, "f32", False, "runs"),     # 64x32 tiles
+    (2, 9, 11, 48, 33, 3, 3, 1, "bf16", False, ""),        # six runs of eight per tap: tap chunks
+    (1, 40, 41, 8, 17, 1, 1, 0, "bf16", False, "one_step"),  # one run
+    (2, 20, 21, 32, 70, 1, 1, 0, "f32", True, "one_step"),   # eight runs
+    (1, 17, 19, 8, 64, 2, 4, 1, "bf16", False, "one_step"),  # eight taps
+    (13, 34, 35, 40, 481, 1, 1, 0, "bf16", True, "one_step"),  # 64x64 tiles, odd F
+])
+def test_conv_tiles_few_channels(cuda, N, H, W, C, F, KH, KW, pad, dtype, res, walk):
+    """Filters of few channels, whose steps walk the runs of all taps, and
+    filters of one step."""
+    assert _conv_tiles(N, H, W, C, F, KH, KW, pad, dtype, res) == "conv2d_nhwc" + ("_" + walk if walk else "")
 
 
 @pytest.mark.parametrize("N,H,W,C,F,dtype", [(2, 9, 13, 24, 40, "f32"), (1, 7, 7, 48, 24, "bf16")])
