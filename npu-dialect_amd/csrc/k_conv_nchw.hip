@@ -27,6 +27,7 @@
 // 56x56x64 31.7 -> 8.5 us, 28x28x128 57.6 -> 10.4, 14x14x256 110 -> 16,
 // 7x7x512 215 -> 20, the 7x7/2 stem 31.7 -> 9.5; 56x56x64 at batch 8
 // 79 -> 32 us.
+#include <cmath>
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -46,6 +47,8 @@ struct NchwArgs {
   int tiles;             // pixel tiles per strip
   int npt, grid;         // pixel tiles of the launch, workgroups
   int hc, ps, npl;       // patch columns, patch words per channel, loads per channel
+  int pstep, istep;      // between neighbouring pixels in the patch, patch words in the image
+  int words;             // patch words past this are not loaded
   int cc, nchunks;       // channels per chunk
   FastDiv by_hc, by_tw, by_t, by_kw;
 };
@@ -115,8 +118,8 @@ void conv2d_nchw_split_kernel(const NchwArgs a) {
 #pragma unroll
   for (int i = 0; i < NPL; ++i) {
     const int e = 64 * i + lane, hy = a.by_hc.div(e), hx = e - hy * a.hc;
-    const int iy = oy0 * a.st - a.pad + hy, ix = ox0 * a.st - a.pad + hx;
-    const bool in = (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
+    const int iy = oy0 * a.st - a.pad + __mul24(hy, a.istep), ix = ox0 * a.st - a.pad + __mul24(hx, a.istep);
+    const bool in = e < a.words && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
     off[i] = in ? iy * a.W + ix : 0;
     keep |= (uint32_t)in << i;
   }
@@ -180,7 +183,7 @@ void conv2d_nchw_split_kernel(const NchwArgs a) {
   for (int i = 0; i < NB; ++i) {
     const int p = min(p0 + 16 * i + r, npx - 1);
     const int oy = a.by_tw.div(p), ox = p - oy * a.tw;
-    pb[i] = ((oy - oy0) * a.hc + min(ox, tw - 1)) * a.st * 4;
+    pb[i] = ((oy - oy0) * a.hc + min(ox, tw - 1)) * a.pstep * 4;
   }
   f32x4 acc[NB];
 #pragma unroll
@@ -287,11 +290,21 @@ bool split_shape(const ConvArgs &c, NchwArgs &a, size_t &lds) {
   a.grid = (int)grid;
   int span = PX % a.tw == 0 ? PX / a.tw : (PX - 2) / a.tw + 2;  // output rows a tile touches
   if (span > c.Ho) span = c.Ho;
-  const long long hr = (long long)(span - 1) * c.stride + c.KH;
-  a.hc = (a.tw - 1) * c.stride + c.KW;
+  // A 1x1 filter's patch holds the pixels it reads only; with few channels the
+  // whole rows, whose channels' loads are fewer (16 -> 16 1x1/4 4.5 against 5.3
+  // us).  us, the kernel before / whole rows / so: 1x1/2 56x56x64 -> 64 at batch 8
+  // 9.3 / 11.0 / 7.0, 1x1/3 64 -> 256 24.4 / 50.5 / 8.7, 1x1/4 256 -> 128 at
+  // 112x112 and batch 2 74 / 93 / 19.
+  const bool skip = a.T == 1 && c.C > 24 && c.stride < 4096;
+  a.pstep = skip ? 1 : c.stride;
+  a.istep = skip ? c.stride : 1;
+  const long long hr = (long long)(span - 1) * a.pstep + c.KH;
+  const long long hc = (long long)(a.tw - 1) * a.pstep + c.KW;
   const long long wwords = (long long)c.F * a.K;  // filter indices stay below 2^31 past a row's end
-  if (hr * a.hc > 64 * kStage || a.T > 4096 || wwords < 4 || wwords > (1LL << 31) - 4096) return false;
-  a.ps = (int)hr * a.hc;
+  if (hr * hc > 64 * kStage || a.T > 4096 || wwords < 4 || wwords > (1LL << 31) - 4096) return false;
+  a.hc = (int)hc;
+  a.ps = (int)(hr * hc);
+  a.words = skip ? a.ps : 64 * kStage;  // (other patches end near a load's end)
   const int need = (a.ps + 63) / 64;
   for (int v : {1, 2, 3, 4, 5, 8, 16})
     if (need <= (a.npl = v)) break;
@@ -330,8 +343,8 @@ hipError_t launch_split(const ConvArgs &c, const NchwArgs &a, size_t lds, hipStr
   if (!ok) return hipErrorInvalidValue;
   const dim3 grid((a.grid + kXcds - 1) / kXcds * kXcds);
   const double units = NW / 4.0, steps = (a.K + 15) / 16;
-  npu_launch_plan p = make_plan("conv2d_nchw", (int)(a.grid * units), wg_per_cu(kern, 64 * NW),
-                                (int)(a.grid * units), 32);
+  const int wgs = (int)std::ceil(a.grid * units);
+  npu_launch_plan p = make_plan("conv2d_nchw", wgs, wg_per_cu(kern, 64 * NW), wgs, 32);
   p.load_phases = a.nchunks;
   p.tile_macs = 16.0 * WF * PX * a.K / units;
   p.tile_valu = 4.0 * (steps / WK * (8.0 + 4.0 * (NB + 2)) + 12.0 * kStage * a.nchunks + 120.0);
@@ -442,6 +455,73 @@ hipError_t launch_dot(const ConvArgs &a, int K, hipStream_t s) {
   hipLaunchKernelGGL((conv2d_nchw_dot_kernel<FW, NI, VEC>), grid, dim3(512), 0, s,
                      static_cast<const float *>(a.x), static_cast<const float *>(a.w), a.bias,
                      static_cast<const float *>(a.res), static_cast<float *>(a.out), a.N, a.F, K, a.act);
+  return hipGetLastError();
+}
+
+// 1x1 filters of at most CMAX channels: a lane per output pixel, its channels in
+// registers, kPwF filters (uniform: scalar loads) multiplied into them and
+// stored along the pixels.  What bounds it: the outputs' stores, and below a few
+// thousand pixels the launch; the split kernel's table, staging and partial
+// sums cost more than such a product.  us, 64-pixel x 64-filter MFMA tiles (the
+// kernel before) / split / here: 67x67x2 -> 59 5.2 / 7.2 / 3.7, 88x88x1 -> 3 with
+// residual at batch 12 13.6 / 16.9 / 3.6, 112x112x8 -> 8 at batch 4 8.8 / 8.4 /
+// 4.4, 111x111x4 -> 253 at batch 2 21.2 / 17.8 / 12.4.
+constexpr int kPwF = 4, kPwThreads = 128;
+
+template <int CMAX>
+__global__ __launch_bounds__(kPwThreads) void conv2d_nchw_pointwise_kernel(
+    const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
+    const float *__restrict__ res, float *__restrict__ out, int P, int C, int H, int W, int F, int st,
+    int pad, int Ho, int Wo, int act) {
+  const int p = blockIdx.x * kPwThreads + threadIdx.x;
+  if (p >= P) return;
+  const int n = p / (Ho * Wo), hw = p - n * Ho * Wo, oy = hw / Wo, ox = hw - oy * Wo;
+  const int iy = oy * st - pad, ix = ox * st - pad, plane = H * W;
+  const bool in = (unsigned)iy < (unsigned)H && (unsigned)ix < (unsigned)W;
+  const float *const xp = x + (size_t)n * C * plane + (in ? iy * W + ix : 0);
+  float v[CMAX];
+#pragma unroll
+  for (int c = 0; c < CMAX; ++c) {
+    const float u = xp[(size_t)min(c, C - 1) * plane];
+    v[c] = in ? u : 0.0f;
+  }
+  const int f0 = blockIdx.y * kPwF;
+  const size_t map = (size_t)Ho * Wo, o = ((size_t)n * F + f0) * map + hw;
+  float r[kPwF], acc[kPwF];
+#pragma unroll
+  for (int j = 0; j < kPwF; ++j) r[j] = res && f0 + j < F ? res[o + j * map] : 0.0f;
+#pragma unroll
+  for (int j = 0; j < kPwF; ++j) {
+    const int f = min(f0 + j, F - 1);
+    acc[j] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CMAX; ++c) acc[j] = c < C ? fmaf(v[c], w[(size_t)f * C + min(c, C - 1)], acc[j]) : acc[j];
+    if (bias) acc[j] += bias[f];
+  }
+  const ActBounds ab = act_bounds(act);
+#pragma unroll
+  for (int j = 0; j < kPwF; ++j)
+    if (f0 + j < F) out[o + j * map] = act_clamp(res ? acc[j] + r[j] : acc[j], ab);
+}
+
+template <int CMAX>
+hipError_t launch_pointwise(const ConvArgs &a, hipStream_t s) {
+  const int P = a.N * a.Ho * a.Wo;
+  const dim3 grid((P + kPwThreads - 1) / kPwThreads, (a.F + kPwF - 1) / kPwF);
+  // in units of four waves
+  const int wgs = (int)(((long long)grid.x * grid.y * kPwThreads + 255) / 256);
+  npu_launch_plan p = make_plan("conv2d_nchw_pointwise", wgs, wg_per_cu(conv2d_nchw_pointwise_kernel<CMAX>, kPwThreads),
+                                wgs, 32);
+  p.tile_valu = 4.0 * (60.0 + 3.0 * CMAX + kPwF * (12.0 + a.C));
+  p.tile_load_bytes = 256.0 * 4 * (a.C + (a.res ? kPwF : 0));
+  p.tile_store_bytes = 256.0 * 4 * kPwF;
+  p.hbm_bytes = 4.0 * ((double)a.N * a.C * a.H * a.W + (double)a.F * a.C + (double)P * a.F * (a.res ? 2 : 1)) +
+                (a.bias ? 4.0 * a.F : 0.0);
+  plans_add(p);
+  hipLaunchKernelGGL((conv2d_nchw_pointwise_kernel<CMAX>), grid, dim3(kPwThreads), 0, s,
+                     static_cast<const float *>(a.x), static_cast<const float *>(a.w), a.bias,
+                     static_cast<const float *>(a.res), static_cast<float *>(a.out), P, a.C, a.H, a.W, a.F,
+                     a.stride, a.pad, a.Ho, a.Wo, a.act);
   return hipGetLastError();
 }
 
@@ -596,6 +676,7 @@ constexpr long long kMinWgs = 160;
 // 2048, dot 205 at 512, 388 at 1024, direct 677 at 2200; of 25088, dot 1375 at
 // 512, 5469 at 2048, direct 3503 and 5449: there the two end at the same rate.
 // kDotImages: the launch's y range.
+constexpr long long kPwPixels = 4096;  // pointwise kernel past 8 channels: see below
 constexpr long long kDotOutputs = 1 << 19, kDotShort = 2048;
 constexpr int kDotImages = 8 * 65535;
 template <int NB, int WF, int WK>
@@ -604,6 +685,19 @@ bool try_split(const ConvArgs &a, long long min_wgs, hipStream_t s, hipError_t &
   size_t lds;
   if (!split_shape<NB, WF, WK>(a, n, lds)) return false;
   if (n.grid < min_wgs) return false;
+  // Patches past 512 words hold at most eight channels, each staged by one wave:
+  // the workgroups' time is the staging's, and many of them take longer than the
+  // direct kernel on a short reduction.  Both estimates in us, from 7x7/4, 5x5/5
+  // and 9x9/3 filters of 1 to 8 channels; split / direct: 7x7/4 168x168x1 -> 42 at
+  // batch 13 37.7 / 17.0, 224x224x3 -> 64 at batch 8 52.8 / 31.2 and at batch 2
+  // 17.8 / 26.3, 112x112x8 -> 64 at batch 32 66 / 78.
+  if (n.npl == 16) {
+    const double steps = (n.K + 15) / 16, tiles = ((double)a.N * a.Ho * a.Wo / 64 + 1) * ((a.F + 63) / 64);
+    if (7.0 + steps * (1.8 + 0.0033 * tiles) < 4.0 + 0.0085 * n.grid) {
+      e = launch_nchw_direct(a, s);
+      return true;
+    }
+  }
   switch (n.npl) {
     case 1: e = launch_split<NB, WF, WK, 1>(a, n, lds, s); break;
     case 2: e = launch_split<NB, WF, WK, 2>(a, n, lds, s); break;
@@ -625,8 +719,19 @@ hipError_t launch_conv2d_nchw_f32(const ConvArgs &a, hipStream_t s) {
     if (K % 4 == 0) return a.N == 1 ? launch_dot<4, 1, true>(a, (int)K, s) : launch_dot<4, 8, true>(a, (int)K, s);
     return launch_dot<4, 8, false>(a, (int)K, s);
   }
+  // The pointwise kernel's time grows with the channels that a lane loads one
+  // after the other: of 16, 5.0 us at 67x67 against 6.5, but 5.1 against 4.5 at
+  // 28x28; of 25 -> 13 filters 13.1 against 10.1 (its channels are loaded again
+  // for every four), of 24 -> 2 10.4 against 31.6.
+  const long long pixels = (long long)a.N * a.Ho * a.Wo;
+  if (K == a.C && a.F <= kPwF * 65535 && (a.C <= 8 || (pixels >= (a.stride > 1 ? 2 : 1) * kPwPixels &&
+                                (a.C <= 16 || (a.C <= 32 && a.F <= 8)))))
+    return a.C <= 4    ? launch_pointwise<4>(a, s)
+           : a.C <= 8  ? launch_pointwise<8>(a, s)
+           : a.C <= 16 ? launch_pointwise<16>(a, s)
+                       : launch_pointwise<32>(a, s);
   hipError_t e = hipSuccess;
-  if (try_split<4, 4, 1>(a, 2 * kMinWgs, s, e) || try_split<4, 4, 2>(a, kMinWgs, s, e) || 
+  if (try_split<4, 4, 1>(a, 2 * kMinWgs, s, e) || try_split<4, 4, 2>(a, kMinWgs, s, e) ||
       try_split<4, 2, 4>(a, kMinWgs, s, e) || try_split<4, 1, 8>(a, kMinWgs, s, e) ||
       try_split<2, 1, 8>(a, kMinWgs, s, e) || try_split<1, 1, 8>(a, 1, s, e))
     return e;

@@ -1216,9 +1216,30 @@ def test_nchw_conv_shapes(cuda, N, C, H, W, F, K, pad, st, act, bias, res):
                 what=f"nchw conv {N}x{C}x{H}x{W} -> {F} {K}x{K}/{st}")
 
 
+def _nchw_conv(N, C, H, W, F, KH, KW, pad, st, bias, res):
+    """An NCHW conv against the oracle; returns the kernel it ran on."""
+    x = rng.uniform(34, 0, (N, C, H, W), -1, 1)
+    w = rng.normal(34, 1, (F, C, KH, KW), 0, math.sqrt(2 / (KH * KW * C)))
+    b = rng.uniform(34, 2, (F,), -0.1, 0.1) if bias else None
+    Ho, Wo = (H + 2 * pad - KH) // st + 1, (W + 2 * pad - KW) // st + 1
+    r = rng.uniform(34, 3, (N, F, Ho, Wo), -1, 1) if res else None
+    out = torch.full((N, F, Ho, Wo), float("nan"), device="cuda")
+    args = (_dev(x), _dev(w), None if b is None else _dev(b))
+    if res:
+        name = _plan_name(lambda: groups.fused_conv2d_nchw_bias_res_act(*args, _dev(r), out, pad, "relu", stride=st))
+    else:
+        name = _plan_name(lambda: groups.fused_conv2d_nchw_bias_act(*args, out, pad, "relu", stride=st))
+    torch.cuda.synchronize()
+    with oracle.threaded():
+        ref, mag = refs.conv_nchw_act(x, w, b, r, pad, "relu", stride=st)
+    check_bound(_host(out), ref, mag, RTOL_F32,
+                what=f"nchw conv {N}x{C}x{H}x{W} -> {F} {KH}x{KW}/{st}")
+    return name
+
+
 @pytest.mark.parametrize("N,C,H,W,F,KH,KW,pad,st,bias,res", [
-    (1, 1, 1, 1, 3, 1, 1, 0, 1, True, False),      # fewer than four filter words: the direct kernel
-    (1, 1, 4, 5, 4, 1, 1, 0, 1, False, False),     # one k; the last filter's run moved back by 3
+    (1, 1, 1, 1, 3, 1, 1, 0, 1, True, False),      # window = input, one word
+    (1, 1, 4, 5, 4, 1, 1, 0, 1, False, False),     # one k: the pointwise kernel
     (1, 3, 9, 11, 5, 3, 3, 1, 1, True, True),      # K = 27: a ragged end of K, rows not 16-byte aligned
     (2, 5, 6, 6, 17, 3, 1, 1, 2, False, False),    # K = 15, a 3x1 filter
     (1, 300, 7, 7, 33, 3, 3, 1, 1, False, True),   # several channel chunks, the last one partial
@@ -1238,21 +1259,30 @@ def test_nchw_conv_shapes(cuda, N, C, H, W, F, K, pad, st, act, bias, res):
 def test_nchw_conv_tiles(cuda, N, C, H, W, F, KH, KW, pad, st, bias, res):
     """Edges of the split-K kernel's tiles, chunks and filter runs, of the
     whole-window dot kernel and of the rule between them."""
-    x = rng.uniform(34, 0, (N, C, H, W), -1, 1)
-    w = rng.normal(34, 1, (F, C, KH, KW), 0, math.sqrt(2 / (KH * KW * C)))
-    b = rng.uniform(34, 2, (F,), -0.1, 0.1) if bias else None
-    Ho, Wo = (H + 2 * pad - KH) // st + 1, (W + 2 * pad - KW) // st + 1
-    r = rng.uniform(34, 3, (N, F, Ho, Wo), -1, 1) if res else None
-    out = torch.full((N, F, Ho, Wo), float("nan"), device="cuda")
-    args = (_dev(x), _dev(w), None if b is None else _dev(b))
-    if res:
-        groups.fused_conv2d_nchw_bias_res_act(*args, _dev(r), out, pad, "relu", stride=st)
-    else:
-        groups.fused_conv2d_nchw_bias_act(*args, out, pad, "relu", stride=st)
-    torch.cuda.synchronize()
-    ref, mag = refs.conv_nchw_act(x, w, b, r, pad, "relu", stride=st)
-    check_bound(_host(out), ref, mag, RTOL_F32,
-                what=f"nchw conv {N}x{C}x{H}x{W} -> {F} {KH}x{KW}/{st}")
+    assert _nchw_conv(N, C, H, W, F, KH, KW, pad, st, bias, res).startswith("conv2d_nchw")
+
+
+@pytest.mark.parametrize("N,C,H,W,F,KH,KW,pad,st,bias,res,kernel", [
+    (1, 1, 5, 7, 1, 1, 1, 0, 1, True, False, "_pointwise"),     # one channel, one filter
+    (2, 4, 9, 11, 5, 1, 1, 1, 1, True, True, "_pointwise"),     # a pad round a 1x1 filter
+    (3, 8, 13, 9, 10, 1, 1, 0, 3, False, True, "_pointwise"),   # stride 3, filters past a block of four
+    (1, 16, 64, 64, 7, 1, 1, 0, 1, True, False, "_pointwise"),  # the fewest pixels for 16 channels
+    (1, 16, 63, 65, 7, 1, 1, 0, 1, True, False, ""),            # and one less
+    (2, 13, 70, 61, 9, 1, 1, 0, 1, True, True, "_pointwise"),
+    (2, 32, 64, 90, 8, 1, 1, 0, 1, False, False, "_pointwise"),  # the most channels and filters
+    (1, 32, 64, 90, 9, 1, 1, 0, 1, False, True, ""),
+    (2, 16, 130, 127, 33, 1, 1, 0, 2, True, False, "_pointwise"),
+    (2, 25, 31, 29, 70, 1, 1, 0, 2, True, True, ""),            # 1x1/2 over the pixels it reads
+    (1, 64, 57, 55, 20, 1, 1, 1, 3, False, False, ""),          # the same, the pad at a stride of 3
+    (1, 300, 9, 50, 33, 1, 1, 0, 4, True, False, ""),           # and several channel chunks
+    (1, 1, 9, 4, 4, 5, 1, 0, 1, True, False, ""),               # K = 5: the last run moved back by 3
+    (1, 1, 5, 7, 1, 1, 3, 0, 1, False, False, "_direct"),       # fewer than four filter words
+    (13, 1, 168, 168, 42, 7, 7, 3, 4, True, False, "_direct"),  # many large patches of one channel
+    (2, 3, 112, 112, 64, 7, 7, 3, 4, False, True, ""),          # few of them
+])
+def test_nchw_conv_rule(cuda, N, C, H, W, F, KH, KW, pad, st, bias, res, kernel):
+    """The kernel that each shape runs on, at the edges of the pointwise one."""
+    assert _nchw_conv(N, C, H, W, F, KH, KW, pad, st, bias, res) == "conv2d_nchw" + kernel
 
 
 def test_nchw_conv_non_finite(cuda):
