@@ -27,9 +27,9 @@ namespace npu {
 namespace {
 
 // Output tile TH x TW: 8 x 8 or 8 x 7 when the batch has tiles enough for every
-// CU (8 x 7 has 90 halo pixels, 6 MFMA blocks against 7), 4 x 4 below that (more workgroups, each with a shorter serial chain; the
-// expand conv is recomputed on 36 halo pixels for 16 outputs instead of 100
-// for 64, which idle CUs pay for).
+// CU (8 x 7 has 90 halo pixels, 6 MFMA blocks against 7), 4 x 4 below that (more
+// workgroups, each with a shorter serial chain; the expand conv is recomputed on
+// 36 halo pixels for 16 outputs instead of 100 for 64, which idle CUs pay for).
 template <int TH, int TW>
 struct IrbTile {
   static constexpr int HW = TW + 2;           // halo tile width
@@ -357,9 +357,7 @@ hipError_t launch_irb_tile(const IrbArgs &a, hipStream_t s) {
 // 16/96 21.5 / 19.3, 32/192 66.1 / 61.4, batch 16 24/144 25.6 / 24.5.
 template <int C, int E>
 hipError_t launch_irb_t(const IrbArgs &a, hipStream_t s) {
-  int dev = 0, cus = 256;
-  if (hipGetDevice(&dev) == hipSuccess)
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  const int cus = device_cus();
   auto tiles = [&](int tw) { return (long long)a.N * ((a.H + 7) / 8) * ((a.W + tw - 1) / tw); };
   if (tiles(8) < cus) return launch_irb_tile<C, E, 4, 4>(a, s);
   auto busiest = [&](int tw, int hpb) {  // MFMAs / 4: expand on hpb blocks, project on four
@@ -607,15 +605,30 @@ hipError_t launch_irb_stream(const IrbArgs &a, hipStream_t s) {
 
 // 4 x 7 tiles (4 blocks of halo pixels and 2 of output pixels) or 4 x 4 (3 and
 // 1), whichever takes the busiest CU fewer blocks: 4 x 7 at 14x14 and batch
-// 32 (256 tiles, one per CU, against 512), 4 x 4 for small batches.
+// 32 (256 tiles, one per CU, against 512), 4 x 4 for small batches.  With fewer
+// chunks than waves most of a tile is not blocks, and 4 x 7 has to save a fifth
+// more: 43x45x44/32 at batch 13 12.3 us in 4 x 4, 13.4 in 4 x 7, 36x39x4/16 at
+// batch 21 7.7 and 8.0.
 template <int CB, int NW>
 hipError_t launch_irb_stream_t(const IrbArgs &a, hipStream_t s) {
+  const int cus = device_cus();
   auto rounds = [&](int tw) {
     const long long tiles = (long long)a.N * ((a.H + 3) / 4) * ((a.W + tw - 1) / tw);
-    return (tiles + 255) / 256;
+    return (tiles + cus - 1) / cus;
   };
-  if (6 * rounds(7) < 4 * rounds(4)) return launch_irb_stream<CB, 4, 7, NW>(a, s);
+  if ((a.E < 64 ? 30 : 24) * rounds(7) < 16 * rounds(4)) return launch_irb_stream<CB, 4, 7, NW>(a, s);
   return launch_irb_stream<CB, 4, 4, NW>(a, s);
+}
+
+// Eight waves, from 49 channels on, where the chunks keep most of them busy in
+// every round or every tile has a CU of its own; else four.  us, four waves /
+// eight: 14x14x64/384 at batch 32 20.4 / 19.3, 96/576 35.3 / 32.4, 28x28x40/240
+// 31.6 / 34.7, 40x40x56/160 (ten chunks) at batch 8 18.2 / 19.0, 35x38x48/144
+// (nine) at batch 25 33.7 / 39.5; one tile each: 10x11x148/144 17.1 / 15.6.
+bool irb_wide(const IrbArgs &a) {
+  const int chunks = a.E / 16, rounds = (chunks + 7) / 8;
+  if (10 * chunks >= 7 * 8 * rounds) return true;
+  return chunks >= 8 && (long long)a.N * ((a.H + 3) / 4) * ((a.W + 3) / 4) <= device_cus();
 }
 
 bool irb_tuned(int C, int E) {
@@ -633,17 +646,24 @@ hipError_t launch_irb_f32(const IrbArgs &a, hipStream_t s) {
   if (a.C == 16 && a.E == 96) return launch_irb_t<16, 96>(a, s);
   if (a.C == 32 && a.E == 192) return launch_irb_t<32, 192>(a, s);
   if (!irb_supported(a.C, a.E)) return hipErrorInvalidValue;
-  // eight waves where E has a chunk for each (up to 32 channels four are
-  // enough: 32x28x29x20/112 15.8 us against 17.4); past 160 channels the
-  // registers and LDS of eight do not hold a pixel block's sums
-  const bool wide = a.E >= 128;
-  if (a.C <= 16) return launch_irb_stream_t<1, 4>(a, s);
-  if (a.C <= 32) return launch_irb_stream_t<2, 4>(a, s);
-  if (a.C <= 64) return wide ? launch_irb_stream_t<4, 8>(a, s) : launch_irb_stream_t<4, 4>(a, s);
-  if (a.C <= 96) return wide ? launch_irb_stream_t<6, 8>(a, s) : launch_irb_stream_t<6, 4>(a, s);
-  if (a.C <= 128) return wide ? launch_irb_stream<8, 4, 4, 8>(a, s) : launch_irb_stream<8, 4, 4, 4>(a, s);
-  if (a.C <= 160) return wide ? launch_irb_stream<10, 4, 4, 8>(a, s) : launch_irb_stream<10, 4, 4, 4>(a, s);
-  return launch_irb_stream<20, 4, 4, 4>(a, s);
+  // The channel blocks exactly: in the next larger even count, a third of the
+  // products of 40 channels were padding (28x28x40/240 at batch 23 42 us, 31 so).
+  // Past 96 channels 4 x 7 tiles' sums, past 160 those of eight waves, do not
+  // fit the registers and LDS.
+  const bool wide = irb_wide(a);
+  switch ((a.C + 15) / 16) {
+    case 1: return launch_irb_stream_t<1, 4>(a, s);
+    case 2: return launch_irb_stream_t<2, 4>(a, s);
+    case 3: return launch_irb_stream_t<3, 4>(a, s);
+    case 4: return wide ? launch_irb_stream_t<4, 8>(a, s) : launch_irb_stream_t<4, 4>(a, s);
+    case 5: return wide ? launch_irb_stream_t<5, 8>(a, s) : launch_irb_stream_t<5, 4>(a, s);
+    case 6: return wide ? launch_irb_stream_t<6, 8>(a, s) : launch_irb_stream_t<6, 4>(a, s);
+    case 7: return wide ? launch_irb_stream<7, 4, 4, 8>(a, s) : launch_irb_stream<7, 4, 4, 4>(a, s);
+    case 8: return wide ? launch_irb_stream<8, 4, 4, 8>(a, s) : launch_irb_stream<8, 4, 4, 4>(a, s);
+    case 9:
+    case 10: return wide ? launch_irb_stream<10, 4, 4, 8>(a, s) : launch_irb_stream<10, 4, 4, 4>(a, s);
+    default: return launch_irb_stream<20, 4, 4, 4>(a, s);
+  }
 }
 
 }  // namespace npu

@@ -626,6 +626,9 @@ def test_c3_irb_shapes(cuda, N, H, W, C, E):
     (33, 10, 14, 28, 80),   # four waves
     (2, 9, 10, 12, 64),     # one channel block
     (2, 7, 9, 124, 112), (2, 7, 9, 112, 144), (2, 7, 9, 144, 96), (2, 7, 9, 80, 64),
+    # three, five and seven channel blocks: 4 x 4 and 4 x 7 tiles, four and eight waves
+    (9, 21, 22, 36, 48), (33, 14, 14, 48, 144), (32, 13, 14, 72, 240), (14, 19, 18, 68, 64),
+    (9, 21, 22, 100, 384), (9, 21, 22, 104, 80),
 ])
 def test_c3_irb_any_channels(cuda, N, H, W, C, E):
     """(C, E) outside the tuned instances run on the kernel that streams the
