@@ -704,8 +704,8 @@ hipError_t launch_qb_stream(const QBottleneckArgs &c, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Small filters that the tuned instances above do not cover (M1 = 64, or
-// M1 = 128 with few channels): every filter block is read from L2 where it is
+// Small filters that the tuned instances above do not cover (M1 = 64, M1 = 128
+// with few channels, see launch_qbottleneck_i8): every filter block is read from L2 where it is
 // used, so nothing scales the registers with the channel counts.  A workgroup
 // walks 4 x 4 output tiles; per tile: the x halo (6 x 6 pixels, all C channels,
 // zero outside the image) to LDS; conv1 on the halo, one unit = 16 output
@@ -714,13 +714,14 @@ hipError_t launch_qb_stream(const QBottleneckArgs &c, hipStream_t s) {
 // pixels, into y2; conv3, one unit = 16 output channels, with requant, the
 // residual from the halo and the clamp, stored.  The units of a phase are dealt
 // round-robin over the four waves, one barrier per phase.
+template <int MMAX>
 __global__ __launch_bounds__(256, 1) void qb_direct_kernel(
     const int8_t *__restrict__ x, const int8_t *__restrict__ w1, const int8_t *__restrict__ w2,
     const int8_t *__restrict__ w3, const int32_t *__restrict__ m1, const int32_t *__restrict__ s1,
     const int32_t *__restrict__ m2, const int32_t *__restrict__ s2,
     const int32_t *__restrict__ m3, const int32_t *__restrict__ s3, int8_t *__restrict__ out,
     int H, int W, int C, int M1, int tiles_w, int tiles_img, int ntiles) {
-  constexpr int SHW = 6, SHP = 36, SHPB = 3, CMAX = 2048, MMAX = 128;
+  constexpr int SHW = 6, SHP = 36, SHPB = 3, CMAX = 2048;
   __shared__ __attribute__((aligned(16))) int8_t xs[SHP * (CMAX + 32)];
   __shared__ __attribute__((aligned(16))) int8_t y1[SHPB * 16 * (MMAX + 32)];
   __shared__ __attribute__((aligned(16))) int8_t y2[16 * (MMAX + 32)];
@@ -796,13 +797,15 @@ __global__ __launch_bounds__(256, 1) void qb_direct_kernel(
   }
 }
 
+template <int MMAX>
 hipError_t launch_qb_direct(const QBottleneckArgs &a, hipStream_t s) {
   const int tiles_w = (a.W + 3) / 4, tiles_img = tiles_w * ((a.H + 3) / 4), ntiles = a.N * tiles_img;
-  const int full = persistent_grid(qb_direct_kernel);
+  auto kern = qb_direct_kernel<MMAX>;
+  const int full = persistent_grid(kern);
   if (full <= 0) return hipErrorInvalidValue;
   const int grid = ntiles < full ? (ntiles + kXcds - 1) / kXcds * kXcds : full;
   {
-    npu_launch_plan p = make_plan("int8_bottleneck_direct", grid, wg_per_cu(qb_direct_kernel), ntiles, 8);
+    npu_launch_plan p = make_plan("int8_bottleneck_direct", grid, wg_per_cu(kern), ntiles, 8);
     p.load_phases = 4;  // the halo, then each phase's filters from L2
     p.tile_macs = 48.0 * a.M1 * a.C + 16.0 * 9 * a.M1 * a.M1 + 16.0 * a.C * a.M1;
     p.tile_valu = 4.0 * (40.0 + 30.0 * (3 * a.M1 / 16 + a.M1 / 16 + a.C / 16) / 4.0);
@@ -814,7 +817,7 @@ hipError_t launch_qb_direct(const QBottleneckArgs &a, hipStream_t s) {
                   4.0 * 2 * (2 * a.M1 + a.C);
     plans_add(p);
   }
-  hipLaunchKernelGGL(qb_direct_kernel, dim3(grid), dim3(256), 0, s, a.x, a.w1, a.w2, a.w3, a.m1,
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, a.x, a.w1, a.w2, a.w3, a.m1,
                      a.s1, a.m2, a.s2, a.m3, a.s3, a.out, a.H, a.W, a.C, a.M1, tiles_w, tiles_img,
                      ntiles);
   return hipGetLastError();
@@ -839,9 +842,21 @@ hipError_t launch_qbottleneck_i8(const QBottleneckArgs &a, hipStream_t s) {
   // from L2: 512/128 (279 KB) one 14x14 image 17.7 / 20.4, batch 32 of 7x7
   // 18.1 / 20.5; 192/192 (406 KB) 17.9 / 19.7; 1024/256 (1.1 MB) one 7x7 image
   // 30.7 / 59.6; 320/128 (229 KB) 17.5 / 15.3; 320/64 (78 KB) 14.4 / 9.2.
-  if (a.M1 >= 128 && 2 * a.M1 * a.C + 9 * a.M1 * a.M1 >= 256 * 1024)
-    return a.M1 >= 192 ? launch_qb_stream<1>(a, s) : launch_qb_stream<2>(a, s);
-  return launch_qb_direct(a, s);
+  const double bytes = 2.0 * a.M1 * a.C + 9.0 * a.M1 * a.M1;
+  if (a.M1 < 128 || bytes < 256 * 1024) return launch_qb_direct<128>(a, s);
+  // With a CU for every 4 x 4 tile, row groups that fill little of their last
+  // chunks (320 filters are chunks of 256 and 64, 192 one of 192) are not worth
+  // streaming for few channels: 64/320 36.1 from L2 / 41.9 streamed, 192/320 40.6
+  // / 42.3, 256/320 44.0 / 42.3, 64/192 17.1 / 18.3, 128/192 19.0 / 18.5, 64/384
+  // 49.8 / 47.1; in rounds 64/320 14x14 at batch 32 72.6 / 47.2.  The estimates,
+  // in us: a tile's filters and channels at L2's rate, or its chunks.
+  if (a.M1 <= 320 && (long long)a.N * ((a.H + 3) / 4) * ((a.W + 3) / 4) <= device_cus()) {
+    const int rg = (a.M1 + SROWS - 1) / SROWS;
+    const int chunks = 2 * (rg * ((a.C + 255) / 256 + (9 * a.M1 + 255) / 256) +
+                            (a.C + SROWS - 1) / SROWS * ((a.M1 + 255) / 256));
+    if (a.M1 >= 192 && 4.3 + 31.8e-6 * bytes + 0.0175 * a.C < 6.5 + 0.635 * chunks) return launch_qb_direct<320>(a, s);
+  }
+  return a.M1 >= 192 ? launch_qb_stream<1>(a, s) : launch_qb_stream<2>(a, s);
 }
 
 }  // namespace npu

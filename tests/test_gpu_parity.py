@@ -585,6 +585,22 @@ def test_c4_qbottleneck_streamed_filters(cuda, N, H, W, C, M1):
     assert np.array_equal(_qb_run(inp), ref)
 
 
+@pytest.mark.parametrize("N,H,W,C,M1,kernel", [
+    (2, 9, 13, 64, 320, "direct"), (1, 7, 7, 192, 320, "direct"), (3, 6, 5, 64, 192, "direct"),
+    (2, 9, 13, 256, 320, "stream"), (1, 7, 7, 128, 192, "stream"), (1, 5, 5, 64, 256, "stream"),
+    (17, 14, 14, 64, 320, "stream"),  # more 4 x 4 tiles than CUs
+    (1, 6, 6, 384, 128, "direct"), (1, 6, 6, 512, 128, "stream"),
+])
+def test_c4_qbottleneck_rule(cuda, N, H, W, C, M1, kernel):
+    """Which of the kernels for any channel counts runs, bit-exact on each."""
+    inp = _qb_wide_inputs(N, H, W, C, M1, 130 + C // 64)
+    with oracle.threaded():
+        ref = oracle.block_qbottleneck(**inp)
+    assert np.array_equal(_qb_run(inp), ref)
+    (p,) = _lib.last_launch_plans()
+    assert p.kernel.decode() == f"int8_bottleneck_{kernel}"
+
+
 @pytest.mark.parametrize("N,H,W,C,E", [
     (2, 9, 13, 24, 144),   # ragged tiles (4 x 4 tiles: fewer 8 x 8 tiles than CUs)
     (1, 3, 5, 24, 144),    # image smaller than a tile
