@@ -344,7 +344,7 @@ hipError_t launch_split(const ConvArgs &c, const NchwArgs &a, size_t lds, hipStr
   const dim3 grid((a.grid + kXcds - 1) / kXcds * kXcds);
   const double units = NW / 4.0, steps = (a.K + 15) / 16;
   const int wgs = (int)std::ceil(a.grid * units);
-  npu_launch_plan p = make_plan("conv2d_nchw", wgs, wg_per_cu(kern, 64 * NW), wgs, 32);
+  npu_launch_plan p = make_plan("conv2d_nchw", wgs, wg_per_cu(kern, 64 * NW, lds), wgs, 32);
   p.load_phases = a.nchunks;
   p.tile_macs = 16.0 * WF * PX * a.K / units;
   p.tile_valu = 4.0 * (steps / WK * (8.0 + 4.0 * (NB + 2)) + 12.0 * kStage * a.nchunks + 120.0);

@@ -1019,7 +1019,7 @@ void plan_gemm(const char *name, Kern kern, const LlamaGemmArgs &a, int grid, in
   // (K > 512 for the RMSNorm GEMMs) reuse these figures.
   const double BM = Sh::kBM, BN = Sh::kBN, units = 4.0;
   const double ksteps = a.K / 32.0;
-  npu_launch_plan p = make_plan(name, grid * 4, wg_per_cu(kern, GT), grid * 4, 16);
+  npu_launch_plan p = make_plan(name, grid * 4, wg_per_cu(kern, GT, Sh::lds_bytes(a.K)), grid * 4, 16);
   p.load_phases = a.K > (int)Sh::SB / 32 ? 2 : 1;  // one exposed load round trip per chunk beyond one
   p.tile_macs = BM * BN * Sh::NB * a.K / units;
   const double bpieces = a.K * BN * Sh::NB / 8.0, apieces = BM * a.K / 8.0;
@@ -1089,7 +1089,7 @@ hipError_t run_tile(const char *name, const LlamaGemmArgs &a, hipStream_t s) {
   if (!ok) return hipErrorInvalidValue;
   {
     const double steps = a.K / S::KC;
-    npu_launch_plan p = make_plan(name, G, wg_per_cu(kern, S::NT), G, 16);
+    npu_launch_plan p = make_plan(name, G, wg_per_cu(kern, S::NT, 2 * S::BUF), G, 16);
     p.unit_waves = WR * WC;
     p.tile_macs = (double)BM * BN * S::NB * a.K;
     p.tile_valu = WR * WC * (steps * ((PRO == kProRmsnorm ? 32.0 : 2.0) * S::AR + 3.0 * S::BR + 20.0) +

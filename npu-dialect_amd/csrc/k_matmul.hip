@@ -396,7 +396,7 @@ hipError_t launch_x6(const char *name, const MatmulArgs &a, hipStream_t s) {
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
   const int G = tiles_m * tiles_n, grid = (G + kXcds - 1) / kXcds * kXcds;
   const double steps = (a.K + S::KC - 1) / S::KC;
-  npu_launch_plan p = make_plan(name, G, wg_per_cu(kern, S::NT), G, 16);
+  npu_launch_plan p = make_plan(name, G, wg_per_cu(kern, S::NT, 2 * S::BUF), G, 16);
   p.unit_waves = WR * WC;
   p.load_phases = 1;
   p.tile_macs = 6.0 * BM * BN * S::KC * steps;

@@ -273,7 +273,7 @@ hipError_t launch_planned_matmul(const PlannedMatmulArgs &a, hipStream_t s) {
   {
     // per tile: the K loop's DMA and MFMAs, then the generic and the copy back
     const double nk = (a.K + a.tk - 1) / a.tk, tiles = (double)grid.x * grid.y;
-    npu_launch_plan p = make_plan("planned_matmul_bias_act", (int)tiles, wg_per_cu(planned_matmul_kernel),
+    npu_launch_plan p = make_plan("planned_matmul_bias_act", (int)tiles, wg_per_cu(planned_matmul_kernel, kPT, a.lds_bytes),
                                   (int)tiles, 32);
     p.load_phases = 1 + 1;  // the first DMA-in, and the copy back's wait
     p.tile_macs = (double)a.tm * a.tn * nk * a.tk;
@@ -308,7 +308,7 @@ hipError_t launch_planned_conv(const PlannedConvArgs &a, hipStream_t s) {
     // per workgroup (one output row): every tile's scalar MACs, the generic
     // and the copy back; the DMA of the input rows and filter slices
     const double nt = (a.F + a.tco - 1) / a.tco, macs = (double)a.tco * a.Wo * a.C * a.KH * a.KW;
-    npu_launch_plan p = make_plan("planned_conv2d_nchw_bias_act", grid, wg_per_cu(planned_conv_kernel),
+    npu_launch_plan p = make_plan("planned_conv2d_nchw_bias_act", grid, wg_per_cu(planned_conv_kernel, kPT, a.lds_bytes),
                                   grid, 32);
     p.load_phases = 1 + 1;
     p.tile_macs = 0.0;  // scalar FMAs, priced as vector work below

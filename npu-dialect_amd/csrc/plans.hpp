@@ -8,7 +8,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
-#include <utility>
+#include <tuple>
 
 #include "../../include/npu_amd.h"
 
@@ -25,21 +25,22 @@ void set_last_error(const char *msg);
 npu_status memref_check(const npu_memref *m, const char *name, int32_t rank, int32_t dtype);
 
 // Per-kernel, per-device launch facts cached by kernel address (kernels of
-// one signature share a function type, so the type cannot be the key).
-// Returns the cached value of (kernel, current device), computing it with
-// `compute(device)` the first time; 0 if the device cannot be queried or
-// `compute` reports 0.
+// one signature share a function type, so the type cannot be the key) and, where
+// the fact depends on it, a launch parameter.  Returns the cached value of
+// (kernel, current device, parameter), computing it with `compute(device)` the
+// first time; 0 if the device cannot be queried or `compute` reports 0.
 template <class F>
-int cached_per_kernel(const void *kernel, F compute) {
+int cached_per_kernel(const void *kernel, F compute, int param = 0) {
   static std::mutex mu;
-  static std::map<std::pair<const void *, int>, int> cache;
+  static std::map<std::tuple<const void *, int, int>, int> cache;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 0;
   std::lock_guard<std::mutex> lock(mu);
-  auto it = cache.find({kernel, dev});
+  const std::tuple<const void *, int, int> key(kernel, dev, param);
+  auto it = cache.find(key);
   if (it != cache.end()) return it->second;
   const int v = compute(dev);
-  if (v > 0) cache[{kernel, dev}] = v;
+  if (v > 0) cache[key] = v;
   return v;
 }
 
@@ -54,17 +55,19 @@ inline int device_cus() {
 }
 
 // Resident four-wave units per CU for `kernel` launched with `threads`
-// lanes per workgroup (resident workgroups x threads / 256), from the
-// runtime's occupancy calculator (registers and LDS decide it): the waves
-// each SIMD holds.
+// lanes and `lds` bytes of dynamic LDS per workgroup (resident workgroups x
+// threads / 256), from the runtime's occupancy calculator (registers and LDS
+// decide it): the waves each SIMD holds.  The hardware allocates LDS in pieces
+// of 1 280 bytes, which bounds what is cached to 128 values a kernel.
 template <class K>
-int wg_per_cu(K kernel, int threads = 256) {
+int wg_per_cu(K kernel, int threads = 256, size_t lds = 0) {
+  const int pieces = (int)((lds + 1279) / 1280);
   return cached_per_kernel(reinterpret_cast<const void *>(kernel), [&](int) {
     int v = 0;
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, kernel, threads, 0) == hipSuccess
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, kernel, threads, lds) == hipSuccess
                ? v * threads / 256
                : 0;
-  });
+  }, pieces);
 }
 
 inline npu_launch_plan make_plan(const char *kernel, int grid, int per_cu, int tiles,

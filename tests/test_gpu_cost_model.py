@@ -71,3 +71,18 @@ def test_plan_vector_instructions_match_the_counters(cuda, w):
         errs.append((kernel, pred, measured, err))
     bad = [e for e in errs if abs(e[3]) > TOL]
     assert not bad, f"{w.name}: {bad}"
+
+
+@pytest.mark.parametrize("C,H,F,units", [
+    (512, 7, 512, 4),   # 74 KB: two workgroups of eight waves, where the registers would hold three
+    (16, 14, 16, 6),    # 17 KB: three
+])
+def test_plan_residency_counts_dynamic_lds(cuda, C, H, F, units):
+    """wg_per_cu of a kernel whose LDS is given at the launch: the four-wave
+    units that fit into a CU's 160 KiB."""
+    x, w = torch.zeros(1, C, H, H, device="cuda"), torch.zeros(F, C, 3, 3, device="cuda")
+    with groups.collect_plans() as cp:
+        groups.fused_conv2d_nchw_bias_act(x, w, None, torch.empty(1, F, H, H, device="cuda"), 1, "relu")
+    torch.cuda.synchronize()
+    (p,) = cp.plans
+    assert (p.kernel, p.wg_per_cu) == (b"conv2d_nchw", units)
