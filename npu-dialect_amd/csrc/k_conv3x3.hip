@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256) void conv3x3_rows_kernel(
   }
 }
 
-// Persistent variant for reductions that fit one stage (C = NCH chunks):
+// Persistent variant for reductions of two chunks, one stage (bf16, 64 channels):
 // each workgroup loads its 64 filters' fragments into registers once, then
 // walks a contiguous range of output rows in 2-row tiles (a 1-row tile where
 // the range or an image ends), fetching the next tile's halo into registers
@@ -249,14 +249,16 @@ __global__ __launch_bounds__(256) void conv3x3_rows_kernel(
 // is a scalar base plus one loop-invariant lane offset, and the LDS addresses
 // are loop-invariant plus immediates: the per-tile vector-ALU work is the
 // epilogue's clamp and conversion, not index arithmetic.
-// Two workgroups per CU where their registers fit (two chunks, rows of up
-// to 56 pixels), else one.
-template <class MM, typename T, int WMAX, int NCH, int WFIX>
-__global__ __launch_bounds__(256, NCH <= 2 && WMAX <= 56 ? 2 : 1) void conv3x3_stream_kernel(
+// Two workgroups per CU where their registers fit (rows of up to 56 pixels),
+// else one.
+constexpr int kStreamChunks = 2;
+
+template <class MM, typename T, int WMAX, int WFIX>
+__global__ __launch_bounds__(256, WMAX <= 56 ? 2 : 1) void conv3x3_stream_kernel(
     const T *__restrict__ x, const T *__restrict__ w, const float *__restrict__ bias,
     T *__restrict__ out, int H, int w_rt, int F, int act, int nrows) {
   const int W = WFIX > 0 ? WFIX : w_rt;
-  constexpr int ES = sizeof(T);
+  constexpr int ES = sizeof(T), NCH = kStreamChunks;
   constexpr int C = NCH * MM::kPerFrag;
   constexpr int TR = 2, HR = TR + 2;
   constexpr int KPL = MM::kPerLane;
@@ -940,8 +942,9 @@ constexpr double STREAM_VALU_TILE_FIXED = 105.0;
 constexpr double STREAM_VALU_TILE_PER_CHUNK = 20.0;
 constexpr double STREAM_VALU_SETUP = 196.0;
 
-template <class MM, typename T, int WMAX, int NCH, int WFIX>
+template <class MM, typename T, int WMAX, int WFIX>
 hipError_t launch_stream(const ConvArgs &a, int wgs, hipStream_t s) {
+  constexpr int NCH = kStreamChunks;
   if (a.W > WMAX || (WFIX > 0 && a.W != WFIX) || a.C != MM::kPerFrag * NCH || a.F % 64 != 0 ||
       wgs % kXcds != 0)
     return hipErrorInvalidValue;
@@ -954,7 +957,7 @@ hipError_t launch_stream(const ConvArgs &a, int wgs, hipStream_t s) {
     const double es = sizeof(T);
     npu_launch_plan p =
         make_plan("conv3x3_persistent", wgs * grid.y,
-                  wg_per_cu(conv3x3_stream_kernel<MM, T, WMAX, NCH, WFIX>), nrows * grid.y, 8 * sizeof(T));
+                  wg_per_cu(conv3x3_stream_kernel<MM, T, WMAX, WFIX>), nrows * grid.y, 8 * sizeof(T));
     p.load_phases = 0;  // the next tile's halo is fetched during this tile
     p.tile_macs = 4.0 * (PBW / 2.0) * 256 * 9 * a.C;
     // vector-ALU instructions per row, summed over the four waves
@@ -970,7 +973,7 @@ hipError_t launch_stream(const ConvArgs &a, int wgs, hipStream_t s) {
                   (a.bias ? 4.0 * a.F : 0.0);
     plans_add(p);
   }
-  hipLaunchKernelGGL((conv3x3_stream_kernel<MM, T, WMAX, NCH, WFIX>), grid, dim3(256), 0, s,
+  hipLaunchKernelGGL((conv3x3_stream_kernel<MM, T, WMAX, WFIX>), grid, dim3(256), 0, s,
                      static_cast<const T *>(a.x), static_cast<const T *>(a.w), a.bias,
                      static_cast<T *>(a.out), a.H, a.W, a.F, a.act, nrows);
   return hipGetLastError();
@@ -1070,11 +1073,11 @@ hipError_t launch_rows(const ConvArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <class MM, typename T, int WMAX, int NCH, int WFIX>
+template <class MM, typename T, int WMAX, int WFIX>
 hipError_t launch_persistent(const ConvArgs &a, hipStream_t s) {
-  const int g = persistent_grid(conv3x3_stream_kernel<MM, T, WMAX, NCH, WFIX>);
+  const int g = persistent_grid(conv3x3_stream_kernel<MM, T, WMAX, WFIX>);
   if (g == 0) return hipErrorInvalidDeviceFunction;
-  return launch_stream<MM, T, WMAX, NCH, WFIX>(a, g, s);
+  return launch_stream<MM, T, WMAX, WFIX>(a, g, s);
 }
 
 // Launch shapes.  With F a multiple of 64 and at least 48 row pairs (two
@@ -1089,8 +1092,8 @@ hipError_t launch_persistent(const ConvArgs &a, hipStream_t s) {
 // k_conv.hip.  Measured, us, here against those tiles: bf16 batch 32
 // 56x56x64 13.5 / 24.2; batch 1 56x56x64 (224 workgroups) 3.8 / 5.8, 14x14x96
 // (84) 5.3 / 7.9, 28x28x128 (224) 8.0 / 8.1; f32 batch 1 56x56x64 6.3 / 9.6,
-// batch 4 13.0 / 19.7, 14x14x160 (140) 16.9 / 18.7.  Past 256 workgroups, and
-// for the bf16 stream kernel with 128 channels, the tiles win: bf16 28x28x64 at
+// batch 4 13.0 / 19.7, 14x14x160 (140) 16.9 / 18.7.  Past a workgroup per CU,
+// and for the bf16 stream kernel with 128 channels, the tiles win: bf16 28x28x64 at
 // batch 4 (448) 7.8 / 5.9, 28x28x128 at batch 4 17.8 / 9.3 and at batch 32
 // 29.3 / 22.5; 14x14x256 at batch 32 249 / 26 (f32 498 / 105).  Rows of up to
 // 56 pixels use tiles sized for 56 (7 pixel blocks for 2 rows, none wasted); a
@@ -1106,7 +1109,7 @@ hipError_t launch_w(const ConvArgs &a, hipStream_t s) {
     if constexpr (sizeof(T) == 4)  // f32: on the bf16 pipe
       return a.C == 32 ? launch_x6<WMAX, 1, WFIX>(a, s) : launch_x6<WMAX, 2, WFIX>(a, s);
     else
-      return launch_persistent<MM, T, WMAX, 2, WFIX>(a, s);
+      return launch_persistent<MM, T, WMAX, WFIX>(a, s);
   }
   if (a.C == 2 * MM::kPerFrag) return launch_rows<MM, T, WMAX, 2, 1, WFIX>(a, s);
   if constexpr (sizeof(T) == 4)
@@ -1125,7 +1128,7 @@ hipError_t launch_conv3x3(const ConvArgs &a, hipStream_t s) {
 bool conv3x3_rows_supported(const ConvArgs &a, int elem_bytes) {
   const int kc = 64 / elem_bytes;
   if (!(a.KH == 3 && a.KW == 3 && a.pad == 1 && a.W <= 64 && a.C % kc == 0 && a.F % 16 == 0)) return false;
-  return persistent_shape(a, kc) || (long long)a.N * a.H * (a.F / 16) <= 256;
+  return persistent_shape(a, kc) || (long long)a.N * a.H * (a.F / 16) <= device_cus();
 }
 
 hipError_t launch_conv3x3_f32(const ConvArgs &a, hipStream_t s) {

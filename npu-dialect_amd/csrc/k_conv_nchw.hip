@@ -21,12 +21,13 @@
 //
 // What bounds it: at batch 1 the patches' loads, one word per lane (about 28
 // clocks of the CU's load path each), and the fetch of code that runs once;
-// at larger batches the f32 MFMAs (half of their rate).  Measured against the
+// at larger batches the chain of a k step (its LDS reads, then its MFMAs: a
+// third of the f32 matrix rate).  Measured against the
 // kernel before it (row segments of 32 or 64 pixels x 64 filters, 16-channel
 // chunks of halo and filters staged between two barriers): 3x3 at batch 1
 // 56x56x64 31.7 -> 8.5 us, 28x28x128 57.6 -> 10.4, 14x14x256 110 -> 16,
-// 7x7x512 215 -> 20, the 7x7/2 stem 31.7 -> 9.5; 56x56x64 at batch 8
-// 79 -> 32 us.
+// 7x7x512 215 -> 20, the 7x7/2 stem 31.7 -> 9.5; 56x56x64 at batch 8 with
+// residual 84 -> 36 us, without 82 -> 34.
 #include <cmath>
 #include <type_traits>
 
@@ -65,7 +66,7 @@ constexpr int patch_stride(int npl) { return 64 * npl + 4; }
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int NB, int WF, int WK, int NPL>
-__global__ __launch_bounds__(64 * WF * WK, WF * WK == 16 || (WF * WK == 8 && NB * NPL <= 16) ? 4 : 2)
+__global__ __launch_bounds__(64 * WF * WK, WF * WK == 8 && NB * NPL <= 16 ? 4 : 2)
 void conv2d_nchw_split_kernel(const NchwArgs a) {
   constexpr int NW = WF * WK, NT = 64 * NW, PX = 16 * NB;
   constexpr int CPW = kStage / NPL;  // channels a wave stages per chunk
@@ -649,10 +650,6 @@ hipError_t launch_nchw_direct(const ConvArgs &a, hipStream_t s) {
                      a.W, a.F, a.KH, a.KW, a.stride, a.pad, a.Ho, a.Wo, a.act);
   return hipGetLastError();
 }
-
-}  // namespace
-
-namespace {
 
 // The split kernel's shapes, largest tile first (pixels x filters per
 // workgroup 64 x 64, 64 x 32, 64 x 16, 32 x 16, 16 x 16): the first that has

@@ -42,7 +42,7 @@ def _matmul_cases(n=12, seed=2026):
 
 def _conv_cases(n=16, seed=2027):
     r = random.Random(seed)
-    cases = []
+    cases, narrow = [], []
     while len(cases) < n:
         dtype = r.choice(("f32", "bf16"))
         step = 4 if dtype == "f32" else 8
@@ -50,7 +50,8 @@ def _conv_cases(n=16, seed=2027):
         pad = 0 if K == 1 else r.choice((0, 1, 1))
         if r.random() < 0.35:
             # the persistent kernels' range: >= 48 row pairs, F % 64 == 0,
-            # two or four 64-byte channel chunks, rows up to 64 pixels
+            # two (f32: also four) 64-byte channel chunks, rows up to 64 pixels;
+            # bf16 of 128 channels runs on the tiles, and again with 64 below
             N, H = r.randint(4, 10), r.randint(10, 24)
             W = r.randint(20, 64)
             C = r.choice((32, 64)) if dtype == "f32" else r.choice((64, 128))
@@ -61,7 +62,9 @@ def _conv_cases(n=16, seed=2027):
         if H + 2 * pad - K + 1 < 1 or W + 2 * pad - K + 1 < 1:
             continue
         cases.append((N, H, W, C, F, K, pad, r.choice(ACTS), r.random() < 0.75, dtype))
-    return cases
+        if dtype == "bf16" and C == 128 and F % 64 == 0:
+            narrow.append((N, H, W, 64) + cases[-1][4:])
+    return cases + narrow
 
 
 def _irb_cases(n=6, seed=2028):
