@@ -1126,7 +1126,8 @@ hipError_t launch_llama_gemm(const LlamaGemmArgs &a, int pro, int epi, hipStream
   //   QKV S x D: 2048x768 55.4 / 31.2 / 31.5, 2048x1024 80.9 / 38.9 / 46,
   //     1024x512 13.1 / 11.4 / 12.5, 2100x512 23.5 / 17.5 / 24.7, 1400x256
   //     11.4 / 9.0 / 9.8, 700x704 19.2 / - / 14.4, 2047x448 18.8 / - / 15.1,
-  //     600x960 29.6 / - / 22.1; not taken: 300x768 (240 workgroups) 10.6 / 13.1;
+  //     600x960 29.6 / - / 22.1; not taken: 300x768 (240 workgroups) 10.6 / 13.1,
+  //     1392x448 (462; 308 of 32x192) 12.9 / - / 14.6;
   //   SwiGLU S x D x F, 16 waves / 64x64 tiles: 2048x768x2048 60.0 / 33.0,
   //     2100x512x1280 22.2 / 18.6, 1024x512x1408 15.1 / 12.8, 300x768x2048
   //     16.3 / 11.4, 700x704x1024 15.9 / 11.0; not taken: 2048x192x512 (256)
@@ -1139,13 +1140,14 @@ hipError_t launch_llama_gemm(const LlamaGemmArgs &a, int pro, int epi, hipStream
   const int cus = device_cus();
   if (pro == kProRmsnorm && epi == kEpiQkvRope && a.K <= 1024) {
     const int cols = a.Npart * a.nparts;
-    if (tiles(64, a.K <= 512 ? 64 : 48, cols) > cus) {
-      if (cols % 128 != 0)
-        return a.K <= 512 ? run_tile<kProRmsnorm, kEpiQkvRope, 32, 192, 1, 4, 1, 2, 1>("llama_rmsnorm_qkv_rope_tiles", a, s)
-                          : run_tile<kProRmsnorm, kEpiQkvRope, 32, 192, 1, 4, 4, 2, 1>("llama_rmsnorm_qkv_rope_tiles", a, s);
+    const long long small = tiles(64, a.K <= 512 ? 64 : 48, cols);
+    if (cols % 128 == 0 && small > cus)
       return a.K <= 512 ? run_tile<kProRmsnorm, kEpiQkvRope, 64, 128, 2, 4, 1, 4, 1>("llama_rmsnorm_qkv_rope_tiles", a, s)
                         : run_tile<kProRmsnorm, kEpiQkvRope, 64, 128, 2, 4, 4, 4, 1>("llama_rmsnorm_qkv_rope_tiles", a, s);
-    }
+    // past one 32x192 tile a CU, only where the shapes above need a third round
+    if (small > (tiles(32, 192, cols) <= cus ? 1 : 2) * cus)
+      return a.K <= 512 ? run_tile<kProRmsnorm, kEpiQkvRope, 32, 192, 1, 4, 1, 2, 1>("llama_rmsnorm_qkv_rope_tiles", a, s)
+                        : run_tile<kProRmsnorm, kEpiQkvRope, 32, 192, 1, 4, 4, 2, 1>("llama_rmsnorm_qkv_rope_tiles", a, s);
   }
   if (pro == kProRmsnorm && epi == kEpiSwiglu && a.K <= 1024 && tiles(a.K <= 512 ? 64 : 32, 64, a.Npart) > cus)
     return a.K <= 512 ? run_tile<kProRmsnorm, kEpiSwiglu, 64, 64, 2, 4, 1, 4, 1>("llama_rmsnorm_swiglu_tiles", a, s)

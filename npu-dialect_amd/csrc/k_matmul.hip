@@ -421,15 +421,16 @@ hipError_t launch_x6(const char *name, const MatmulArgs &a, hipStream_t s) {
 // rates measured for each (us per k step of 32 and round, and per tile of
 // 16 x 16).  A count of tiles alone does not tell: one row against 32 000
 // columns counts 334 tiles of 256 x 96, of which hardly anything lies inside
-// the matrix.  So the split-K tiles of 16 x 16 are kept below 32 rows or
-// columns (half a 64 x 64 tile), and below kMinMid tiles of 64 x 64, where the
-// rates are least certain, for anything thinner than a tile or without a fifth
-// to gain.  Over 260 shapes the choice takes 1.2 % longer than the fastest of
-// the three (geometric mean).  Measured, us, as 16x16 / 64x64 / 256x96:
+// the matrix.  So the split-K tiles of 16 x 16 are kept below 48 rows or 32
+// columns (three quarters and half of a 64 x 64 tile), and below kMinMid tiles of
+// 64 x 64, where the rates are least certain, for anything thinner than a tile
+// or without a fifth to gain.  Over 260 shapes the choice takes 1.2 % longer than
+// the fastest of the three (geometric mean).  Measured, us, as 16x16 / 64x64 / 256x96:
 // 2000x1024x3000 (256 tiles of 256 x 96) 420 / 124 / 83; 1500x1024x4096 (258)
 // 255 / 119 / 147; 2026x384x6040 (504) 318 / 94 / 69; 1024x1024x1024 (256 of
 // 64 x 64) 43 / 29 / 73; 225x1520x2234 (140) 87 / 51 / 117; 1x512x32000 (500)
-// 12.7 / 22.7 / 76; 16x512x32000 15.5 / 23.1 / 76; 64x512x32000 48 / 24 / 79;
+// 12.7 / 22.7 / 76; 16x512x32000 15.5 / 23.1 / 76; 32x512x32000 26.2 / 24.4 / 77;
+// 64x512x32000 48 / 24 / 79; 50000x256x32 (782) 36.5 / 24.7 / 24;
 // 50000x256x10 (782) 27.3 / 27.5 / 25; 4521x508x36 (71) 8.3 / 16.0 / -;
 // 1x484x28358 (444) 23.9 / 27.3 / -; 1980x360x158 (93) 14.3 / 16.3 / -.
 // Error against 64 bits, relative 2-norm, x6 tiles / 16x16: K = 4 2.9e-8 /
@@ -444,7 +445,7 @@ MatmulTile matmul_tile(const MatmulArgs &a) {
   auto rounds = [&](long long t) { return (double)((t + cus - 1) / cus); };
   const long long mid = tiles(64, 64);
   const int least = mid < kMinMid ? 64 : 32;
-  if (a.M < least || a.N < least) return MatmulTile::k16x16;
+  if (a.M < (least > 48 ? least : 48) || a.N < least) return MatmulTile::k16x16;
   const double steps = (a.K + 31) / 32;
   // a row of B that is no multiple of 16 bytes is loaded word by word
   const double t16 = 4.0 + tiles(16, 16) * (a.N % 4 == 0 ? 0.003 + 0.0003 * steps : 0.004 + 0.0006 * steps);

@@ -111,7 +111,8 @@ def test_c1_matmul_large_tiles(cuda, M, K, N, act, bias):
     (1, 512, 32000, "matmul_bias_act_f32"), (16, 1024, 32000, "matmul_bias_act_f32"),
     (1, 1024, 16384, "matmul_bias_act_f32"), (8, 512, 11264, "matmul_bias_act_f32"),
     (11300, 1024, 16, "matmul_bias_act_f32"), (4521, 508, 36, "matmul_bias_act_f32"),
-    (256, 512, 256, "matmul_bias_act_f32"),
+    (256, 512, 256, "matmul_bias_act_f32"), (47, 512, 32000, "matmul_bias_act_f32"),
+    (20000, 256, 31, "matmul_bias_act_f32"), (50000, 256, 32, "matmul_f32_bf16x6_64x64"),
     (64, 512, 32000, "matmul_f32_bf16x6_64x64"), (1024, 1024, 1024, "matmul_f32_bf16x6_64x64"),
     # a few more 256x96 tiles than CUs: a second round
     (1500, 1024, 4096, "matmul_f32_bf16x6_64x64"), (1100, 1000, 5001, "matmul_f32_bf16x6_64x64"),
