@@ -32,8 +32,10 @@ class NpuError(RuntimeError):
 def _stream(stream):
     if stream is None:
         import torch
-        # the raw handle of torch.cuda.current_stream(), without the Stream object
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        # the raw handle of torch.cuda.current_stream() without the Stream object
+        # (0.3 us against 2.7), by a private function that a torch may not have
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        return raw(torch.cuda.current_device()) if raw else torch.cuda.current_stream().cuda_stream
     return getattr(stream, "cuda_stream", stream)
 
 

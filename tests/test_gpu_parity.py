@@ -1326,6 +1326,35 @@ def test_nchw_conv_non_finite(cuda):
     check_bound(got[~hit], ref[~hit], mag[~hit], RTOL_F32, what="nchw conv next to NaN / Inf")
 
 
+@pytest.mark.parametrize("layout,C,k,pad,kernel", [("nchw", 5, 1, 1, "conv2d_nchw_pointwise"),
+                                                   ("nhwc", 8, 3, 1, "conv2d_nhwc_runs"),
+                                                   ("nhwc", 12, 1, 0, "conv2d_nhwc_one_step")])
+def test_conv_few_channels_non_finite(cuda, layout, C, k, pad, kernel):
+    """NaN and +-Inf in the last channel, where a step's lanes past the channels
+    are zeroed, and in the first: where the oracle's f32 loops have them."""
+    N, H, W, F = 1, 41, 70, 30
+    x = rng.uniform(36, 0, (N, H, W, C), 0, 1)
+    x[0, 4, 5, C - 1], x[0, 9, 15, 0], x[0, H - 1, W - 1, C - 1] = np.nan, np.inf, -np.inf
+    w = rng.normal(36, 1, (F, k, k, C), 0, 0.1)
+    Ho, Wo = H + 2 * pad - k + 1, W + 2 * pad - k + 1
+    if layout == "nchw":
+        x, w = (np.ascontiguousarray(t.transpose(0, 3, 1, 2)) for t in (x, w))
+        out = torch.empty(N, F, Ho, Wo, device="cuda")
+        call = groups.fused_conv2d_nchw_bias_act
+        ref, mag = refs.conv_nchw_act(x, w, None, None, pad, "none")
+    else:
+        out = torch.empty(N, Ho, Wo, F, device="cuda")
+        call = groups.fused_conv2d_nhwc_bias_act
+        ref, mag = refs.conv_bias_act(x, w, None, pad, "none")
+    assert _plan_name(lambda: call(_dev(x), _dev(w), None, out, pad, "none")) == kernel
+    torch.cuda.synchronize()
+    got, hit = _host(out), ~np.isfinite(ref)
+    assert hit.sum() >= 3 * F and np.array_equal(np.isnan(got), np.isnan(ref))
+    fin = hit & ~np.isnan(ref)
+    assert np.array_equal(got[fin], ref[fin])
+    check_bound(got[~hit], ref[~hit], mag[~hit], RTOL_F32, what=f"{kernel} next to NaN / Inf")
+
+
 @pytest.mark.parametrize("name", ["resnet18", "resnet50", "vgg11", "srcnn", "espcn",
                                   "dcgan_generator", "autoencoder", "autoencoder_deep"])
 def test_model_zoo_networks_run_on_the_gpu(cuda, name):
